@@ -247,7 +247,6 @@ template <typename S> static int set_media(Ctx *c, const S *const alpha[3], cons
   const S *e6[6] = {alpha[0], beta[0], alpha[1], beta[1], alpha[2], beta[2]};
   build_classes<6, S>(c, e6, c->ecls, c->etab);
   build_classes<3, S>(c, gamma, c->hcls, c->htab);
-  c->edslot.assign(c->etab.size() / 6 * 3, -1);
   c->media_set = true;
   return VGPU_OK;
 }
@@ -298,13 +297,12 @@ int vgpu_create(const vgpu_grid_desc *g, vgpu_prec prec, int device, vgpu_ctx **
   c->grid.idhx = c->grid.idhy = c->grid.idhz = nullptr;
   {
     const int N[3] = {c->NX, c->NY, c->NZ};
-    // The fused leapfrog sweep with VGPU_LEAP=1 (not with the fused Debye
-    // layer, VGPU_DEBYE_FUSION=1, which only the separate sweeps have; its
-    // kernel indexes cells with 32-bit offsets).  The separate E and H
+    // The fused leapfrog sweep with VGPU_LEAP=1 (its kernel indexes cells with
+    // 32-bit offsets).  The separate E and H
     // sweeps are the default: on the Debye volume at 256^3 the fused sweep
     // and the H cells it leaves to k_h_fix measured slower.
-    const char *lp = getenv("VGPU_LEAP"), *df = getenv("VGPU_DEBYE_FUSION");
-    c->leap = lp && lp[0] == '1' && !(df && df[0] == '1') && c->ncell + FIELD_DISCARD < (1ull << 31);
+    const char *lp = getenv("VGPU_LEAP");
+    c->leap = lp && lp[0] == '1' && c->ncell + FIELD_DISCARD < (1ull << 31);
     if (c->leap) {
       int fb[6];
       leap_box(g->gfilim, N, fb);
@@ -318,7 +316,9 @@ int vgpu_create(const vgpu_grid_desc *g, vgpu_prec prec, int device, vgpu_ctx **
       fast_boxes(g->gfilim, N, c->fastE, c->fastH, al && al[0] == '0' ? 0 : (int)(128 / c->esz));
     }
   }
-  c->NCH = c->fastE[0] <= c->fastE[1] ? (c->fastE[1] - c->fastE[0] + 64) / 64 : 0;
+  // Corrections go in line with the sweeps, which index cells in 32 bits for
+  // them; the fused sweep, whose E other tiles recompute, keeps its own launches.
+  c->inl = !c->leap && c->ncell < (1ull << 31);
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     delete c;
     return VGPU_EDEVICE;
@@ -611,6 +611,30 @@ static int build_debye(Ctx *c)
     }
     blockMedium[b] = it->second;
   }
+  c->d_dalpha = upload_vec(c, da);
+  c->d_dbeta = upload_vec(c, db);
+  c->d_dnp = upload_vec(c, np);
+  if (!c->d_dalpha || !c->d_dbeta || !c->d_dnp) return set_error(c, VGPU_ENOMEM, "Debye media");
+  if (c->inl) {
+    for (size_t m = 0; m < np.size(); ++m) {
+      const size_t at = m * maxP * 2;
+      c->dsimple.push_back(np[m] == 1 && da[at + 1] == 0.0 && db[at + 1] == 0.0);
+      c->dhost[0].push_back(da[at]);
+      c->dhost[1].push_back(db[at]);
+    }
+    for (size_t b = 0; b < c->debye.size(); ++b)
+      for (int f = 0; f < 3; ++f) {
+        const int *l = c->debye[b].flim[f];
+        if (box_empty(l)) continue;
+        if (l[0] < 0 || l[2] < 0 || l[4] < 0 || l[1] >= c->NX || l[3] >= c->NY || l[5] >= c->NZ)
+          return set_error(c, VGPU_EINVAL, "Debye block outside the grid");
+        for (int k = l[4]; k <= l[5]; ++k)
+          for (int j = l[2]; j <= l[3]; ++j)
+            for (int i = l[0]; i <= l[1]; ++i) c->xsite.push_back({c->lin(i, j, k), f, blockMedium[b]});
+      }
+    c->debyeAll = (long long)c->xsite.size();
+    return VGPU_OK;
+  }
   // Sites in block order; a cell already covered by an earlier block goes to
   // the next layer so corrections apply in block order (debye.c:243-307
   // loops block by block).
@@ -628,9 +652,9 @@ static int build_debye(Ctx *c)
               return set_error(c, VGPU_EINVAL, "Debye block outside the grid");
             const long long cell = c->lin(i, j, k);
             int &cnt = seen[cell * 3 + f];
-            // layer 0: first block of a cell inside the fast E box (applied
-            // by the fast sweep); layer 1: first block elsewhere; then the
-            // later blocks of a cell, one layer each
+            // layer 0: first block of a cell inside the fused box; layer 1:
+            // first block elsewhere; then the later blocks of a cell, one
+            // layer each
             const int layer = cnt == 0 ? (in_fast(c->fastE, i, j, k) ? 0 : 1) : cnt + 1;
             ++cnt;
             layers = std::max(layers, layer + 1);
@@ -654,68 +678,7 @@ static int build_debye(Ctx *c)
     if (c->debyeLayerStart[l] > c->debyeLayerStart[l + 1]) c->debyeLayerStart[l] = c->debyeLayerStart[l + 1];
   for (long long s = 0; s < n; ++s) { comp[s] = sites[s].comp; cell[s] = sites[s].cell; med[s] = sites[s].med; }
   c->debyeLayers = layers;
-  c->debyeSites = n;
-  c->debyeL0 = layers > 1 ? c->debyeLayerStart[1] : n;
-
-  // Refine the E coefficient classes with each component's layer-0 Debye
-  // medium, so the E sweep can apply layer 0 itself.
-  std::unordered_map<long long, std::array<int, 3>> slot;
-  for (long long s = 0; s < c->debyeL0; ++s) {
-    auto it = slot.find(cell[s]);
-    if (it == slot.end()) it = slot.emplace(cell[s], std::array<int, 3>{-1, -1, -1}).first;
-    it->second[comp[s]] = med[s];
-  }
-  std::map<std::array<int, 4>, uint32_t> refined;
-  for (auto &kv : slot) {
-    const uint32_t old = c->ecls[kv.first];
-    const std::array<int, 4> key{(int)old, kv.second[0], kv.second[1], kv.second[2]};
-    auto it = refined.find(key);
-    if (it == refined.end()) {
-      const uint32_t id = (uint32_t)(c->etab.size() / 6);
-      for (int q = 0; q < 6; ++q) c->etab.push_back(c->etab[(size_t)old * 6 + q]);
-      for (int q = 0; q < 3; ++q) c->edslot.push_back(kv.second[q]);
-      it = refined.emplace(key, id).first;
-    }
-    c->ecls[kv.first] = it->second;
-  }
-  // First layer-0 site of every (component, row, 64-cell x chunk of the fast
-  // box), for the fast sweep's in-wavefront site numbering.
-  const size_t nrow = (size_t)c->NZ * c->NY * c->NCH;
-  std::vector<int> dbase(3 * nrow + 1, 0);
-  for (long long s = 0; s < c->debyeL0; ++s) {
-    const long long cl = cell[s];
-    const int i = (int)(cl % c->PX);
-    const long long row = cl / c->PX;  // k*NY + j
-    const size_t q = (size_t)comp[s] * nrow + (size_t)row * c->NCH + (i - c->fastE[0]) / 64;
-    dbase[q + 1]++;
-  }
-  if (c->debyeL0 > INT32_MAX) return set_error(c, VGPU_EINVAL, "too many Debye sites");
-  for (size_t q = 1; q < dbase.size(); ++q) dbase[q] += dbase[q - 1];
-  // dbase[q] is the first site of chunk q; dbase[3*nrow] the layer-0 count.
-  // The E sweep numbers layer-0 sites by counting, in x order within each
-  // 64-cell chunk, the cells whose class carries a Debye medium for the
-  // component.  Check here that this numbering reproduces the site list
-  // exactly, so the sweep can never address a site outside it.
-  const int *fb = c->fastE;
-  for (int f = 0; f < 3; ++f) {
-    long long g = dbase[(size_t)f * nrow];
-    for (int k = fb[4]; k <= fb[5]; ++k)
-      for (int j = fb[2]; j <= fb[3]; ++j)
-        for (int i = fb[0]; i <= fb[1]; ++i) {
-          const long long cl = c->lin(i, j, k);
-          const size_t row = (size_t)f * nrow + ((size_t)k * c->NY + j) * c->NCH + (i - fb[0]) / 64;
-          if ((i - fb[0]) % 64 == 0 && dbase[row] != g)
-            return set_error(c, VGPU_EINVAL, "Debye site numbering (chunk start)");
-          const int ds = c->edslot[(size_t)c->ecls[cl] * 3 + f];
-          if (ds < 0) continue;
-          if (g >= c->debyeL0 || cell[g] != cl || comp[g] != f || med[g] != ds)
-            return set_error(c, VGPU_EINVAL, "Debye site numbering (site %lld)", g);
-          ++g;
-        }
-    const long long end = dbase[(size_t)(f + 1) * nrow];
-    if (g != end) return set_error(c, VGPU_EINVAL, "Debye site numbering (component %d count)", f);
-  }
-  c->d_dbase = upload_vec(c, dbase);
+  c->debyeSites = c->debyeAll = n;
 
   std::vector<long long> key(n);
   for (long long g = 0; g < n; ++g) {
@@ -727,10 +690,7 @@ static int build_debye(Ctx *c)
   c->d_dsbeta = dev_alloc(c, (size_t)n * c->esz);
   c->d_dlast = dev_alloc(c, (size_t)n * c->esz);
   c->d_dJ = dev_alloc(c, (size_t)n * maxP * (cplx ? 2 : 1) * c->esz);
-  c->d_dalpha = upload_vec(c, da);
-  c->d_dbeta = upload_vec(c, db);
-  c->d_dnp = upload_vec(c, np);
-  if (!c->d_dkey || !c->d_dsbeta || !c->d_dlast || !c->d_dJ || !c->d_dbase)
+  if (!c->d_dkey || !c->d_dsbeta || !c->d_dlast || !c->d_dJ)
     return set_error(c, VGPU_ENOMEM, "Debye state allocation");
   return VGPU_OK;
 }
@@ -740,7 +700,8 @@ static int build_class_tables(Ctx *c)
 {
   c->nEcls = (int)(c->etab.size() / 6);
   c->nHcls = (int)(c->htab.size() / 3);
-  c->indexed = c->nEcls <= 65536 && c->nHcls <= 65536 && getenv("VGPU_NO_INDEXED_MEDIA") == nullptr;
+  // (with in-line corrections decided with their own classes, build_inline)
+  if (!c->inl) c->indexed = c->nEcls <= 65536 && c->nHcls <= 65536 && getenv("VGPU_NO_INDEXED_MEDIA") == nullptr;
   if (c->indexed) {
     std::vector<uint16_t> e(c->ncell), h(c->ncell);
     for (size_t q = 0; q < c->ncell; ++q) { e[q] = (uint16_t)c->ecls[q]; h[q] = (uint16_t)c->hcls[q]; }
@@ -754,17 +715,9 @@ static int build_class_tables(Ctx *c)
       for (int q = 0; q < 3; ++q) h4[(size_t)k * HTAB_STRIDE + q] = c->htab[(size_t)k * 3 + q];
     c->d_etab = upload_reals(c, e8);
     c->d_htab = upload_reals(c, h4);
-    c->d_edslot = upload_vec(c, c->edslot);
-    if (!c->d_ecls || !c->d_hcls || !c->d_etab || !c->d_htab || !c->d_edslot)
+    if (!c->d_ecls || !c->d_hcls || !c->d_etab || !c->d_htab)
       return set_error(c, VGPU_ENOMEM, "coefficient class allocation");
   }
-  // Applying the first Debye layer inside the fast E kernel saves the
-  // separate pass's field traffic but serialises three dependent table
-  // look-ups per component on Debye rows; measured on the Debye-sphere
-  // workload it is slower, so the separate pass is the default and the
-  // fused one is kept behind VGPU_DEBYE_FUSION=1.
-  const char *df = getenv("VGPU_DEBYE_FUSION");
-  c->debyeFused = c->indexed && c->debyeSites > 0 && df && df[0] == '1';
   std::vector<uint32_t>().swap(c->ecls);
   std::vector<uint32_t>().swap(c->hcls);
   return VGPU_OK;
@@ -827,18 +780,18 @@ static int build_sibc(Ctx *c)
               f0 + ((long long)(k - d.gbbox[4]) * nj + (j - d.gbbox[2])) * ni + (i - d.gbbox[0]);
           ijk[3 * f] = i; ijk[3 * f + 1] = j; ijk[3 * f + 2] = k;
           surf[f] = s;
-          if (c->leap) {
-            // the tangential E that k_sibc_e sets to zero on this face
+          {
+            // the tangential E that the face sets to zero
             const long long id = c->lin(i, j, k), P = c->plane, SJ = c->PX;
             const int t1 = (d.normal + 1) % 3, t2 = (d.normal + 2) % 3;
             // each tangential component at the face cell and at its next
             // cell along the other tangential axis
             const long long o1 = d.normal == 0 ? P : d.normal == 1 ? 1 : SJ;
             const long long o2 = d.normal == 0 ? SJ : d.normal == 1 ? P : 1;
-            c->eTouched.push_back(id * 3 + t1);
-            c->eTouched.push_back((id + o1) * 3 + t1);
-            c->eTouched.push_back(id * 3 + t2);
-            c->eTouched.push_back((id + o2) * 3 + t2);
+            for (const auto &[at, comp] : {std::pair<long long, int>(id, t1), {id + o1, t1}, {id, t2}, {id + o2, t2}}) {
+              if (c->leap) c->eTouched.push_back(at * 3 + comp);
+              if (c->inl) c->xent[0].push_back({at, 0, comp, 1, XO_ZERO, 0, 0, 0});
+            }
           }
           const unsigned char *a = &c->sibc[s].adjA[4 * lf], *b = &c->sibc[s].adjB[4 * lf];
           for (int r = 0; r < 4; ++r) { adjA[4 * f + r] = a[r]; adjB[4 * f + r] = b[r]; }
@@ -917,6 +870,18 @@ static int build_sibc(Ctx *c)
   std::stable_sort(hents.begin(), hents.end(), [](const HE &a, const HE &b) { return a.key < b.key; });
   std::sort(zeroKeys.begin(), zeroKeys.end());
   zeroKeys.erase(std::unique(zeroKeys.begin(), zeroKeys.end()), zeroKeys.end());
+  if (c->inl) {
+    // a normal H set to zero takes no other term
+    for (long long key : zeroKeys) c->xent[1].push_back({key / 6, 0, (int)(key % 6 - 3), 0, XO_ZERO, 0, 0, 0});
+    for (const HE &h : hents) {
+      if (std::binary_search(zeroKeys.begin(), zeroKeys.end(), h.key)) continue;
+      const std::vector<double> &id = *ide[(h.e.bits >> 9) & 3];
+      c->xent[1].push_back({h.key / 6, h.seq, (int)(h.key % 6 - 3), 1, XO_SIBC | h.e.bits << 3, h.e.face, id[h.e.ia],
+                            id[h.e.ib]});
+    }
+    hents.clear();
+    zeroKeys.clear();
+  }
   std::vector<int> rstart;
   std::vector<long long> rkey;
   std::vector<SibcHEnt> ents;
@@ -1106,7 +1071,42 @@ static int build_corrections(Ctx *c)
     }
   if (c->leap)
     for (const RowEntry &r : rows[0]) c->eTouched.push_back(r.key);
-  for (int e = 0; e < 2; ++e) {
+  for (int e = 0; e < 2 && c->inl; ++e) {
+    // operations on the rows' values; sources' and analytic waves' values are
+    // evaluated ahead, a source's once for all its cells
+    std::vector<XVal> &val = c->xval[e];
+    std::vector<int> srcVal(c->src.size(), -1);
+    for (size_t s = 0; s < c->src.size(); ++s)
+      if ((c->src[s].field < 3 ? 0 : 1) == e) {
+        srcVal[s] = (int)val.size();
+        val.push_back({0.0, c->src[s].delay, c->src[s].size, c->src[s].waveform, 0});
+      }
+    for (const RowEntry &r : rows[e]) {
+      const CorrEntry &ce = r.e;
+      if (ce.idx < 0 || ce.idx >= (1 << 23)) return set_error(c, VGPU_EINVAL, "too many sources or plane waves");
+      Ctx::XEnt x{r.key / 3, r.seq, (int)(r.key % 3), 2, 0, 0, 0, 0};
+      if (ce.kind <= 1) {
+        x.code = XO_SRC | ce.kind << 3 | c->src[ce.idx].soft << 4;
+        x.arg = srcVal[ce.idx];
+      } else if (ce.kind == 2) {
+        x.code = XO_AUX | ce.inc << 3 | (ce.sign < 0 ? 1 : 0) << 6 | ce.idx << 8;
+        x.arg = ce.auxid;
+        x.a = ce.geo;
+        x.b = ce.il;
+      } else {
+        x.code = XO_WAVE | (ce.sign < 0 ? 1 : 0) << 6;
+        x.arg = (int)val.size();
+        x.b = ce.il;
+        val.push_back({ce.geo, c->pw[ce.idx].d.delay, c->pw[ce.idx].d.Finc[ce.inc], c->pw[ce.idx].d.waveform, 1});
+      }
+      c->xent[e].push_back(x);
+    }
+    std::vector<long long> keys;
+    for (const RowEntry &r : rows[e]) keys.push_back(r.key);
+    std::sort(keys.begin(), keys.end());
+    c->corrRows[e] = std::unique(keys.begin(), keys.end()) - keys.begin();
+  }
+  for (int e = 0; e < 2 && !c->inl; ++e) {
     std::stable_sort(rows[e].begin(), rows[e].end(), [](const RowEntry &a, const RowEntry &b) { return a.key < b.key; });
     std::vector<int> rstart;
     std::vector<long long> rkey;
@@ -1295,11 +1295,12 @@ int vgpu_finalize(vgpu_ctx *c, uint64_t total_steps, uint64_t max_steps_per_run)
   c->d_step = dev_alloc(c, 64);
   if (!c->d_step) return set_error(c, VGPU_ENOMEM, "step counter");
   int r;
-  if ((r = build_debye(c)) || (r = build_class_tables(c)) || (r = build_sibc(c)) || (r = build_corrections(c)) ||
-      (r = build_observers(c)) || (r = build_leap(c)))
+  if ((r = build_debye(c)) || (r = build_sibc(c)) || (r = build_corrections(c)) || (r = build_observers(c)) ||
+      (r = c->prec == VGPU_FP64 ? build_inline<double>(c) : build_inline<float>(c)) || (r = build_class_tables(c)) ||
+      (r = build_leap(c)))
     return r;
   if ((r = c->prec == VGPU_FP64 ? prepare_sweeps<double>(c) : prepare_sweeps<float>(c))) return r;
-  if (!c->leap && !c->debyeFused && (r = c->prec == VGPU_FP64 ? upload_pack<double>(c) : upload_pack<float>(c)))
+  if (c->inl && (r = c->prec == VGPU_FP64 ? upload_pack<double>(c) : upload_pack<float>(c)))
     return r;
   // set-up copies are synchronous and its kernels ran on the solve's stream
   if (hipStreamSynchronize(c->stream) != hipSuccess || hipGetLastError() != hipSuccess)
@@ -1427,7 +1428,7 @@ int vgpu_run_group(vgpu_ctx *const *ctxs, int n, const uint64_t *first, uint64_t
     Ctx *c = ctxs[i];
     int r = check_run(c, first[i], nsteps);
     if (r) return r;
-    if (!c->d_pack) return set_error(c, VGPU_EINVAL, "group runs need the separate sweeps");
+    if (c->leap) return set_error(c, VGPU_EINVAL, "group runs need the separate sweeps");
     if (c->device != ctxs[0]->device || c->prec != ctxs[0]->prec)
       return set_error(c, VGPU_EINVAL, "group members differ in device or precision");
     for (int j = 0; j < i; ++j)
@@ -1687,7 +1688,7 @@ int vgpu_get_stats(const vgpu_ctx *c, vgpu_stats *out)
   const int *go = c->grid.gobox, *gi = c->grid.gibox;
   out->cells = (uint64_t)(go[1] - go[0]) * (uint64_t)(go[3] - go[2]) * (uint64_t)(go[5] - go[4]);
   out->mesh_cells = (uint64_t)(gi[1] - gi[0]) * (uint64_t)(gi[3] - gi[2]) * (uint64_t)(gi[5] - gi[4]);
-  out->debye_sites = (uint64_t)c->debyeSites;
+  out->debye_sites = (uint64_t)c->debyeAll;
   out->debye_poles = c->debye.empty() ? 0 : c->debyeMaxPoles;
   out->debye_complex = c->debyeCplx;
   out->sibc_faces = (uint64_t)c->sibcFaces;
@@ -1700,9 +1701,9 @@ int vgpu_get_stats(const vgpu_ctx *c, vgpu_stats *out)
                              ? (uint64_t)(fb[1] - fb[0] + 1) * (uint64_t)(fb[3] - fb[2] + 1) * (uint64_t)(fb[5] - fb[4] + 1)
                              : 0;
   }
-  out->debye_fused_sites = c->debyeFused ? (uint64_t)c->debyeL0 : 0;
+  out->debye_fused_sites = (uint64_t)c->debyeSimple;
   out->indexed_media = c->indexed ? 1 : 0;
-  out->debye_fused = c->debyeFused ? 1 : 0;
+  out->debye_fused = c->debyeSimple > 0 ? 1 : 0;
   out->sibc_state = c->sibcFactored ? 2 : c->sibcReal ? 1 : 0;
   out->leap = c->leap ? 1 : 0;
   out->fix_cells = (uint64_t)c->fixCells;

@@ -26,6 +26,9 @@ namespace vgpu {
 
 // ---- kernel argument blocks (passed by value) ----
 
+struct WaveformDev;
+struct PwDev;
+
 // Full argument block of the E sweep, kept in device memory and read through
 // a pointer by the shell kernel and the fused Debye step.
 template <typename T> struct EArgs {
@@ -42,18 +45,9 @@ template <typename T> struct EArgs {
   T *PP[6][3], *P[6][3]; // UPML auxiliaries, x-fastest within each slab box
   T *PPpool, *Ppool;     // the pools holding them (same layout: a slab is at the same offset in both)
   const T *ad[3], *bd[3], *ah[3], *ibh[3];
-  // coefficient classes: per-cell class, [class][8] alpha/beta (6 used), [class][3] Debye medium
+  // coefficient classes: per-cell class, [class][8] alpha/beta (6 used)
   const uint16_t *ecls;
   const T *etab;
-  const int *edslot;
-  // layer-0 Debye sites applied in the sweep
-  int dfuse;
-  const int *dbase;      // [3][NZ][NY][NCH] first site of each 64-cell chunk of the fast box
-  T *dlast, *dJ;
-  long long dstride;
-  const double *dalpha, *dbeta;
-  const int *dnp;
-  int dmaxP, dcplx;
   unsigned *vis[3];      // update-once check: visit counts per component (null in ordinary runs)
 };
 
@@ -76,6 +70,96 @@ template <typename T> struct HArgs {
   unsigned *vis[3];      // update-once check (null in ordinary runs)
 };
 
+// ---- corrections ----
+//
+// The updates that follow a sweep (Debye sites, SIBC edges and faces, sources,
+// TF/SF, ghost planes) each change single field values and read no field but
+// that value, or a ghost's source.  Two forms:
+//
+//  - In line: the thread that sweeps a cell applies them right after its
+//    update, with no second pass over the field.  This takes what needs no
+//    look-up chain: a single one-pole Debye site per value (its alpha and beta
+//    in the class table, its J in a dense array, its previous E the old E the
+//    sweep has in a register), an E to zero (SIBC), and Mur's E, which the
+//    thread of the face's inner neighbour writes, having both of that
+//    neighbour's values Mur's equation takes.  Such cells have coefficient
+//    classes of their own (from `flag0` on), so the others pay one comparison.
+//  - Rows: one launch per half-step, a thread per field value and its
+//    operations in the reference's order, ghosts behind the row of their
+//    source.  (Rows walked by the sweep's threads measured slower: each costs
+//    four dependent loads, one lane of a wavefront at a time at the x faces.)
+enum XKind { XO_SRC, XO_AUX, XO_WAVE, XO_ZERO, XO_DEBYE, XO_GHOST, XO_SIBC };
+// flags of a flagged class (dtab slot 6): one-pole Debye sites of components
+// 0-2 (bits 0-2), Mur faces (3), zeroed components (4-6)
+enum XFlag { XF_DEBYE = 1, XF_MUR = 8, XF_ZERO = 16 };
+constexpr int DTAB_STRIDE = 8;
+
+// code: kind (bits 0-2), then
+//   SRC:   density (3), soft (4); arg value
+//   AUX:   incident component (3-5), negative sign (6), plane wave (8-); arg aux cell, a dp, b inverse edge length
+//   WAVE:  negative sign (6); arg value, b inverse edge length
+//   DEBYE: medium (8-); arg site
+//   GHOST: arg source cell, a sign
+//   SIBC:  SibcHEnt's bits (3-); arg face, a/b the two inverse edge lengths
+template <typename T> struct XOp {
+  int code, arg;
+  T a, b;
+};
+
+struct XRow {
+  int cell;
+  unsigned opc;          // first operation << 2 | component
+};
+
+// A value of the incident field or of a source at one time: scale *
+// wf_value(t) in double, rounded once (a source), or its two factors rounded
+// first, the time less `geo` (an analytic plane wave's, at one edge).
+struct XVal {
+  double geo, delay, scale;
+  int wf, wave;
+};
+
+template <typename T> struct XArgs {
+  unsigned flag0;        // first flagged class (E)
+  const uint16_t *cls;   // per cell: class, or without classes 0 / 1 + dtab row
+  const T *dtab;         // [class - flag0][8]: alpha, beta of J per component, flags
+  T *J;                  // [component][cell] (null without one-pole sites)
+  long long nJ;          // cells
+  int PX;
+  long long plane;
+  unsigned murmask;      // Mur faces written in line
+  int mbox[6][3][6];     // their limits [face][component]
+  T mzeta[6];
+  long long nrow, ngroup;  // rows on their own, then groups of rows (a row and its ghosts)
+  const int *gstart;     // first row of each group
+  const XRow *row;
+  const XOp<T> *op;
+  T *F[3];               // the half-step's fields
+  const T *tab;          // class table (null: per-cell arrays)
+  const T *ca[3], *cb[3];  // alpha and beta, or gamma in cb
+  const T *val;          // source and analytic incident values
+  const T *aux;          // aux grids [pw][2][auxmax]
+  int auxmax;
+  const PwDev *pw;
+  T eta0;
+  T *dlast, *dJ;         // Debye sites of rows
+  long long dstride;
+  const double *dalpha, *dbeta;
+  const int *dnp;
+  int dmaxP, dcplx;
+  const T *Etan;
+};
+
+// Values of a half-step's sources and analytic plane waves, evaluated ahead
+// of it at t = (n + half) * dt.
+template <typename T> struct ValArgs {
+  long long n;
+  const XVal *v;
+  T *out;
+  const WaveformDev *wf;
+  double half;
+};
+
 // Lean by-value arguments of the fast sweep kernels.
 template <typename T> struct FastE {
   int NX, NY, NZ, PX;
@@ -90,8 +174,6 @@ template <typename T> struct FastE {
   const uint16_t *ecls;  // coefficient classes
   const T *etab;
   const T *alpha[3], *beta[3];  // per-cell arrays when there are no classes
-  int dfuse;             // apply layer-0 Debye sites
-  const EArgs<T> *ap;    // full argument block in device memory (Debye state)
   unsigned *vis[3];      // update-once check (null in ordinary runs)
 };
 
@@ -165,7 +247,7 @@ template <typename T> struct FixArgs {
 // consecutive cells of the piece's x-y plane (x fastest) and marches over
 // `kc` planes; block b of the piece is x-y block b % nxyb of z chunk
 // b / nxyb.
-constexpr int SHELL_RUNS = 8;
+constexpr int SHELL_RUNS = 4;
 constexpr int SHELL_KC = 4;  // planes a shell thread marches over
 struct ShellRun {
   int xa, xb;            // inclusive x range
@@ -184,9 +266,22 @@ struct ShellPiece {
   ShellRun run[3][SHELL_RUNS];
 };
 
+// A piece as the kernels read it: everything a block needs in consecutive
+// words, so one batch of scalar loads brings it, in place of one load after
+// another along the runs.  A run's q0 is its element offset in the
+// auxiliaries' pools at x = 0, row 0, plane 0 of the piece; a run past the
+// component's last has xa > xb.
+struct ShellDevRun {
+  int xa, xb, reg, q0, psy, psz;
+};
+struct ShellDev {
+  int x0, y0, z0, ni, nip, xo, nxy, nxyb, kc, nk;
+  int pad_[2];
+  ShellDevRun run[3][SHELL_RUNS];
+};
+
 // One block of a shell launch: its piece and the piece's block (piece < 0:
 // nothing to do).
-
 struct ShellWork {
   int piece, block;
 };
@@ -388,6 +483,23 @@ template <typename T> struct VolObsArgs {
   unsigned long long ring;   // staging rows: two runs' worth
 };
 
+// What rides along with a half-step's sweep, in blocks of its own: things the
+// sweep neither reads nor writes.  The E sweep carries the H half of the
+// observers' samples of its step, the aux grids' E update and the values of
+// its step's E sources and analytic waves (its rows, a launch later, read
+// those); the H sweep the E half of the next step's samples -- E is final
+// then -- and the aux grids' H update and H values.  A run's first E samples
+// have a launch of their own before it, and its last step takes none.
+template <typename T> struct SideArgs {
+  ObsArgs<T> o;
+  VolObsArgs<T> v;
+  AuxArgs<T> x;
+  ValArgs<T> val;
+  int electric;          // rides with the E sweep
+  int nfb;               // 256-frequency blocks per observer
+  int b[4];              // first block past the observers, volume samples, aux grids, values
+};
+
 // ---- packed launches over several solves (vgpu_run_group) ----
 
 constexpr int PACK_MAX = VGPU_GROUP_MAX;  // solves in one group run
@@ -398,16 +510,13 @@ constexpr int PACK_MAX = VGPU_GROUP_MAX;  // solves in one group run
 template <typename T> struct PackArgs {
   FastE<T> fe;
   FastH<T> fh;
-  const ShellPiece *epc, *hpc;
+  const ShellDev *epc, *hpc;
   const ShellWork *ewk, *hwk;
   const EArgs<T> *ea;
   const HArgs<T> *ha;
-  DebyeArgs<T> da;
-  CorrArgs<T> ce, ch;    // E and H corrections
-  ObsArgs<T> oa;
-  AuxArgs<T> xa;
-  VolObsArgs<T> va;
-  int headGx;            // x blocks of the solve's own k_head launch
+  const XArgs<T> *xe, *xh;  // corrections
+  unsigned nEside, nHside, nEshell, nHshell;  // blocks
+  SideArgs<T> se, sh;
 };
 
 // Argument of a packed launch: the solves it covers, in launch order, and
@@ -416,11 +525,9 @@ template <typename T> struct PackArgs {
 // 0 .. start[d+1]-start[d]-1.
 struct PackMap {
   int n;                         // solves in this launch
-  int soff;                      // step offset within the run
+  int soff, last;                // step offset within the run, its last step
   unsigned start[PACK_MAX + 1];
   const void *args[PACK_MAX];    // each solve's PackArgs
-  long long base[PACK_MAX];      // Debye launches: first site of the layer
-  long long cnt[PACK_MAX];       // Debye: sites in the layer; H corrections: correction blocks
 };
 
 template <typename T> struct GhostArgs {
@@ -516,13 +623,28 @@ struct Ctx {
   // tables fit.
   std::vector<uint32_t> ecls, hcls;          // host, per device cell
   std::vector<double> etab, htab;            // host: [class][6] alpha/beta, [class][3] gamma (device: padded to 8, 4)
-  std::vector<int> edslot;                   // [class][3] layer-0 Debye medium or -1
   bool indexed = false;
-  void *d_ecls = nullptr, *d_hcls = nullptr, *d_etab = nullptr, *d_htab = nullptr, *d_edslot = nullptr;
+  void *d_ecls = nullptr, *d_hcls = nullptr, *d_etab = nullptr, *d_htab = nullptr;
   int nEcls = 0, nHcls = 0;
-  // layer-0 Debye sites handled inside the E sweep
-  bool debyeFused = false;
-  long long debyeL0 = 0;
+  // corrections as XArgs has them: every context but those with the fused sweep
+  bool inl = false;
+  bool murPush = false;                      // Mur E written by its inner neighbour's thread
+  int xlevel() const { return debyeSimple ? 2 : xflag0 != ~0u ? 1 : 0; }  // in-line corrections of the E sweep
+  long long debyeSimple = 0;                 // one-pole Debye sites applied from the class table
+  // an operation on one field value, before rows are made of them
+  struct XEnt { long long cell, seq; int comp, order, code, arg; double a, b; };
+  std::vector<XEnt> xent[2];
+  struct XSite { long long cell; int comp, med; };
+  std::vector<XSite> xsite;                  // Debye sites in block order
+  long long debyeAll = 0;                    // all Debye sites
+  std::vector<char> dsimple;                 // per Debye medium: one real pole
+  std::vector<double> dhost[2];              // its alpha and beta (real part)
+  std::vector<XVal> xval[2];
+  unsigned xflag0 = ~0u;
+  void *d_xargs[2] = {}, *d_xval[2] = {}, *d_xvals[2] = {}, *d_xcls = nullptr;
+  void *d_xgstart[2] = {}, *d_xrow[2] = {}, *d_xop[2] = {};
+  void *d_xdtab = nullptr, *d_xJ = nullptr;
+  long long nXval[2] = {}, nXrow[2] = {}, nXgroup[2] = {};
   // fused leapfrog sweep: the fast boxes are its fused box, H cells to
   // update again after the E corrections
   bool leap = false;
@@ -530,7 +652,6 @@ struct Ctx {
   long long nFix = 0, fixCells = 0;
   void *d_fix = nullptr;
   std::vector<long long> eTouched;           // E values (cell * 3 + component) changed after the E sweep
-  int NCH = 0;                               // 64-cell x chunks of the fast E box
   int fastE[6] = {}, fastH[6] = {};          // boxes of the sweeps' fast kernels
   void *d_eargs[2] = {}, *d_hargs[2] = {};   // argument blocks in device memory, by the set read
   void *d_epcs = nullptr, *d_ework = nullptr;   // E shell: pieces, launch blocks
@@ -541,7 +662,6 @@ struct Ctx {
   void *d_epcsPk = nullptr, *d_eworkPk = nullptr, *d_hpcsPk = nullptr, *d_hworkPk = nullptr;
   int nEworkPk = 0, nHworkPk = 0;
   long long shellCells[2] = {};              // cells of the E and H shell pieces
-  void *d_dbase = nullptr;                   // [3][NZ][NY][NCH] + 1: first layer-0 site
 
   // UPML
   unsigned pmlmask = 0;
@@ -657,6 +777,10 @@ struct VisitRun {
   unsigned *vis[6];
   void *eargs, *hargs;
 };
+
+// Corrections of a finalized set-up: rows, flagged classes, device arrays
+// (vgpu_inline.h).
+template <typename T> int build_inline(Ctx *c);
 
 // Per-precision step driver, instantiated for double and float.
 // Enqueues nsteps steps that start at the device step counter, then advances

@@ -88,8 +88,8 @@ VG_HD int classify(const A &a, const int (*in)[6], int C, int i, int j, int k, l
   return -1;
 }
 
-// Debye ADE correction of one site (debye.c:243-307); shared by the fused E
-// sweep (layer 0) and k_debye (later layers).  g is the site, m its medium.
+// Debye ADE correction of one site (debye.c:243-307).  g is the site, m its
+// medium.
 template <typename T>
 VG_DEV T debye_site(T e, T beta, long long g, int m, T *lastE_, T *J_, long long stride, const double *dalpha_,
                     const double *dbeta_, const int *npoles_, int maxPoles, int cplx)
@@ -132,6 +132,102 @@ VG_DEV T debye_site(T e, T beta, long long g, int m, T *lastE_, T *J_, long long
   return e;
 }
 
+// ---------------------------------------------------------------------------
+// Waveforms (waveform.c:413-638) on the device, in double.
+// ---------------------------------------------------------------------------
+VG_DEV double wf_compact(double pi, double time, double width, double span)
+{
+  if (time <= 0.0) return 0.0;
+  if (time < span * width)
+    return 1.0 / 32.0 * (10.0 - 15.0 * cos(pi / width * time) + 6.0 * cos(2.0 * pi / width * time) -
+                         cos(3.0 * pi / width * time));
+  return span < 1.5 ? 1.0 : 0.0;
+}
+
+VG_DEV double wf_value(const WaveformDev &w, double t, double delay, double pi)
+{
+  const double tt = t - delay - w.delay;
+  const double width = w.width;
+  switch (w.type) {
+  case 0:
+  case 1: return w.size * exp(-0.5 * (pow(tt / width, 2.0)));
+  case 2: return w.size * (-tt / width * exp(-0.5 * (pow(tt / width, 2.0))));
+  case 3: return w.size * ((1.0 - pow(tt / width, 2)) * exp(-0.5 * (pow(tt / width, 2.0))));
+  case 4: return w.size * (exp(-0.5 * (pow(tt / width, 2.0))) * sin(2.0 * pi * w.frequency * tt));
+  case 5: return w.size * wf_compact(pi, tt, width, 2.0);
+  case 6:
+    if (tt <= 0.0 || tt >= 2.0 * width) return 0.0;
+    return w.size * (1.0 / 32.0 * (15.0 * sin(pi / width * tt) - 12.0 * sin(2.0 * pi / width * tt) +
+                                   3.0 * sin(3.0 * pi / width * tt)));
+  case 7: return w.size * (wf_compact(pi, tt, width, 2.0) * sin(2.0 * pi * w.frequency * tt));
+  case 8: return w.size * (wf_compact(pi, tt, width, 1.0) * sin(2.0 * pi * w.frequency * tt));
+  case 9: {
+    const double *T3 = w.table;
+    const unsigned long n = w.n;
+    if (n < 2 || tt < T3[0] || tt > T3[3 * (n - 1)]) return 0.0;
+    unsigned long lo = 0, hi = n - 1;
+    while (hi - lo > 1) {
+      const unsigned long m = (hi + lo) >> 1;
+      if (T3[3 * m] > tt) hi = m;
+      else lo = m;
+    }
+    const double h = T3[3 * hi] - T3[3 * lo];
+    const double aa = (T3[3 * hi] - tt) / h, bb = (tt - T3[3 * lo]) / h;
+    return w.size * (aa * T3[3 * lo + 1] + bb * T3[3 * hi + 1] +
+                     ((aa * aa * aa - aa) * T3[3 * lo + 2] + (bb * bb * bb - bb) * T3[3 * hi + 2]) * (h * h) / 6.0);
+  }
+  default: return 0.0;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 1-D auxiliary grids of the TF/SF plane waves (planewave.c:1315-1372).
+// One block per plane wave; the blocks ride in other launches (k_head for E,
+// the H corrections' k_corr for H), whose own work they do not touch.
+// ---------------------------------------------------------------------------
+template <typename T> VG_DEV void aux_e_block(const AuxArgs<T> &a, int p, double t, double pi)
+{
+  const PwDev &pw = a.pw[p];
+  if (!pw.use_aux) return;
+  T *Eyi = a.aux + (long long)p * 2 * a.auxmax, *Hzi = Eyi + a.auxmax;
+  T *PPy = a.pml + p * 30, *Py = PPy + 10;
+  const T *adx = a.prof + p * 40, *bdx = adx + 10;
+  const T beta = T(pw.beta);
+  for (int i = 1 + threadIdx.x; i < pw.nx; i += blockDim.x) {
+    if (i < pw.xb) {
+      Eyi[i] = Eyi[i] + beta * (Hzi[i - 1] - Hzi[i]);
+    } else {
+      const int L = i - pw.xb;
+      const T oldPP = PPy[L];
+      PPy[L] = PPy[L] + beta * (Hzi[i - 1] - Hzi[i]);
+      const T oldP = Py[L];
+      Py[L] = Py[L] + (PPy[L] - oldPP);
+      Eyi[i] = adx[L] * Eyi[i] + bdx[L] * (Py[L] - oldP);
+    }
+  }
+  if (threadIdx.x == 0) Eyi[0] = T(wf_value(a.wf[pw.waveform], t, pw.delay, pi));
+}
+
+template <typename T> VG_DEV void aux_h_block(const AuxArgs<T> &a, int p)
+{
+  const PwDev &pw = a.pw[p];
+  if (!pw.use_aux) return;
+  T *Eyi = a.aux + (long long)p * 2 * a.auxmax, *Hzi = Eyi + a.auxmax;
+  T *Bz = a.pml + p * 30 + 20;
+  const T *ahx = a.prof + p * 40 + 20, *bhx = ahx + 10;
+  const T gamma = T(pw.gamma);
+  for (int i = threadIdx.x; i < pw.nx; i += blockDim.x) {
+    if (i < pw.xb) {
+      Hzi[i] = Hzi[i] + gamma * (Eyi[i] - Eyi[i + 1]);
+    } else {
+      const int L = i - pw.xb;
+      const T oldB = Bz[L];
+      Bz[L] = ahx[L] * Bz[L] + gamma * bhx[L] * (-Eyi[i + 1] + Eyi[i]);
+      Hzi[i] = Hzi[i] + (Bz[L] - oldB);
+    }
+  }
+}
+
 // ===========================================================================
 // Volume sweeps.  Each half-step is two kernels over disjoint cells:
 //  - the fast kernel over the fast box, where every component takes the
@@ -158,43 +254,170 @@ VG_DEV unsigned xcd_block(unsigned b, unsigned n)
 }
 VG_DEV unsigned xcd_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
-// Layer-0 Debye correction inside the fast E kernel (debye.c:243-307).  The
-// chunk's first site comes from dbase (uniform over the wavefront, so rows
-// without Debye sites skip this entirely); a site's number is that plus the
-// count of lower lanes whose class carries a Debye medium for C, which is
-// the site list's (component, cell) order.
-template <typename T, int C>
-VG_DEV void debye_fused(const FastE<T> &f, int bx, int j, int k, bool vx, unsigned cls, T be, T &e)
+// ===========================================================================
+// Corrections (XArgs): rows in a launch of their own after the sweep, and
+// what a sweep's thread does itself after its cell's update.
+// ===========================================================================
+
+// One field value's operations, in order.  Coefficients of the value's cell
+// come from its class, as the sweep's do.
+template <typename T, bool IDX, bool ELEC>
+VG_DEV void x_row(const VG_CONST XArgs<T> *x, const VG_GLOBAL XRow *row)
 {
-  const EArgs<T> &a = *f.ap;
-  const long long row = ((long long)(C * f.NZ + k) * f.NY + j) * f.nchx + bx;
-  const VG_GLOBAL int *dbase = gp(a.dbase);
-  const int g0 = dbase[row];
-  if (dbase[row + 1] == g0) return;
-  const int ds = vx ? gp(a.edslot)[cls * 3 + C] : -1;
-  const unsigned long long m = __ballot(ds >= 0);
-  if (ds < 0) return;
-  const long long g = g0 + __popcll(m & ((1ull << __lane_id()) - 1ull));
-  e = debye_site<T>(e, be, g, ds, a.dlast, a.dJ, a.dstride, a.dalpha, a.dbeta, a.dnp, a.dmaxP, a.dcplx);
+  const int id = row[0].cell, c = (int)(row[0].opc & 3u);
+  VG_GLOBAL T *F = gp(c == 0 ? x->F[0] : c == 1 ? x->F[1] : x->F[2]);
+  T v = F[id], al = T(1), be = T(0);
+  const unsigned o1 = row[1].opc >> 2;
+  bool coef = false;
+  for (unsigned o = row[0].opc >> 2; o < o1; ++o) {
+    const VG_GLOBAL XOp<T> *po = gp(x->op) + o;
+    const struct { int code, arg; T a, b; } op{po->code, po->arg, po->a, po->b};
+    const int kind = op.code & 7;
+    if (kind != XO_ZERO && kind != XO_GHOST && !coef) {
+      coef = true;
+      if (IDX) {
+        const unsigned cl = (unsigned)gp(x->cls)[id];
+        if (ELEC) load_pair(x->tab + cl * ETAB_STRIDE + 2 * c, al, be);
+        else be = gp(x->tab)[cl * HTAB_STRIDE + c];
+      } else {
+        if (ELEC) al = gp(c == 0 ? x->ca[0] : c == 1 ? x->ca[1] : x->ca[2])[id];
+        be = gp(c == 0 ? x->cb[0] : c == 1 ? x->cb[1] : x->cb[2])[id];
+      }
+    }
+    if (kind == XO_ZERO) {
+      v = T(0);
+    } else if (kind == XO_GHOST) {
+      v = op.a * F[op.arg];
+    } else if (kind == XO_DEBYE) {
+      if (ELEC)
+        v = debye_site<T>(v, be, op.arg, op.code >> 8, x->dlast, x->dJ, x->dstride, x->dalpha, x->dbeta, x->dnp,
+                          x->dmaxP, x->dcplx);
+    } else if (kind == XO_SRC) {
+      const T source = gp(x->val)[op.arg], soft = T((op.code >> 4) & 1);
+      if ((op.code >> 3) & 1) v = soft * v - be * source;
+      else v = soft * v + source;
+    } else if (kind == XO_SIBC) {
+      if (!ELEC) {
+        const int b = op.code >> 3, ea = (b >> 1) & 3, eb = (b >> 3) & 3;
+        const T w = (b >> 6) & 1 ? T(1) : T(0.5);
+        const VG_GLOBAL T *Et = gp(x->Etan) + 4 * (long long)op.arg;
+        T t;
+        if (!(b & 1)) t = (be * w) * (op.a * Et[ea]);
+        else t = ((be * T(0.5)) * w) * (T((b >> 7) & 1) * (op.a * Et[ea]) + T((b >> 8) & 1) * (op.b * Et[eb]));
+        v = v + ((b >> 5) & 1 ? T(-1) : T(1)) * t;
+      }
+    } else {
+      T incv;
+      if (kind == XO_AUX) {
+        const int inc = (op.code >> 3) & 7, p = op.code >> 8;
+        const T dp = op.a;
+        const VG_GLOBAL T *Eyi = gp(x->aux) + (long long)p * 2 * x->auxmax, *Hzi = Eyi + x->auxmax;
+        T value;
+        if (inc < 3) value = (T(1) - dp) * Eyi[2 + op.arg] + dp * Eyi[2 + op.arg + 1];
+        else value = x->eta0 * ((T(1) - dp) * Hzi[1 + op.arg] + dp * Hzi[2 + op.arg]);
+        incv = T(gp(x->pw)[p].Finc[inc]) * value;
+      } else {
+        incv = gp(x->val)[op.arg];
+      }
+      const T term = be * (op.b * incv);
+      const T sign = (op.code >> 6) & 1 ? T(-1) : T(1);
+      if (ELEC) v = al * v + sign * term;
+      else v = v + sign * term;
+    }
+  }
+  F[id] = v;
 }
 
-// One E component of a fast-box cell: its coefficients and old value, then
-// the ordinary update (and, with FUSE, the first Debye layer).  All three
-// components are computed before any is stored, so the stores do not hold
-// back the next component's loads.
-template <typename T, bool IDX, bool FUSE, int C>
-VG_DEV T e_fast(const FastE<T> &f, int bx, int j, int k, bool vx, long long id, unsigned cls, T curl)
+// A row on its own, or a group's rows in order.
+template <typename T, bool IDX, bool ELEC> VG_DEV void x_rows(const VG_CONST XArgs<T> *x, unsigned b)
 {
-  T al, be;
-  if (IDX) {
-    load_pair(f.etab + cls * ETAB_STRIDE + 2 * C, al, be);
-  } else {
-    al = f.alpha[C][id];
-    be = f.beta[C][id];
+  const long long q = b * 256ll + threadIdx.x;
+  const VG_GLOBAL XRow *row = gp(x->row);
+  if (q < x->nrow) {
+    x_row<T, IDX, ELEC>(x, row + q);
+  } else if (q < x->nrow + x->ngroup) {
+    const VG_GLOBAL int *gs = gp(x->gstart) + (q - x->nrow);
+    for (int r = gs[0], r1 = gs[1]; r < r1; ++r) x_row<T, IDX, ELEC>(x, row + r);
   }
-  T e = al * f.Ein[C][id] + be * curl;
-  if (FUSE) debye_fused<T, C>(f, bx, j, k, vx, cls, be, e);
+}
+
+template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) void k_rows(const XArgs<T> *x)
+{
+  x_rows<T, IDX, ELEC>(cp(x), blockIdx.x);
+}
+
+// A one-pole Debye site (debye.c:243-307, as debye_site with one real pole):
+// j is its J, the previous E is the old E of the update.
+template <typename T> VG_DEV T x_debye(VG_GLOBAL T *J, T j, T da, T db, T be, T eo, T e)
+{
+  const T jsum = T(0) + (T(1) + da) * j;
+  e = e - be * jsum;
+  const T de = e - eo;
+  *J = da * j + db * de;
   return e;
+}
+
+// What a flagged cell's corrections read, loaded together with the update's
+// own operands: J is dense, so its address needs nothing but the cell.
+template <typename T> struct XPre {
+  T j0, j1, j2;
+  typename Vec2<T>::type d0, d1, d2;
+  unsigned fl;
+  template <bool DEBYE> VG_DEV void load(const VG_CONST XArgs<T> *x, long long id, unsigned cls)
+  {
+    using V2 = typename Vec2<T>::type;
+    const VG_GLOBAL T *d = gp(x->dtab) + (cls - x->flag0) * DTAB_STRIDE;
+    fl = (unsigned)d[6];
+    if (DEBYE) {
+      const VG_GLOBAL T *J = gp(x->J) + id;
+      j0 = J[0];
+      j1 = J[x->nJ];
+      j2 = J[2 * x->nJ];
+      d0 = ((const VG_GLOBAL V2 *)d)[0];
+      d1 = ((const VG_GLOBAL V2 *)d)[1];
+      d2 = ((const VG_GLOBAL V2 *)d)[2];
+    }
+  }
+};
+
+// A flagged cell's E before it is stored (o* old, e* updated, b* the update's
+// beta): the Mur faces that take its update (mur.c:135-395), its one-pole
+// Debye sites, its zeroed components.
+template <typename T, bool DEBYE>
+VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, int i, int j, int k, long long id, const XPre<T> &p, T o0, T o1,
+                       T o2, T b0, T b1, T b2, T &e0, T &e1, T &e2)
+{
+  const unsigned fl = p.fl;
+  if (fl & XF_MUR) {
+    const unsigned mask = x->murmask;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      const int a = f >> 1, up = f & 1;
+      if (!((mask >> f) & 1u)) continue;
+#pragma unroll
+      for (int s = 1; s < 3; ++s) {
+        const int C = (a + s) % 3;
+        const VG_CONST int *b = x->mbox[f][C];
+        const int n = a == 0 ? i : a == 1 ? j : k;
+        if (n != b[2 * a + up] + (up ? -1 : 1)) continue;
+        if ((a != 0 && (i < b[0] || i > b[1])) || (a != 1 && (j < b[2] || j > b[3])) || (a != 2 && (k < b[4] || k > b[5])))
+          continue;
+        const long long st = a == 0 ? 1 : a == 1 ? (long long)x->PX : x->plane;
+        VG_GLOBAL T *F = gp(x->F[C]) + (up ? id + st : id - st);
+        const T o = C == 0 ? o0 : C == 1 ? o1 : o2, t = C == 0 ? e0 : C == 1 ? e1 : e2;
+        *F = o + x->mzeta[f] * (t - *F);
+      }
+    }
+  }
+  if (DEBYE) {
+    VG_GLOBAL T *J = gp(x->J) + id;
+    if (fl & XF_DEBYE) e0 = x_debye(J, p.j0, p.d0.x, p.d0.y, b0, o0, e0);
+    if (fl & (XF_DEBYE << 1)) e1 = x_debye(J + x->nJ, p.j1, p.d1.x, p.d1.y, b1, o1, e1);
+    if (fl & (XF_DEBYE << 2)) e2 = x_debye(J + 2 * x->nJ, p.j2, p.d2.x, p.d2.y, b2, o2, e2);
+  }
+  if (fl & XF_ZERO) e0 = T(0);
+  if (fl & (XF_ZERO << 1)) e1 = T(0);
+  if (fl & (XF_ZERO << 2)) e2 = T(0);
 }
 
 // Update-once check (the reference's CHECK_LIMITS build, grid.h:181-191):
@@ -202,15 +425,18 @@ VG_DEV T e_fast(const FastE<T> &f, int bx, int j, int k, bool vx, long long id, 
 // instead of storing them, and leaves every field and auxiliary untouched.
 VG_DEV void visit(unsigned *v, long long id) { atomicAdd(v + id, 1u); }
 
-// Fast E tile: inner grid (grid.c:709-797) and, with FUSE, the first Debye
-// layer.  L is the logical block (in XCD order).
-template <typename T, bool IDX, bool FUSE, bool CHK>
-VG_DEV void e_fast_tile(const FastE<T> &f, unsigned L)
+// Fast E tile: inner grid (grid.c:709-797).  X: in-line corrections, 0 none,
+// 1 Mur faces and zeroed E, 2 Debye sites as well.
+// L is the logical block (in XCD order).  All three components are computed
+// before any is stored, so the stores do not hold back the next component's
+// loads.
+template <typename T, bool IDX, int X, bool CHK>
+VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned L)
 {
   if (L >= (unsigned)(f.nchx * f.gy * f.gz)) return;
   const int bx = (int)(L % f.nchx), by = (int)((L / f.nchx) % f.gy), bz = (int)(L / (f.nchx * f.gy));
-  const int i = f.box[0] + bx * 64 + (int)threadIdx.x;
-  const int j = f.box[2] + by * (int)blockDim.y + (int)threadIdx.y;
+  const int i = f.box[0] + bx * 64 + (int)(threadIdx.x & 63u);
+  const int j = f.box[2] + by * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6);
   if (j > f.box[3]) return;  // whole wavefront
   const bool vx = i <= f.box[1];
   const int ic = vx ? i : f.box[1];
@@ -218,28 +444,50 @@ VG_DEV void e_fast_tile(const FastE<T> &f, unsigned L)
   const int ke = min(kb + f.kchunk, f.box[5] + 1);
   if (kb >= ke) return;
   const long long P = f.plane, SJ = f.PX;
-  const T *__restrict__ Hx = f.H[0];
-  const T *__restrict__ Hy = f.H[1];
-  const T *__restrict__ Hz = f.H[2];
+  const T *Hx = f.H[0], *Hy = f.H[1], *Hz = f.H[2];
   const T idhx = f.idh[0][ic], idhy = f.idh[1][j];
+  const unsigned flag0 = X ? x->flag0 : ~0u;
   long long id = ((long long)kb * f.NY + j) * SJ + ic;
   // The fast box starts at index 1 or more on every axis, so the i-1, j-1
   // and k-1 neighbours are inside the allocation.
   T hxm = Hx[id - P], hym = Hy[id - P];
+  // the next plane's class is loaded a plane ahead (the box ends at N-2): what
+  // it selects then loads with the plane's fields, not after them
+  const uint16_t *pc = IDX ? f.ecls : X && flag0 != ~0u ? (const uint16_t *)x->cls : nullptr;
+  unsigned cnext = pc ? (unsigned)pc[id] : 0u;
   for (int k = kb; k < ke; ++k, id += P) {
+    const unsigned cls = cnext;
+    XPre<T> pre{};
+    const bool flagged = X && cls >= flag0;
+    if (flagged) pre.template load<X == 2>(x, id, cls);
     const T hx = Hx[id], hy = Hy[id], hz = Hz[id];
     const T hzy = Hz[id - SJ], hzx = Hz[id - 1], hyx = Hy[id - 1], hxy = Hx[id - SJ];
-    const unsigned cls = IDX ? (unsigned)f.ecls[id] : 0u;
+    if (pc) cnext = (unsigned)pc[id + P];
     const T idhz = cp(f.idh[2])[k];
-    const T e0 = e_fast<T, IDX, FUSE, 0>(f, bx, j, k, vx, id, cls, idhy * (hz - hzy) + idhz * (hym - hy));
-    const T e1 = e_fast<T, IDX, FUSE, 1>(f, bx, j, k, vx, id, cls, idhz * (hx - hxm) + idhx * (hzx - hz));
-    const T e2 = e_fast<T, IDX, FUSE, 2>(f, bx, j, k, vx, id, cls, idhx * (hy - hyx) + idhy * (hxy - hx));
+    T a0, a1, a2, b0, b1, b2;
+    if (IDX) {
+      load_pair(f.etab + cls * ETAB_STRIDE, a0, b0);
+      load_pair(f.etab + cls * ETAB_STRIDE + 2, a1, b1);
+      load_pair(f.etab + cls * ETAB_STRIDE + 4, a2, b2);
+    } else {
+      a0 = f.alpha[0][id];
+      a1 = f.alpha[1][id];
+      a2 = f.alpha[2][id];
+      b0 = f.beta[0][id];
+      b1 = f.beta[1][id];
+      b2 = f.beta[2][id];
+    }
+    const T o0 = f.Ein[0][id], o1 = f.Ein[1][id], o2 = f.Ein[2][id];
+    T e0 = a0 * o0 + b0 * (idhy * (hz - hzy) + idhz * (hym - hy));
+    T e1 = a1 * o1 + b1 * (idhz * (hx - hxm) + idhx * (hzx - hz));
+    T e2 = a2 * o2 + b2 * (idhx * (hy - hyx) + idhy * (hxy - hx));
     if (vx) {
       if (CHK) {
         visit(f.vis[0], id);
         visit(f.vis[1], id);
         visit(f.vis[2], id);
       } else {
+        if (flagged) x_inline_e<T, X == 2>(x, i, j, k, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
         f.E[0][id] = e0;
         f.E[1][id] = e1;
         f.E[2][id] = e2;
@@ -250,10 +498,10 @@ VG_DEV void e_fast_tile(const FastE<T> &f, unsigned L)
   }
 }
 
-template <typename T, bool IDX, bool FUSE, bool CHK = false>
-__global__ __launch_bounds__(512) void k_e_fast(FastE<T> f)
+template <typename T, bool IDX, int X, bool CHK = false>
+__global__ __launch_bounds__(512) void k_e_fast(FastE<T> f, const XArgs<T> *x)
 {
-  e_fast_tile<T, IDX, FUSE, CHK>(f, xcd_block());
+  e_fast_tile<T, IDX, X, CHK>(f, cp(x), xcd_block());
 }
 
 // Fast H tile: inner grid (grid.c:800-888).
@@ -261,8 +509,8 @@ template <typename T, bool IDX, bool CHK> VG_DEV void h_fast_tile(const FastH<T>
 {
   if (L >= (unsigned)(f.nchx * f.gy * f.gz)) return;
   const int bx = (int)(L % f.nchx), by = (int)((L / f.nchx) % f.gy), bz = (int)(L / (f.nchx * f.gy));
-  const int i = f.box[0] + bx * 64 + (int)threadIdx.x;
-  const int j = f.box[2] + by * (int)blockDim.y + (int)threadIdx.y;
+  const int i = f.box[0] + bx * 64 + (int)(threadIdx.x & 63u);
+  const int j = f.box[2] + by * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6);
   if (j > f.box[3]) return;
   const bool vx = i <= f.box[1];
   const int ic = vx ? i : f.box[1];
@@ -270,23 +518,19 @@ template <typename T, bool IDX, bool CHK> VG_DEV void h_fast_tile(const FastH<T>
   const int ke = min(kb + f.kchunk, f.box[5] + 1);
   if (kb >= ke) return;
   const long long P = f.plane, SJ = f.PX;
-  const T *__restrict__ Ex = f.E[0];
-  const T *__restrict__ Ey = f.E[1];
-  const T *__restrict__ Ez = f.E[2];
-  T *__restrict__ H0 = f.H[0];
-  T *__restrict__ H1 = f.H[1];
-  T *__restrict__ H2 = f.H[2];
-  const T *__restrict__ I0 = f.Hin[0];
-  const T *__restrict__ I1 = f.Hin[1];
-  const T *__restrict__ I2 = f.Hin[2];
+  const T *Ex = f.E[0], *Ey = f.E[1], *Ez = f.E[2];
+  T *H0 = f.H[0], *H1 = f.H[1], *H2 = f.H[2];
+  const T *I0 = f.Hin[0], *I1 = f.Hin[1], *I2 = f.Hin[2];
   const T idex = f.ide[0][ic], idey = f.ide[1][j];
   long long id = ((long long)kb * f.NY + j) * SJ + ic;
   // The fast box ends at index N-2 or less, so i+1, j+1 and k+1 are inside.
   T ex = Ex[id], ey = Ey[id];
+  unsigned cnext = IDX ? (unsigned)f.hcls[id] : 0u;  // a plane ahead, as in the E tile
   for (int k = kb; k < ke; ++k, id += P) {
+    const unsigned cls = cnext;
     const T exp1 = Ex[id + P], eyp1 = Ey[id + P];
     const T ez = Ez[id], ezy = Ez[id + SJ], ezx = Ez[id + 1], exy = Ex[id + SJ], eyx = Ey[id + 1];
-    const unsigned cls = IDX ? (unsigned)f.hcls[id] : 0u;
+    if (IDX) cnext = (unsigned)f.hcls[id + P];
     const T idez = cp(f.ide[2])[k];
     T g0, g1, g2;
     if (IDX) {
@@ -564,13 +808,13 @@ template <typename T, bool IDX> __global__ __launch_bounds__(256) void k_h_fix(F
 // registers, and each plane issues all its loads before its first store.  The
 // launch order of the blocks (ShellWork) gives each XCD one contiguous eighth
 // of every piece.
-VG_DEV bool shell_column(const ShellPiece *pcs, const ShellWork *work, unsigned b, const ShellPiece *&pc, int &di,
+VG_DEV bool shell_column(const ShellDev *pcs, const ShellWork *work, unsigned b, const VG_CONST ShellDev *&pc, int &di,
                          int &dj, int &dk0, int &dk1)
 {
-  const ShellWork w = work[b];
-  if (w.piece < 0) return false;
-  pc = pcs + w.piece;
-  const int zc = w.block / pc->nxyb, xyb = w.block - zc * pc->nxyb;
+  const VG_CONST ShellWork *w = cp(work) + b;
+  if (w->piece < 0) return false;
+  pc = cp(pcs) + w->piece;
+  const int zc = w->block / pc->nxyb, xyb = w->block - zc * pc->nxyb;
   const int l = xyb * 256 + (int)threadIdx.x;
   if (l >= pc->nxy) return false;
   dj = l / pc->nip;
@@ -589,21 +833,6 @@ struct ColRegion {
   long long p, psz;
   void *a, *b;
 };
-// A lane's region in the kernels: reg as above, and for a UPML slab the
-// 32-bit element offset q of the lane's current cell in the auxiliaries'
-// pools (the slab's offset in the pool plus its slab index), advanced by psz
-// per plane.  Three 32-bit values per component instead of a 64-bit index,
-// stride and two 64-bit slab addresses keep the shell kernels' register
-// count, and so their occupancy, lower.
-struct LaneRegion {
-  int reg, q, psz;
-  template <typename T> VG_DEV LaneRegion(const ColRegion &r, const T *pool)
-      : reg(r.reg), q(r.reg >= 0 && r.reg < 6 ? (int)(static_cast<const T *>(r.a) - pool + r.p) : 0),
-        psz((int)r.psz)
-  {
-  }
-};
-
 template <int C> VG_HD ColRegion shell_region(const ShellPiece *pc, int i, int dj, int dk)
 {
   ColRegion r{-1, 0, 0, nullptr, nullptr};
@@ -619,6 +848,25 @@ template <int C> VG_HD ColRegion shell_region(const ShellPiece *pc, int i, int d
   }
   return r;
 }
+
+// A lane's region in the kernels: reg as above, and for a UPML slab the
+// 32-bit element offset q of the lane's current cell in the auxiliaries'
+// pools, advanced by psz per plane.  Three 32-bit values per component instead
+// of a 64-bit index, stride and two 64-bit slab addresses keep the shell
+// kernels' register count, and so their occupancy, lower.
+struct LaneRegion {
+  int reg, q, psz;
+  VG_DEV LaneRegion(const VG_CONST ShellDevRun *run, int i, int dj, int dk) : reg(-1), q(0), psz(0)
+  {
+#pragma unroll
+    for (int s = 0; s < SHELL_RUNS; ++s) {
+      const bool in = i >= run[s].xa && i <= run[s].xb;
+      reg = in ? run[s].reg : reg;
+      q = in ? run[s].q0 + i + dj * run[s].psy + dk * run[s].psz : q;
+      psz = in ? run[s].psz : psz;
+    }
+  }
+};
 
 // The E shell's arrays as global pointers, read from the argument block
 // once, before the plane loop.
@@ -694,41 +942,41 @@ template <typename T, bool IDX, int C> struct EShellCell {
       coef(g, n3, true);
     }
   }
-  VG_DEV void store(const EShellPtrs<T> &g, const LaneRegion &rg, long long id, T curl) const
+  // the new E (the auxiliaries stored), to be stored by the caller
+  VG_DEV T value(const EShellPtrs<T> &g, const LaneRegion &rg, T curl) const
   {
-    if (rg.reg == 6) {
-      g.E[C][id] = al * e + be * curl;
-    } else if (rg.reg >= 0) {
-      const T ppn = al * opp + be * curl;
-      g.PP[rg.q] = ppn;
-      const T pn = cf[0] * op + cf[1] * (ppn - opp);
-      g.Pa[rg.q] = pn;
-      g.E[C][id] = cf[2] * e + cf[3] * cf[4] * (pn - cf[5] * op);
-    }
+    if (rg.reg == 6) return al * e + be * curl;
+    if (rg.reg < 0) return T(0);
+    const T ppn = al * opp + be * curl;
+    g.PP[rg.q] = ppn;
+    const T pn = cf[0] * op + cf[1] * (ppn - opp);
+    g.Pa[rg.q] = pn;
+    return cf[2] * e + cf[3] * cf[4] * (pn - cf[5] * op);
   }
 };
 
-template <typename T, bool IDX, bool CHK, bool SEP>
-VG_DEV void e_shell_column(const ShellPiece *pcs, const ShellWork *work, const EArgs<T> *ap, unsigned b)
+template <typename T, bool IDX, int X, bool CHK, bool SEP>
+VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EArgs<T> *ap,
+                           const VG_CONST XArgs<T> *x, unsigned b)
 {
-  const ShellPiece *pc;
+  const VG_CONST ShellDev *pc;
   int di, dj, dk0, dk1;
   if (!shell_column(pcs, work, b, pc, di, dj, dk0, dk1)) return;
   const EArgs<T> &a = *ap;
   const EShellPtrs<T> g(a, SEP);
   const int NY = a.NY;
   const long long P = a.plane, SJ = a.PX;
-  const int i = pc->box[0] + di, j = pc->box[2] + dj;
-  LaneRegion rg[3] = {LaneRegion(shell_region<0>(pc, i, dj, dk0), a.PPpool),
-                      LaneRegion(shell_region<1>(pc, i, dj, dk0), a.PPpool),
-                      LaneRegion(shell_region<2>(pc, i, dj, dk0), a.PPpool)};
+  const int i = pc->x0 + di, j = pc->y0 + dj;
+  LaneRegion rg[3] = {LaneRegion(pc->run[0], i, dj, dk0), LaneRegion(pc->run[1], i, dj, dk0),
+                      LaneRegion(pc->run[2], i, dj, dk0)};
   if (rg[0].reg < 0 && rg[1].reg < 0 && rg[2].reg < 0) return;
   const VG_GLOBAL T *Hx = g.H[0], *Hy = g.H[1], *Hz = g.H[2];
   // (the sweep never updates index 0 of any axis; the guards keep every read
   // inside the allocation regardless)
   const bool xm = i > 0, ym = j > 0;
   const T idh0 = g.idh[0][i], idh1 = g.idh[1][j];
-  int k = pc->box[4] + dk0;
+  const unsigned flag0 = X ? x->flag0 : ~0u;
+  int k = pc->z0 + dk0;
   long long id = ((long long)k * NY + j) * SJ + i;
   T hxm = k > 0 ? Hx[id - P] : T(0), hym = k > 0 ? Hy[id - P] : T(0);  // plane k-1, carried
   EShellCell<T, IDX, 0> c0;
@@ -740,13 +988,19 @@ VG_DEV void e_shell_column(const ShellPiece *pcs, const ShellWork *work, const E
     c1.init(g, rg[1], n3);
     c2.init(g, rg[2], n3);
   }
+  const VG_GLOBAL uint16_t *pcl = IDX ? g.ecls : X && flag0 != ~0u ? gp((const uint16_t *)x->cls) : nullptr;
+  unsigned cnext = pcl ? (unsigned)pcl[id] : 0u;  // a plane ahead, as in the fast tile
   for (int dk = dk0; dk < dk1; ++dk, ++k, id += P) {
+    const unsigned cls = cnext;
+    if (pcl && dk + 1 < dk1) cnext = (unsigned)pcl[id + P];
     const T hx = Hx[id], hy = Hy[id], hz = Hz[id];
     const T hzy = ym ? Hz[id - SJ] : T(0), hzx = xm ? Hz[id - 1] : T(0);
     const T hyx = xm ? Hy[id - 1] : T(0), hxy = ym ? Hx[id - SJ] : T(0);
     const T idh2 = cp(g.idh[2])[k];
-    const unsigned cls = IDX ? (unsigned)g.ecls[id] : 0u;
     const int n3[3] = {i, j, k};
+    XPre<T> pre{};
+    const bool flagged = X && cls >= flag0;
+    if (flagged) pre.template load<X == 2>(x, id, cls);
     c0.load(g, rg[0], n3, id, cls);
     c1.load(g, rg[1], n3, id, cls);
     c2.load(g, rg[2], n3, id, cls);
@@ -754,9 +1008,13 @@ VG_DEV void e_shell_column(const ShellPiece *pcs, const ShellWork *work, const E
       for (int C = 0; C < 3; ++C)
         if (rg[C].reg >= 0) visit(a.vis[C], id);
     } else {
-      c0.store(g, rg[0], id, idh1 * (hz - hzy) + idh2 * (hym - hy));
-      c1.store(g, rg[1], id, idh2 * (hx - hxm) + idh0 * (hzx - hz));
-      c2.store(g, rg[2], id, idh0 * (hy - hyx) + idh1 * (hxy - hx));
+      T e0 = c0.value(g, rg[0], idh1 * (hz - hzy) + idh2 * (hym - hy));
+      T e1 = c1.value(g, rg[1], idh2 * (hx - hxm) + idh0 * (hzx - hz));
+      T e2 = c2.value(g, rg[2], idh0 * (hy - hyx) + idh1 * (hxy - hx));
+      if (flagged) x_inline_e<T, X == 2>(x, i, j, k, id, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
+      if (rg[0].reg >= 0) g.E[0][id] = e0;
+      if (rg[1].reg >= 0) g.E[1][id] = e1;
+      if (rg[2].reg >= 0) g.E[2][id] = e2;
     }
     hxm = hx;
     hym = hy;
@@ -766,10 +1024,10 @@ VG_DEV void e_shell_column(const ShellPiece *pcs, const ShellWork *work, const E
   }
 }
 
-template <typename T, bool IDX, bool CHK = false, bool SEP = true>
-__global__ __launch_bounds__(256) void k_e_shell(const ShellPiece *pcs, const ShellWork *work, const EArgs<T> *ap)
+template <typename T, bool IDX, bool CHK = false>
+__global__ __launch_bounds__(256) void k_e_shell(const ShellDev *pcs, const ShellWork *work, const EArgs<T> *ap)
 {
-  e_shell_column<T, IDX, CHK, SEP>(pcs, work, ap, blockIdx.x);
+  e_shell_column<T, IDX, 0, CHK, true>(pcs, work, ap, nullptr, blockIdx.x);
 }
 
 // The H shell's arrays as global pointers.
@@ -778,12 +1036,13 @@ template <typename T> struct HShellPtrs {
   VG_GLOBAL T *B;  // UPML auxiliary pool
   VG_GLOBAL const T *Hin[3], *E[3], *gamma[3], *ad[3], *ah[3], *bh[3], *ibd[3], *ide[3], *htab;
   VG_GLOBAL const uint16_t *hcls;
-  VG_DEV explicit HShellPtrs(const HArgs<T> &a)
+  // sep as in EShellPtrs
+  VG_DEV explicit HShellPtrs(const HArgs<T> &a, bool sep)
   {
     B = gp(a.Bpool);
     for (int d = 0; d < 3; ++d) {
       H[d] = gp(a.H[d]);
-      Hin[d] = gp(a.Hin[d]);
+      Hin[d] = sep ? gp(a.Hin[d]) : H[d];
       E[d] = gp(a.E[d]);
       gamma[d] = gp(a.gamma[d]);
       ad[d] = gp(a.ad[d]);
@@ -844,25 +1103,24 @@ template <typename T, bool IDX, int C> struct HShellCell {
   }
 };
 
-template <typename T, bool IDX, bool CHK>
-VG_DEV void h_shell_column(const ShellPiece *pcs, const ShellWork *work, const HArgs<T> *ap, unsigned b)
+template <typename T, bool IDX, bool CHK, bool SEP>
+VG_DEV void h_shell_column(const ShellDev *pcs, const ShellWork *work, const HArgs<T> *ap, unsigned b)
 {
-  const ShellPiece *pc;
+  const VG_CONST ShellDev *pc;
   int di, dj, dk0, dk1;
   if (!shell_column(pcs, work, b, pc, di, dj, dk0, dk1)) return;
   const HArgs<T> &a = *ap;
-  const HShellPtrs<T> q(a);
+  const HShellPtrs<T> q(a, SEP);
   const int NX = a.NX, NY = a.NY, NZ = a.NZ;
   const long long P = a.plane, SJ = a.PX;
-  const int i = pc->box[0] + di, j = pc->box[2] + dj;
-  LaneRegion rg[3] = {LaneRegion(shell_region<0>(pc, i, dj, dk0), a.Bpool),
-                      LaneRegion(shell_region<1>(pc, i, dj, dk0), a.Bpool),
-                      LaneRegion(shell_region<2>(pc, i, dj, dk0), a.Bpool)};
+  const int i = pc->x0 + di, j = pc->y0 + dj;
+  LaneRegion rg[3] = {LaneRegion(pc->run[0], i, dj, dk0), LaneRegion(pc->run[1], i, dj, dk0),
+                      LaneRegion(pc->run[2], i, dj, dk0)};
   if (rg[0].reg < 0 && rg[1].reg < 0 && rg[2].reg < 0) return;
   const VG_GLOBAL T *Ex = q.E[0], *Ey = q.E[1], *Ez = q.E[2];
   const bool xin = i + 1 < NX, yin = j + 1 < NY;
   const T ide0 = q.ide[0][i], ide1 = q.ide[1][j];
-  int k = pc->box[4] + dk0;
+  int k = pc->z0 + dk0;
   long long id = ((long long)k * NY + j) * SJ + i;
   T exc = Ex[id], eyc = Ey[id];  // this plane's Ex, Ey: carried from the previous plane's k+1 loads
   HShellCell<T, IDX, 0> c0;
@@ -874,13 +1132,15 @@ VG_DEV void h_shell_column(const ShellPiece *pcs, const ShellWork *work, const H
     c1.init(q, rg[1], n3);
     c2.init(q, rg[2], n3);
   }
+  unsigned cnext = IDX ? (unsigned)q.hcls[id] : 0u;
   for (int dk = dk0; dk < dk1; ++dk, ++k, id += P) {
+    const unsigned cls = cnext;
+    if (IDX && dk + 1 < dk1) cnext = (unsigned)q.hcls[id + P];
     const bool zin = k + 1 < NZ;
     const T exp1 = zin ? Ex[id + P] : T(0), eyp1 = zin ? Ey[id + P] : T(0);
     const T ez = Ez[id], ezy = yin ? Ez[id + SJ] : T(0), ezx = xin ? Ez[id + 1] : T(0);
     const T eyx = xin ? Ey[id + 1] : T(0), exy = yin ? Ex[id + SJ] : T(0);
     const T ide2 = cp(q.ide[2])[k];
-    const unsigned cls = IDX ? (unsigned)q.hcls[id] : 0u;
     const int n3[3] = {i, j, k};
     c0.load(q, rg[0], n3, id, cls);
     c1.load(q, rg[1], n3, id, cls);
@@ -902,9 +1162,9 @@ VG_DEV void h_shell_column(const ShellPiece *pcs, const ShellWork *work, const H
 }
 
 template <typename T, bool IDX, bool CHK = false>
-__global__ __launch_bounds__(256) void k_h_shell(const ShellPiece *pcs, const ShellWork *work, const HArgs<T> *ap)
+__global__ __launch_bounds__(256) void k_h_shell(const ShellDev *pcs, const ShellWork *work, const HArgs<T> *ap)
 {
-  h_shell_column<T, IDX, CHK>(pcs, work, ap, blockIdx.x);
+  h_shell_column<T, IDX, CHK, true>(pcs, work, ap, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1017,7 +1277,7 @@ __global__ void k_debye_gather(long long n, const long long *key, const T *const
 // SIBC: E pass per face (sibc.c:443-586) with FP64 recursive convolution
 // (filter.c:309-327).
 // ---------------------------------------------------------------------------
-template <typename T> __global__ __launch_bounds__(128) void k_sibc_e(SibcEArgs<T> a)
+template <typename T, bool ZERO> __global__ __launch_bounds__(128) void k_sibc_e(SibcEArgs<T> a)
 {
   const SibcBlock w = a.blocks[blockIdx.x];  // one surface per block: s is uniform
   const long long f = w.f0 + threadIdx.x;
@@ -1036,19 +1296,19 @@ template <typename T> __global__ __launch_bounds__(128) void k_sibc_e(SibcEArgs<
   const T *Hx = a.H[0], *Hy = a.H[1], *Hz = a.H[2];
   T *Ex = a.E[0], *Ey = a.E[1], *Ez = a.E[2];
   if (nrm == 0) {
-    Ey[id] = T(0); Ey[id + P] = T(0); Ez[id] = T(0); Ez[id + SJ] = T(0);
+    if (ZERO) { Ey[id] = T(0); Ey[id + P] = T(0); Ez[id] = T(0); Ez[id + SJ] = T(0); }
     Htan[0] = T(0.5 * (1 + A[0] + A[1]) * (double)(Hy[id - 1] + Hy[id - 1 + SJ]));
     Htan[1] = T(0.5 * (1 + B[0] + B[1]) * (double)(Hy[id] + Hy[id + SJ]));
     Htan[2] = T(0.5 * (1 + A[2] + A[3]) * (double)(Hz[id - 1] + Hz[id - 1 + P]));
     Htan[3] = T(0.5 * (1 + B[2] + B[3]) * (double)(Hz[id] + Hz[id + P]));
   } else if (nrm == 1) {
-    Ez[id] = T(0); Ez[id + 1] = T(0); Ex[id] = T(0); Ex[id + P] = T(0);
+    if (ZERO) { Ez[id] = T(0); Ez[id + 1] = T(0); Ex[id] = T(0); Ex[id + P] = T(0); }
     Htan[0] = T(0.5 * (1 + A[0] + A[1]) * (double)(Hz[id - SJ] + Hz[id - SJ + P]));
     Htan[1] = T(0.5 * (1 + B[0] + B[1]) * (double)(Hz[id] + Hz[id + P]));
     Htan[2] = T(0.5 * (1 + A[2] + A[3]) * (double)(Hx[id - SJ] + Hx[id - SJ + 1]));
     Htan[3] = T(0.5 * (1 + B[2] + B[3]) * (double)(Hx[id] + Hx[id + 1]));
   } else {
-    Ex[id] = T(0); Ex[id + SJ] = T(0); Ey[id] = T(0); Ey[id + 1] = T(0);
+    if (ZERO) { Ex[id] = T(0); Ex[id + SJ] = T(0); Ey[id] = T(0); Ey[id + 1] = T(0); }
     Htan[0] = T(0.5 * (1 + A[0] + A[1]) * (double)(Hx[id - P] + Hx[id - P + 1]));
     Htan[1] = T(0.5 * (1 + B[0] + B[1]) * (double)(Hx[id] + Hx[id + 1]));
     Htan[2] = T(0.5 * (1 + A[2] + A[3]) * (double)(Hy[id - P] + Hy[id - P + SJ]));
@@ -1194,103 +1454,6 @@ template <typename T> __global__ void k_sibc_h(SibcHArgs<T> a)
 }
 
 // ---------------------------------------------------------------------------
-// Waveforms (waveform.c:413-638) on the device, in double.
-// ---------------------------------------------------------------------------
-VG_DEV double wf_compact(double pi, double time, double width, double span)
-{
-  if (time <= 0.0) return 0.0;
-  if (time < span * width)
-    return 1.0 / 32.0 * (10.0 - 15.0 * cos(pi / width * time) + 6.0 * cos(2.0 * pi / width * time) -
-                         cos(3.0 * pi / width * time));
-  return span < 1.5 ? 1.0 : 0.0;
-}
-
-VG_DEV double wf_value(const WaveformDev &w, double t, double delay, double pi)
-{
-  const double tt = t - delay - w.delay;
-  const double width = w.width;
-  switch (w.type) {
-  case 0:
-  case 1: return w.size * exp(-0.5 * (pow(tt / width, 2.0)));
-  case 2: return w.size * (-tt / width * exp(-0.5 * (pow(tt / width, 2.0))));
-  case 3: return w.size * ((1.0 - pow(tt / width, 2)) * exp(-0.5 * (pow(tt / width, 2.0))));
-  case 4: return w.size * (exp(-0.5 * (pow(tt / width, 2.0))) * sin(2.0 * pi * w.frequency * tt));
-  case 5: return w.size * wf_compact(pi, tt, width, 2.0);
-  case 6:
-    if (tt <= 0.0 || tt >= 2.0 * width) return 0.0;
-    return w.size * (1.0 / 32.0 * (15.0 * sin(pi / width * tt) - 12.0 * sin(2.0 * pi / width * tt) +
-                                   3.0 * sin(3.0 * pi / width * tt)));
-  case 7: return w.size * (wf_compact(pi, tt, width, 2.0) * sin(2.0 * pi * w.frequency * tt));
-  case 8: return w.size * (wf_compact(pi, tt, width, 1.0) * sin(2.0 * pi * w.frequency * tt));
-  case 9: {
-    const double *T3 = w.table;
-    const unsigned long n = w.n;
-    if (n < 2 || tt < T3[0] || tt > T3[3 * (n - 1)]) return 0.0;
-    unsigned long lo = 0, hi = n - 1;
-    while (hi - lo > 1) {
-      const unsigned long m = (hi + lo) >> 1;
-      if (T3[3 * m] > tt) hi = m;
-      else lo = m;
-    }
-    const double h = T3[3 * hi] - T3[3 * lo];
-    const double aa = (T3[3 * hi] - tt) / h, bb = (tt - T3[3 * lo]) / h;
-    return w.size * (aa * T3[3 * lo + 1] + bb * T3[3 * hi + 1] +
-                     ((aa * aa * aa - aa) * T3[3 * lo + 2] + (bb * bb * bb - bb) * T3[3 * hi + 2]) * (h * h) / 6.0);
-  }
-  default: return 0.0;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 1-D auxiliary grids of the TF/SF plane waves (planewave.c:1315-1372).
-// One block per plane wave; the blocks ride in other launches (k_head for E,
-// the H corrections' k_corr for H), whose own work they do not touch.
-// ---------------------------------------------------------------------------
-template <typename T> VG_DEV void aux_e_block(const AuxArgs<T> &a, int p, double pi)
-{
-  const PwDev &pw = a.pw[p];
-  if (!pw.use_aux) return;
-  T *Eyi = a.aux + (long long)p * 2 * a.auxmax, *Hzi = Eyi + a.auxmax;
-  T *PPy = a.pml + p * 30, *Py = PPy + 10;
-  const T *adx = a.prof + p * 40, *bdx = adx + 10;
-  const T beta = T(pw.beta);
-  for (int i = 1 + threadIdx.x; i < pw.nx; i += blockDim.x) {
-    if (i < pw.xb) {
-      Eyi[i] = Eyi[i] + beta * (Hzi[i - 1] - Hzi[i]);
-    } else {
-      const int L = i - pw.xb;
-      const T oldPP = PPy[L];
-      PPy[L] = PPy[L] + beta * (Hzi[i - 1] - Hzi[i]);
-      const T oldP = Py[L];
-      Py[L] = Py[L] + (PPy[L] - oldPP);
-      Eyi[i] = adx[L] * Eyi[i] + bdx[L] * (Py[L] - oldP);
-    }
-  }
-  const double t = (double)(*a.step + (unsigned long long)a.soff) * a.dt;
-  if (threadIdx.x == 0) Eyi[0] = T(wf_value(a.wf[pw.waveform], t, pw.delay, pi));
-}
-
-template <typename T> VG_DEV void aux_h_block(const AuxArgs<T> &a, int p)
-{
-  const PwDev &pw = a.pw[p];
-  if (!pw.use_aux) return;
-  T *Eyi = a.aux + (long long)p * 2 * a.auxmax, *Hzi = Eyi + a.auxmax;
-  T *Bz = a.pml + p * 30 + 20;
-  const T *ahx = a.prof + p * 40 + 20, *bhx = ahx + 10;
-  const T gamma = T(pw.gamma);
-  for (int i = threadIdx.x; i < pw.nx; i += blockDim.x) {
-    if (i < pw.xb) {
-      Hzi[i] = Hzi[i] + gamma * (Eyi[i] - Eyi[i + 1]);
-    } else {
-      const int L = i - pw.xb;
-      const T oldB = Bz[L];
-      Bz[L] = ahx[L] * Bz[L] + gamma * bhx[L] * (-Eyi[i + 1] + Eyi[i]);
-      Hzi[i] = Hzi[i] + (Bz[L] - oldB);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Sources and TF/SF corrections, one thread per touched cell, entries in
 // reference order (source.c:602-753, planewave.c:576-1007).
 // ---------------------------------------------------------------------------
@@ -1373,29 +1536,41 @@ template <typename T> __global__ void k_corr_aux(CorrArgs<T> a, double pi, AuxAr
 // samples for impulse.dat (observer.c:1164-1198).  One thread per
 // (observer, frequency); thread f==0 also stores the time sample.
 // ---------------------------------------------------------------------------
-template <typename T> VG_DEV void observe_block(const ObsArgs<T> &a, int o)
+// C0..C0+NC-1: the components to take, sampled at step n.
+template <typename T, int C0, int NC>
+VG_DEV void observe_block(const ObsArgs<T> &a, int o, int fb, unsigned long long n)
 {
-  const unsigned long long n = *a.step + (unsigned long long)a.soff;
   if (n < a.first[o] || n > a.last[o]) return;
   const double t = (double)n * a.dt;
   const long long id = a.cell[o];
-  double v[6];
-  for (int c = 0; c < 6; ++c) v[c] = (double)a.F[c][id];
-  const int f = blockIdx.x * blockDim.x + threadIdx.x;
+  double v[NC];
+  for (int c = 0; c < NC; ++c) v[c] = (double)a.F[C0 + c][id];
+  const int f = fb * (int)blockDim.x + (int)threadIdx.x;
   if (f == 0) {
-    double *td = a.td + ((long long)o * a.tdsteps + (n - a.first[o])) * 6;
-    for (int c = 0; c < 6; ++c) td[c] = v[c];
+    double *td = a.td + ((long long)o * a.tdsteps + (n - a.first[o])) * 6 + C0;
+    for (int c = 0; c < NC; ++c) td[c] = v[c];
   }
   const int nf = a.nfreq[o];
   if (f >= nf) return;
   const double ot = a.omega[a.dftoff[o] / 6 + f] * t;
   double si, co;
   sincos(ot, &si, &co);
-  double *re = a.dre + a.dftoff[o], *im = a.dim + a.dftoff[o];
-  for (int c = 0; c < 6; ++c) {
+  double *re = a.dre + a.dftoff[o] + C0 * nf, *im = a.dim + a.dftoff[o] + C0 * nf;
+  for (int c = 0; c < NC; ++c) {
     re[c * nf + f] += v[c] * co;
     im[c * nf + f] -= v[c] * si;
   }
+}
+
+// Values of a half-step's sources and analytic plane waves (XVal).
+template <typename T> VG_DEV void value_block(const ValArgs<T> &a, unsigned long long n, double dt, double pi, int b)
+{
+  const long long q = b * (long long)blockDim.x + threadIdx.x;
+  if (q >= a.n) return;
+  const XVal v = a.v[q];
+  const double t = ((double)n + a.half) * dt;
+  if (v.wave) a.out[q] = T(v.scale) * T(wf_value(a.wf[v.wf], t - v.geo, v.delay, pi));
+  else a.out[q] = T(v.scale * wf_value(a.wf[v.wf], t, v.delay, pi));
 }
 
 // Head of a step: the observers sample the fields (blocks y < nobs) and each
@@ -1405,8 +1580,9 @@ template <typename T> VG_DEV void observe_block(const ObsArgs<T> &a, int o)
 // (planewave.c:576-590 runs it just before the E corrections).
 template <typename T> VG_DEV void head_block(const ObsArgs<T> &oa, const AuxArgs<T> &xa, double pi, int y)
 {
-  if (y < oa.nobs) observe_block(oa, y);
-  else if (blockIdx.x == 0) aux_e_block(xa, y - oa.nobs, pi);
+  if (y < oa.nobs) observe_block<T, 0, 6>(oa, y, (int)blockIdx.x, *oa.step + (unsigned long long)oa.soff);
+  else if (blockIdx.x == 0)
+    aux_e_block(xa, y - oa.nobs, (double)(*xa.step + (unsigned long long)xa.soff) * xa.dt, pi);
 }
 
 template <typename T> __global__ void k_head(ObsArgs<T> oa, AuxArgs<T> xa, double pi)
@@ -1414,20 +1590,75 @@ template <typename T> __global__ void k_head(ObsArgs<T> oa, AuxArgs<T> xa, doubl
   head_block(oa, xa, pi, (int)blockIdx.y);
 }
 
-template <typename T> VG_DEV void observe_volume_node(const VolObsArgs<T> &a, long long nd)
+template <typename T, int C0, int NC>
+VG_DEV void observe_volume_node(const VolObsArgs<T> &a, long long nd, unsigned long long n)
 {
   if (nd >= a.nnodes) return;
   const int o = a.nodeobs[nd];
-  const unsigned long long n = *a.step + (unsigned long long)a.soff;
   if (n < a.first[o] || n > a.last[o]) return;
   const long long id = a.nodecell[nd];
-  float *out = a.stage + ((long long)(n % a.ring) * a.nnodes + nd) * 6;
-  for (int c = 0; c < 6; ++c) out[c] = (float)a.F[c][id];
+  float *out = a.stage + ((long long)(n % a.ring) * a.nnodes + nd) * 6 + C0;
+  for (int c = 0; c < NC; ++c) out[c] = (float)a.F[C0 + c][id];
 }
 
 template <typename T> __global__ void k_observe_volume(VolObsArgs<T> a)
 {
-  observe_volume_node(a, blockIdx.x * (long long)blockDim.x + threadIdx.x);
+  observe_volume_node<T, 0, 6>(a, blockIdx.x * (long long)blockDim.x + threadIdx.x,
+                               *a.step + (unsigned long long)a.soff);
+}
+
+// Samples of a half's components at step n: blocks b < a.b[1] of the side.
+template <typename T, int C0> VG_DEV void sample_block(const SideArgs<T> &a, int b, unsigned long long n)
+{
+  if (b < a.b[0]) observe_block<T, C0, 3>(a.o, b / a.nfb, b % a.nfb, n);
+  else observe_volume_node<T, C0, 3>(a.v, (b - a.b[0]) * 256ll + threadIdx.x, n);
+}
+
+// A side block of step `soff` of the run.
+template <typename T, bool ELEC>
+VG_DEV void side_block(const SideArgs<T> &a, int b, int soff, bool last, double pi)
+{
+  const unsigned long long n = *a.o.step + (unsigned long long)soff;
+  if (b < a.b[1]) {
+    if (ELEC) sample_block<T, 3>(a, b, n);
+    else if (!last) sample_block<T, 0>(a, b, n + 1);
+  } else if (b < a.b[2]) {
+    if (ELEC) aux_e_block(a.x, b - a.b[1], (double)n * a.x.dt, pi);
+    else aux_h_block(a.x, b - a.b[1]);
+  } else if (b < a.b[3]) {
+    value_block(a.val, n, a.o.dt, pi, b - a.b[2]);
+  }
+}
+
+// The E samples of a run's first step.
+template <typename T> __global__ __launch_bounds__(256) void k_first_samples(SideArgs<T> a)
+{
+  sample_block<T, 0>(a, (int)blockIdx.x, *a.o.step);
+}
+
+// A half-step's sweep: the side blocks, the shell's (each a multiple of eight,
+// so that what follows keeps its XCD order), then the fast tiles, unless those
+// have a launch of their own.
+template <typename T, bool IDX, int X>
+__global__ __launch_bounds__(256) void k_e_sweep(FastE<T> f, const ShellDev *pcs, const ShellWork *work,
+                                                 const EArgs<T> *ap, const XArgs<T> *x, unsigned nSide, unsigned nShell,
+                                                 SideArgs<T> sd, int soff, int last, double pi)
+{
+  const unsigned b = blockIdx.x, n1 = nSide + nShell;
+  if (b < nSide) side_block<T, true>(sd, (int)b, soff, last, pi);
+  else if (b < n1) e_shell_column<T, IDX, X, false, false>(pcs, work, ap, cp(x), b - nSide);
+  else e_fast_tile<T, IDX, X, false>(f, cp(x), xcd_block(b - n1, gridDim.x - n1));
+}
+
+template <typename T, bool IDX>
+__global__ __launch_bounds__(256) void k_h_sweep(FastH<T> f, const ShellDev *pcs, const ShellWork *work,
+                                                 const HArgs<T> *ap, unsigned nSide, unsigned nShell, SideArgs<T> sd,
+                                                 int soff, int last, double pi)
+{
+  const unsigned b = blockIdx.x, n1 = nSide + nShell;
+  if (b < nSide) side_block<T, false>(sd, (int)b, soff, last, pi);
+  else if (b < n1) h_shell_column<T, IDX, false, false>(pcs, work, ap, b - nSide);
+  else h_fast_tile<T, IDX, false>(f, xcd_block(b - n1, gridDim.x - n1));
 }
 
 // Ghost plane copy for one face (surface.c:569-812).
@@ -1479,83 +1710,48 @@ template <typename S> VG_DEV S ld_args(const VG_CONST S *p)
   return out;
 }
 
-template <typename T, bool IDX> __global__ __launch_bounds__(512) void k_e_fast_pk(PackMap m)
-{
-  const int d = pack_member(m, blockIdx.x);
-  const FastE<T> f = ld_args(&pack_args<T>(m, d)->fe);
-  e_fast_tile<T, IDX, false, false>(f, xcd_block(blockIdx.x - m.start[d], m.start[d + 1] - m.start[d]));
-}
-
-template <typename T, bool IDX> __global__ __launch_bounds__(512) void k_h_fast_pk(PackMap m)
-{
-  const int d = pack_member(m, blockIdx.x);
-  const FastH<T> f = ld_args(&pack_args<T>(m, d)->fh);
-  h_fast_tile<T, IDX, false>(f, xcd_block(blockIdx.x - m.start[d], m.start[d + 1] - m.start[d]));
-}
-
-template <typename T, bool IDX> __global__ __launch_bounds__(256) void k_e_shell_pk(PackMap m)
+template <typename T, bool IDX, int X> __global__ __launch_bounds__(256) void k_e_sweep_pk(PackMap m, double pi)
 {
   const int d = pack_member(m, blockIdx.x);
   const VG_CONST PackArgs<T> *a = pack_args<T>(m, d);
-  e_shell_column<T, IDX, false, false>(a->epc, a->ewk, a->ea, blockIdx.x - m.start[d]);
+  const unsigned b = blockIdx.x - m.start[d], nSide = a->nEside, n1 = nSide + a->nEshell;
+  if (b < nSide) {
+    side_block<T, true>(ld_args(&a->se), (int)b, m.soff, m.last, pi);
+  } else if (b < n1) {
+    e_shell_column<T, IDX, X, false, false>(a->epc, a->ewk, a->ea, cp(a->xe), b - nSide);
+  } else {
+    const FastE<T> f = ld_args(&a->fe);
+    e_fast_tile<T, IDX, X, false>(f, cp(a->xe), xcd_block(b - n1, m.start[d + 1] - m.start[d] - n1));
+  }
 }
 
-template <typename T, bool IDX> __global__ __launch_bounds__(256) void k_h_shell_pk(PackMap m)
+template <typename T, bool IDX> __global__ __launch_bounds__(256) void k_h_sweep_pk(PackMap m, double pi)
 {
   const int d = pack_member(m, blockIdx.x);
   const VG_CONST PackArgs<T> *a = pack_args<T>(m, d);
-  h_shell_column<T, IDX, false>(a->hpc, a->hwk, a->ha, blockIdx.x - m.start[d]);
+  const unsigned b = blockIdx.x - m.start[d], nSide = a->nHside, n1 = nSide + a->nHshell;
+  if (b < nSide) {
+    side_block<T, false>(ld_args(&a->sh), (int)b, m.soff, m.last, pi);
+  } else if (b < n1) {
+    h_shell_column<T, IDX, false, false>(a->hpc, a->hwk, a->ha, b - nSide);
+  } else {
+    const FastH<T> f = ld_args(&a->fh);
+    h_fast_tile<T, IDX, false>(f, xcd_block(b - n1, m.start[d + 1] - m.start[d] - n1));
+  }
 }
 
-// The Debye and correction kernels pick a component's array by an index read
-// from memory; from a copy in registers that would be an indexed read of
-// scratch, so they read their argument blocks in place.
-template <typename T> VG_DEV const PackArgs<T> &pack_ref(const PackMap &m, int d)
-{
-  return *static_cast<const PackArgs<T> *>(m.args[d]);
-}
-
-template <typename T> __global__ void k_debye_pk(PackMap m)
-{
-  const int d = pack_member(m, blockIdx.x);
-  debye_layer_site(pack_ref<T>(m, d).da, m.base[d], m.cnt[d],
-                   (blockIdx.x - m.start[d]) * (long long)blockDim.x + threadIdx.x);
-}
-
-template <typename T> __global__ void k_corr_e_pk(PackMap m, double pi)
+template <typename T> __global__ __launch_bounds__(256) void k_first_samples_pk(PackMap m)
 {
   const int d = pack_member(m, blockIdx.x);
-  corr_rows(pack_ref<T>(m, d).ce, pi, (blockIdx.x - m.start[d]) * (long long)blockDim.x + threadIdx.x, m.soff);
+  const SideArgs<T> a = ld_args(&pack_args<T>(m, d)->sh);
+  sample_block<T, 0>(a, (int)(blockIdx.x - m.start[d]), *a.o.step);
 }
 
-// H corrections, and the aux grids' H update in each solve's blocks from
-// cnt[d] on (none when the solve has no aux grid).
-template <typename T> __global__ void k_corr_h_pk(PackMap m, double pi)
+template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) void k_rows_pk(PackMap m)
 {
   const int d = pack_member(m, blockIdx.x);
-  const PackArgs<T> &p = pack_ref<T>(m, d);
-  corr_aux_block(p.ch, pi, p.xa, (int)m.cnt[d], (int)(blockIdx.x - m.start[d]), m.soff);
-}
-
-// Head of a step: block rows are the solves' own k_head rows; x blocks past
-// a solve's own launch width return.
-template <typename T> __global__ void k_head_pk(PackMap m, double pi)
-{
-  const int d = pack_member(m, blockIdx.y);
-  const VG_CONST PackArgs<T> *p = pack_args<T>(m, d);
-  if ((int)blockIdx.x >= p->headGx) return;
-  ObsArgs<T> oa = ld_args(&p->oa);
-  AuxArgs<T> xa = ld_args(&p->xa);
-  oa.soff = xa.soff = m.soff;
-  head_block(oa, xa, pi, (int)(blockIdx.y - m.start[d]));
-}
-
-template <typename T> __global__ void k_observe_volume_pk(PackMap m)
-{
-  const int d = pack_member(m, blockIdx.x);
-  VolObsArgs<T> a = ld_args(&pack_args<T>(m, d)->va);
-  a.soff = m.soff;
-  observe_volume_node(a, (blockIdx.x - m.start[d]) * (long long)blockDim.x + threadIdx.x);
+  const VG_CONST PackArgs<T> *a = pack_args<T>(m, d);
+  x_rows<T, IDX, ELEC>(cp(ELEC ? a->xe : a->xh), blockIdx.x - m.start[d]);
 }
 
 // Device step counter: set before a run that does not continue the previous

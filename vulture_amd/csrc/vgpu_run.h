@@ -64,15 +64,8 @@ template <typename T> static void fill_volume_args(Ctx *c, EArgs<T> &ea, HArgs<T
     ha.bh[d] = P<T>(c->prof[3][d]);
     ha.ibd[d] = P<T>(c->prof[4][d]);
   }
-  ea.ecls = P<uint16_t>(c->d_ecls); ea.etab = P<T>(c->d_etab); ea.edslot = P<int>(c->d_edslot);
+  ea.ecls = P<uint16_t>(c->d_ecls); ea.etab = P<T>(c->d_etab);
   ha.hcls = P<uint16_t>(c->d_hcls); ha.htab = P<T>(c->d_htab);
-  ea.dfuse = c->debyeFused ? 1 : 0;
-  if (c->debyeFused) {
-    ea.dbase = P<int>(c->d_dbase);
-    ea.dlast = P<T>(c->d_dlast); ea.dJ = P<T>(c->d_dJ); ea.dstride = c->debyeSites;
-    ea.dalpha = P<double>(c->d_dalpha); ea.dbeta = P<double>(c->d_dbeta); ea.dnp = P<int>(c->d_dnp);
-    ea.dmaxP = c->debyeMaxPoles; ea.dcplx = c->debyeCplx;
-  }
   ea.pmlmask = ha.pmlmask = c->pmlmask;
   for (int r = 0; r < 6; ++r)
     for (int d = 0; d < 3; ++d) {
@@ -310,12 +303,40 @@ static int build_shell(const A &a, const int (*in)[NB][6], const int *fb, const 
   return 0;
 }
 
+// Pieces as the kernels read them; pool: the pool holding their auxiliaries.
+template <typename T> static std::vector<ShellDev> shell_dev(const std::vector<ShellPiece> &pcs, const T *pool)
+{
+  std::vector<ShellDev> out;
+  for (const ShellPiece &p : pcs) {
+    ShellDev d{};
+    d.x0 = p.box[0]; d.y0 = p.box[2]; d.z0 = p.box[4];
+    d.ni = p.ni; d.nip = p.nip; d.xo = p.xo; d.nxy = p.nxy; d.nxyb = p.nxyb; d.kc = p.kc; d.nk = p.nk;
+    for (int C = 0; C < 3; ++C)
+      for (int r = 0; r < SHELL_RUNS; ++r) {
+        ShellDevRun &o = d.run[C][r];
+        o.xa = 1;
+        if (r >= p.nrun[C]) continue;
+        const ShellRun &n = p.run[C][r];
+        o.xa = n.xa; o.xb = n.xb; o.reg = n.reg;
+        if (n.reg < 6) {
+          // the pools hold at most 2^31 elements (vgpu_set_pml)
+          o.q0 = (int)(static_cast<const T *>(n.a) - pool + n.p0 - n.xa);
+          o.psy = (int)n.psy;
+          o.psz = (int)n.psz;
+        }
+      }
+    out.push_back(d);
+  }
+  return out;
+}
+
 // The E and H shells of a context (build_shell); kcPlan > 0 fixes the planes
 // per block.
 template <typename T>
-static int plan_shells(Ctx *c, int kcPlan, std::vector<ShellPiece> &ep, std::vector<ShellWork> &ew,
-                       std::vector<ShellPiece> &hp, std::vector<ShellWork> &hw, long long cells[2], std::string &err)
+static int plan_shells(Ctx *c, int kcPlan, std::vector<ShellDev> &ep, std::vector<ShellWork> &ew,
+                       std::vector<ShellDev> &hp, std::vector<ShellWork> &hw, long long cells[2], std::string &err)
 {
+  std::vector<ShellPiece> pe, ph;
   EArgs<T> ea{};
   HArgs<T> ha{};
   fill_volume_args<T>(c, ea, ha, 0);
@@ -324,12 +345,47 @@ static int plan_shells(Ctx *c, int kcPlan, std::vector<ShellPiece> &ep, std::vec
   for (int C = 0; C < 3; ++C)
     for (int q = 0; q < 6; ++q) ein[C][0][q] = ea.in[C][q];
   const int lw = getenv("VGPU_SHELL_ROWS") && getenv("VGPU_SHELL_ROWS")[0] == '0' ? 0 : (int)(128 / sizeof(T));
-  return build_shell<1>(ea, ein, c->fastE, N, ep, ew, cells[0], err, lw, kcPlan) ||
-         build_shell<3>(ha, ha.in, c->fastH, N, hp, hw, cells[1], err, lw, kcPlan);
+  if (build_shell<1>(ea, ein, c->fastE, N, pe, ew, cells[0], err, lw, kcPlan) ||
+      build_shell<3>(ha, ha.in, c->fastH, N, ph, hw, cells[1], err, lw, kcPlan))
+    return -1;
+  ep = shell_dev<T>(pe, ea.PPpool);
+  hp = shell_dev<T>(ph, ha.Bpool);
+  return 0;
+}
+
+// Argument block of the corrections of half-step e.
+template <typename T> static void fill_correction_args(Ctx *c, XArgs<T> &x, int e)
+{
+  x.cls = P<uint16_t>(c->indexed ? (e == 0 ? c->d_ecls : c->d_hcls) : c->d_xcls);
+  x.PX = c->PX; x.plane = c->plane;
+  x.nrow = c->nXrow[e]; x.ngroup = c->nXgroup[e];
+  x.gstart = P<int>(c->d_xgstart[e]); x.row = P<XRow>(c->d_xrow[e]); x.op = P<XOp<T>>(c->d_xop[e]);
+  for (int d = 0; d < 3; ++d) {
+    x.F[d] = P<T>(c->fld(0, 3 * e + d));
+    x.ca[d] = P<T>(e == 0 ? c->alpha[d] : nullptr);
+    x.cb[d] = P<T>(e == 0 ? c->beta[d] : c->gamma[d]);
+  }
+  x.tab = P<T>(e == 0 ? c->d_etab : c->d_htab);
+  x.val = P<T>(c->d_xvals[e]);
+  x.aux = P<T>(c->d_aux); x.auxmax = c->auxmax; x.pw = P<PwDev>(c->d_pw); x.eta0 = T(c->grid.eta0);
+  x.Etan = P<T>(c->d_setan);
+  x.flag0 = ~0u;
+  if (e) return;
+  x.flag0 = c->xflag0;
+  x.dtab = P<T>(c->d_xdtab); x.J = P<T>(c->d_xJ); x.nJ = (long long)c->ncell;
+  x.murmask = c->murPush ? c->murmask : 0u;
+  for (int f = 0; f < 6; ++f) {
+    x.mzeta[f] = T(c->zeta[f]);
+    for (int C = 0; C < 3; ++C)
+      for (int q = 0; q < 6; ++q) x.mbox[f][C][q] = c->fmlim[f][C][q];
+  }
+  x.dlast = P<T>(c->d_dlast); x.dJ = P<T>(c->d_dJ); x.dstride = c->debyeSites;
+  x.dalpha = P<double>(c->d_dalpha); x.dbeta = P<double>(c->d_dbeta); x.dnp = P<int>(c->d_dnp);
+  x.dmaxP = c->debyeMaxPoles; x.dcplx = c->debyeCplx;
 }
 
 // Once per context (at finalize): the sweeps' argument blocks go to device
-// memory, where the shell kernels and the fused Debye step read them.
+// memory, where the shell kernels and the corrections read them.
 template <typename T> int prepare_sweeps(Ctx *c)
 {
   for (int e = 0; e < 2; ++e) {
@@ -342,7 +398,7 @@ template <typename T> int prepare_sweeps(Ctx *c)
   HArgs<T> ha{}, ha1{};
   fill_volume_args<T>(c, ea, ha, 0);
   fill_volume_args<T>(c, ea1, ha1, 1);
-  std::vector<ShellPiece> ep, hp;
+  std::vector<ShellDev> ep, hp;
   std::vector<ShellWork> ew, hw;
   std::string err;
   if (plan_shells<T>(c, 0, ep, ew, hp, hw, c->shellCells, err)) return set_error(c, VGPU_EINVAL, "%s", err.c_str());
@@ -352,8 +408,8 @@ template <typename T> int prepare_sweeps(Ctx *c)
     c->d_eargs[q] = dev_alloc(c, sizeof(ea));
     c->d_hargs[q] = dev_alloc(c, sizeof(ha));
   }
-  c->d_epcs = dev_alloc(c, ep.size() * sizeof(ShellPiece));
-  c->d_hpcs = dev_alloc(c, hp.size() * sizeof(ShellPiece));
+  c->d_epcs = dev_alloc(c, ep.size() * sizeof(ShellDev));
+  c->d_hpcs = dev_alloc(c, hp.size() * sizeof(ShellDev));
   c->d_ework = dev_alloc(c, ew.size() * sizeof(ShellWork));
   c->d_hwork = dev_alloc(c, hw.size() * sizeof(ShellWork));
   if (!c->d_eargs[0] || !c->d_hargs[0] || !c->d_eargs[1] || !c->d_hargs[1] || !c->d_epcs || !c->d_hpcs ||
@@ -362,11 +418,21 @@ template <typename T> int prepare_sweeps(Ctx *c)
   auto up = [](void *d, const void *h, size_t n) { return n == 0 || hipMemcpy(d, h, n, hipMemcpyHostToDevice) == hipSuccess; };
   if (!up(c->d_eargs[0], &ea, sizeof(ea)) || !up(c->d_hargs[0], &ha, sizeof(ha)) ||
       !up(c->d_eargs[1], &ea1, sizeof(ea1)) || !up(c->d_hargs[1], &ha1, sizeof(ha1)) ||
-      !up(c->d_epcs, ep.data(), ep.size() * sizeof(ShellPiece)) ||
-      !up(c->d_hpcs, hp.data(), hp.size() * sizeof(ShellPiece)) ||
+      !up(c->d_epcs, ep.data(), ep.size() * sizeof(ShellDev)) ||
+      !up(c->d_hpcs, hp.data(), hp.size() * sizeof(ShellDev)) ||
       !up(c->d_ework, ew.data(), ew.size() * sizeof(ShellWork)) ||
       !up(c->d_hwork, hw.data(), hw.size() * sizeof(ShellWork)))
     return set_error(c, VGPU_EDEVICE, "sweep arguments upload");
+  if (c->inl) {
+    for (int e = 0; e < 2; ++e) {
+      XArgs<T> x{};
+      fill_correction_args<T>(c, x, e);
+      c->d_xargs[e] = dev_alloc(c, sizeof(x));
+      if (!c->d_xargs[e]) return set_error(c, VGPU_ENOMEM, "corrections");
+      if (!up(c->d_xargs[e], &x, sizeof(x))) return set_error(c, VGPU_EDEVICE, "corrections upload");
+    }
+    return VGPU_OK;
+  }
   // Debye sites, correction rows and SIBC H rows: each one's coefficients, gathered once
   if (c->debyeSites) {
     const T *b[3] = {P<T>(c->beta[0]), P<T>(c->beta[1]), P<T>(c->beta[2])};
@@ -422,7 +488,7 @@ template <typename T> struct StepArgs {
   FastH<T> fh[2];
   const EArgs<T> *eap[2];              // argument blocks in device memory (shells)
   const HArgs<T> *hap[2];
-  const ShellPiece *epc, *hpc;
+  const ShellDev *epc, *hpc;
   const ShellWork *ewk, *hwk;
   LeapArgs<T> la[2];
   FixArgs<T> fx[2];
@@ -437,6 +503,8 @@ template <typename T> struct StepArgs {
   bool anyAux;
   ObsArgs<T> oa[2];
   int maxnf;
+  SideArgs<T> side[2];                 // what rides with the E and H sweeps
+  unsigned nside[2];                   // their blocks
   VolObsArgs<T> va[2];
   unsigned long long *stepp;           // device step counter
 };
@@ -453,7 +521,7 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   // rows per block (tuning override VGPU_FAST_TY: 1..8)
   int ty = 4;
   if (const char *ev = getenv("VGPU_FAST_TY")) ty = std::max(1, std::min(atoi(ev), 8));
-  A.vblk = dim3(64, ty, 1);
+  A.vblk = dim3(64 * ty);
   auto fast_grid = [&](const int *fb, int &kchunk) {
     if (fb[0] > fb[1] || fb[2] > fb[3] || fb[4] > fb[5]) return dim3(0, 0, 0);
     const int gx = (fb[1] - fb[0] + 64) / 64, gy = (fb[3] - fb[2] + ty) / ty, nz = fb[5] - fb[4] + 1;
@@ -485,7 +553,7 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
       h.H[d] = ha[q].H[d]; h.Hin[d] = ha[q].Hin[d]; h.E[d] = ha[q].E[d]; h.ide[d] = ha[q].ide[d];
       h.gamma[d] = ha[q].gamma[d];
     }
-    e.ecls = ea[q].ecls; e.etab = ea[q].etab; e.dfuse = ea[q].dfuse; e.ap = P<EArgs<T>>(c->d_eargs[q]);
+    e.ecls = ea[q].ecls; e.etab = ea[q].etab;
     h.hcls = ha[q].hcls; h.htab = ha[q].htab;
     if (chk)
       for (int d = 0; d < 3; ++d) { e.vis[d] = chk->vis[d]; h.vis[d] = chk->vis[3 + d]; }
@@ -496,8 +564,8 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
     eap[q] = P<EArgs<T>>(chk ? chk->eargs : c->d_eargs[q]);
     hap[q] = P<HArgs<T>>(chk ? chk->hargs : c->d_hargs[q]);
   }
-  A.epc = P<ShellPiece>(c->d_epcs);
-  A.hpc = P<ShellPiece>(c->d_hpcs);
+  A.epc = P<ShellDev>(c->d_epcs);
+  A.hpc = P<ShellDev>(c->d_hpcs);
   A.ewk = P<ShellWork>(c->d_ework);
   A.hwk = P<ShellWork>(c->d_hwork);
   // fused leapfrog sweep: 4 waves of R rows per block, 63-cell x tiles, kz-plane z chunks
@@ -677,6 +745,21 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
     for (int e = 0; e < 2; ++e) { ce[q][e].step = stepp; ce[q][e].dt = dt; ce[q][e].half = e == 0 ? 0.0 : 0.5; }
   }
   xa.step = stepp; xa.dt = dt;
+  for (int e = 0; e < 2; ++e) {
+    SideArgs<T> &d = A.side[e];
+    d.o = oa[0];
+    d.v = va[0];
+    d.x = xa;
+    d.val.n = c->nXval[e]; d.val.v = P<XVal>(c->d_xval[e]); d.val.out = P<T>(c->d_xvals[e]);
+    d.val.wf = P<WaveformDev>(c->d_wf); d.val.half = e == 0 ? 0.0 : 0.5;
+    d.electric = e == 0;
+    d.nfb = (maxnf + 255) / 256;
+    d.b[0] = d.o.nobs * d.nfb;
+    d.b[1] = d.b[0] + (int)((d.v.nnodes + 255) / 256);
+    d.b[2] = d.b[1] + (anyAux ? xa.npw : 0);
+    d.b[3] = d.b[2] + (int)((d.val.n + 255) / 256);
+    A.nside[e] = (unsigned)(d.b[3] + 7) / 8 * 8;
+  }
 }
 
 // Ghost planes of one half-step (surface.c:569-812), copied within the field
@@ -709,6 +792,16 @@ template <typename T> void launch_ghosts(Ctx *c, int electric, int q, hipStream_
   }
 }
 
+// Whether a context's fast tiles have launches of their own.  In one launch
+// the tiles share the shell's register count (FP32 E 104 and H 62 VGPRs
+// against 62 and 53 alone), but its blocks fill the device together with
+// theirs and one launch fewer is on the step's critical path: 48.6 -> 39.8 us
+// a step on a 53x41x62 request, 82 -> 71 on 101x115x108, 298 -> 283 on the
+// FP64 200x160x120 enclosure, 377 -> 368 on the 256x256x160 box.  Where the
+// fields are past the 256 MB last-level cache the tiles' own occupancy counts
+// for more: 537 against 529 us at 272^3 in FP32 (85 MB a field).
+static bool sweeps_apart(const Ctx *c) { return c->ncell * c->esz > ((size_t)64 << 20); }
+
 // The loop (simulation.c:136-230).  With chk, one step of the field sweeps
 // only (Mur E, the E sweep, the H sweep), in their update-counting form.
 // With the fused sweep, step q of the run reads field set c->par ^ (q & 1)
@@ -725,50 +818,77 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   const dim3 egrid = A.egrid, hgrid = A.hgrid, eg1 = A.eg1, hg1 = A.hg1, vblk = A.vblk;
   const auto &eap = A.eap;
   const auto &hap = A.hap;
-  const ShellPiece *epc = A.epc, *hpc = A.hpc;
+  const ShellDev *epc = A.epc, *hpc = A.hpc;
   const ShellWork *ewk = A.ewk, *hwk = A.hwk;
+  const XArgs<T> *xe = P<XArgs<T>>(c->d_xargs[0]), *xh = P<XArgs<T>>(c->d_xargs[1]);
+  const unsigned nHshell = (unsigned)c->nHwork;
   auto fast_e = [&](int q) {
     const FastE<T> &f = fe[q];
-    if (egrid.x && chk) {
-      if (c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, false, true>), eg1, vblk, 0, s, f);
-      else hipLaunchKernelGGL((k_e_fast<T, false, false, true>), eg1, vblk, 0, s, f);
-    } else if (egrid.x) {
-      if (c->indexed && c->debyeFused) hipLaunchKernelGGL((k_e_fast<T, true, true>), eg1, vblk, 0, s, f);
-      else if (c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, false>), eg1, vblk, 0, s, f);
-      else hipLaunchKernelGGL((k_e_fast<T, false, false>), eg1, vblk, 0, s, f);
-    }
+    if (!egrid.x) return;
+    const int x = c->xlevel();
+    if (chk && c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 0, true>), eg1, vblk, 0, s, f, xe);
+    else if (chk) hipLaunchKernelGGL((k_e_fast<T, false, 0, true>), eg1, vblk, 0, s, f, xe);
+    else if (c->indexed && x == 2) hipLaunchKernelGGL((k_e_fast<T, true, 2>), eg1, vblk, 0, s, f, xe);
+    else if (c->indexed && x == 1) hipLaunchKernelGGL((k_e_fast<T, true, 1>), eg1, vblk, 0, s, f, xe);
+    else if (c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 0>), eg1, vblk, 0, s, f, xe);
+    else if (x) hipLaunchKernelGGL((k_e_fast<T, false, 1>), eg1, vblk, 0, s, f, xe);
+    else hipLaunchKernelGGL((k_e_fast<T, false, 0>), eg1, vblk, 0, s, f, xe);
   };
   auto shell_e = [&](int q) {
-    if (c->nEwork) {
-      const dim3 g((unsigned)c->nEwork);
-      const EArgs<T> *a = eap[q];
-      if (chk && c->indexed) hipLaunchKernelGGL((k_e_shell<T, true, true>), g, dim3(256), 0, s, epc, ewk, a);
-      else if (chk) hipLaunchKernelGGL((k_e_shell<T, false, true>), g, dim3(256), 0, s, epc, ewk, a);
-      else if (c->indexed && !c->leap) hipLaunchKernelGGL((k_e_shell<T, true, false, false>), g, dim3(256), 0, s, epc, ewk, a);
-      else if (c->indexed) hipLaunchKernelGGL((k_e_shell<T, true>), g, dim3(256), 0, s, epc, ewk, a);
-      else if (!c->leap) hipLaunchKernelGGL((k_e_shell<T, false, false, false>), g, dim3(256), 0, s, epc, ewk, a);
-      else hipLaunchKernelGGL((k_e_shell<T, false>), g, dim3(256), 0, s, epc, ewk, a);
-    }
+    const EArgs<T> *a = eap[q];
+    const dim3 b(256), g((unsigned)c->nEwork);
+    if (!g.x) return;
+    if (chk && c->indexed) hipLaunchKernelGGL((k_e_shell<T, true, true>), g, b, 0, s, epc, ewk, a);
+    else if (chk) hipLaunchKernelGGL((k_e_shell<T, false, true>), g, b, 0, s, epc, ewk, a);
+    else if (c->indexed) hipLaunchKernelGGL((k_e_shell<T, true>), g, b, 0, s, epc, ewk, a);
+    else hipLaunchKernelGGL((k_e_shell<T, false>), g, b, 0, s, epc, ewk, a);
   };
   auto fast_h = [&](int q) {
     const FastH<T> &f = fh[q];
-    if (hgrid.x && chk) {
-      if (c->indexed) hipLaunchKernelGGL((k_h_fast<T, true, true>), hg1, vblk, 0, s, f);
-      else hipLaunchKernelGGL((k_h_fast<T, false, true>), hg1, vblk, 0, s, f);
-    } else if (hgrid.x) {
-      if (c->indexed) hipLaunchKernelGGL((k_h_fast<T, true>), hg1, vblk, 0, s, f);
-      else hipLaunchKernelGGL((k_h_fast<T, false>), hg1, vblk, 0, s, f);
-    }
+    if (!hgrid.x) return;
+    if (chk && c->indexed) hipLaunchKernelGGL((k_h_fast<T, true, true>), hg1, vblk, 0, s, f);
+    else if (chk) hipLaunchKernelGGL((k_h_fast<T, false, true>), hg1, vblk, 0, s, f);
+    else if (c->indexed) hipLaunchKernelGGL((k_h_fast<T, true>), hg1, vblk, 0, s, f);
+    else hipLaunchKernelGGL((k_h_fast<T, false>), hg1, vblk, 0, s, f);
   };
   auto shell_h = [&](int q) {
-    if (c->nHwork) {
-      const dim3 g((unsigned)c->nHwork);
-      const HArgs<T> *a = hap[q];
-      if (chk && c->indexed) hipLaunchKernelGGL((k_h_shell<T, true, true>), g, dim3(256), 0, s, hpc, hwk, a);
-      else if (chk) hipLaunchKernelGGL((k_h_shell<T, false, true>), g, dim3(256), 0, s, hpc, hwk, a);
-      else if (c->indexed) hipLaunchKernelGGL((k_h_shell<T, true>), g, dim3(256), 0, s, hpc, hwk, a);
-      else hipLaunchKernelGGL((k_h_shell<T, false>), g, dim3(256), 0, s, hpc, hwk, a);
-    }
+    const HArgs<T> *a = hap[q];
+    const dim3 b(256), g((unsigned)c->nHwork);
+    if (!g.x) return;
+    if (chk && c->indexed) hipLaunchKernelGGL((k_h_shell<T, true, true>), g, b, 0, s, hpc, hwk, a);
+    else if (chk) hipLaunchKernelGGL((k_h_shell<T, false, true>), g, b, 0, s, hpc, hwk, a);
+    else if (c->indexed) hipLaunchKernelGGL((k_h_shell<T, true>), g, b, 0, s, hpc, hwk, a);
+    else hipLaunchKernelGGL((k_h_shell<T, false>), g, b, 0, s, hpc, hwk, a);
+  };
+  // A half-step's sweep in one launch (side blocks, shell, fast tiles), or
+  // with `apart` without the fast tiles.
+  const bool apart = sweeps_apart(c);
+  auto sweep_e = [&](int soff, int last) {
+    const unsigned ns = A.nside[0], nw = (unsigned)c->nEwork;
+    const dim3 b(256), g(ns + nw + (apart ? 0u : eg1.x));
+    if (!g.x) return;
+    const int x = c->xlevel();
+    const FastE<T> &f = fe[0];
+    const SideArgs<T> &sd = A.side[0];
+    if (c->indexed && x == 2) hipLaunchKernelGGL((k_e_sweep<T, true, 2>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
+    else if (c->indexed && x == 1) hipLaunchKernelGGL((k_e_sweep<T, true, 1>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
+    else if (c->indexed) hipLaunchKernelGGL((k_e_sweep<T, true, 0>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
+    else hipLaunchKernelGGL((k_e_sweep<T, false, 1>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
+  };
+  auto sweep_h = [&](int soff, int last) {
+    const unsigned ns = A.nside[1], nw = (unsigned)c->nHwork;
+    const dim3 b(256), g(ns + nw + (apart ? 0u : hg1.x));
+    if (!g.x) return;
+    if (c->indexed) hipLaunchKernelGGL((k_h_sweep<T, true>), g, b, 0, s, fh[0], hpc, hwk, hap[0], ns, nw, A.side[1], soff, last, pi);
+    else hipLaunchKernelGGL((k_h_sweep<T, false>), g, b, 0, s, fh[0], hpc, hwk, hap[0], ns, nw, A.side[1], soff, last, pi);
+  };
+  auto rows = [&](int e) {
+    const dim3 b(256), g((unsigned)((c->nXrow[e] + c->nXgroup[e] + 255) / 256));
+    if (!g.x) return;
+    if (c->indexed && e == 0) hipLaunchKernelGGL((k_rows<T, true, true>), g, b, 0, s, xe);
+    else if (c->indexed) hipLaunchKernelGGL((k_rows<T, true, false>), g, b, 0, s, xh);
+    else if (e == 0) hipLaunchKernelGGL((k_rows<T, false, true>), g, b, 0, s, xe);
+    else hipLaunchKernelGGL((k_rows<T, false, false>), g, b, 0, s, xh);
   };
 
   const auto &la = A.la;
@@ -837,7 +957,35 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   unsigned long long *stepp = A.stepp;
   auto ghost = [&](int electric, int q) { launch_ghosts<T>(c, electric, q, s); };
   int ne = 0, nh = 0;
-  for (uint64_t n = 0; n < nsteps; ++n) {
+  auto mark = [&](std::vector<hipEvent_t> &ev, int k) {  // times the fast kernels of the first steps
+    if (timeKernels && k < (int)ev.size()) hipEventRecord(ev[k], s);
+  };
+  // A step: the E sweep and rows, the H sweep and rows, the sweeps with what
+  // rides along (SideArgs).  SIBC faces read the old H and write only their
+  // own state, so their place before the H sweep is all that matters; so
+  // with Mur faces their inner neighbours' threads cannot write, which read
+  // the old E.
+  if (c->inl && nsteps && A.side[1].b[1])
+    hipLaunchKernelGGL(k_first_samples<T>, dim3((unsigned)A.side[1].b[1]), dim3(256), 0, s, A.side[1]);
+  for (uint64_t n = 0; c->inl && n < nsteps; ++n) {
+    const int soff = (int)n, last = n + 1 == nsteps;
+    if (c->murmask && !c->murPush) hipLaunchKernelGGL(k_mur_e<T>, murGrid, dim3(16, 16), 0, s, ma[0]);
+    mark(c->evE, 2 * ne);
+    if (apart) fast_e(0);
+    else sweep_e(soff, last);
+    mark(c->evE, 2 * ne++ + 1);
+    if (apart) sweep_e(soff, last);
+    rows(0);
+    if (c->sibcFaces) hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)c->sibcBlocks), dim3(128), 0, s, se[0]);
+    mark(c->evH, 2 * nh);
+    if (apart) fast_h(0);
+    else sweep_h(soff, last);
+    mark(c->evH, 2 * nh++ + 1);
+    if (apart) sweep_h(soff, last);
+    rows(1);
+  }
+  // Steps with the fused leapfrog sweep.
+  for (uint64_t n = 0; !c->inl && n < nsteps; ++n) {
     const int soff = (int)n;
     const int q = c->leap ? c->par ^ (int)(n & 1) : c->par;  // field set this step reads
     // observers, and the aux grids' E update as extra blocks (k_head)
@@ -860,17 +1008,17 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     if (timeKernels && ne < (int)c->evE.size() / 2) { hipEventRecord(c->evE[2 * ne + 1], s); ++ne; }
     shell_e(q);
     // Layers 0 and 1 hold each cell's first block, inside and outside the
-    // fast E box, so their sites never share an edge: without fusion they
-    // go in one launch.  Later layers follow one launch each, in block order.
-    for (int l = c->debyeFused ? 1 : 0; l < c->debyeLayers;) {
-      const int l1 = (!c->debyeFused && l == 0 && c->debyeLayers > 1) ? 2 : l + 1;
+    // fast E box, so their sites never share an edge: they go in one launch.
+    // Later layers follow one launch each, in block order.
+    for (int l = 0; l < c->debyeLayers;) {
+      const int l1 = l == 0 && c->debyeLayers > 1 ? 2 : l + 1;
       da[q].base = c->debyeLayerStart[l];
       da[q].n = c->debyeLayerStart[l1] - c->debyeLayerStart[l];
       l = l1;
       if (da[q].n == 0) continue;
       hipLaunchKernelGGL(k_debye<T>, dim3((unsigned)((da[q].n + 255) / 256)), dim3(256), 0, s, da[q]);
     }
-    if (c->sibcFaces) hipLaunchKernelGGL(k_sibc_e<T>, dim3((unsigned)c->sibcBlocks), dim3(128), 0, s, se[q]);
+    if (c->sibcFaces) hipLaunchKernelGGL((k_sibc_e<T, true>), dim3((unsigned)c->sibcBlocks), dim3(128), 0, s, se[q]);
     if (ce[q][0].nrows) {
       ce[q][0].soff = soff;
       hipLaunchKernelGGL(k_corr<T>, dim3((unsigned)((ce[q][0].nrows + 255) / 256)), dim3(256), 0, s, ce[q][0], pi);
@@ -908,13 +1056,13 @@ template <typename T> int upload_pack(Ctx *c)
   fill_step_args<T>(c, A, nullptr);
   // shells at SHELL_KC planes per block: a packed launch fills the device
   // with many grids' blocks, where a small grid's own plan used one plane
-  std::vector<ShellPiece> ep, hp;
+  std::vector<ShellDev> ep, hp;
   std::vector<ShellWork> ew, hw;
   std::string err;
   long long cells[2];
   if (plan_shells<T>(c, SHELL_KC, ep, ew, hp, hw, cells, err)) return set_error(c, VGPU_EINVAL, "%s", err.c_str());
-  c->d_epcsPk = dev_alloc(c, ep.size() * sizeof(ShellPiece));
-  c->d_hpcsPk = dev_alloc(c, hp.size() * sizeof(ShellPiece));
+  c->d_epcsPk = dev_alloc(c, ep.size() * sizeof(ShellDev));
+  c->d_hpcsPk = dev_alloc(c, hp.size() * sizeof(ShellDev));
   c->d_eworkPk = dev_alloc(c, ew.size() * sizeof(ShellWork));
   c->d_hworkPk = dev_alloc(c, hw.size() * sizeof(ShellWork));
   if (!c->d_epcsPk || !c->d_hpcsPk || !c->d_eworkPk || !c->d_hworkPk)
@@ -922,8 +1070,8 @@ template <typename T> int upload_pack(Ctx *c)
   auto up = [](void *d, const void *h, size_t n) {
     return n == 0 || hipMemcpy(d, h, n, hipMemcpyHostToDevice) == hipSuccess;
   };
-  if (!up(c->d_epcsPk, ep.data(), ep.size() * sizeof(ShellPiece)) ||
-      !up(c->d_hpcsPk, hp.data(), hp.size() * sizeof(ShellPiece)) ||
+  if (!up(c->d_epcsPk, ep.data(), ep.size() * sizeof(ShellDev)) ||
+      !up(c->d_hpcsPk, hp.data(), hp.size() * sizeof(ShellDev)) ||
       !up(c->d_eworkPk, ew.data(), ew.size() * sizeof(ShellWork)) ||
       !up(c->d_hworkPk, hw.data(), hw.size() * sizeof(ShellWork)))
     return set_error(c, VGPU_EDEVICE, "group-run shells upload");
@@ -932,16 +1080,13 @@ template <typename T> int upload_pack(Ctx *c)
   PackArgs<T> p{};
   p.fe = A.fe[0];
   p.fh = A.fh[0];
-  p.epc = P<ShellPiece>(c->d_epcsPk); p.hpc = P<ShellPiece>(c->d_hpcsPk);
+  p.epc = P<ShellDev>(c->d_epcsPk); p.hpc = P<ShellDev>(c->d_hpcsPk);
   p.ewk = P<ShellWork>(c->d_eworkPk); p.hwk = P<ShellWork>(c->d_hworkPk);
   p.ea = A.eap[0]; p.ha = A.hap[0];
-  p.da = A.da[0];
-  p.ce = A.ce[0][0];
-  p.ch = A.ce[0][1];
-  p.oa = A.oa[0];
-  p.xa = A.xa;
-  p.va = A.va[0];
-  p.headGx = A.oa[0].nobs ? (A.maxnf + 63) / 64 : 1;
+  p.xe = P<XArgs<T>>(c->d_xargs[0]); p.xh = P<XArgs<T>>(c->d_xargs[1]);
+  p.nEside = A.nside[0]; p.nHside = A.nside[1];
+  p.nEshell = (unsigned)c->nEworkPk; p.nHshell = (unsigned)c->nHworkPk;
+  p.se = A.side[0]; p.sh = A.side[1];
   c->d_pack = dev_alloc(c, sizeof(p));
   if (!c->d_pack) return set_error(c, VGPU_ENOMEM, "group-run arguments");
   if (hipMemcpy(c->d_pack, &p, sizeof(p), hipMemcpyHostToDevice) != hipSuccess)
@@ -950,15 +1095,23 @@ template <typename T> int upload_pack(Ctx *c)
 }
 
 // Steps of several solves in lockstep on one stream (vgpu_run_group): the
-// same kernels in the same order per solve as run_steps, with the fast and
-// shell sweeps, Debye layers, corrections and observers of all solves in one
-// packed launch each per half-step; Mur, SIBC and ghost launches stay one
-// per solve.  Solves share no memory, so only each solve's own order
-// matters, and every block does what it does in the solve's own launch.
-// Every context uses the separate sweeps (set 0) and has its PackArgs.
-template <typename T> int run_group_steps(Ctx *const *cs, int n, uint64_t nsteps, hipStream_t s)
+// same kernels in the same order per solve as run_steps, with the sweeps and
+// what rides along, and the rows, of all solves in one packed launch each; SIBC E, and Mur E where it keeps its launch, stay one per
+// solve.  Solves share no memory, so only each solve's own order matters, and
+// every block does what it does in the solve's own launch.  Members without
+// PackArgs (grids too large to index in line) run their own launches.
+template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t nsteps, hipStream_t s)
 {
   const double pi = 4.0 * atan(1.0);
+  Ctx *cs[PACK_MAX];
+  int n = 0;
+  for (int i = 0; i < nall; ++i) {
+    if (all[i]->d_pack) {
+      cs[n++] = all[i];
+    } else if (const int r = run_steps<T>(all[i], nsteps, s, false)) {
+      return r;
+    }
+  }
   std::vector<StepArgs<T>> A(n);
   for (int i = 0; i < n; ++i) fill_step_args<T>(cs[i], A[i], nullptr);
   // One packed launch: the solves with a positive block count, in order.
@@ -966,100 +1119,55 @@ template <typename T> int run_group_steps(Ctx *const *cs, int n, uint64_t nsteps
     PackMap m{};
     unsigned tot = 0;
     for (int i = 0; i < n; ++i) {
-      long long base = 0, cnt = 0;
-      const long long k = blocks(i, base, cnt);
+      const long long k = blocks(i);
       if (k <= 0) continue;
       m.args[m.n] = cs[i]->d_pack;
-      m.base[m.n] = base;
-      m.cnt[m.n] = cnt;
       m.start[m.n++] = tot;
       tot += (unsigned)k;
     }
     m.start[m.n] = tot;
     return m;
   };
-  PackMap fastE[2], fastH[2], shellE[2], shellH[2];
+  // packs by kernel form: with classes, the E sweep's by the level of its
+  // in-line corrections
+  PackMap sweepE[4], sweepH[2], rowE[2], rowH[2];
+  for (int x = 0; x < 4; ++x)
+    sweepE[x] = plan([&](int i) {
+      return (cs[i]->indexed ? cs[i]->xlevel() : 3) == x ? (long long)A[i].nside[0] + cs[i]->nEworkPk + A[i].eg1.x : 0LL; });
   for (int x = 0; x < 2; ++x) {
     const bool idx = x == 0;
-    fastE[x] = plan([&](int i, long long &, long long &) {
-      return cs[i]->indexed == idx && A[i].egrid.x ? (long long)A[i].eg1.x : 0LL; });
-    fastH[x] = plan([&](int i, long long &, long long &) {
-      return cs[i]->indexed == idx && A[i].hgrid.x ? (long long)A[i].hg1.x : 0LL; });
-    shellE[x] = plan([&](int i, long long &, long long &) {
-      return cs[i]->indexed == idx ? (long long)cs[i]->nEworkPk : 0LL; });
-    shellH[x] = plan([&](int i, long long &, long long &) {
-      return cs[i]->indexed == idx ? (long long)cs[i]->nHworkPk : 0LL; });
+    sweepH[x] = plan([&](int i) {
+      return cs[i]->indexed == idx ? (long long)A[i].nside[1] + cs[i]->nHworkPk + A[i].hg1.x : 0LL; });
+    auto nrows = [&](int i, int e) {
+      return cs[i]->indexed == idx ? (cs[i]->nXrow[e] + cs[i]->nXgroup[e] + 255) / 256 : 0LL; };
+    rowE[x] = plan([&](int i) { return nrows(i, 0); });
+    rowH[x] = plan([&](int i) { return nrows(i, 1); });
   }
-  unsigned headGx = 1;
-  for (int i = 0; i < n; ++i)
-    if (A[i].oa[0].nobs) headGx = std::max(headGx, (unsigned)((A[i].maxnf + 63) / 64));
-  PackMap head = plan([&](int i, long long &, long long &) {
-    return A[i].oa[0].nobs || A[i].anyAux ? (long long)A[i].oa[0].nobs + (A[i].anyAux ? A[i].xa.npw : 0) : 0LL; });
-  PackMap vol = plan([&](int i, long long &, long long &) { return (A[i].va[0].nnodes + 255) / 256; });
-  PackMap corrE = plan([&](int i, long long &, long long &) { return (A[i].ce[0][0].nrows + 255) / 256; });
-  PackMap corrH = plan([&](int i, long long &, long long &cnt) {
-    cnt = (A[i].ce[0][1].nrows + 255) / 256;
-    return A[i].ce[0][1].nrows || A[i].anyAux ? cnt + (A[i].anyAux ? A[i].xa.npw : 0) : 0LL; });
-  // Debye launches of each solve (run_steps' order: layers 0 and 1 together,
-  // then one per layer), packed by launch number
-  std::vector<std::vector<std::pair<long long, long long>>> dl(n);
-  size_t ndl = 0;
-  for (int i = 0; i < n; ++i) {
-    const Ctx *c = cs[i];
-    for (int l = 0; l < c->debyeLayers;) {
-      const int l1 = (l == 0 && c->debyeLayers > 1) ? 2 : l + 1;
-      const long long b = c->debyeLayerStart[l], k = c->debyeLayerStart[l1] - b;
-      l = l1;
-      if (k) dl[i].push_back({b, k});
-    }
-    ndl = std::max(ndl, dl[i].size());
-  }
-  std::vector<PackMap> debye(ndl);
-  for (size_t j = 0; j < ndl; ++j)
-    debye[j] = plan([&](int i, long long &base, long long &cnt) {
-      if (j >= dl[i].size()) return 0LL;
-      base = dl[i][j].first;
-      cnt = dl[i][j].second;
-      return (cnt + 255) / 256; });
-  const dim3 vblk = A[0].vblk;
+  const PackMap first = plan([&](int i) { return (long long)A[i].side[1].b[1]; });
   auto blocks = [](const PackMap &m) { return dim3(m.start[m.n]); };  // a packed launch's 1-D grid
-  for (uint64_t st = 0; st < nsteps; ++st) {
-    const int soff = (int)st;
-    if (head.n) {
-      head.soff = soff;
-      hipLaunchKernelGGL(k_head_pk<T>, dim3(headGx, head.start[head.n]), dim3(64), 0, s, head, pi);
-    }
-    if (vol.n) {
-      vol.soff = soff;
-      hipLaunchKernelGGL(k_observe_volume_pk<T>, blocks(vol), dim3(256), 0, s, vol);
+  const dim3 b(256);
+  if (first.n && nsteps) hipLaunchKernelGGL(k_first_samples_pk<T>, blocks(first), b, 0, s, first);
+  for (uint64_t st = 0; n && st < nsteps; ++st) {
+    for (PackMap *m : {sweepE, sweepE + 1, sweepE + 2, sweepE + 3, sweepH, sweepH + 1}) {
+      m->soff = (int)st;
+      m->last = st + 1 == nsteps;
     }
     for (int i = 0; i < n; ++i)
-      if (cs[i]->murmask) hipLaunchKernelGGL(k_mur_e<T>, A[i].murGrid, dim3(16, 16), 0, s, A[i].ma[0]);
-    if (fastE[0].n) hipLaunchKernelGGL((k_e_fast_pk<T, true>), blocks(fastE[0]), vblk, 0, s, fastE[0]);
-    if (fastE[1].n) hipLaunchKernelGGL((k_e_fast_pk<T, false>), blocks(fastE[1]), vblk, 0, s, fastE[1]);
-    if (shellE[0].n) hipLaunchKernelGGL((k_e_shell_pk<T, true>), blocks(shellE[0]), dim3(256), 0, s, shellE[0]);
-    if (shellE[1].n) hipLaunchKernelGGL((k_e_shell_pk<T, false>), blocks(shellE[1]), dim3(256), 0, s, shellE[1]);
-    for (const PackMap &m : debye) hipLaunchKernelGGL(k_debye_pk<T>, blocks(m), dim3(256), 0, s, m);
-    for (int i = 0; i < n; ++i)
-      if (cs[i]->sibcFaces)
-        hipLaunchKernelGGL(k_sibc_e<T>, dim3((unsigned)cs[i]->sibcBlocks), dim3(128), 0, s, A[i].se[0]);
-    if (corrE.n) {
-      corrE.soff = soff;
-      hipLaunchKernelGGL(k_corr_e_pk<T>, blocks(corrE), dim3(256), 0, s, corrE, pi);
-    }
-    for (int i = 0; i < n; ++i) launch_ghosts<T>(cs[i], 1, 0, s);
-    if (fastH[0].n) hipLaunchKernelGGL((k_h_fast_pk<T, true>), blocks(fastH[0]), vblk, 0, s, fastH[0]);
-    if (fastH[1].n) hipLaunchKernelGGL((k_h_fast_pk<T, false>), blocks(fastH[1]), vblk, 0, s, fastH[1]);
-    if (shellH[0].n) hipLaunchKernelGGL((k_h_shell_pk<T, true>), blocks(shellH[0]), dim3(256), 0, s, shellH[0]);
-    if (shellH[1].n) hipLaunchKernelGGL((k_h_shell_pk<T, false>), blocks(shellH[1]), dim3(256), 0, s, shellH[1]);
+      if (cs[i]->murmask && !cs[i]->murPush)
+        hipLaunchKernelGGL(k_mur_e<T>, A[i].murGrid, dim3(16, 16), 0, s, A[i].ma[0]);
+    if (sweepE[0].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 0>), blocks(sweepE[0]), b, 0, s, sweepE[0], pi);
+    if (sweepE[1].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 1>), blocks(sweepE[1]), b, 0, s, sweepE[1], pi);
+    if (sweepE[2].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 2>), blocks(sweepE[2]), b, 0, s, sweepE[2], pi);
+    if (sweepE[3].n) hipLaunchKernelGGL((k_e_sweep_pk<T, false, 1>), blocks(sweepE[3]), b, 0, s, sweepE[3], pi);
+    if (rowE[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, true>), blocks(rowE[0]), b, 0, s, rowE[0]);
+    if (rowE[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, true>), blocks(rowE[1]), b, 0, s, rowE[1]);
     for (int i = 0; i < n; ++i)
       if (cs[i]->sibcFaces)
-        hipLaunchKernelGGL(k_sibc_h<T>, dim3((unsigned)((A[i].sh[0].nrows + 255) / 256)), dim3(256), 0, s, A[i].sh[0]);
-    if (corrH.n) {
-      corrH.soff = soff;
-      hipLaunchKernelGGL(k_corr_h_pk<T>, blocks(corrH), dim3(256), 0, s, corrH, pi);
-    }
-    for (int i = 0; i < n; ++i) launch_ghosts<T>(cs[i], 0, 0, s);
+        hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)cs[i]->sibcBlocks), dim3(128), 0, s, A[i].se[0]);
+    if (sweepH[0].n) hipLaunchKernelGGL((k_h_sweep_pk<T, true>), blocks(sweepH[0]), b, 0, s, sweepH[0], pi);
+    if (sweepH[1].n) hipLaunchKernelGGL((k_h_sweep_pk<T, false>), blocks(sweepH[1]), b, 0, s, sweepH[1], pi);
+    if (rowH[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, false>), blocks(rowH[0]), b, 0, s, rowH[0]);
+    if (rowH[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, false>), blocks(rowH[1]), b, 0, s, rowH[1]);
   }
   for (int i = 0; i < n; ++i)
     hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(64), 0, s, A[i].stepp, (unsigned long long)nsteps);

@@ -275,7 +275,7 @@ vh_dsolve *vh_dsolve_open(vh_solve *s, int prec, int device, unsigned long chunk
   for (int o = 0; o < s->numObs; o++) d->nbin += s->obs[o].format == OF_BINARY;
   s->binaryStreamed = d->nbin > 0;
   vgpu_stats st;
-  d->packable = vgpu_get_stats(d->c, &st) == 0 && !st.leap && !st.debye_fused;
+  d->packable = vgpu_get_stats(d->c, &st) == 0 && !st.leap;
   return d;
 }
 

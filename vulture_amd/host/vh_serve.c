@@ -94,6 +94,7 @@ static size_t estimate_bytes(const vh_solve *s, int prec)
   const size_t gi = (size_t)(s->gibox[XHI] - s->gibox[XLO]) * (s->gibox[YHI] - s->gibox[YLO]) *
                     (s->gibox[ZHI] - s->gibox[ZLO]);
   b += (go - gi) * 9 * esz;
+  if (s->numDebye > 0) b += ncell * 3 * esz;  /* dense polarisation currents */
   for (int d = 0; d < s->numDebye; d++) {
     size_t n = 0;
     for (int f = 0; f < 3; f++) {
