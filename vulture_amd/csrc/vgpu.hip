@@ -743,7 +743,7 @@ static int build_sibc(Ctx *c)
     const vgpu_sibc_desc &d = c->sibc[s].d;
     {
       const long long nfs = (long long)(d.gbbox[1] - d.gbbox[0]) * (d.gbbox[3] - d.gbbox[2]) * (d.gbbox[5] - d.gbbox[4]);
-      for (long long f0 = 0; f0 < nfs; f0 += 128) blocks.push_back({s, 0, f + f0, f + nfs});
+      for (long long f0 = 0; f0 < nfs; f0 += SIBC_FACES) blocks.push_back({s, 0, f + f0, f + nfs});
     }
     normal[s] = d.normal;
     set[s] = s;

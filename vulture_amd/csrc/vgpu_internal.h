@@ -320,7 +320,7 @@ template <typename T> struct DebyeArgs {
   int cplx;
 };
 
-// A block of the SIBC E launch: up to 128 faces of one surface, so the
+// A block of the SIBC E launch: up to SIBC_FACES faces of one surface, so the
 // surface, its filters and its matrices are uniform across the block.
 struct SibcBlock {
   int surf, pad_;

@@ -1275,131 +1275,136 @@ __global__ void k_debye_gather(long long n, const long long *key, const T *const
 
 // ---------------------------------------------------------------------------
 // SIBC: E pass per face (sibc.c:443-586) with FP64 recursive convolution
-// (filter.c:309-327).
+// (filter.c:309-327).  A block is 64 faces of one surface by four wavefronts.
+// The filter states are the bytes; a thread per face walked them one group of
+// loads after another (a 14-pole slab in FP64: 8 filters, 112 states), with a
+// few hundred wavefronts on the device.  Here wavefront w takes a quarter of
+// a face's states -- output w's filters, or with one state per (input, pole)
+// input w's -- and the four meet in LDS, in the reference's order of sums.
+// The surface's matrices and filter tables are the same for every face of the
+// block and every lane of a wavefront: read through the constant address
+// space they are scalar loads.
 // ---------------------------------------------------------------------------
-template <typename T, bool ZERO> __global__ __launch_bounds__(128) void k_sibc_e(SibcEArgs<T> a)
+constexpr int SIBC_FACES = 64, SIBC_GROUP = 16;  // faces per block, states loaded together
+
+template <typename T, bool ZERO> VG_DEV void sibc_e_block(const SibcEArgs<T> &a, unsigned b)
 {
-  const SibcBlock w = a.blocks[blockIdx.x];  // one surface per block: s is uniform
-  const long long f = w.f0 + threadIdx.x;
-  if (f >= w.f1) return;
-  const int i = a.ijk[3 * f], j = a.ijk[3 * f + 1], k = a.ijk[3 * f + 2];
-  const int s = w.surf;
-  // the surface's matrices and filter tables are the same for every face of
-  // the block: read through the constant address space they are scalar loads
+  __shared__ T sh[4][SIBC_FACES];       // Htan, then Eout
+  __shared__ double sy[16][SIBC_FACES]; // filter outputs (one state per input and pole)
+  const SibcBlock bk = a.blocks[b];     // one surface per block: s is uniform
+  const int lane = (int)(threadIdx.x & 63u), w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const long long f = bk.f0 + lane;
+  const bool in = f < bk.f1;
+  const int s = bk.surf;
   const VG_CONST double *qtab = cp(a.q), *frat = cp(a.fratio), *asym = cp(a.asymp);
   const VG_CONST int *npol = cp(a.npoles), *fbas = cp(a.fbase);
   const int nrm = cp(a.normal)[s];
   const long long SJ = a.PX, P = a.plane;
-  const long long id = ((long long)k * a.NY + j) * SJ + i;
-  const unsigned char *A = a.adjA + 4 * f, *B = a.adjB + 4 * f;
-  T Htan[4];
-  const T *Hx = a.H[0], *Hy = a.H[1], *Hz = a.H[2];
-  T *Ex = a.E[0], *Ey = a.E[1], *Ez = a.E[2];
-  if (nrm == 0) {
-    if (ZERO) { Ey[id] = T(0); Ey[id + P] = T(0); Ez[id] = T(0); Ez[id + SJ] = T(0); }
-    Htan[0] = T(0.5 * (1 + A[0] + A[1]) * (double)(Hy[id - 1] + Hy[id - 1 + SJ]));
-    Htan[1] = T(0.5 * (1 + B[0] + B[1]) * (double)(Hy[id] + Hy[id + SJ]));
-    Htan[2] = T(0.5 * (1 + A[2] + A[3]) * (double)(Hz[id - 1] + Hz[id - 1 + P]));
-    Htan[3] = T(0.5 * (1 + B[2] + B[3]) * (double)(Hz[id] + Hz[id + P]));
-  } else if (nrm == 1) {
-    if (ZERO) { Ez[id] = T(0); Ez[id + 1] = T(0); Ex[id] = T(0); Ex[id + P] = T(0); }
-    Htan[0] = T(0.5 * (1 + A[0] + A[1]) * (double)(Hz[id - SJ] + Hz[id - SJ + P]));
-    Htan[1] = T(0.5 * (1 + B[0] + B[1]) * (double)(Hz[id] + Hz[id + P]));
-    Htan[2] = T(0.5 * (1 + A[2] + A[3]) * (double)(Hx[id - SJ] + Hx[id - SJ + 1]));
-    Htan[3] = T(0.5 * (1 + B[2] + B[3]) * (double)(Hx[id] + Hx[id + 1]));
-  } else {
-    if (ZERO) { Ex[id] = T(0); Ex[id + SJ] = T(0); Ey[id] = T(0); Ey[id + 1] = T(0); }
-    Htan[0] = T(0.5 * (1 + A[0] + A[1]) * (double)(Hx[id - P] + Hx[id - P + 1]));
-    Htan[1] = T(0.5 * (1 + B[0] + B[1]) * (double)(Hx[id] + Hx[id + 1]));
-    Htan[2] = T(0.5 * (1 + A[2] + A[3]) * (double)(Hy[id - P] + Hy[id - P + SJ]));
-    Htan[3] = T(0.5 * (1 + B[2] + B[3]) * (double)(Hy[id] + Hy[id + SJ]));
+  const int t1 = (nrm + 1) % 3, t2 = (nrm + 2) % 3;
+  // Htan[0], [1]: H along axis nrm+1 below and above the face, averaged along
+  // axis nrm+2's partner; [2], [3]: H along axis nrm+2
+  if (in) {
+    const int i = a.ijk[3 * f], j = a.ijk[3 * f + 1], k = a.ijk[3 * f + 2];
+    const long long id = ((long long)k * a.NY + j) * SJ + i;
+    auto st = [&](int ax) { return ax == 0 ? 1ll : ax == 1 ? SJ : P; };
+    const long long s1 = st(t1), s2 = st(t2);
+    const long long at = (w & 1) ? id : id - st(nrm), along = w < 2 ? s1 : s2;
+    const VG_GLOBAL T *H = gp(a.H[w < 2 ? t1 : t2]);
+    const unsigned char *A = ((w & 1) ? a.adjB : a.adjA) + 4 * f + (w & 2);
+    sh[w][lane] = T(0.5 * (1 + A[0] + A[1]) * (double)(H[at] + H[at + along]));
+    if (ZERO) {
+      T *E = a.E[w < 2 ? t1 : t2];
+      E[(w & 1) ? id + (w < 2 ? s2 : s1) : id] = T(0);
+    }
   }
+  __syncthreads();
+  T Hin[4];
   const VG_CONST double *Am = cp(a.A) + 16 * s, *Bm = cp(a.B) + 16 * s;
-  T Hin[4], Eout[4];
-  for (int p = 0; p < 4; ++p) {
-    Hin[p] = T(0);
-    for (int q = 0; q < 4; ++q) Hin[p] = Hin[p] + T(Am[4 * p + q]) * Htan[q];
-  }
+  if (in)
+    for (int p = 0; p < 4; ++p) {
+      Hin[p] = T(0);
+      for (int q = 0; q < 4; ++q) Hin[p] = Hin[p] + T(Am[4 * p + q]) * sh[q][lane];
+    }
   const int set = cp(a.filtset)[s];
   const long long NF = a.nfaces;
   // every filter fed by input q saw the same input last step: one stored
   // previous input per (input, face), read before and written after all
-  double xo4[4];
-  bool fed[4] = {false, false, false, false};
-  for (int q = 0; q < 4; ++q) {
-    xo4[q] = a.old[q * NF + f];
-    for (int p = 0; p < 4; ++p) fed[q] = fed[q] || npol[16 * set + 4 * p + q] > 0;
+  double xo4[4] = {0.0, 0.0, 0.0, 0.0};
+  if (in) {
+    if (a.factored) {
+      xo4[w] = a.old[w * NF + f];
+    } else {
+      for (int q = 0; q < 4; ++q) xo4[q] = a.old[q * NF + f];
+    }
   }
+  T Eout = T(0);
   if (a.factored) {
-    // one state per (input, pole), scaled by each filter's residue ratio
-    double y16[16];
-    for (int flt = 0; flt < 16; ++flt) y16[flt] = asym[16 * set + flt] * (double)Hin[flt & 3];
-    for (int q = 0; q < 4; ++q) {
-      const int b = fbas[4 * set + q];
-      if (b < 0) continue;
-      const double x = (double)Hin[q], xo = xo4[q];
-      const int np = npol[16 * set + b];
-      const VG_CONST double *qq = qtab + ((long long)(16 * set + b) * a.maxPoles) * 6;
-      VG_GLOBAL double *zq = gp(a.zeta) + (long long)q * a.maxPoles * NF + f;
-      // states in groups of eight: all loads of a group issued before its math
-      for (int k0 = 0; k0 < np; k0 += 8) {
-        double zs[8];
+    // one state per (input w, pole), scaled by each filter's residue ratio
+    const T x0 = w == 0 ? Hin[0] : w == 1 ? Hin[1] : w == 2 ? Hin[2] : Hin[3];
+    const double x = (double)x0, xo = w == 0 ? xo4[0] : w == 1 ? xo4[1] : w == 2 ? xo4[2] : xo4[3];
+    if (in) {
+      double y[4];
+      for (int p = 0; p < 4; ++p) y[p] = asym[16 * set + 4 * p + w] * x;
+      const int base = fbas[4 * set + w];
+      if (base >= 0) {
+        const int np = npol[16 * set + base];
+        const VG_CONST double *qq = qtab + ((long long)(16 * set + base) * a.maxPoles) * 6;
+        VG_GLOBAL double *zq = gp(a.zeta) + (long long)w * a.maxPoles * NF + f;
+        for (int k0 = 0; k0 < np; k0 += SIBC_GROUP) {
+          double zs[SIBC_GROUP];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (k0 + u < np) zs[u] = zq[(long long)(k0 + u) * NF];
+          for (int u = 0; u < SIBC_GROUP; ++u)
+            if (k0 + u < np) zs[u] = zq[(long long)(k0 + u) * NF];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int kp = k0 + u;
-          if (kp >= np) break;
-          const double xi = (qq[6 * kp] * zs[u] + qq[6 * kp + 2] * xo) + qq[6 * kp + 4] * x;
-          zq[(long long)kp * NF] = xi;
-          for (int p = 0; p < 4; ++p) {
-            const int flt = 4 * p + q;
-            if (npol[16 * set + flt] > 0) y16[flt] += frat[((long long)(16 * set + flt)) * a.maxPoles + kp] * xi;
+          for (int u = 0; u < SIBC_GROUP; ++u) {
+            const int kp = k0 + u;
+            if (kp >= np) break;
+            const double xi = (qq[6 * kp] * zs[u] + qq[6 * kp + 2] * xo) + qq[6 * kp + 4] * x;
+            zq[(long long)kp * NF] = xi;
+            for (int p = 0; p < 4; ++p) {
+              const int flt = 4 * p + w;
+              if (npol[16 * set + flt] > 0) y[p] += frat[((long long)(16 * set + flt)) * a.maxPoles + kp] * xi;
+            }
           }
         }
       }
+      for (int p = 0; p < 4; ++p) sy[4 * p + w][lane] = y[p];
     }
-    for (int p = 0; p < 4; ++p) {
-      Eout[p] = T(0);
+    __syncthreads();
+    if (in)
       for (int q = 0; q < 4; ++q) {
-        const int flt = 4 * p + q;
+        const int flt = 4 * w + q;
         if (npol[16 * set + flt] == 0 && asym[16 * set + flt] == 0.0) continue;
-        Eout[p] = T((double)Eout[p] + y16[flt]);
+        Eout = T((double)Eout + sy[flt][lane]);
       }
-    }
-  } else
-  for (int p = 0; p < 4; ++p) {
-    Eout[p] = T(0);
+  } else if (in) {
     for (int q = 0; q < 4; ++q) {
-      const int flt = 4 * p + q;
+      const int flt = 4 * w + q;
       const int np = npol[16 * set + flt];
       const double asy = asym[16 * set + flt];
       if (np == 0 && asy == 0.0) continue;
-      const double x = (double)Hin[q];
+      const double x = (double)Hin[q], xo = xo4[q];
       double y = asy * x;
-      if (np > 0) {
-        const double xo = xo4[q];
-        const VG_CONST double *qq = qtab + ((long long)(16 * set + flt) * a.maxPoles) * 6;
-        if (a.real) {
-          // real coefficients: the complex step below with zero imaginary
-          // parts, which leave the same real part bit for bit
-          VG_GLOBAL double *zf = gp(a.zeta) + (long long)flt * a.maxPoles * NF + f;
-          for (int k0 = 0; k0 < np; k0 += 8) {
-            double zs[8];
+      const VG_CONST double *qq = qtab + ((long long)(16 * set + flt) * a.maxPoles) * 6;
+      if (a.real) {
+        // real coefficients: the complex step below with zero imaginary
+        // parts, which leave the same real part bit for bit
+        VG_GLOBAL double *zf = gp(a.zeta) + (long long)flt * a.maxPoles * NF + f;
+        for (int k0 = 0; k0 < np; k0 += SIBC_GROUP) {
+          double zs[SIBC_GROUP];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-              if (k0 + u < np) zs[u] = zf[(long long)(k0 + u) * NF];
+          for (int u = 0; u < SIBC_GROUP; ++u)
+            if (k0 + u < np) zs[u] = zf[(long long)(k0 + u) * NF];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-              const int kp = k0 + u;
-              if (kp >= np) break;
-              const double nr = (qq[6 * kp] * zs[u] + qq[6 * kp + 2] * xo) + qq[6 * kp + 4] * x;
-              zf[(long long)kp * NF] = nr;
-              y = y + nr;
-            }
+          for (int u = 0; u < SIBC_GROUP; ++u) {
+            const int kp = k0 + u;
+            if (kp >= np) break;
+            const double nr = (qq[6 * kp] * zs[u] + qq[6 * kp + 2] * xo) + qq[6 * kp + 4] * x;
+            zf[(long long)kp * NF] = nr;
+            y = y + nr;
           }
-        } else
+        }
+      } else {
         for (int kp = 0; kp < np; ++kp) {
           double *z = &a.zeta[(((long long)flt * a.maxPoles + kp) * NF + f) * 2];
           const double q0r = qq[6 * kp], q0i = qq[6 * kp + 1], q1r = qq[6 * kp + 2], q1i = qq[6 * kp + 3];
@@ -1412,17 +1417,35 @@ template <typename T, bool ZERO> __global__ __launch_bounds__(128) void k_sibc_e
           y = y + nr;
         }
       }
-      Eout[p] = T((double)Eout[p] + y);
+      Eout = T((double)Eout + y);
     }
   }
-  for (int q = 0; q < 4; ++q)
-    if (fed[q]) a.old[q * NF + f] = (double)Hin[q];
-  T *Et = a.Etan + 4 * f;
-  for (int p = 0; p < 4; ++p) {
+  __syncthreads();  // every wavefront has read Htan and the previous inputs
+  sh[w][lane] = Eout;
+  bool fed = false;
+  for (int p = 0; p < 4; ++p) fed = fed || npol[16 * set + 4 * p + w] > 0;
+  if (in && fed) a.old[w * NF + f] = (double)(w == 0 ? Hin[0] : w == 1 ? Hin[1] : w == 2 ? Hin[2] : Hin[3]);
+  __syncthreads();
+  // Etan of face f, slot p: four consecutive lanes a face
+  const int ft = (int)(threadIdx.x >> 2), p = (int)(threadIdx.x & 3u);
+  if (bk.f0 + ft < bk.f1) {
     T v = T(0);
-    for (int q = 0; q < 4; ++q) v = v + T(Bm[4 * p + q]) * Eout[q];
-    Et[p] = v;
+    for (int q = 0; q < 4; ++q) v = v + T(Bm[4 * p + q]) * sh[q][ft];
+    a.Etan[4 * (bk.f0 + ft) + p] = v;
   }
+}
+
+template <typename T, bool ZERO> __global__ __launch_bounds__(256) void k_sibc_e(SibcEArgs<T> a)
+{
+  sibc_e_block<T, ZERO>(a, blockIdx.x);
+}
+
+// The SIBC faces' blocks, then the E rows.
+template <typename T, bool IDX>
+__global__ __launch_bounds__(256) void k_sibc_rows(SibcEArgs<T> a, const XArgs<T> *x, unsigned nSibc)
+{
+  if (blockIdx.x < nSibc) sibc_e_block<T, false>(a, blockIdx.x);
+  else x_rows<T, IDX, true>(cp(x), blockIdx.x - nSibc);
 }
 
 // SIBC: gathered H corrections (sibc.c:616-776).

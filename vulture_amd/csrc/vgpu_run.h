@@ -948,6 +948,12 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   auto &da = A.da;
   const auto &se = A.se;
   const auto &sh = A.sh;
+  auto sibc_rows = [&]() {
+    const unsigned nb = (unsigned)c->sibcBlocks;
+    const dim3 b(256), g(nb + (unsigned)((c->nXrow[0] + c->nXgroup[0] + 255) / 256));
+    if (c->indexed) hipLaunchKernelGGL((k_sibc_rows<T, true>), g, b, 0, s, se[0], xe, nb);
+    else hipLaunchKernelGGL((k_sibc_rows<T, false>), g, b, 0, s, se[0], xe, nb);
+  };
   auto &ce = A.ce;
   auto &xa = A.xa;
   const bool anyAux = A.anyAux;
@@ -975,8 +981,8 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     else sweep_e(soff, last);
     mark(c->evE, 2 * ne++ + 1);
     if (apart) sweep_e(soff, last);
-    rows(0);
-    if (c->sibcFaces) hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)c->sibcBlocks), dim3(128), 0, s, se[0]);
+    if (c->sibcFaces) sibc_rows();
+    else rows(0);
     mark(c->evH, 2 * nh);
     if (apart) fast_h(0);
     else sweep_h(soff, last);
@@ -1018,7 +1024,7 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
       if (da[q].n == 0) continue;
       hipLaunchKernelGGL(k_debye<T>, dim3((unsigned)((da[q].n + 255) / 256)), dim3(256), 0, s, da[q]);
     }
-    if (c->sibcFaces) hipLaunchKernelGGL((k_sibc_e<T, true>), dim3((unsigned)c->sibcBlocks), dim3(128), 0, s, se[q]);
+    if (c->sibcFaces) hipLaunchKernelGGL((k_sibc_e<T, true>), dim3((unsigned)c->sibcBlocks), dim3(256), 0, s, se[q]);
     if (ce[q][0].nrows) {
       ce[q][0].soff = soff;
       hipLaunchKernelGGL(k_corr<T>, dim3((unsigned)((ce[q][0].nrows + 255) / 256)), dim3(256), 0, s, ce[q][0], pi);
@@ -1163,7 +1169,7 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
     if (rowE[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, true>), blocks(rowE[1]), b, 0, s, rowE[1]);
     for (int i = 0; i < n; ++i)
       if (cs[i]->sibcFaces)
-        hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)cs[i]->sibcBlocks), dim3(128), 0, s, A[i].se[0]);
+        hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)cs[i]->sibcBlocks), dim3(256), 0, s, A[i].se[0]);
     if (sweepH[0].n) hipLaunchKernelGGL((k_h_sweep_pk<T, true>), blocks(sweepH[0]), b, 0, s, sweepH[0], pi);
     if (sweepH[1].n) hipLaunchKernelGGL((k_h_sweep_pk<T, false>), blocks(sweepH[1]), b, 0, s, sweepH[1], pi);
     if (rowH[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, false>), blocks(rowH[0]), b, 0, s, rowH[0]);
