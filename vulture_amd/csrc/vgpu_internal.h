@@ -166,7 +166,8 @@ template <typename T> struct FastE {
   long long plane;
   int box[6];            // fast box (every E component inner-grid)
   int kchunk, nchx;      // planes per block; 64-cell x chunks from box[0]
-  int gy, gz;            // y blocks (blockDim.y rows), z chunks (blocks = nchx*gy*gz, launched in XCD order)
+  int gy, gz;            // y blocks, z chunks
+  int per;               // blocks of a z chunk per XCD
   T *E[3];               // new E (written)
   const T *Ein[3];       // old E
   const T *H[3];         // old H
@@ -182,7 +183,7 @@ template <typename T> struct FastH {
   long long plane;
   int box[6];
   int kchunk, nchx;
-  int gy, gz;
+  int gy, gz, per;
   T *H[3];               // new H (written)
   const T *Hin[3];       // old H
   const T *E[3];         // new E

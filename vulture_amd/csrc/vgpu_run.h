@@ -265,11 +265,11 @@ static int build_shell(const A &a, const int (*in)[NB][6], const int *fb, const 
       return -1;
     }
     pc.cells = (int)n;
-    // Rows shorter than half a line are padded to whole lines of lw
+    // With lw, rows shorter than half a line are padded to whole lines of lw
     // elements, each starting on a line, so a wavefront's loads touch one
-    // line per row instead of one line per lane (a piece of one- or
-    // two-cell rows, as at a Mur face's x end).  Longer rows stay unpadded:
-    // there the idle lanes cost more than the split lines (measured).
+    // line per row.  Off by default: since the pieces are read in one batch of
+    // scalar loads, the idle lanes' wavefronts cost more (53x41x62 request
+    // 40.4 us a step padded, 36.0 packed; 256x256x160 box 342 and 335).
     const bool pad = lw > 0 && 2 * pc.ni < lw;
     pc.xo = pad ? pc.box[0] % lw : 0;
     pc.nip = pad ? (pc.xo + pc.ni + lw - 1) / lw * lw : pc.ni;
@@ -344,7 +344,8 @@ static int plan_shells(Ctx *c, int kcPlan, std::vector<ShellDev> &ep, std::vecto
   int ein[3][1][6];
   for (int C = 0; C < 3; ++C)
     for (int q = 0; q < 6; ++q) ein[C][0][q] = ea.in[C][q];
-  const int lw = getenv("VGPU_SHELL_ROWS") && getenv("VGPU_SHELL_ROWS")[0] == '0' ? 0 : (int)(128 / sizeof(T));
+  // VGPU_SHELL_ROWS=1 pads rows shorter than half a line to whole lines
+  const int lw = getenv("VGPU_SHELL_ROWS") && getenv("VGPU_SHELL_ROWS")[0] == '1' ? (int)(128 / sizeof(T)) : 0;
   if (build_shell<1>(ea, ein, c->fastE, N, pe, ew, cells[0], err, lw, kcPlan) ||
       build_shell<3>(ha, ha.in, c->fastH, N, ph, hw, cells[1], err, lw, kcPlan))
     return -1;
@@ -509,6 +510,16 @@ template <typename T> struct StepArgs {
   unsigned long long *stepp;           // device step counter
 };
 
+// Whether a context's fast tiles have launches of their own.  In one launch
+// the tiles share the shell's register count (FP32 E 104 and H 62 VGPRs
+// against 62 and 53 alone), but its blocks fill the device together with
+// theirs and one launch fewer is on the step's critical path: 48.6 -> 39.8 us
+// a step on a 53x41x62 request, 82 -> 71 on 101x115x108, 298 -> 283 on the
+// FP64 200x160x120 enclosure, 377 -> 368 on the 256x256x160 box.  Where the
+// fields are past the 256 MB last-level cache the tiles' own occupancy counts
+// for more: 537 against 529 us at 272^3 in FP32 (85 MB a field).
+static bool sweeps_apart(const Ctx *c) { return c->ncell * c->esz > ((size_t)64 << 20); }
+
 template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun *chk)
 {
   const double dt = c->grid.dt;
@@ -516,8 +527,9 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   auto &ea = A.ea;
   auto &ha = A.ha;
   for (int q = 0; q < 2; ++q) fill_volume_args<T>(c, ea[q], ha[q], q);
-  // Fast kernels: 64x4 tiles (64 x ty) over the fast boxes, marching z in chunks of 4
-  // planes (measured best from 272^3 to 386x386x258; 16k blocks and more at those sizes).
+  // Fast kernels: 64x4 tiles (64 x ty) over the fast boxes, marching z in
+  // chunks of 4 planes, or 2 where they have launches of their own (272^3 FP32:
+  // 505 us a step with 4, 501 with 2, 514 with 8; merged grids within 1 %).
   // rows per block (tuning override VGPU_FAST_TY: 1..8)
   int ty = 4;
   if (const char *ev = getenv("VGPU_FAST_TY")) ty = std::max(1, std::min(atoi(ev), 8));
@@ -525,7 +537,7 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   auto fast_grid = [&](const int *fb, int &kchunk) {
     if (fb[0] > fb[1] || fb[2] > fb[3] || fb[4] > fb[5]) return dim3(0, 0, 0);
     const int gx = (fb[1] - fb[0] + 64) / 64, gy = (fb[3] - fb[2] + ty) / ty, nz = fb[5] - fb[4] + 1;
-    kchunk = std::min(4, nz);
+    kchunk = std::min(sweeps_apart(c) ? 2 : 4, nz);
     if (const char *ev = getenv("VGPU_FAST_KCHUNK"))  // tuning override: planes per block
       kchunk = std::max(1, std::min(atoi(ev), nz));
     return dim3(gx, gy, (nz + kchunk - 1) / kchunk);
@@ -534,16 +546,17 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   auto &fh = A.fh;
   int ekc = 1, hkc = 1;
   const dim3 egrid = A.egrid = fast_grid(c->fastE, ekc), hgrid = A.hgrid = fast_grid(c->fastH, hkc);
-  // 1-D launches padded to a multiple of eight blocks (XCD order, xcd_block)
+  // 1-D launches: an eighth of each z chunk's tiles per XCD (fast_block)
   auto pad8 = [](unsigned long long n) { return dim3((unsigned)((n + 7) / 8 * 8)); };
-  A.eg1 = pad8((unsigned long long)egrid.x * egrid.y * egrid.z);
-  A.hg1 = pad8((unsigned long long)hgrid.x * hgrid.y * hgrid.z);
+  const int eper = (int)(egrid.x * egrid.y + 7) / 8, hper = (int)(hgrid.x * hgrid.y + 7) / 8;
+  A.eg1 = dim3(8u * eper * egrid.z);
+  A.hg1 = dim3(8u * hper * hgrid.z);
   for (int q = 0; q < 2; ++q) {
     FastE<T> &e = fe[q];
     FastH<T> &h = fh[q];
     e.NX = h.NX = c->NX; e.NY = h.NY = c->NY; e.NZ = h.NZ = c->NZ; e.PX = h.PX = c->PX;
     e.plane = h.plane = c->plane;
-    e.kchunk = ekc; h.kchunk = hkc;
+    e.kchunk = ekc; h.kchunk = hkc; e.per = eper; h.per = hper;
     for (int f = 0; f < 6; ++f) { e.box[f] = c->fastE[f]; h.box[f] = c->fastH[f]; }
     e.nchx = egrid.x; h.nchx = hgrid.x;
     e.gy = egrid.y; e.gz = egrid.z; h.gy = hgrid.y; h.gz = hgrid.z;
@@ -792,16 +805,6 @@ template <typename T> void launch_ghosts(Ctx *c, int electric, int q, hipStream_
   }
 }
 
-// Whether a context's fast tiles have launches of their own.  In one launch
-// the tiles share the shell's register count (FP32 E 104 and H 62 VGPRs
-// against 62 and 53 alone), but its blocks fill the device together with
-// theirs and one launch fewer is on the step's critical path: 48.6 -> 39.8 us
-// a step on a 53x41x62 request, 82 -> 71 on 101x115x108, 298 -> 283 on the
-// FP64 200x160x120 enclosure, 377 -> 368 on the 256x256x160 box.  Where the
-// fields are past the 256 MB last-level cache the tiles' own occupancy counts
-// for more: 537 against 529 us at 272^3 in FP32 (85 MB a field).
-static bool sweeps_apart(const Ctx *c) { return c->ncell * c->esz > ((size_t)64 << 20); }
-
 // The loop (simulation.c:136-230).  With chk, one step of the field sweeps
 // only (Mur E, the E sweep, the H sweep), in their update-counting form.
 // With the fused sweep, step q of the run reads field set c->par ^ (q & 1)
@@ -976,11 +979,13 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   for (uint64_t n = 0; c->inl && n < nsteps; ++n) {
     const int soff = (int)n, last = n + 1 == nsteps;
     if (c->murmask && !c->murPush) hipLaunchKernelGGL(k_mur_e<T>, murGrid, dim3(16, 16), 0, s, ma[0]);
+    // the fast tiles last here and first in the H sweep, which runs them from
+    // the top plane down: what the E tiles touched last is still in cache
+    if (apart) sweep_e(soff, last);
     mark(c->evE, 2 * ne);
     if (apart) fast_e(0);
     else sweep_e(soff, last);
     mark(c->evE, 2 * ne++ + 1);
-    if (apart) sweep_e(soff, last);
     if (c->sibcFaces) sibc_rows();
     else rows(0);
     mark(c->evH, 2 * nh);
