@@ -94,7 +94,8 @@ template <typename T> int build_inline(Ctx *c)
   // Mur faces: each E value on one is written by the thread of its inner
   // neighbour when that takes the ordinary update; else the whole context
   // keeps Mur's own launch before the sweep
-  std::vector<long long> mur;  // the neighbours
+  struct Mur { long long cell; unsigned fl; };  // a neighbour, its flag of one face and component
+  std::vector<Mur> mur;
   c->murPush = c->murmask != 0;
   for (int f = 0; f < 6 && c->murPush; ++f)
     for (int C = 0; C < 3 && c->murPush; ++C) {
@@ -111,12 +112,11 @@ template <typename T> int build_inline(Ctx *c)
               c->murPush = false;
               continue;
             }
-            mur.push_back(c->lin(nb[0], nb[1], nb[2]));
+            mur.push_back({c->lin(nb[0], nb[1], nb[2]), (unsigned)XF_MUR << (2 * f + (C - a + 5) % 3)});
           }
     }
   if (!c->murPush) mur.clear();
-  std::sort(mur.begin(), mur.end());
-  mur.erase(std::unique(mur.begin(), mur.end()), mur.end());
+  std::sort(mur.begin(), mur.end(), [](const Mur &a, const Mur &b) { return a.cell < b.cell; });
 
   // E operations but Debye, then the Debye sites: one one-pole site alone on a
   // swept value goes to the class table, others are listed
@@ -242,7 +242,7 @@ template <typename T> int build_inline(Ctx *c)
       long long cell = INT64_MAX;
       if (qs < simple.size()) cell = std::min(cell, simple[qs].cell);
       if (qz < zero.size()) cell = std::min(cell, zero[qz].cell);
-      if (qm < mur.size()) cell = std::min(cell, mur[qm]);
+      if (qm < mur.size()) cell = std::min(cell, mur[qm].cell);
       if (cell == INT64_MAX) break;
       Entry x{(int)cell, {-1, -1, -1}, 0};
       for (; qs < simple.size() && simple[qs].cell == cell; ++qs) {
@@ -250,7 +250,7 @@ template <typename T> int build_inline(Ctx *c)
         x.fl |= XF_DEBYE << simple[qs].comp;
       }
       for (; qz < zero.size() && zero[qz].cell == cell; ++qz) x.fl |= XF_ZERO << zero[qz].comp;
-      for (; qm < mur.size() && mur[qm] == cell; ++qm) x.fl |= XF_MUR;
+      for (; qm < mur.size() && mur[qm].cell == cell; ++qm) x.fl |= mur[qm].fl;
       ent.push_back(x);
     }
   };

@@ -90,8 +90,9 @@ template <typename T> struct HArgs {
 //    four dependent loads, one lane of a wavefront at a time at the x faces.)
 enum XKind { XO_SRC, XO_AUX, XO_WAVE, XO_ZERO, XO_DEBYE, XO_GHOST, XO_SIBC };
 // flags of a flagged class (dtab slot 6): one-pole Debye sites of components
-// 0-2 (bits 0-2), Mur faces (3), zeroed components (4-6)
-enum XFlag { XF_DEBYE = 1, XF_MUR = 8, XF_ZERO = 16 };
+// 0-2 (bits 0-2), zeroed components (3-5), and per Mur face f the components
+// (f/2 + 1) % 3 and (f/2 + 2) % 3 it takes from the cell (bits 6+2f, 7+2f)
+enum XFlag { XF_DEBYE = 1, XF_ZERO = 8, XF_MUR = 64 };
 constexpr int DTAB_STRIDE = 8;
 
 // code: kind (bits 0-2), then
@@ -123,13 +124,10 @@ template <typename T> struct XArgs {
   unsigned flag0;        // first flagged class (E)
   const uint16_t *cls;   // per cell: class, or without classes 0 / 1 + dtab row
   const T *dtab;         // [class - flag0][8]: alpha, beta of J per component, flags
-  T *J;                  // [component][cell] (null without one-pole sites)
-  long long nJ;          // cells
+  T *J;                  // [cell][component] (null without one-pole sites)
   int PX;
   long long plane;
-  unsigned murmask;      // Mur faces written in line
-  int mbox[6][3][6];     // their limits [face][component]
-  T mzeta[6];
+  T mzeta[6];            // Mur factors
   long long nrow, ngroup;  // rows on their own, then groups of rows (a row and its ghosts)
   const int *gstart;     // first row of each group
   const XRow *row;

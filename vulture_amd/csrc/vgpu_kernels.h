@@ -371,35 +371,47 @@ template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) voi
 }
 
 // A one-pole Debye site (debye.c:243-307, as debye_site with one real pole):
-// j is its J, the previous E is the old E of the update.
-template <typename T> VG_DEV T x_debye(VG_GLOBAL T *J, T j, T da, T db, T be, T eo, T e)
+// the previous E is the old E of the update.
+template <typename T> VG_DEV void x_debye(T &j, T da, T db, T be, T eo, T &e)
 {
   const T jsum = T(0) + (T(1) + da) * j;
   e = e - be * jsum;
   const T de = e - eo;
-  *J = da * j + db * de;
-  return e;
+  j = da * j + db * de;
 }
 
 // What a flagged cell's corrections read, loaded together with the update's
-// own operands: J is dense, so its address needs nothing but the cell.
+// own operands: its class's row of dtab, J -- dense and interleaved, so its
+// address needs nothing but the cell and it is one stream -- and the E of the
+// first Mur face beside it.
 template <typename T> struct XPre {
-  T j0, j1, j2;
-  typename Vec2<T>::type d0, d1, d2;
+  T j[3], d[6], m0, m1, mz;
   unsigned fl;
+  VG_DEV static long long mur_at(const VG_CONST XArgs<T> *x, long long id, int f)
+  {
+    const long long st = f < 2 ? 1 : f < 4 ? (long long)x->PX : x->plane;
+    return (f & 1) ? id + st : id - st;
+  }
+  VG_DEV static VG_GLOBAL T *mur_e(const VG_CONST XArgs<T> *x, int f, int s)
+  {
+    const int C = ((f >> 1) + 1 + s) % 3;
+    return gp(C == 0 ? x->F[0] : C == 1 ? x->F[1] : x->F[2]);
+  }
   template <bool DEBYE> VG_DEV void load(const VG_CONST XArgs<T> *x, long long id, unsigned cls)
   {
-    using V2 = typename Vec2<T>::type;
-    const VG_GLOBAL T *d = gp(x->dtab) + (cls - x->flag0) * DTAB_STRIDE;
-    fl = (unsigned)d[6];
+    const VG_GLOBAL T *q = gp(x->dtab) + (cls - x->flag0) * DTAB_STRIDE;
+    fl = (unsigned)q[6];
     if (DEBYE) {
-      const VG_GLOBAL T *J = gp(x->J) + id;
-      j0 = J[0];
-      j1 = J[x->nJ];
-      j2 = J[2 * x->nJ];
-      d0 = ((const VG_GLOBAL V2 *)d)[0];
-      d1 = ((const VG_GLOBAL V2 *)d)[1];
-      d2 = ((const VG_GLOBAL V2 *)d)[2];
+      const VG_GLOBAL T *J = gp(x->J) + 3 * id;
+      for (int c = 0; c < 3; ++c) j[c] = J[c];
+      for (int c = 0; c < 6; ++c) d[c] = q[c];
+    }
+    if (fl >= XF_MUR) {
+      const int f = (__ffs((int)(fl >> 6)) - 1) >> 1;
+      const long long at = mur_at(x, id, f);
+      m0 = mur_e(x, f, 0)[at];
+      m1 = mur_e(x, f, 1)[at];
+      mz = f == 0 ? x->mzeta[0] : f == 1 ? x->mzeta[1] : f == 2 ? x->mzeta[2] : f == 3 ? x->mzeta[3] : f == 4 ? x->mzeta[4] : x->mzeta[5];
     }
   }
 };
@@ -408,36 +420,35 @@ template <typename T> struct XPre {
 // beta): the Mur faces that take its update (mur.c:135-395), its one-pole
 // Debye sites, its zeroed components.
 template <typename T, bool DEBYE>
-VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, int i, int j, int k, long long id, const XPre<T> &p, T o0, T o1,
-                       T o2, T b0, T b1, T b2, T &e0, T &e1, T &e2)
+VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, XPre<T> &p, T o0, T o1, T o2, T b0, T b1, T b2, T &e0,
+                       T &e1, T &e2)
 {
   const unsigned fl = p.fl;
-  if (fl & XF_MUR) {
-    const unsigned mask = x->murmask;
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-      const int a = f >> 1, up = f & 1;
-      if (!((mask >> f) & 1u)) continue;
-#pragma unroll
-      for (int s = 1; s < 3; ++s) {
-        const int C = (a + s) % 3;
-        const VG_CONST int *b = x->mbox[f][C];
-        const int n = a == 0 ? i : a == 1 ? j : k;
-        if (n != b[2 * a + up] + (up ? -1 : 1)) continue;
-        if ((a != 0 && (i < b[0] || i > b[1])) || (a != 1 && (j < b[2] || j > b[3])) || (a != 2 && (k < b[4] || k > b[5])))
-          continue;
-        const long long st = a == 0 ? 1 : a == 1 ? (long long)x->PX : x->plane;
-        VG_GLOBAL T *F = gp(x->F[C]) + (up ? id + st : id - st);
-        const T o = C == 0 ? o0 : C == 1 ? o1 : o2, t = C == 0 ? e0 : C == 1 ? e1 : e2;
-        *F = o + x->mzeta[f] * (t - *F);
-      }
+  bool first = true;
+  for (unsigned m = fl >> 6; m;) {
+    const int f = (__ffs((int)m) - 1) >> 1, a = f >> 1;
+    const unsigned on = (m >> (2 * f)) & 3u;
+    m &= ~(3u << (2 * f));
+    const long long at = XPre<T>::mur_at(x, id, f);
+    VG_GLOBAL T *F0 = XPre<T>::mur_e(x, f, 0) + at, *F1 = XPre<T>::mur_e(x, f, 1) + at;
+    T v0 = p.m0, v1 = p.m1, z = p.mz;
+    if (!first) {
+      v0 = *F0;
+      v1 = *F1;
+      z = f == 1 ? x->mzeta[1] : f == 2 ? x->mzeta[2] : f == 3 ? x->mzeta[3] : f == 4 ? x->mzeta[4] : x->mzeta[5];
     }
+    first = false;
+    const T oa = a == 0 ? o1 : a == 1 ? o2 : o0, ta = a == 0 ? e1 : a == 1 ? e2 : e0;
+    const T ob = a == 0 ? o2 : a == 1 ? o0 : o1, tb = a == 0 ? e2 : a == 1 ? e0 : e1;
+    if (on & 1u) *F0 = oa + z * (ta - v0);
+    if (on & 2u) *F1 = ob + z * (tb - v1);
   }
-  if (DEBYE) {
-    VG_GLOBAL T *J = gp(x->J) + id;
-    if (fl & XF_DEBYE) e0 = x_debye(J, p.j0, p.d0.x, p.d0.y, b0, o0, e0);
-    if (fl & (XF_DEBYE << 1)) e1 = x_debye(J + x->nJ, p.j1, p.d1.x, p.d1.y, b1, o1, e1);
-    if (fl & (XF_DEBYE << 2)) e2 = x_debye(J + 2 * x->nJ, p.j2, p.d2.x, p.d2.y, b2, o2, e2);
+  if (DEBYE && (fl & 7u)) {
+    if (fl & XF_DEBYE) x_debye(p.j[0], p.d[0], p.d[1], b0, o0, e0);
+    if (fl & (XF_DEBYE << 1)) x_debye(p.j[1], p.d[2], p.d[3], b1, o1, e1);
+    if (fl & (XF_DEBYE << 2)) x_debye(p.j[2], p.d[4], p.d[5], b2, o2, e2);
+    VG_GLOBAL T *J = gp(x->J) + 3 * id;  // this thread's alone: the others go back as they came
+    for (int c = 0; c < 3; ++c) J[c] = p.j[c];
   }
   if (fl & XF_ZERO) e0 = T(0);
   if (fl & (XF_ZERO << 1)) e1 = T(0);
@@ -511,7 +522,7 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
         visit(f.vis[1], id);
         visit(f.vis[2], id);
       } else {
-        if (flagged) x_inline_e<T, X == 2>(x, i, j, k, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
+        if (flagged) x_inline_e<T, X == 2>(x, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
         f.E[0][id] = e0;
         f.E[1][id] = e1;
         f.E[2][id] = e2;
@@ -1035,7 +1046,7 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
       T e0 = c0.value(g, rg[0], idh1 * (hz - hzy) + idh2 * (hym - hy));
       T e1 = c1.value(g, rg[1], idh2 * (hx - hxm) + idh0 * (hzx - hz));
       T e2 = c2.value(g, rg[2], idh0 * (hy - hyx) + idh1 * (hxy - hx));
-      if (flagged) x_inline_e<T, X == 2>(x, i, j, k, id, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
+      if (flagged) x_inline_e<T, X == 2>(x, id, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
       if (rg[0].reg >= 0) g.E[0][id] = e0;
       if (rg[1].reg >= 0) g.E[1][id] = e1;
       if (rg[2].reg >= 0) g.E[2][id] = e2;

@@ -373,13 +373,8 @@ template <typename T> static void fill_correction_args(Ctx *c, XArgs<T> &x, int 
   x.flag0 = ~0u;
   if (e) return;
   x.flag0 = c->xflag0;
-  x.dtab = P<T>(c->d_xdtab); x.J = P<T>(c->d_xJ); x.nJ = (long long)c->ncell;
-  x.murmask = c->murPush ? c->murmask : 0u;
-  for (int f = 0; f < 6; ++f) {
-    x.mzeta[f] = T(c->zeta[f]);
-    for (int C = 0; C < 3; ++C)
-      for (int q = 0; q < 6; ++q) x.mbox[f][C][q] = c->fmlim[f][C][q];
-  }
+  x.dtab = P<T>(c->d_xdtab); x.J = P<T>(c->d_xJ);
+  for (int f = 0; f < 6; ++f) x.mzeta[f] = T(c->zeta[f]);
   x.dlast = P<T>(c->d_dlast); x.dJ = P<T>(c->d_dJ); x.dstride = c->debyeSites;
   x.dalpha = P<double>(c->d_dalpha); x.dbeta = P<double>(c->d_dbeta); x.dnp = P<int>(c->d_dnp);
   x.dmaxP = c->debyeMaxPoles; x.dcplx = c->debyeCplx;
