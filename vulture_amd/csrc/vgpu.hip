@@ -630,7 +630,7 @@ static int build_debye(Ctx *c)
           return set_error(c, VGPU_EINVAL, "Debye block outside the grid");
         for (int k = l[4]; k <= l[5]; ++k)
           for (int j = l[2]; j <= l[3]; ++j)
-            for (int i = l[0]; i <= l[1]; ++i) c->xsite.push_back({c->lin(i, j, k), f, blockMedium[b]});
+            for (int i = l[0]; i <= l[1]; ++i) c->xsite.push_back({c->lin(i, j, k) * 3 + f, blockMedium[b]});
       }
     c->debyeAll = (long long)c->xsite.size();
     return VGPU_OK;
@@ -713,6 +713,7 @@ static int build_class_tables(Ctx *c)
       for (int q = 0; q < 6; ++q) e8[(size_t)k * ETAB_STRIDE + q] = c->etab[(size_t)k * 6 + q];
     for (int k = 0; k < c->nHcls; ++k)
       for (int q = 0; q < 3; ++q) h4[(size_t)k * HTAB_STRIDE + q] = c->htab[(size_t)k * 3 + q];
+    for (size_t k = 0; k < c->hflags.size(); ++k) h4[k * HTAB_STRIDE + 3] = c->hflags[k];
     c->d_etab = upload_reals(c, e8);
     c->d_htab = upload_reals(c, h4);
     if (!c->d_ecls || !c->d_hcls || !c->d_etab || !c->d_htab)
@@ -790,7 +791,7 @@ static int build_sibc(Ctx *c)
             const long long o2 = d.normal == 0 ? SJ : d.normal == 1 ? P : 1;
             for (const auto &[at, comp] : {std::pair<long long, int>(id, t1), {id + o1, t1}, {id, t2}, {id + o2, t2}}) {
               if (c->leap) c->eTouched.push_back(at * 3 + comp);
-              if (c->inl) c->xent[0].push_back({at, 0, comp, 1, XO_ZERO, 0, 0, 0});
+              if (c->inl) c->xent[0].push_back({(at * 3 + comp) * 4 + 1, XO_ZERO, 0, 0, 0});
             }
           }
           const unsigned char *a = &c->sibc[s].adjA[4 * lf], *b = &c->sibc[s].adjB[4 * lf];
@@ -867,21 +868,24 @@ static int build_sibc(Ctx *c)
         }
     f = f0 + lf;
   }
-  std::stable_sort(hents.begin(), hents.end(), [](const HE &a, const HE &b) { return a.key < b.key; });
-  std::sort(zeroKeys.begin(), zeroKeys.end());
-  zeroKeys.erase(std::unique(zeroKeys.begin(), zeroKeys.end()), zeroKeys.end());
   if (c->inl) {
     // a normal H set to zero takes no other term
-    for (long long key : zeroKeys) c->xent[1].push_back({key / 6, 0, (int)(key % 6 - 3), 0, XO_ZERO, 0, 0, 0});
+    std::sort(zeroKeys.begin(), zeroKeys.end());
+    zeroKeys.erase(std::unique(zeroKeys.begin(), zeroKeys.end()), zeroKeys.end());
+    for (long long key : zeroKeys) c->xent[1].push_back({(key / 6 * 3 + key % 6 - 3) * 4, XO_ZERO, 0, 0, 0});
+    c->xent[1].reserve(zeroKeys.size() + hents.size());
     for (const HE &h : hents) {
       if (std::binary_search(zeroKeys.begin(), zeroKeys.end(), h.key)) continue;
       const std::vector<double> &id = *ide[(h.e.bits >> 9) & 3];
-      c->xent[1].push_back({h.key / 6, h.seq, (int)(h.key % 6 - 3), 1, XO_SIBC | h.e.bits << 3, h.e.face, id[h.e.ia],
+      c->xent[1].push_back({(h.key / 6 * 3 + h.key % 6 - 3) * 4 + 1, XO_SIBC | h.e.bits << 3, h.e.face, id[h.e.ia],
                             id[h.e.ib]});
     }
     hents.clear();
     zeroKeys.clear();
   }
+  std::stable_sort(hents.begin(), hents.end(), [](const HE &a, const HE &b) { return a.key < b.key; });
+  std::sort(zeroKeys.begin(), zeroKeys.end());
+  zeroKeys.erase(std::unique(zeroKeys.begin(), zeroKeys.end()), zeroKeys.end());
   std::vector<int> rstart;
   std::vector<long long> rkey;
   std::vector<SibcHEnt> ents;
@@ -1084,7 +1088,7 @@ static int build_corrections(Ctx *c)
     for (const RowEntry &r : rows[e]) {
       const CorrEntry &ce = r.e;
       if (ce.idx < 0 || ce.idx >= (1 << 23)) return set_error(c, VGPU_EINVAL, "too many sources or plane waves");
-      Ctx::XEnt x{r.key / 3, r.seq, (int)(r.key % 3), 2, 0, 0, 0, 0};
+      Ctx::XEnt x{r.key * 4 + 2, 0, 0, 0, 0};
       if (ce.kind <= 1) {
         x.code = XO_SRC | ce.kind << 3 | c->src[ce.idx].soft << 4;
         x.arg = srcVal[ce.idx];

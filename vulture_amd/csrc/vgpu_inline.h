@@ -73,29 +73,51 @@ template <typename T> struct InlineGeom {
   }
 };
 
+// Stable sort by the 64-bit key of each element, least significant digit first.
+template <typename V> static void sort_by_key(std::vector<V> &v)
+{
+  long long top = 0;
+  bool sorted = true;
+  for (size_t k = 0; k < v.size(); ++k) {
+    top = std::max(top, v[k].key);
+    sorted = sorted && (k == 0 || v[k - 1].key <= v[k].key);
+  }
+  if (sorted) return;
+  constexpr int BITS = 11;
+  std::vector<V> w(v.size());
+  std::vector<size_t> at(1 << BITS);
+  for (int shift = 0; shift < 63 && (top >> shift) > 0; shift += BITS) {
+    std::fill(at.begin(), at.end(), 0);
+    for (const V &x : v) ++at[(x.key >> shift) & ((1 << BITS) - 1)];
+    size_t sum = 0;
+    for (size_t &n : at) {
+      const size_t m = n;
+      n = sum;
+      sum += m;
+    }
+    for (const V &x : v) w[at[(x.key >> shift) & ((1 << BITS) - 1)]++] = x;
+    v.swap(w);
+  }
+}
+
 template <typename T> int build_inline(Ctx *c)
 {
   if (!c->inl) return VGPU_OK;
   using Ent = Ctx::XEnt;
   const InlineGeom<T> geo(c);
+  const int N[3] = {c->NX, c->NY, c->NZ};
   auto fail = [&](const char *what) { return set_error(c, VGPU_ENOMEM, "corrections: %s", what); };
   auto up = [&](void *&d, const void *h, size_t bytes) {
     d = dev_alloc(c, bytes);
     return d && (bytes == 0 || hipMemcpy(d, h, bytes, hipMemcpyHostToDevice) == hipSuccess);
   };
-  auto less = [](const Ent &a, const Ent &b) {
-    if (a.cell != b.cell) return a.cell < b.cell;
-    if (a.comp != b.comp) return a.comp < b.comp;
-    if (a.order != b.order) return a.order < b.order;
-    return a.seq < b.seq;
-  };
-  auto same = [](const Ent &a, const Ent &b) { return a.cell == b.cell && a.comp == b.comp; };
+  auto kind = [](const Ent &x) { return x.code & 7; };
 
   // Mur faces: each E value on one is written by the thread of its inner
   // neighbour when that takes the ordinary update; else the whole context
   // keeps Mur's own launch before the sweep
-  struct Mur { long long cell; unsigned fl; };  // a neighbour, its flag of one face and component
-  std::vector<Mur> mur;
+  struct Flag { long long key; unsigned fl; };  // key: cell
+  std::vector<Flag> flags[2];
   c->murPush = c->murmask != 0;
   for (int f = 0; f < 6 && c->murPush; ++f)
     for (int C = 0; C < 3 && c->murPush; ++C) {
@@ -112,60 +134,65 @@ template <typename T> int build_inline(Ctx *c)
               c->murPush = false;
               continue;
             }
-            mur.push_back({c->lin(nb[0], nb[1], nb[2]), (unsigned)XF_MUR << (2 * f + (C - a + 5) % 3)});
+            flags[0].push_back({c->lin(nb[0], nb[1], nb[2]), (unsigned)XF_MUR << (2 * f + (C - a + 5) % 3)});
           }
     }
-  if (!c->murPush) mur.clear();
-  std::sort(mur.begin(), mur.end(), [](const Mur &a, const Mur &b) { return a.cell < b.cell; });
-
-  // E operations but Debye, then the Debye sites: one one-pole site alone on a
-  // swept value goes to the class table, others are listed
-  auto tidy = [&](int e) {
-    std::vector<Ent> &v = c->xent[e];
-    std::sort(v.begin(), v.end(), less);
-    v.erase(std::unique(v.begin(), v.end(),
-                        [&](const Ent &a, const Ent &b) {
-                          return same(a, b) && (a.code & 7) == XO_ZERO && (b.code & 7) == XO_ZERO;
-                        }),
-            v.end());
-    // a ghost value takes its source's: what else would change it is lost
-    v.erase(std::remove_if(v.begin(), v.end(),
-                           [&](const Ent &a) {
-                             int n[3];
-                             geo.unlin(a.cell, n);
-                             return geo.ghost_dst(3 * e + a.comp, n);
-                           }),
-            v.end());
+  if (!c->murPush) flags[0].clear();
+  sort_by_key(flags[0]);
+  // whether a Mur face takes component C of a cell
+  auto feeds_mur = [&](long long cell, int C) {
+    auto it = std::lower_bound(flags[0].begin(), flags[0].end(), cell, [](const Flag &x, long long k) { return x.key < k; });
+    for (; it != flags[0].end() && it->key == cell; ++it)
+      for (int f = 0; f < 6; ++f)
+        for (int s = 0; s < 2; ++s)
+          if (((it->fl >> (XF_MUR_SHIFT + 2 * f + s)) & 1u) && (f / 2 + 1 + s) % 3 == C) return true;
+    return false;
   };
-  tidy(0);
-  tidy(1);
-  struct Simple { long long cell; int comp, med; };
-  std::vector<Simple> simple;
+
+  // operations but Debye, by value; a ghost value takes its source's, so what
+  // else would change it is lost
+  for (int e = 0; e < 2; ++e) {
+    std::vector<Ent> &v = c->xent[e];
+    sort_by_key(v);
+    size_t k = 0;
+    for (const Ent &x : v) {
+      if (k && kind(x) == XO_ZERO && kind(v[k - 1]) == XO_ZERO && v[k - 1].key == x.key) continue;
+      if (!geo.ghosts[3 * e + x.comp()].empty()) {
+        int n[3];
+        geo.unlin(x.cell(), n);
+        if (geo.ghost_dst(3 * e + x.comp(), n)) continue;
+      }
+      v[k++] = x;
+    }
+    v.resize(k);
+  }
+
+  // Debye sites: one one-pole site alone on a swept value goes to the class
+  // table, the others are operations
+  std::vector<Ctx::XSite> simple;
   long long listed = 0;
   {
     std::vector<Ctx::XSite> &st = c->xsite;
-    std::stable_sort(st.begin(), st.end(), [](const Ctx::XSite &a, const Ctx::XSite &b) {
-      return a.cell != b.cell ? a.cell < b.cell : a.comp < b.comp;
-    });
+    sort_by_key(st);
     std::vector<Ent> add;
     const std::vector<Ent> &v = c->xent[0];
     size_t q = 0;
     simple.reserve(st.size());
     for (size_t a = 0; a < st.size();) {
       size_t b = a;
-      while (b < st.size() && st[b].cell == st[a].cell && st[b].comp == st[a].comp) ++b;
-      while (q < v.size() && (v[q].cell < st[a].cell || (v[q].cell == st[a].cell && v[q].comp < st[a].comp))) ++q;
-      const bool rows = q < v.size() && v[q].cell == st[a].cell && v[q].comp == st[a].comp;
+      while (b < st.size() && st[b].key == st[a].key) ++b;
+      while (q < v.size() && v[q].value() < st[a].key) ++q;
+      const bool ops = q < v.size() && v[q].value() == st[a].key;
+      const int C = (int)(st[a].key % 3), m = st[a].med;
       int n[3];
-      geo.unlin(st[a].cell, n);
-      if (!geo.ghost_dst(st[a].comp, n)) {
-        const int m = st[a].med;
-        if (b == a + 1 && !rows && c->dsimple[m] && geo.region(st[a].comp, n) >= 0) {
-          simple.push_back({st[a].cell, st[a].comp, m});
+      geo.unlin(st[a].key / 3, n);
+      if (!geo.ghost_dst(C, n)) {
+        if (b == a + 1 && !ops && c->dsimple[m] && geo.region(C, n) >= 0) {
+          simple.push_back(st[a]);
         } else {
           for (size_t k = a; k < b; ++k) {
             if (st[k].med >= 1 << 21) return set_error(c, VGPU_EINVAL, "Debye site index out of range");
-            add.push_back({st[k].cell, (long long)k, st[k].comp, 0, XO_DEBYE | st[k].med << 8, (int)listed++, 0, 0});
+            add.push_back({st[k].key * 4, XO_DEBYE | st[k].med << 8, (int)listed++, 0, 0});
           }
         }
       }
@@ -173,29 +200,13 @@ template <typename T> int build_inline(Ctx *c)
     }
     std::vector<Ctx::XSite>().swap(st);
     c->xent[0].insert(c->xent[0].end(), add.begin(), add.end());
-    std::sort(c->xent[0].begin(), c->xent[0].end(), less);
   }
-  // zeroed E of swept values, when nothing comes before: a flag of the class
-  struct Zero { long long cell; int comp; };
-  std::vector<Zero> zero;
-  {
-    std::vector<Ent> &v = c->xent[0];
-    std::vector<Ent> keep;
-    keep.reserve(v.size());
-    for (size_t a = 0; a < v.size(); ++a) {
-      int n[3];
-      geo.unlin(v[a].cell, n);
-      if ((v[a].code & 7) == XO_ZERO && (a == 0 || !same(v[a - 1], v[a])) && geo.region(v[a].comp, n) >= 0)
-        zero.push_back({v[a].cell, v[a].comp});
-      else keep.push_back(v[a]);
-    }
-    v.swap(keep);
-  }
+
   // ghosts of every value that changes
   for (int e = 0; e < 2; ++e) {
+    sort_by_key(c->xent[e]);
     std::vector<Ent> add;
     const std::vector<Ent> &v = c->xent[e];
-    const int N[3] = {c->NX, c->NY, c->NZ};
     for (int C = 0; C < 3; ++C) {
       const auto &gs = geo.ghosts[3 * e + C];
       for (size_t g = 0; g < gs.size(); ++g) {
@@ -218,39 +229,76 @@ template <typename T> int build_inline(Ctx *c)
               if (!first) continue;
               if (geo.region(3 * e + C, n) >= 0)
                 return set_error(c, VGPU_EINVAL, "ghost plane inside the sweeps' limits");
-              const long long cell = c->lin(n[0], n[1], n[2]), src = c->lin(s[0], s[1], s[2]);
-              const Ent key{src, -1, C, -1, 0, 0, 0, 0};
-              auto it = std::lower_bound(v.begin(), v.end(), key, less);
-              if (geo.region(3 * e + C, s) < 0 && !(e == 0 && geo.mur_face(C, s, nb) >= 0) &&
-                  !(it != v.end() && it->cell == src && it->comp == C))
-                continue;
-              add.push_back({cell, 0, C, 3, XO_GHOST, (int)src, sign, 0});
+              const long long src = c->lin(s[0], s[1], s[2]), val = src * 3 + C;
+              if (geo.region(3 * e + C, s) < 0 && !(e == 0 && geo.mur_face(C, s, nb) >= 0)) {
+                auto it = std::lower_bound(v.begin(), v.end(), val, [](const Ent &x, long long k) { return x.value() < k; });
+                if (it == v.end() || it->value() != val) continue;
+              }
+              add.push_back({(c->lin(n[0], n[1], n[2]) * 3 + C) * 4 + 3, XO_GHOST, (int)src, sign, 0});
             }
       }
     }
     c->xent[e].insert(c->xent[e].end(), add.begin(), add.end());
-    std::sort(c->xent[e].begin(), c->xent[e].end(), less);
+    sort_by_key(c->xent[e]);
   }
 
-  // the cells the E sweep corrects in line, in cell order
+  // The cells the sweeps correct in line, in cell order: their flags and Debye
+  // media; and each value's operations [a, b): update rows, rows, and zeros
+  // alone on a swept value, which are a flag.  Update rows take values of the
+  // ordinary update with both neighbours inside on every axis, unless a Mur
+  // face takes them too: its thread, the sweep's, reads the old value.
+  // They pay where a launch is what a step waits for, in grids up to a million
+  // cells: 53x41x62 request 35.6 -> 28.9 us a step, 40^3 free space FP64 28.6
+  // -> 26.5.  Beyond, reading the other field's neighbours again costs more
+  // than the rows' launch: 256^3 Debye volume 497 -> 531, 173x211x158 request
+  // 204 -> 215, FP64 128^3 Debye volume 159 -> 168.
+  const bool small = c->xskip = c->ncell <= 1000000;
+  struct Value { size_t a, b; bool ghost; };
   struct Entry { int cell; int med[3]; unsigned fl; };
-  std::vector<Entry> ent;
-  auto plan = [&] {
-    ent.clear();
-    size_t qs = 0, qz = 0, qm = 0;
-    for (;;) {
-      long long cell = INT64_MAX;
-      if (qs < simple.size()) cell = std::min(cell, simple[qs].cell);
-      if (qz < zero.size()) cell = std::min(cell, zero[qz].cell);
-      if (qm < mur.size()) cell = std::min(cell, mur[qm].cell);
-      if (cell == INT64_MAX) break;
-      Entry x{(int)cell, {-1, -1, -1}, 0};
-      for (; qs < simple.size() && simple[qs].cell == cell; ++qs) {
-        x.med[simple[qs].comp] = simple[qs].med;
-        x.fl |= XF_DEBYE << simple[qs].comp;
+  std::vector<Value> upd[2], rest[2];
+  std::vector<Entry> ents[2];
+  auto plan = [&](int e) {
+    const std::vector<Ent> &v = c->xent[e];
+    std::vector<Flag> fl = flags[e];
+    upd[e].clear();
+    rest[e].clear();
+    for (size_t a = 0; a < v.size();) {
+      size_t b = a;
+      while (b < v.size() && v[b].value() == v[a].value()) ++b;
+      const long long cell = v[a].cell();
+      const int C = v[a].comp();
+      int n[3];
+      geo.unlin(cell, n);
+      const int reg = geo.region(3 * e + C, n);
+      const bool inside = n[0] > 0 && n[1] > 0 && n[2] > 0 && n[0] < N[0] - 1 && n[1] < N[1] - 1 && n[2] < N[2] - 1;
+      size_t from = a;
+      if (reg >= 0 && kind(v[a]) == XO_ZERO && (small || e == 0) && (b == a + 1 || !small || reg != 6 || !inside)) {
+        fl.push_back({cell, (unsigned)XF_ZERO << C});
+        ++from;
       }
-      for (; qz < zero.size() && zero[qz].cell == cell; ++qz) x.fl |= XF_ZERO << zero[qz].comp;
-      for (; qm < mur.size() && mur[qm].cell == cell; ++qm) x.fl |= mur[qm].fl;
+      if (from < b) {
+        if (small && reg == 6 && inside && !(e == 0 && feeds_mur(cell, C))) {
+          fl.push_back({cell, (unsigned)XF_SKIP << C});
+          upd[e].push_back({from, b, false});
+        } else {
+          rest[e].push_back({from, b, kind(v[a]) == XO_GHOST});
+        }
+      }
+      a = b;
+    }
+    sort_by_key(fl);
+    std::vector<Entry> &ent = ents[e];
+    ent.clear();
+    const size_t ns = e == 0 ? simple.size() : 0;
+    for (size_t qs = 0, qf = 0; qs < ns || qf < fl.size();) {
+      const long long cs = qs < ns ? simple[qs].key / 3 : INT64_MAX, cf = qf < fl.size() ? fl[qf].key : INT64_MAX;
+      const long long cell = std::min(cs, cf);
+      Entry x{(int)cell, {-1, -1, -1}, 0};
+      for (; qs < ns && simple[qs].key / 3 == cell; ++qs) {
+        x.med[simple[qs].key % 3] = simple[qs].med;
+        x.fl |= XF_DEBYE << simple[qs].key % 3;
+      }
+      for (; qf < fl.size() && fl[qf].key == cell; ++qf) x.fl |= fl[qf].fl;
       ent.push_back(x);
     }
   };
@@ -264,103 +312,109 @@ template <typename T> int build_inline(Ctx *c)
       return (size_t)(h ^ h >> 29);
     }
   };
-  std::vector<Kind> made;
-  std::vector<int> of;
-  auto kinds = [&](bool withOld) {
+  std::vector<Kind> made[2];
+  std::vector<int> of[2];
+  auto kinds = [&](int e, bool withOld) {
+    const std::vector<uint32_t> &cls = e == 0 ? c->ecls : c->hcls;
+    const std::vector<Entry> &ent = ents[e];
     std::unordered_map<Kind, int, Hash> ids;
-    made.clear();
-    of.resize(ent.size());
+    made[e].clear();
+    of[e].resize(ent.size());
     Kind prev{};
     int prevId = -1;
     for (size_t k = 0; k < ent.size(); ++k) {
-      const Kind key{withOld ? (int)c->ecls[ent[k].cell] : 0, ent[k].med[0], ent[k].med[1], ent[k].med[2], (int)ent[k].fl};
+      const Kind key{withOld ? (int)cls[ent[k].cell] : 0, ent[k].med[0], ent[k].med[1], ent[k].med[2], (int)ent[k].fl};
       if (prevId < 0 || key != prev) {
         auto it = ids.find(key);
         if (it == ids.end()) {
-          it = ids.emplace(key, (int)made.size()).first;
-          made.push_back(key);
+          it = ids.emplace(key, (int)made[e].size()).first;
+          made[e].push_back(key);
         }
         prev = key;
         prevId = it->second;
       }
-      of[k] = prevId;
+      of[e][k] = prevId;
     }
   };
   // Coefficient classes are kept when the flagged cells' own fit beside them:
-  // with the one-pole sites' media in them, else with those sites in rows.
-  // Without classes every site is in a row, and a flagged cell's number is
-  // its flags'.
-  const size_t baseE = c->etab.size() / 6;
-  bool indexed = baseE <= 65536 && c->htab.size() / 3 <= 65536 && !getenv("VGPU_NO_INDEXED_MEDIA");
+  // with the one-pole sites' media in them, else with those sites as
+  // operations.  Without classes every site is one, and a flagged cell's number
+  // is its flags'.
+  const size_t baseE = c->etab.size() / 6, baseH = c->htab.size() / 3;
+  bool indexed = baseE <= 65536 && baseH <= 65536 && !getenv("VGPU_NO_INDEXED_MEDIA");
   auto fits = [&] {
-    kinds(true);
-    return baseE + made.size() <= 65536;
+    kinds(0, true);
+    kinds(1, true);
+    return baseE + made[0].size() <= 65536 && baseH + made[1].size() <= 65536;
   };
-  plan();
+  plan(0);
+  plan(1);
   if (!(indexed && fits())) {
-    long long seq = 0;
-    for (const Simple &s : simple)
-      c->xent[0].push_back({s.cell, seq++, s.comp, 0, XO_DEBYE | s.med << 8, (int)listed++, 0, 0});
+    for (const Ctx::XSite &s : simple) c->xent[0].push_back({s.key * 4, XO_DEBYE | s.med << 8, (int)listed++, 0, 0});
     simple.clear();
-    std::sort(c->xent[0].begin(), c->xent[0].end(), less);
-    plan();
+    sort_by_key(c->xent[0]);
+    plan(0);
     indexed = indexed && fits();
-    if (!indexed) kinds(false);
+    if (!indexed) {
+      kinds(0, false);
+      kinds(1, false);
+    }
   }
   c->indexed = indexed;
   c->debyeSimple = (long long)simple.size();
   c->debyeSites = listed;
+  if (listed > INT32_MAX) return set_error(c, VGPU_EINVAL, "too many Debye sites");
   if (listed) {
     c->d_dlast = dev_alloc(c, (size_t)listed * c->esz);
     c->d_dJ = dev_alloc(c, (size_t)listed * c->debyeMaxPoles * (c->debyeCplx ? 2 : 1) * c->esz);
     if (!c->d_dlast || !c->d_dJ) return fail("Debye state");
   }
 
-  // rows, those with ghosts behind them in groups
   for (int e = 0; e < 2; ++e) {
     const std::vector<Ent> &v = c->xent[e];
     if (v.size() > (1u << 30) - 1) return set_error(c, VGPU_EINVAL, "too many corrections");
-    struct Row { long long src; int ghost; size_t a, b; };  // src: value the row changes, or its ghosts' source
-    std::vector<Row> R;
-    for (size_t a = 0; a < v.size();) {
-      size_t b = a;
-      while (b < v.size() && same(v[b], v[a])) ++b;
-      const bool g = (v[a].code & 7) == XO_GHOST;
-      R.push_back({(g ? v[a].arg : v[a].cell) * 3 + v[a].comp, g, a, b});
-      a = b;
-    }
-    std::vector<size_t> by(R.size());
-    for (size_t q = 0; q < by.size(); ++q) by[q] = q;
-    std::sort(by.begin(), by.end(), [&](size_t a, size_t b) {
-      return R[a].src != R[b].src ? R[a].src < R[b].src : R[a].ghost != R[b].ghost ? R[a].ghost < R[b].ghost : a < b;
-    });
+    // rows with ghosts behind them go in groups
+    struct Src { long long key; size_t q; };  // the value a row changes, or its ghosts' source
+    std::vector<Src> by;
+    const std::vector<Value> &R = rest[e];
+    bool ghosts = false;
+    for (size_t q = 0; q < R.size(); ++q) ghosts = ghosts || R[q].ghost;
     std::vector<char> grouped(R.size(), 0);
-    for (size_t a = 0; a < by.size();) {
-      size_t b = a;
-      while (b < by.size() && R[by[b]].src == R[by[a]].src) ++b;
-      if (b > a + 1 && !R[by[a]].ghost)
-        for (size_t q = a; q < b; ++q) grouped[by[q]] = 1;
-      a = b;
+    if (ghosts) {
+      for (size_t q = 0; q < R.size(); ++q) {
+        const Ent &x = v[R[q].a];
+        by.push_back({(R[q].ghost ? (long long)x.arg * 3 + x.comp() : x.value()) * 2 + R[q].ghost, q});
+      }
+      sort_by_key(by);
+      for (size_t a = 0; a < by.size();) {
+        size_t b = a;
+        while (b < by.size() && by[b].key / 2 == by[a].key / 2) ++b;
+        if (b > a + 1 && !R[by[a].q].ghost)
+          for (size_t q = a; q < b; ++q) grouped[by[q].q] = 1;
+        a = b;
+      }
     }
     std::vector<XRow> row;
     std::vector<XOp<T>> op;
     std::vector<int> gstart;
-    row.reserve(R.size() + 1);
+    row.reserve(upd[e].size() + R.size() + 1);
     op.reserve(v.size());
-    auto take = [&](const Row &r) {
-      row.push_back({(int)v[r.a].cell, (unsigned)op.size() << 2 | (unsigned)v[r.a].comp});
+    auto take = [&](const Value &r) {
+      row.push_back({(int)v[r.a].cell(), (unsigned)op.size() << 2 | (unsigned)v[r.a].comp()});
       for (size_t k = r.a; k < r.b; ++k) op.push_back({v[k].code, v[k].arg, T(v[k].a), T(v[k].b)});
     };
+    for (const Value &r : upd[e]) take(r);
+    c->nXupd[e] = (long long)row.size();
     for (size_t q = 0; q < R.size(); ++q)
       if (!grouped[q]) take(R[q]);
-    c->nXrow[e] = (long long)row.size();
-    for (size_t q = 0; q < by.size(); ++q)
-      if (grouped[by[q]]) {
-        if (!R[by[q]].ghost) gstart.push_back((int)row.size());
-        take(R[by[q]]);
+    c->nXrow[e] = (long long)row.size() - c->nXupd[e];
+    for (const Src &s : by)
+      if (grouped[s.q]) {
+        if (!R[s.q].ghost) gstart.push_back((int)(row.size() - c->nXupd[e]));
+        take(R[s.q]);
       }
     c->nXgroup[e] = (long long)gstart.size();
-    gstart.push_back((int)row.size());
+    gstart.push_back((int)(row.size() - c->nXupd[e]));
     row.push_back({0, (unsigned)op.size() << 2});
     if (!up(c->d_xgstart[e], gstart.data(), gstart.size() * sizeof(int)) ||
         !up(c->d_xrow[e], row.data(), row.size() * sizeof(XRow)) || !up(c->d_xop[e], op.data(), op.size() * sizeof(op[0])))
@@ -373,31 +427,42 @@ template <typename T> int build_inline(Ctx *c)
       if (!c->d_xvals[e] || !up(c->d_xval[e], c->xval[e].data(), c->xval[e].size() * sizeof(XVal))) return fail("values");
     }
     std::vector<XVal>().swap(c->xval[e]);
-  }
-  if (ent.empty()) return VGPU_OK;
 
-  if (!simple.empty() && !(c->d_xJ = dev_alloc(c, 3 * c->ncell * sizeof(T)))) return fail("Debye state");
-  // classes of the flagged cells: their coefficients, Debye media and flags
-  c->xflag0 = indexed ? (unsigned)baseE : 1u;
-  if (indexed) {
-    for (const Kind &k : made)
-      for (int s = 0; s < 6; ++s) c->etab.push_back(c->etab[(size_t)k[0] * 6 + s]);
-    for (size_t k = 0; k < ent.size(); ++k) c->ecls[ent[k].cell] = (uint32_t)(baseE + of[k]);
-  } else {
-    std::vector<uint16_t> f(c->ncell, 0);
-    for (size_t k = 0; k < ent.size(); ++k) f[ent[k].cell] = (uint16_t)(1 + of[k]);
-    if (!up(c->d_xcls, f.data(), f.size() * sizeof(uint16_t))) return fail("flags");
+    // classes of the flagged cells: their coefficients, Debye media and flags
+    const std::vector<Entry> &ent = ents[e];
+    if (ent.empty()) continue;
+    if (indexed) {
+      std::vector<uint32_t> &cls = e == 0 ? c->ecls : c->hcls;
+      std::vector<double> &tab = e == 0 ? c->etab : c->htab;
+      const size_t base = e == 0 ? baseE : baseH, w = e == 0 ? 6 : 3;
+      for (const Kind &k : made[e])
+        for (size_t s = 0; s < w; ++s) tab.push_back(tab[(size_t)k[0] * w + s]);
+      for (size_t k = 0; k < ent.size(); ++k) cls[ent[k].cell] = (uint32_t)(base + of[e][k]);
+    } else {
+      std::vector<uint16_t> f(c->ncell, 0);
+      for (size_t k = 0; k < ent.size(); ++k) f[ent[k].cell] = (uint16_t)(e == 0 ? 1 + of[e][k] : ent[k].fl);
+      if (!up(c->d_xcls[e], f.data(), f.size() * sizeof(uint16_t))) return fail("flags");
+    }
+    if (e == 1) {
+      c->xflagH = true;
+      c->hflags.assign(baseH, 0.0);
+      if (indexed)
+        for (const Kind &k : made[e]) c->hflags.push_back((double)k[4]);
+      continue;
+    }
+    c->xflag0 = indexed ? (unsigned)baseE : 1u;
+    std::vector<T> dt(made[e].size() * DTAB_STRIDE, T(0));
+    for (size_t k = 0; k < made[e].size(); ++k) {
+      for (int C = 0; C < 3; ++C)
+        if (made[e][k][1 + C] >= 0) {
+          dt[k * DTAB_STRIDE + 2 * C] = T(c->dhost[0][made[e][k][1 + C]]);
+          dt[k * DTAB_STRIDE + 2 * C + 1] = T(c->dhost[1][made[e][k][1 + C]]);
+        }
+      dt[k * DTAB_STRIDE + 6] = T(made[e][k][4]);
+    }
+    if (!up(c->d_xdtab, dt.data(), dt.size() * sizeof(T))) return fail("class table");
+    if (!simple.empty() && !(c->d_xJ = dev_alloc(c, 3 * c->ncell * sizeof(T)))) return fail("Debye state");
   }
-  std::vector<T> dt(made.size() * DTAB_STRIDE, T(0));
-  for (size_t k = 0; k < made.size(); ++k) {
-    for (int C = 0; C < 3; ++C)
-      if (made[k][1 + C] >= 0) {
-        dt[k * DTAB_STRIDE + 2 * C] = T(c->dhost[0][made[k][1 + C]]);
-        dt[k * DTAB_STRIDE + 2 * C + 1] = T(c->dhost[1][made[k][1 + C]]);
-      }
-    dt[k * DTAB_STRIDE + 6] = T(made[k][4]);
-  }
-  if (!up(c->d_xdtab, dt.data(), dt.size() * sizeof(T))) return fail("class table");
   return VGPU_OK;
 }
 

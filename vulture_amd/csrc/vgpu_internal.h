@@ -84,15 +84,23 @@ template <typename T> struct HArgs {
 //    thread of the face's inner neighbour writes, having both of that
 //    neighbour's values Mur's equation takes.  Such cells have coefficient
 //    classes of their own (from `flag0` on), so the others pay one comparison.
-//  - Rows: one launch per half-step, a thread per field value and its
-//    operations in the reference's order, ghosts behind the row of their
-//    source.  (Rows walked by the sweep's threads measured slower: each costs
-//    four dependent loads, one lane of a wavefront at a time at the x faces.)
+//  - Update rows, for the other operations on values of the ordinary update
+//    (TF/SF faces, sources, SIBC's H terms): the sweep leaves the value alone
+//    (a flag of the cell's class) and a thread of its own, in blocks beside
+//    the sweep's, makes the whole update and then the value's operations in
+//    the reference's order.  An update reads no value of its own kind but its
+//    own, so this needs no order between them.  (Operations walked by the
+//    sweep's threads measured slower: each costs four dependent loads, one
+//    lane of a wavefront at a time at the x faces.)
+//  - Rows, for what is left (ghost planes, values that are not ordinary
+//    updates): a launch after the sweep, a thread per value, ghosts behind the
+//    row of their source.
 enum XKind { XO_SRC, XO_AUX, XO_WAVE, XO_ZERO, XO_DEBYE, XO_GHOST, XO_SIBC };
-// flags of a flagged class (dtab slot 6): one-pole Debye sites of components
-// 0-2 (bits 0-2), zeroed components (3-5), and per Mur face f the components
-// (f/2 + 1) % 3 and (f/2 + 2) % 3 it takes from the cell (bits 6+2f, 7+2f)
-enum XFlag { XF_DEBYE = 1, XF_ZERO = 8, XF_MUR = 64 };
+// flags of a flagged class (E: dtab slot 6, H: the class table's slot 3):
+// one-pole Debye sites of components 0-2 (bits 0-2), zeroed components (3-5),
+// components left to update rows (6-8), and per Mur face f the components
+// (f/2 + 1) % 3 and (f/2 + 2) % 3 it takes from the cell (bits 9+2f, 10+2f)
+enum XFlag { XF_DEBYE = 1, XF_ZERO = 8, XF_SKIP = 64, XF_MUR = 512, XF_MUR_SHIFT = 9 };
 constexpr int DTAB_STRIDE = 8;
 
 // code: kind (bits 0-2), then
@@ -122,17 +130,18 @@ struct XVal {
 
 template <typename T> struct XArgs {
   unsigned flag0;        // first flagged class (E)
-  const uint16_t *cls;   // per cell: class, or without classes 0 / 1 + dtab row
+  const uint16_t *cls;   // per cell: class, or without classes E 0 / 1 + dtab row, H its flags
   const T *dtab;         // [class - flag0][8]: alpha, beta of J per component, flags
   T *J;                  // [cell][component] (null without one-pole sites)
   int PX;
   long long plane;
   T mzeta[6];            // Mur factors
-  long long nrow, ngroup;  // rows on their own, then groups of rows (a row and its ghosts)
+  long long nupd, nrow, ngroup;  // update rows, rows, then groups of rows (a row and its ghosts)
   const int *gstart;     // first row of each group
   const XRow *row;
   const XOp<T> *op;
   T *F[3];               // the half-step's fields
+  const T *G[3], *il[3]; // the other fields, the inverse lengths of the update
   const T *tab;          // class table (null: per-cell arrays)
   const T *ca[3], *cb[3];  // alpha and beta, or gamma in cb
   const T *val;          // source and analytic incident values
@@ -483,12 +492,12 @@ template <typename T> struct VolObsArgs {
 };
 
 // What rides along with a half-step's sweep, in blocks of its own: things the
-// sweep neither reads nor writes.  The E sweep carries the H half of the
-// observers' samples of its step, the aux grids' E update and the values of
-// its step's E sources and analytic waves (its rows, a launch later, read
-// those); the H sweep the E half of the next step's samples -- E is final
-// then -- and the aux grids' H update and H values.  A run's first E samples
-// have a launch of their own before it, and its last step takes none.
+// sweep neither reads nor writes: its update rows; in the E sweep the H half
+// of the observers' samples of its step, the aux grids' E update and the values
+// of its step's H sources and analytic waves; in the H sweep the E half of the
+// next step's samples and the next step's E values -- E is final then -- and the
+// aux grids' H update.  A run's first E samples and values have a launch of
+// their own before it, and its last step takes none.
 template <typename T> struct SideArgs {
   ObsArgs<T> o;
   VolObsArgs<T> v;
@@ -496,7 +505,7 @@ template <typename T> struct SideArgs {
   ValArgs<T> val;
   int electric;          // rides with the E sweep
   int nfb;               // 256-frequency blocks per observer
-  int b[4];              // first block past the observers, volume samples, aux grids, values
+  int b[5];              // first block past the observers, volume samples, values, aux grids, update rows
 };
 
 // ---- packed launches over several solves (vgpu_run_group) ----
@@ -628,22 +637,35 @@ struct Ctx {
   // corrections as XArgs has them: every context but those with the fused sweep
   bool inl = false;
   bool murPush = false;                      // Mur E written by its inner neighbour's thread
-  int xlevel() const { return debyeSimple ? 2 : xflag0 != ~0u ? 1 : 0; }  // in-line corrections of the E sweep
+  // in-line corrections of the E sweep: 0 none, 1 Mur and zeros, 2 Debye
+  // sites as well; 3 and 4 the same with update rows
+  int xlevel() const { return xflag0 == ~0u ? 0 : (debyeSimple ? 2 : 1) + (xskip ? 2 : 0); }
   long long debyeSimple = 0;                 // one-pole Debye sites applied from the class table
   // an operation on one field value, before rows are made of them
-  struct XEnt { long long cell, seq; int comp, order, code, arg; double a, b; };
+  // (key: ((cell * 3 + component) * 4 + order); kept in the reference's order within one key)
+  struct XEnt {
+    long long key;
+    int code, arg;
+    double a, b;
+    long long value() const { return key / 4; }
+    long long cell() const { return key / 12; }
+    int comp() const { return (int)(key / 4 % 3); }
+  };
   std::vector<XEnt> xent[2];
-  struct XSite { long long cell; int comp, med; };
+  struct XSite { long long key; int med; };  // key: cell * 3 + component
   std::vector<XSite> xsite;                  // Debye sites in block order
   long long debyeAll = 0;                    // all Debye sites
   std::vector<char> dsimple;                 // per Debye medium: one real pole
   std::vector<double> dhost[2];              // its alpha and beta (real part)
   std::vector<XVal> xval[2];
   unsigned xflag0 = ~0u;
-  void *d_xargs[2] = {}, *d_xval[2] = {}, *d_xvals[2] = {}, *d_xcls = nullptr;
+  bool xskip = false;                        // values may be left to update rows
+  bool xflagH = false;                       // some H cells are flagged (with xskip)
+  void *d_xargs[2] = {}, *d_xval[2] = {}, *d_xvals[2] = {}, *d_xcls[2] = {};
   void *d_xgstart[2] = {}, *d_xrow[2] = {}, *d_xop[2] = {};
   void *d_xdtab = nullptr, *d_xJ = nullptr;
-  long long nXval[2] = {}, nXrow[2] = {}, nXgroup[2] = {};
+  long long nXval[2] = {}, nXupd[2] = {}, nXrow[2] = {}, nXgroup[2] = {};
+  std::vector<double> hflags;                // [H class] flags
   // fused leapfrog sweep: the fast boxes are its fused box, H cells to
   // update again after the E corrections
   bool leap = false;

@@ -31,7 +31,8 @@ template <typename T> VG_DEV const VG_CONST T *cp(const VG_GLOBAL T *p) { return
 // Coefficient class tables on the device are padded to 8 (E: alpha, beta
 // per component) and 4 (H: gamma per component) entries per class, so a
 // component's (alpha, beta) pair is one aligned 2-vector load and a class's
-// three gammas one 4-vector load (two 2-vectors in FP64).
+// three gammas, with the class's correction flags, one 4-vector load (two
+// 2-vectors in FP64).
 constexpr int ETAB_STRIDE = 8, HTAB_STRIDE = 4;
 typedef float vf2 __attribute__((ext_vector_type(2)));
 typedef float vf4 __attribute__((ext_vector_type(4)));
@@ -46,18 +47,18 @@ template <typename T> VG_DEV void load_pair(const T *p, T &a, T &b)
   b = v.y;
 }
 
-template <typename T> VG_DEV void load_gammas(const T *p, T &g0, T &g1, T &g2)
+template <typename T> VG_DEV void load_gammas(const T *p, T &g0, T &g1, T &g2, T &flags)
 {
-  T u;
   load_pair(p, g0, g1);
-  load_pair(p + 2, g2, u);
+  load_pair(p + 2, g2, flags);
 }
-template <> VG_DEV void load_gammas<float>(const float *p, float &g0, float &g1, float &g2)
+template <> VG_DEV void load_gammas<float>(const float *p, float &g0, float &g1, float &g2, float &flags)
 {
   const vf4 v = *reinterpret_cast<const VG_GLOBAL vf4 *>(gp(p));
   g0 = v.x;
   g1 = v.y;
   g2 = v.z;
+  flags = v.w;
 }
 
 VG_HD bool in_box(const int *b, int i, int j, int k)
@@ -283,30 +284,51 @@ VG_DEV unsigned xcd_block()
 // what a sweep's thread does itself after its cell's update.
 // ===========================================================================
 
-// One field value's operations, in order.  Coefficients of the value's cell
-// come from its class, as the sweep's do.
-template <typename T, bool IDX, bool ELEC>
+// Coefficients of component c of a cell: alpha and beta, or gamma in be.
+template <typename T, bool IDX, bool ELEC> VG_DEV void x_coef(const VG_CONST XArgs<T> *x, int id, int c, T &al, T &be)
+{
+  if (IDX) {
+    const unsigned cl = (unsigned)gp(x->cls)[id];
+    if (ELEC) load_pair(x->tab + cl * ETAB_STRIDE + 2 * c, al, be);
+    else be = gp(x->tab)[cl * HTAB_STRIDE + c];
+  } else {
+    if (ELEC) al = gp(c == 0 ? x->ca[0] : c == 1 ? x->ca[1] : x->ca[2])[id];
+    be = gp(c == 0 ? x->cb[0] : c == 1 ? x->cb[1] : x->cb[2])[id];
+  }
+}
+
+// One field value's operations, in order, with UPD after the ordinary update
+// of it (grid.c:709-888), the operands in the sweep's order.  Coefficients of
+// the value's cell come from its class, as the sweep's do.
+template <typename T, bool IDX, bool ELEC, bool UPD>
 VG_DEV void x_row(const VG_CONST XArgs<T> *x, const VG_GLOBAL XRow *row)
 {
   const int id = row[0].cell, c = (int)(row[0].opc & 3u);
   VG_GLOBAL T *F = gp(c == 0 ? x->F[0] : c == 1 ? x->F[1] : x->F[2]);
   T v = F[id], al = T(1), be = T(0);
   const unsigned o1 = row[1].opc >> 2;
-  bool coef = false;
+  bool coef = UPD;
+  if (UPD) {
+    const int P = (int)x->plane, SJ = x->PX;
+    const int k = id / P, j = (id - k * P) / SJ, i = id - k * P - j * SJ;
+    const int a1 = c == 2 ? 0 : c + 1, a2 = c == 0 ? 2 : c - 1;
+    const int s1 = a1 == 0 ? 1 : a1 == 1 ? SJ : P, s2 = a2 == 0 ? 1 : a2 == 1 ? SJ : P;
+    const VG_GLOBAL T *G1 = gp(a1 == 0 ? x->G[0] : a1 == 1 ? x->G[1] : x->G[2]);
+    const VG_GLOBAL T *G2 = gp(a2 == 0 ? x->G[0] : a2 == 1 ? x->G[1] : x->G[2]);
+    const T l1 = gp(a1 == 0 ? x->il[0] : a1 == 1 ? x->il[1] : x->il[2])[a1 == 0 ? i : a1 == 1 ? j : k];
+    const T l2 = gp(a2 == 0 ? x->il[0] : a2 == 1 ? x->il[1] : x->il[2])[a2 == 0 ? i : a2 == 1 ? j : k];
+    const T g1 = G1[id], g2 = G2[id], n1 = G1[ELEC ? id - s2 : id + s2], n2 = G2[ELEC ? id - s1 : id + s1];
+    x_coef<T, IDX, ELEC>(x, id, c, al, be);
+    if (ELEC) v = al * v + be * (l1 * (g2 - n2) + l2 * (n1 - g1));
+    else v = v + be * (l2 * (n1 - g1) + l1 * (g2 - n2));
+  }
   for (unsigned o = row[0].opc >> 2; o < o1; ++o) {
     const VG_GLOBAL XOp<T> *po = gp(x->op) + o;
     const struct { int code, arg; T a, b; } op{po->code, po->arg, po->a, po->b};
     const int kind = op.code & 7;
     if (kind != XO_ZERO && kind != XO_GHOST && !coef) {
       coef = true;
-      if (IDX) {
-        const unsigned cl = (unsigned)gp(x->cls)[id];
-        if (ELEC) load_pair(x->tab + cl * ETAB_STRIDE + 2 * c, al, be);
-        else be = gp(x->tab)[cl * HTAB_STRIDE + c];
-      } else {
-        if (ELEC) al = gp(c == 0 ? x->ca[0] : c == 1 ? x->ca[1] : x->ca[2])[id];
-        be = gp(c == 0 ? x->cb[0] : c == 1 ? x->cb[1] : x->cb[2])[id];
-      }
+      x_coef<T, IDX, ELEC>(x, id, c, al, be);
     }
     if (kind == XO_ZERO) {
       v = T(0);
@@ -356,13 +378,20 @@ VG_DEV void x_row(const VG_CONST XArgs<T> *x, const VG_GLOBAL XRow *row)
 template <typename T, bool IDX, bool ELEC> VG_DEV void x_rows(const VG_CONST XArgs<T> *x, unsigned b)
 {
   const long long q = b * 256ll + threadIdx.x;
-  const VG_GLOBAL XRow *row = gp(x->row);
+  const VG_GLOBAL XRow *row = gp(x->row) + x->nupd;
   if (q < x->nrow) {
-    x_row<T, IDX, ELEC>(x, row + q);
+    x_row<T, IDX, ELEC, false>(x, row + q);
   } else if (q < x->nrow + x->ngroup) {
     const VG_GLOBAL int *gs = gp(x->gstart) + (q - x->nrow);
-    for (int r = gs[0], r1 = gs[1]; r < r1; ++r) x_row<T, IDX, ELEC>(x, row + r);
+    for (int r = gs[0], r1 = gs[1]; r < r1; ++r) x_row<T, IDX, ELEC, false>(x, row + r);
   }
+}
+
+// An update row.
+template <typename T, bool IDX, bool ELEC> VG_DEV void x_update(const VG_CONST XArgs<T> *x, unsigned b)
+{
+  const long long q = b * 256ll + threadIdx.x;
+  if (q < x->nupd) x_row<T, IDX, ELEC, true>(x, gp(x->row) + q);
 }
 
 template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) void k_rows(const XArgs<T> *x)
@@ -407,7 +436,7 @@ template <typename T> struct XPre {
       for (int c = 0; c < 6; ++c) d[c] = q[c];
     }
     if (fl >= XF_MUR) {
-      const int f = (__ffs((int)(fl >> 6)) - 1) >> 1;
+      const int f = (__ffs((int)(fl >> XF_MUR_SHIFT)) - 1) >> 1;
       const long long at = mur_at(x, id, f);
       m0 = mur_e(x, f, 0)[at];
       m1 = mur_e(x, f, 1)[at];
@@ -425,7 +454,7 @@ VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, XPre<T> &p, T o
 {
   const unsigned fl = p.fl;
   bool first = true;
-  for (unsigned m = fl >> 6; m;) {
+  for (unsigned m = fl >> XF_MUR_SHIFT; m;) {
     const int f = (__ffs((int)m) - 1) >> 1, a = f >> 1;
     const unsigned on = (m >> (2 * f)) & 3u;
     m &= ~(3u << (2 * f));
@@ -461,7 +490,8 @@ VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, XPre<T> &p, T o
 VG_DEV void visit(unsigned *v, long long id) { atomicAdd(v + id, 1u); }
 
 // Fast E tile: inner grid (grid.c:709-797).  X: in-line corrections, 0 none,
-// 1 Mur faces and zeroed E, 2 Debye sites as well.
+// 1 Mur faces and zeroed E, 2 Debye sites as well, 3 and 4 the same with
+// values left to update rows.
 // L is the logical block (in XCD order).  All three components are computed
 // before any is stored, so the stores do not hold back the next component's
 // loads.
@@ -494,7 +524,7 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
     const unsigned cls = cnext;
     XPre<T> pre{};
     const bool flagged = X && cls >= flag0;
-    if (flagged) pre.template load<X == 2>(x, id, cls);
+    if (flagged) pre.template load<(X == 2 || X == 4)>(x, id, cls);
     const T hx = Hx[id], hy = Hy[id], hz = Hz[id];
     const T hzy = Hz[id - SJ], hzx = Hz[id - 1], hyx = Hy[id - 1], hxy = Hx[id - SJ];
     if (pc) cnext = (unsigned)pc[id + P];
@@ -522,10 +552,10 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
         visit(f.vis[1], id);
         visit(f.vis[2], id);
       } else {
-        if (flagged) x_inline_e<T, X == 2>(x, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
-        f.E[0][id] = e0;
-        f.E[1][id] = e1;
-        f.E[2][id] = e2;
+        if (flagged) x_inline_e<T, (X == 2 || X == 4)>(x, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
+        if (X < 3 || !(pre.fl & XF_SKIP)) f.E[0][id] = e0;
+        if (X < 3 || !(pre.fl & (XF_SKIP << 1))) f.E[1][id] = e1;
+        if (X < 3 || !(pre.fl & (XF_SKIP << 2))) f.E[2][id] = e2;
       }
     }
     hxm = hx;
@@ -540,7 +570,8 @@ __global__ __launch_bounds__(512) void k_e_fast(FastE<T> f, const XArgs<T> *x)
 }
 
 // Fast H tile: inner grid (grid.c:800-888).
-template <typename T, bool IDX, bool CHK> VG_DEV void h_fast_tile(const FastH<T> &f, unsigned L)
+// X: some H are zeroed or left to update rows.
+template <typename T, bool IDX, bool X, bool CHK> VG_DEV void h_fast_tile(const FastH<T> &f, unsigned L)
 {
   int bx, by, bz;
   if (!fast_block(L, f.nchx, f.gy, f.gz, f.per, true, bx, by, bz)) return;
@@ -560,33 +591,40 @@ template <typename T, bool IDX, bool CHK> VG_DEV void h_fast_tile(const FastH<T>
   long long id = ((long long)kb * f.NY + j) * SJ + ic;
   // The fast box ends at index N-2 or less, so i+1, j+1 and k+1 are inside.
   T ex = Ex[id], ey = Ey[id];
-  unsigned cnext = IDX ? (unsigned)f.hcls[id] : 0u;  // a plane ahead, as in the E tile
+  unsigned cnext = IDX || X ? (unsigned)f.hcls[id] : 0u;  // a plane ahead, as in the E tile
   for (int k = kb; k < ke; ++k, id += P) {
     const unsigned cls = cnext;
     const T exp1 = Ex[id + P], eyp1 = Ey[id + P];
     const T ez = Ez[id], ezy = Ez[id + SJ], ezx = Ez[id + 1], exy = Ex[id + SJ], eyx = Ey[id + 1];
-    if (IDX) cnext = (unsigned)f.hcls[id + P];
+    if (IDX || X) cnext = (unsigned)f.hcls[id + P];
     const T idez = cp(f.ide[2])[k];
     T g0, g1, g2;
+    unsigned fl = 0u;
     if (IDX) {
-      load_gammas(f.htab + cls * HTAB_STRIDE, g0, g1, g2);
+      T u;
+      load_gammas(f.htab + cls * HTAB_STRIDE, g0, g1, g2, u);
+      if (X) fl = (unsigned)u;
     } else {
       g0 = f.gamma[0][id];
       g1 = f.gamma[1][id];
       g2 = f.gamma[2][id];
+      if (X) fl = cls;
     }
-    const T h0 = I0[id] + g0 * (idez * (eyp1 - ey) + idey * (ez - ezy));
-    const T h1 = I1[id] + g1 * (idex * (ezx - ez) + idez * (ex - exp1));
-    const T h2 = I2[id] + g2 * (idey * (exy - ex) + idex * (ey - eyx));
+    T h0 = I0[id] + g0 * (idez * (eyp1 - ey) + idey * (ez - ezy));
+    T h1 = I1[id] + g1 * (idex * (ezx - ez) + idez * (ex - exp1));
+    T h2 = I2[id] + g2 * (idey * (exy - ex) + idex * (ey - eyx));
     if (vx) {
       if (CHK) {
         visit(f.vis[0], id);
         visit(f.vis[1], id);
         visit(f.vis[2], id);
       } else {
-        H0[id] = h0;
-        H1[id] = h1;
-        H2[id] = h2;
+        if (fl & XF_ZERO) h0 = T(0);
+        if (fl & (XF_ZERO << 1)) h1 = T(0);
+        if (fl & (XF_ZERO << 2)) h2 = T(0);
+        if (!(fl & XF_SKIP)) H0[id] = h0;
+        if (!(fl & (XF_SKIP << 1))) H1[id] = h1;
+        if (!(fl & (XF_SKIP << 2))) H2[id] = h2;
       }
     }
     ex = exp1;
@@ -594,9 +632,9 @@ template <typename T, bool IDX, bool CHK> VG_DEV void h_fast_tile(const FastH<T>
   }
 }
 
-template <typename T, bool IDX, bool CHK = false> __global__ __launch_bounds__(512) void k_h_fast(FastH<T> f)
+template <typename T, bool IDX, bool X, bool CHK = false> __global__ __launch_bounds__(512) void k_h_fast(FastH<T> f)
 {
-  h_fast_tile<T, IDX, CHK>(f, blockIdx.x);
+  h_fast_tile<T, IDX, X, CHK>(f, blockIdx.x);
 }
 
 // ===========================================================================
@@ -629,7 +667,8 @@ template <typename T, bool IDX>
 VG_DEV void leap_gammas(const LeapArgs<T> &a, unsigned cls, int id, T &g0, T &g1, T &g2)
 {
   if (IDX) {
-    load_gammas(a.htab + cls * HTAB_STRIDE, g0, g1, g2);
+    T u;
+    load_gammas(a.htab + cls * HTAB_STRIDE, g0, g1, g2, u);
   } else {
     g0 = a.gamma[0][id];
     g1 = a.gamma[1][id];
@@ -822,7 +861,8 @@ template <typename T, bool IDX> __global__ __launch_bounds__(256) void k_h_fix(F
   const T idex = a.ide[0][i], idey = a.ide[1][j], idez = a.ide[2][k];
   T g0, g1, g2;
   if (IDX) {
-    load_gammas(a.htab + (unsigned)a.hcls[id] * HTAB_STRIDE, g0, g1, g2);
+    T u;
+    load_gammas(a.htab + (unsigned)a.hcls[id] * HTAB_STRIDE, g0, g1, g2, u);
   } else {
     g0 = a.gamma[0][id];
     g1 = a.gamma[1][id];
@@ -1035,7 +1075,7 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
     const int n3[3] = {i, j, k};
     XPre<T> pre{};
     const bool flagged = X && cls >= flag0;
-    if (flagged) pre.template load<X == 2>(x, id, cls);
+    if (flagged) pre.template load<(X == 2 || X == 4)>(x, id, cls);
     c0.load(g, rg[0], n3, id, cls);
     c1.load(g, rg[1], n3, id, cls);
     c2.load(g, rg[2], n3, id, cls);
@@ -1046,10 +1086,10 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
       T e0 = c0.value(g, rg[0], idh1 * (hz - hzy) + idh2 * (hym - hy));
       T e1 = c1.value(g, rg[1], idh2 * (hx - hxm) + idh0 * (hzx - hz));
       T e2 = c2.value(g, rg[2], idh0 * (hy - hyx) + idh1 * (hxy - hx));
-      if (flagged) x_inline_e<T, X == 2>(x, id, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
-      if (rg[0].reg >= 0) g.E[0][id] = e0;
-      if (rg[1].reg >= 0) g.E[1][id] = e1;
-      if (rg[2].reg >= 0) g.E[2][id] = e2;
+      if (flagged) x_inline_e<T, (X == 2 || X == 4)>(x, id, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
+      if (rg[0].reg >= 0 && (X < 3 || !(pre.fl & XF_SKIP))) g.E[0][id] = e0;
+      if (rg[1].reg >= 0 && (X < 3 || !(pre.fl & (XF_SKIP << 1)))) g.E[1][id] = e1;
+      if (rg[2].reg >= 0 && (X < 3 || !(pre.fl & (XF_SKIP << 2)))) g.E[2][id] = e2;
     }
     hxm = hx;
     hym = hy;
@@ -1126,19 +1166,21 @@ template <typename T, bool IDX, int C> struct HShellCell {
       coef(q, n3, true);
     }
   }
-  VG_DEV void store(const HShellPtrs<T> &q, const LaneRegion &rg, long long id, T curl) const
+  VG_DEV void store(const HShellPtrs<T> &q, const LaneRegion &rg, long long id, unsigned fl, T curl) const
   {
     if (rg.reg == 6) {
-      q.H[C][id] = h + g * curl;
+      const T v = h + g * curl;
+      if (!(fl & (XF_SKIP << C))) q.H[C][id] = fl & (XF_ZERO << C) ? T(0) : v;
     } else if (rg.reg >= 0) {
       const T bn = cf[0] * ob + g * cf[1] * curl;
+      const T v = cf[2] * h + cf[3] * cf[4] * (bn - cf[5] * ob);
       q.B[rg.q] = bn;
-      q.H[C][id] = cf[2] * h + cf[3] * cf[4] * (bn - cf[5] * ob);
+      if (!(fl & (XF_SKIP << C))) q.H[C][id] = fl & (XF_ZERO << C) ? T(0) : v;
     }
   }
 };
 
-template <typename T, bool IDX, bool CHK, bool SEP>
+template <typename T, bool IDX, bool X, bool CHK, bool SEP>
 VG_DEV void h_shell_column(const ShellDev *pcs, const ShellWork *work, const HArgs<T> *ap, unsigned b)
 {
   const VG_CONST ShellDev *pc;
@@ -1167,10 +1209,11 @@ VG_DEV void h_shell_column(const ShellDev *pcs, const ShellWork *work, const HAr
     c1.init(q, rg[1], n3);
     c2.init(q, rg[2], n3);
   }
-  unsigned cnext = IDX ? (unsigned)q.hcls[id] : 0u;
+  unsigned cnext = IDX || X ? (unsigned)q.hcls[id] : 0u;
   for (int dk = dk0; dk < dk1; ++dk, ++k, id += P) {
     const unsigned cls = cnext;
-    if (IDX && dk + 1 < dk1) cnext = (unsigned)q.hcls[id + P];
+    if ((IDX || X) && dk + 1 < dk1) cnext = (unsigned)q.hcls[id + P];
+    const unsigned fl = !X ? 0u : IDX ? (unsigned)q.htab[cls * HTAB_STRIDE + 3] : cls;
     const bool zin = k + 1 < NZ;
     const T exp1 = zin ? Ex[id + P] : T(0), eyp1 = zin ? Ey[id + P] : T(0);
     const T ez = Ez[id], ezy = yin ? Ez[id + SJ] : T(0), ezx = xin ? Ez[id + 1] : T(0);
@@ -1184,9 +1227,9 @@ VG_DEV void h_shell_column(const ShellDev *pcs, const ShellWork *work, const HAr
       for (int C = 0; C < 3; ++C)
         if (rg[C].reg >= 0) visit(a.vis[C], id);
     } else {
-      c0.store(q, rg[0], id, ide2 * (eyp1 - eyc) + ide1 * (ez - ezy));
-      c1.store(q, rg[1], id, ide0 * (ezx - ez) + ide2 * (exc - exp1));
-      c2.store(q, rg[2], id, ide1 * (exy - exc) + ide0 * (eyc - eyx));
+      c0.store(q, rg[0], id, fl, ide2 * (eyp1 - eyc) + ide1 * (ez - ezy));
+      c1.store(q, rg[1], id, fl, ide0 * (ezx - ez) + ide2 * (exc - exp1));
+      c2.store(q, rg[2], id, fl, ide1 * (exy - exc) + ide0 * (eyc - eyx));
     }
     exc = exp1;
     eyc = eyp1;
@@ -1199,7 +1242,7 @@ VG_DEV void h_shell_column(const ShellDev *pcs, const ShellWork *work, const HAr
 template <typename T, bool IDX, bool CHK = false>
 __global__ __launch_bounds__(256) void k_h_shell(const ShellDev *pcs, const ShellWork *work, const HArgs<T> *ap)
 {
-  h_shell_column<T, IDX, CHK, true>(pcs, work, ap, blockIdx.x);
+  h_shell_column<T, IDX, false, CHK, true>(pcs, work, ap, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1672,26 +1715,33 @@ template <typename T, int C0> VG_DEV void sample_block(const SideArgs<T> &a, int
   else observe_volume_node<T, C0, 3>(a.v, (b - a.b[0]) * 256ll + threadIdx.x, n);
 }
 
+// Samples and values of step n, one block of b < a.b[2].
+template <typename T, int C0> VG_DEV void sample_value_block(const SideArgs<T> &a, int b, unsigned long long n, double pi)
+{
+  if (b < a.b[1]) sample_block<T, C0>(a, b, n);
+  else value_block(a.val, n, a.o.dt, pi, b - a.b[1]);
+}
+
 // A side block of step `soff` of the run.
-template <typename T, bool ELEC>
-VG_DEV void side_block(const SideArgs<T> &a, int b, int soff, bool last, double pi)
+template <typename T, bool IDX, bool ELEC, bool UPD>
+VG_DEV void side_block(const SideArgs<T> &a, const VG_CONST XArgs<T> *x, int b, int soff, bool last, double pi)
 {
   const unsigned long long n = *a.o.step + (unsigned long long)soff;
-  if (b < a.b[1]) {
-    if (ELEC) sample_block<T, 3>(a, b, n);
-    else if (!last) sample_block<T, 0>(a, b, n + 1);
-  } else if (b < a.b[2]) {
-    if (ELEC) aux_e_block(a.x, b - a.b[1], (double)n * a.x.dt, pi);
-    else aux_h_block(a.x, b - a.b[1]);
+  if (b < a.b[2]) {
+    if (ELEC) sample_value_block<T, 3>(a, b, n, pi);
+    else if (!last) sample_value_block<T, 0>(a, b, n + 1, pi);
   } else if (b < a.b[3]) {
-    value_block(a.val, n, a.o.dt, pi, b - a.b[2]);
+    if (ELEC) aux_e_block(a.x, b - a.b[2], (double)n * a.x.dt, pi);
+    else aux_h_block(a.x, b - a.b[2]);
+  } else if (UPD && b < a.b[4]) {
+    x_update<T, IDX, ELEC>(x, (unsigned)(b - a.b[3]));
   }
 }
 
-// The E samples of a run's first step.
-template <typename T> __global__ __launch_bounds__(256) void k_first_samples(SideArgs<T> a)
+// The E samples and values of a run's first step.
+template <typename T> __global__ __launch_bounds__(256) void k_first_samples(SideArgs<T> a, double pi)
 {
-  sample_block<T, 0>(a, (int)blockIdx.x, *a.o.step);
+  sample_value_block<T, 0>(a, (int)blockIdx.x, *a.o.step, pi);
 }
 
 // A half-step's sweep: the side blocks, the shell's (each a multiple of eight,
@@ -1703,20 +1753,20 @@ __global__ __launch_bounds__(256) void k_e_sweep(FastE<T> f, const ShellDev *pcs
                                                  SideArgs<T> sd, int soff, int last, double pi)
 {
   const unsigned b = blockIdx.x, n1 = nSide + nShell;
-  if (b < nSide) side_block<T, true>(sd, (int)b, soff, last, pi);
+  if (b < nSide) side_block<T, IDX, true, (X >= 3)>(sd, cp(x), (int)b, soff, last, pi);
   else if (b < n1) e_shell_column<T, IDX, X, false, false>(pcs, work, ap, cp(x), b - nSide);
   else e_fast_tile<T, IDX, X, false>(f, cp(x), b - n1);
 }
 
-template <typename T, bool IDX>
+template <typename T, bool IDX, bool X>
 __global__ __launch_bounds__(256) void k_h_sweep(FastH<T> f, const ShellDev *pcs, const ShellWork *work,
-                                                 const HArgs<T> *ap, unsigned nSide, unsigned nShell, SideArgs<T> sd,
-                                                 int soff, int last, double pi)
+                                                 const HArgs<T> *ap, const XArgs<T> *x, unsigned nSide, unsigned nShell,
+                                                 SideArgs<T> sd, int soff, int last, double pi)
 {
   const unsigned b = blockIdx.x, n1 = nSide + nShell;
-  if (b < nSide) side_block<T, false>(sd, (int)b, soff, last, pi);
-  else if (b < n1) h_shell_column<T, IDX, false, false>(pcs, work, ap, b - nSide);
-  else h_fast_tile<T, IDX, false>(f, b - n1);
+  if (b < nSide) side_block<T, IDX, false, X>(sd, cp(x), (int)b, soff, last, pi);
+  else if (b < n1) h_shell_column<T, IDX, X, false, false>(pcs, work, ap, b - nSide);
+  else h_fast_tile<T, IDX, X, false>(f, b - n1);
 }
 
 // Ghost plane copy for one face (surface.c:569-812).
@@ -1774,7 +1824,7 @@ template <typename T, bool IDX, int X> __global__ __launch_bounds__(256) void k_
   const VG_CONST PackArgs<T> *a = pack_args<T>(m, d);
   const unsigned b = blockIdx.x - m.start[d], nSide = a->nEside, n1 = nSide + a->nEshell;
   if (b < nSide) {
-    side_block<T, true>(ld_args(&a->se), (int)b, m.soff, m.last, pi);
+    side_block<T, IDX, true, (X >= 3)>(ld_args(&a->se), cp(a->xe), (int)b, m.soff, m.last, pi);
   } else if (b < n1) {
     e_shell_column<T, IDX, X, false, false>(a->epc, a->ewk, a->ea, cp(a->xe), b - nSide);
   } else {
@@ -1783,26 +1833,26 @@ template <typename T, bool IDX, int X> __global__ __launch_bounds__(256) void k_
   }
 }
 
-template <typename T, bool IDX> __global__ __launch_bounds__(256) void k_h_sweep_pk(PackMap m, double pi)
+template <typename T, bool IDX, bool X> __global__ __launch_bounds__(256) void k_h_sweep_pk(PackMap m, double pi)
 {
   const int d = pack_member(m, blockIdx.x);
   const VG_CONST PackArgs<T> *a = pack_args<T>(m, d);
   const unsigned b = blockIdx.x - m.start[d], nSide = a->nHside, n1 = nSide + a->nHshell;
   if (b < nSide) {
-    side_block<T, false>(ld_args(&a->sh), (int)b, m.soff, m.last, pi);
+    side_block<T, IDX, false, X>(ld_args(&a->sh), cp(a->xh), (int)b, m.soff, m.last, pi);
   } else if (b < n1) {
-    h_shell_column<T, IDX, false, false>(a->hpc, a->hwk, a->ha, b - nSide);
+    h_shell_column<T, IDX, X, false, false>(a->hpc, a->hwk, a->ha, b - nSide);
   } else {
     const FastH<T> f = ld_args(&a->fh);
-    h_fast_tile<T, IDX, false>(f, b - n1);
+    h_fast_tile<T, IDX, X, false>(f, b - n1);
   }
 }
 
-template <typename T> __global__ __launch_bounds__(256) void k_first_samples_pk(PackMap m)
+template <typename T> __global__ __launch_bounds__(256) void k_first_samples_pk(PackMap m, double pi)
 {
   const int d = pack_member(m, blockIdx.x);
   const SideArgs<T> a = ld_args(&pack_args<T>(m, d)->sh);
-  sample_block<T, 0>(a, (int)(blockIdx.x - m.start[d]), *a.o.step);
+  sample_value_block<T, 0>(a, (int)(blockIdx.x - m.start[d]), *a.o.step, pi);
 }
 
 template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) void k_rows_pk(PackMap m)

@@ -65,7 +65,8 @@ template <typename T> static void fill_volume_args(Ctx *c, EArgs<T> &ea, HArgs<T
     ha.ibd[d] = P<T>(c->prof[4][d]);
   }
   ea.ecls = P<uint16_t>(c->d_ecls); ea.etab = P<T>(c->d_etab);
-  ha.hcls = P<uint16_t>(c->d_hcls); ha.htab = P<T>(c->d_htab);
+  // (without classes the H cells' flags, when some are flagged)
+  ha.hcls = P<uint16_t>(c->indexed ? c->d_hcls : c->d_xcls[1]); ha.htab = P<T>(c->d_htab);
   ea.pmlmask = ha.pmlmask = c->pmlmask;
   for (int r = 0; r < 6; ++r)
     for (int d = 0; d < 3; ++d) {
@@ -357,12 +358,14 @@ static int plan_shells(Ctx *c, int kcPlan, std::vector<ShellDev> &ep, std::vecto
 // Argument block of the corrections of half-step e.
 template <typename T> static void fill_correction_args(Ctx *c, XArgs<T> &x, int e)
 {
-  x.cls = P<uint16_t>(c->indexed ? (e == 0 ? c->d_ecls : c->d_hcls) : c->d_xcls);
+  x.cls = P<uint16_t>(c->indexed ? (e == 0 ? c->d_ecls : c->d_hcls) : c->d_xcls[e]);
   x.PX = c->PX; x.plane = c->plane;
-  x.nrow = c->nXrow[e]; x.ngroup = c->nXgroup[e];
+  x.nupd = c->nXupd[e]; x.nrow = c->nXrow[e]; x.ngroup = c->nXgroup[e];
   x.gstart = P<int>(c->d_xgstart[e]); x.row = P<XRow>(c->d_xrow[e]); x.op = P<XOp<T>>(c->d_xop[e]);
   for (int d = 0; d < 3; ++d) {
     x.F[d] = P<T>(c->fld(0, 3 * e + d));
+    x.G[d] = P<T>(c->fld(0, 3 - 3 * e + d));
+    x.il[d] = P<T>(e == 0 ? c->idh[d] : c->ide[d]);
     x.ca[d] = P<T>(e == 0 ? c->alpha[d] : nullptr);
     x.cb[d] = P<T>(e == 0 ? c->beta[d] : c->gamma[d]);
   }
@@ -758,15 +761,17 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
     d.o = oa[0];
     d.v = va[0];
     d.x = xa;
-    d.val.n = c->nXval[e]; d.val.v = P<XVal>(c->d_xval[e]); d.val.out = P<T>(c->d_xvals[e]);
-    d.val.wf = P<WaveformDev>(c->d_wf); d.val.half = e == 0 ? 0.0 : 0.5;
+    const int v = 1 - e;  // the E sweep evaluates H values, the H sweep the next step's E values
+    d.val.n = c->nXval[v]; d.val.v = P<XVal>(c->d_xval[v]); d.val.out = P<T>(c->d_xvals[v]);
+    d.val.wf = P<WaveformDev>(c->d_wf); d.val.half = v == 0 ? 0.0 : 0.5;
     d.electric = e == 0;
     d.nfb = (maxnf + 255) / 256;
     d.b[0] = d.o.nobs * d.nfb;
     d.b[1] = d.b[0] + (int)((d.v.nnodes + 255) / 256);
-    d.b[2] = d.b[1] + (anyAux ? xa.npw : 0);
-    d.b[3] = d.b[2] + (int)((d.val.n + 255) / 256);
-    A.nside[e] = (unsigned)(d.b[3] + 7) / 8 * 8;
+    d.b[2] = d.b[1] + (int)((d.val.n + 255) / 256);
+    d.b[3] = d.b[2] + (anyAux ? xa.npw : 0);
+    d.b[4] = d.b[3] + (int)((c->nXupd[e] + 255) / 256);
+    A.nside[e] = (unsigned)(d.b[4] + 7) / 8 * 8;
   }
 }
 
@@ -826,6 +831,7 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     const int x = c->xlevel();
     if (chk && c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 0, true>), eg1, vblk, 0, s, f, xe);
     else if (chk) hipLaunchKernelGGL((k_e_fast<T, false, 0, true>), eg1, vblk, 0, s, f, xe);
+    // (grids whose fast tiles launch apart have no update rows)
     else if (c->indexed && x == 2) hipLaunchKernelGGL((k_e_fast<T, true, 2>), eg1, vblk, 0, s, f, xe);
     else if (c->indexed && x == 1) hipLaunchKernelGGL((k_e_fast<T, true, 1>), eg1, vblk, 0, s, f, xe);
     else if (c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 0>), eg1, vblk, 0, s, f, xe);
@@ -844,10 +850,10 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   auto fast_h = [&](int q) {
     const FastH<T> &f = fh[q];
     if (!hgrid.x) return;
-    if (chk && c->indexed) hipLaunchKernelGGL((k_h_fast<T, true, true>), hg1, vblk, 0, s, f);
-    else if (chk) hipLaunchKernelGGL((k_h_fast<T, false, true>), hg1, vblk, 0, s, f);
-    else if (c->indexed) hipLaunchKernelGGL((k_h_fast<T, true>), hg1, vblk, 0, s, f);
-    else hipLaunchKernelGGL((k_h_fast<T, false>), hg1, vblk, 0, s, f);
+    if (chk && c->indexed) hipLaunchKernelGGL((k_h_fast<T, true, false, true>), hg1, vblk, 0, s, f);
+    else if (chk) hipLaunchKernelGGL((k_h_fast<T, false, false, true>), hg1, vblk, 0, s, f);
+    else if (c->indexed) hipLaunchKernelGGL((k_h_fast<T, true, false>), hg1, vblk, 0, s, f);
+    else hipLaunchKernelGGL((k_h_fast<T, false, false>), hg1, vblk, 0, s, f);
   };
   auto shell_h = [&](int q) {
     const HArgs<T> *a = hap[q];
@@ -868,17 +874,24 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     const int x = c->xlevel();
     const FastE<T> &f = fe[0];
     const SideArgs<T> &sd = A.side[0];
-    if (c->indexed && x == 2) hipLaunchKernelGGL((k_e_sweep<T, true, 2>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
-    else if (c->indexed && x == 1) hipLaunchKernelGGL((k_e_sweep<T, true, 1>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
-    else if (c->indexed) hipLaunchKernelGGL((k_e_sweep<T, true, 0>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
-    else hipLaunchKernelGGL((k_e_sweep<T, false, 1>), g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi);
+    auto go = [&](auto k) { hipLaunchKernelGGL(k, g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi); };
+    if (!c->indexed) go(k_e_sweep<T, false, 3>);
+    else if (x == 0) go(k_e_sweep<T, true, 0>);
+    else if (x == 1) go(k_e_sweep<T, true, 1>);
+    else if (x == 2) go(k_e_sweep<T, true, 2>);
+    else if (x == 3) go(k_e_sweep<T, true, 3>);
+    else go(k_e_sweep<T, true, 4>);
   };
   auto sweep_h = [&](int soff, int last) {
     const unsigned ns = A.nside[1], nw = (unsigned)c->nHwork;
     const dim3 b(256), g(ns + nw + (apart ? 0u : hg1.x));
     if (!g.x) return;
-    if (c->indexed) hipLaunchKernelGGL((k_h_sweep<T, true>), g, b, 0, s, fh[0], hpc, hwk, hap[0], ns, nw, A.side[1], soff, last, pi);
-    else hipLaunchKernelGGL((k_h_sweep<T, false>), g, b, 0, s, fh[0], hpc, hwk, hap[0], ns, nw, A.side[1], soff, last, pi);
+    const SideArgs<T> &sd = A.side[1];
+    auto go = [&](auto k) { hipLaunchKernelGGL(k, g, b, 0, s, fh[0], hpc, hwk, hap[0], xh, ns, nw, sd, soff, last, pi); };
+    if (c->indexed && c->xflagH) go(k_h_sweep<T, true, true>);
+    else if (c->indexed) go(k_h_sweep<T, true, false>);
+    else if (c->xflagH) go(k_h_sweep<T, false, true>);
+    else go(k_h_sweep<T, false, false>);
   };
   auto rows = [&](int e) {
     const dim3 b(256), g((unsigned)((c->nXrow[e] + c->nXgroup[e] + 255) / 256));
@@ -969,8 +982,8 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   // own state, so their place before the H sweep is all that matters; so
   // with Mur faces their inner neighbours' threads cannot write, which read
   // the old E.
-  if (c->inl && nsteps && A.side[1].b[1])
-    hipLaunchKernelGGL(k_first_samples<T>, dim3((unsigned)A.side[1].b[1]), dim3(256), 0, s, A.side[1]);
+  if (c->inl && nsteps && A.side[1].b[2])
+    hipLaunchKernelGGL(k_first_samples<T>, dim3((unsigned)A.side[1].b[2]), dim3(256), 0, s, A.side[1], pi);
   for (uint64_t n = 0; c->inl && n < nsteps; ++n) {
     const int soff = (int)n, last = n + 1 == nsteps;
     if (c->murmask && !c->murPush) hipLaunchKernelGGL(k_mur_e<T>, murGrid, dim3(16, 16), 0, s, ma[0]);
@@ -1136,42 +1149,46 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
   };
   // packs by kernel form: with classes, the E sweep's by the level of its
   // in-line corrections
-  PackMap sweepE[4], sweepH[2], rowE[2], rowH[2];
-  for (int x = 0; x < 4; ++x)
+  PackMap sweepE[6], sweepH[4], rowE[2], rowH[2];
+  for (int x = 0; x < 6; ++x)
     sweepE[x] = plan([&](int i) {
-      return (cs[i]->indexed ? cs[i]->xlevel() : 3) == x ? (long long)A[i].nside[0] + cs[i]->nEworkPk + A[i].eg1.x : 0LL; });
+      return (cs[i]->indexed ? cs[i]->xlevel() : 5) == x ? (long long)A[i].nside[0] + cs[i]->nEworkPk + A[i].eg1.x : 0LL; });
   for (int x = 0; x < 2; ++x) {
     const bool idx = x == 0;
-    sweepH[x] = plan([&](int i) {
-      return cs[i]->indexed == idx ? (long long)A[i].nside[1] + cs[i]->nHworkPk + A[i].hg1.x : 0LL; });
+    for (int f = 0; f < 2; ++f)  // with flagged H cells or without
+      sweepH[2 * x + f] = plan([&](int i) {
+        return cs[i]->indexed == idx && cs[i]->xflagH == (f == 0)
+                   ? (long long)A[i].nside[1] + cs[i]->nHworkPk + A[i].hg1.x : 0LL; });
     auto nrows = [&](int i, int e) {
       return cs[i]->indexed == idx ? (cs[i]->nXrow[e] + cs[i]->nXgroup[e] + 255) / 256 : 0LL; };
     rowE[x] = plan([&](int i) { return nrows(i, 0); });
     rowH[x] = plan([&](int i) { return nrows(i, 1); });
   }
-  const PackMap first = plan([&](int i) { return (long long)A[i].side[1].b[1]; });
+  const PackMap first = plan([&](int i) { return (long long)A[i].side[1].b[2]; });
   auto blocks = [](const PackMap &m) { return dim3(m.start[m.n]); };  // a packed launch's 1-D grid
   const dim3 b(256);
-  if (first.n && nsteps) hipLaunchKernelGGL(k_first_samples_pk<T>, blocks(first), b, 0, s, first);
+  if (first.n && nsteps) hipLaunchKernelGGL(k_first_samples_pk<T>, blocks(first), b, 0, s, first, pi);
   for (uint64_t st = 0; n && st < nsteps; ++st) {
-    for (PackMap *m : {sweepE, sweepE + 1, sweepE + 2, sweepE + 3, sweepH, sweepH + 1}) {
-      m->soff = (int)st;
-      m->last = st + 1 == nsteps;
-    }
+    for (PackMap &m : sweepE) m.soff = (int)st, m.last = st + 1 == nsteps;
+    for (PackMap &m : sweepH) m.soff = (int)st, m.last = st + 1 == nsteps;
     for (int i = 0; i < n; ++i)
       if (cs[i]->murmask && !cs[i]->murPush)
         hipLaunchKernelGGL(k_mur_e<T>, A[i].murGrid, dim3(16, 16), 0, s, A[i].ma[0]);
     if (sweepE[0].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 0>), blocks(sweepE[0]), b, 0, s, sweepE[0], pi);
     if (sweepE[1].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 1>), blocks(sweepE[1]), b, 0, s, sweepE[1], pi);
     if (sweepE[2].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 2>), blocks(sweepE[2]), b, 0, s, sweepE[2], pi);
-    if (sweepE[3].n) hipLaunchKernelGGL((k_e_sweep_pk<T, false, 1>), blocks(sweepE[3]), b, 0, s, sweepE[3], pi);
+    if (sweepE[3].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 3>), blocks(sweepE[3]), b, 0, s, sweepE[3], pi);
+    if (sweepE[4].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 4>), blocks(sweepE[4]), b, 0, s, sweepE[4], pi);
+    if (sweepE[5].n) hipLaunchKernelGGL((k_e_sweep_pk<T, false, 3>), blocks(sweepE[5]), b, 0, s, sweepE[5], pi);
     if (rowE[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, true>), blocks(rowE[0]), b, 0, s, rowE[0]);
     if (rowE[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, true>), blocks(rowE[1]), b, 0, s, rowE[1]);
     for (int i = 0; i < n; ++i)
       if (cs[i]->sibcFaces)
         hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)cs[i]->sibcBlocks), dim3(256), 0, s, A[i].se[0]);
-    if (sweepH[0].n) hipLaunchKernelGGL((k_h_sweep_pk<T, true>), blocks(sweepH[0]), b, 0, s, sweepH[0], pi);
-    if (sweepH[1].n) hipLaunchKernelGGL((k_h_sweep_pk<T, false>), blocks(sweepH[1]), b, 0, s, sweepH[1], pi);
+    if (sweepH[0].n) hipLaunchKernelGGL((k_h_sweep_pk<T, true, true>), blocks(sweepH[0]), b, 0, s, sweepH[0], pi);
+    if (sweepH[1].n) hipLaunchKernelGGL((k_h_sweep_pk<T, true, false>), blocks(sweepH[1]), b, 0, s, sweepH[1], pi);
+    if (sweepH[2].n) hipLaunchKernelGGL((k_h_sweep_pk<T, false, true>), blocks(sweepH[2]), b, 0, s, sweepH[2], pi);
+    if (sweepH[3].n) hipLaunchKernelGGL((k_h_sweep_pk<T, false, false>), blocks(sweepH[3]), b, 0, s, sweepH[3], pi);
     if (rowH[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, false>), blocks(rowH[0]), b, 0, s, rowH[0]);
     if (rowH[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, false>), blocks(rowH[1]), b, 0, s, rowH[1]);
   }
