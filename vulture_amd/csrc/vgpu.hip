@@ -261,7 +261,7 @@ static void destroy_ctx(vgpu_ctx *c);
 // counts as complete.
 static void wait_last_run(Ctx *c)
 {
-  hipEventSynchronize(c->ev1);
+  hipEventSynchronize(c->last_run().end);
   hipStreamSynchronize(c->stream);
 }
 
@@ -323,8 +323,6 @@ int vgpu_create(const vgpu_grid_desc *g, vgpu_prec prec, int device, vgpu_ctx **
     delete c;
     return VGPU_EDEVICE;
   }
-  hipEventCreate(&c->ev0);
-  hipEventCreate(&c->ev1);
   for (auto &rr : c->runs) {
     hipEventCreate(&rr.start);
     hipEventCreate(&rr.end);
@@ -1201,6 +1199,12 @@ static int build_observers(Ctx *c)
     c->d_odre = dev_alloc(c, (size_t)std::max<long long>(o6, 1) * sizeof(double));
     c->d_odim = dev_alloc(c, (size_t)std::max<long long>(o6, 1) * sizeof(double));
     if (!c->d_otd || !c->d_odre || !c->d_odim) return set_error(c, VGPU_ENOMEM, "observer buffers");
+    const size_t specBytes = 12 * (size_t)*std::max_element(nf.begin(), nf.end()) * sizeof(double);
+    if (specBytes && (hipHostMalloc((void **)&c->h_spec, specBytes, hipHostMallocDefault) != hipSuccess || !c->h_spec)) {
+      c->h_spec = nullptr;
+      (void)hipGetLastError();
+      return set_error(c, VGPU_ENOMEM, "pinned spectrum buffer (%zu bytes)", specBytes);
+    }
   }
   if (!c->vobs.empty()) {
     std::vector<long long> cell;
@@ -1355,7 +1359,6 @@ static int check_run(Ctx *c, uint64_t first, uint64_t nsteps)
 // A run's start events on stream s.
 static void open_run(Ctx *c, hipStream_t s)
 {
-  hipEventRecord(c->ev0, s);
   hipEventRecord(c->runs[c->runCount & 1].start, s);
 }
 
@@ -1367,22 +1370,24 @@ static void set_step(Ctx *c, uint64_t first, hipStream_t s)
                        (unsigned long long)first);
 }
 
+// The last run's slot in the pinned ring, before it closes.
+static float *run_slot(const Ctx *c) { return c->h_vring + (size_t)(c->runCount & 1) * c->maxRun * c->vnodes * 6; }
+
 // A run's close on stream s, after its kernels: its volume samples to its
-// slot of the pinned ring (rows wrap at the end of the device ring), its end
-// events and its record.
-static void close_run(Ctx *c, uint64_t first, uint64_t nsteps, hipStream_t s)
+// slot of the pinned ring (rows wrap at the end of the device ring; not with
+// copy false, where k_group_close has them), its end event and its record.
+static void close_run(Ctx *c, uint64_t first, uint64_t nsteps, hipStream_t s, bool copy)
 {
   Ctx::RunRec &rr = c->runs[c->runCount & 1];
-  if (c->vnodes && nsteps) {
+  if (copy && c->vnodes && nsteps) {
     const size_t row = (size_t)c->vnodes * 6;
-    float *dst = c->h_vring + (size_t)(c->runCount & 1) * c->maxRun * row;
+    float *dst = run_slot(c);
     const uint64_t r0 = first % c->vring, n1 = std::min<uint64_t>(nsteps, c->vring - r0);
     hipMemcpyAsync(dst, (float *)c->d_vstage + r0 * row, n1 * row * sizeof(float), hipMemcpyDeviceToHost, s);
     if (n1 < nsteps)
       hipMemcpyAsync(dst + n1 * row, c->d_vstage, (nsteps - n1) * row * sizeof(float), hipMemcpyDeviceToHost, s);
   }
   hipEventRecord(rr.end, s);
-  hipEventRecord(c->ev1, s);
   rr.first = first;
   rr.n = nsteps;
   rr.valid = true;
@@ -1421,7 +1426,7 @@ int vgpu_run(vgpu_ctx *c, uint64_t first, uint64_t nsteps, void *stream)
     r = c->prec == VGPU_FP64 ? run_steps<double>(c, nsteps, s, true) : run_steps<float>(c, nsteps, s, true);
     c->lastRunTimed = true;
   }
-  close_run(c, first, nsteps, s);
+  close_run(c, first, nsteps, s, true);
   return r;
 }
 
@@ -1522,6 +1527,27 @@ int vgpu_run_group(vgpu_ctx *const *ctxs, int n, const uint64_t *first, uint64_t
   } else {
     r = lead->prec == VGPU_FP64 ? run_group_steps<double>(cs, n, nsteps, s) : run_group_steps<float>(cs, n, nsteps, s);
   }
+  GroupClose gc{};
+  gc.by = nsteps;
+  unsigned blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    Ctx *c = ctxs[i];
+    // a member without a pack ran alone, its counter advanced
+    const bool step = c->d_pack, rows = c->vnodes && nsteps;
+    if (!step && !rows) continue;
+    const int d = gc.n++;
+    gc.start[d] = blocks;
+    gc.step[d] = step ? (unsigned long long *)c->d_step : nullptr;
+    if (rows) {
+      gc.src[d] = (const double *)c->d_vstage;
+      gc.dst[d] = (double *)run_slot(c);
+      gc.at[d] = (long long)(first[i] % c->vring) * c->vnodes * 3;
+      gc.pairs[d] = (long long)nsteps * c->vnodes * 3;
+      gc.ring[d] = (long long)c->vring * c->vnodes * 3;
+    }
+    blocks += (unsigned)std::max(1LL, (gc.pairs[d] + 1023) / 1024);
+  }
+  if (gc.n) hipLaunchKernelGGL(k_group_close, dim3(blocks), dim3(256), 0, s, gc);
   // the first member closes last, so its end follows all of the group's work
   // on its stream
   for (int k = 1; k <= n; ++k) {
@@ -1529,7 +1555,7 @@ int vgpu_run_group(vgpu_ctx *const *ctxs, int n, const uint64_t *first, uint64_t
     Ctx *c = ctxs[i];
     c->lastRunTimed = false;
     hipEvent_t end = c->runs[c->runCount & 1].end;
-    close_run(c, first[i], nsteps, s);
+    close_run(c, first[i], nsteps, s, false);
     if (i) hipStreamWaitEvent(c->stream, end, 0);
   }
   return r;
@@ -1538,10 +1564,10 @@ int vgpu_run_group(vgpu_ctx *const *ctxs, int n, const uint64_t *first, uint64_t
 int vgpu_synchronize(vgpu_ctx *c)
 {
   if (!c) return VGPU_EINVAL;
-  if (hipEventSynchronize(c->ev1) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
+  if (hipEventSynchronize(c->last_run().end) != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
     return set_error(c, VGPU_EDEVICE, "device error: %s", hipGetErrorString(hipGetLastError()));
   float ms = 0;
-  hipEventElapsedTime(&ms, c->ev0, c->ev1);
+  hipEventElapsedTime(&ms, c->last_run().start, c->last_run().end);
   c->last_total_ms = ms;
   double se = 0, sh = 0;
   int ne = 0;
@@ -1563,7 +1589,7 @@ int vgpu_synchronize(vgpu_ctx *c)
 int vgpu_query(vgpu_ctx *c)
 {
   if (!c || !c->finalized) return VGPU_EINVAL;
-  const hipError_t e = hipEventQuery(c->ev1);
+  const hipError_t e = hipEventQuery(c->last_run().end);
   if (e == hipSuccess) return 1;
   if (e == hipErrorNotReady) return 0;
   return set_error(c, VGPU_EDEVICE, "device error: %s", hipGetErrorString(e));
@@ -1573,8 +1599,11 @@ int vgpu_read_point_observer(vgpu_ctx *c, int id, double *td, uint64_t nsteps, d
 {
   if (!c || !c->finalized || id < 0 || id >= (int)c->pobs.size()) return VGPU_EINVAL;
   const DeviceCalls guard(g_capture_mu);
-  wait_last_run(c);
+  // the run may be on a caller's stream; the read below is behind c->stream's
+  // own work by its order
+  hipEventSynchronize(c->last_run().end);
   if (td) {
+    hipStreamSynchronize(c->stream);
     const uint64_t n = std::min<uint64_t>(nsteps, c->totalSteps);
     hipMemcpy(td, (char *)c->d_otd + (size_t)id * c->totalSteps * 6 * sizeof(double), n * 6 * sizeof(double),
               hipMemcpyDeviceToHost);
@@ -1582,8 +1611,17 @@ int vgpu_read_point_observer(vgpu_ctx *c, int id, double *td, uint64_t nsteps, d
   long long off = 0;
   for (int o = 0; o < id; ++o) off += 6 * (long long)c->pobs[o].omega.size();
   const size_t nb = 6 * c->pobs[id].omega.size() * sizeof(double);
-  if (nb && dft_re) hipMemcpy(dft_re, (char *)c->d_odre + off * sizeof(double), nb, hipMemcpyDeviceToHost);
-  if (nb && dft_im) hipMemcpy(dft_im, (char *)c->d_odim + off * sizeof(double), nb, hipMemcpyDeviceToHost);
+  if (nb && (dft_re || dft_im)) {
+    // one launch and one wait; two pageable copies of 3 KB took 37 us
+    std::lock_guard<std::mutex> lock(c->specMu);
+    const int n = (int)(nb / sizeof(double));
+    hipSetDevice(c->device);
+    hipLaunchKernelGGL(k_read_spectrum, dim3((2 * n + 255) / 256), dim3(256), 0, c->stream,
+                       (const double *)c->d_odre + off, (const double *)c->d_odim + off, c->h_spec, n);
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return VGPU_EDEVICE;
+    if (dft_re) memcpy(dft_re, c->h_spec, nb);
+    if (dft_im) memcpy(dft_im, c->h_spec + n, nb);
+  }
   return hipGetLastError() == hipSuccess ? VGPU_OK : VGPU_EDEVICE;
 }
 
@@ -1752,13 +1790,12 @@ static void destroy_ctx(vgpu_ctx *c)
   }
   for (auto e : c->evE) hipEventDestroy(e);
   for (auto e : c->evH) hipEventDestroy(e);
-  if (c->ev0) hipEventDestroy(c->ev0);
-  if (c->ev1) hipEventDestroy(c->ev1);
   for (auto &rr : c->runs) {
     if (rr.start) hipEventDestroy(rr.start);
     if (rr.end) hipEventDestroy(rr.end);
   }
   if (c->h_vring) hipHostFree(c->h_vring);
+  if (c->h_spec) hipHostFree(c->h_spec);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
 }

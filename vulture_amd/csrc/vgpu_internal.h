@@ -19,6 +19,7 @@
 #include <cstdint>
 #include <cstddef>
 #include <string>
+#include <mutex>
 #include <vector>
 #include "vgpu.h"
 
@@ -512,6 +513,18 @@ template <typename T> struct SideArgs {
 
 constexpr int PACK_MAX = VGPU_GROUP_MAX;  // solves in one group run
 
+// The end of a group run, one launch over its solves: the step counters, and
+// the run's rows of volume samples (8-byte pairs: n of them, from `at` on in
+// a ring of `ring`) to their place in pinned host memory.
+struct GroupClose {
+  int n;
+  unsigned start[PACK_MAX + 1];  // first block of each solve; start[n] is the grid
+  unsigned long long by, *step[PACK_MAX];
+  const double *src[PACK_MAX];
+  double *dst[PACK_MAX];
+  long long at[PACK_MAX], pairs[PACK_MAX], ring[PACK_MAX];
+};
+
 // One solve's by-value argument blocks for the packed launches, for field set
 // 0 (the one the separate sweeps read and write), kept in device memory.  A
 // packed launch passes the step offset itself.
@@ -605,7 +618,6 @@ struct Ctx {
   vgpu_grid_desc grid;
   std::vector<double> xl, yl, zl, dex, dey, dez, idex, idey, idez, idhx, idhy, idhz;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::vector<hipEvent_t> evE, evH;
   double last_total_ms = 0, last_e_ms = 0, last_h_ms = 0;
   bool finalized = false;
@@ -785,6 +797,11 @@ struct Ctx {
   struct RunRec { uint64_t first = 0, n = 0; bool valid = false; hipEvent_t start = nullptr, end = nullptr; };
   RunRec runs[2];
   uint64_t runCount = 0;
+  const RunRec &last_run() const { return runs[runCount ? (runCount - 1) & 1 : 0]; }
+  // Point spectra are read through a pinned buffer: one observer's, re then
+  // im, gathered by one kernel on the context's stream.
+  std::mutex specMu;
+  double *h_spec = nullptr;  // [2][6][most frequencies of an observer]
 
   long long lin(int i, int j, int k) const { return ((long long)k * NY + j) * PX + i; }
 };

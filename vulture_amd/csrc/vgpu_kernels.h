@@ -1874,4 +1874,27 @@ static __global__ void k_advance_step(unsigned long long *step, unsigned long lo
   if (threadIdx.x == 0) step[threadIdx.x] = step[threadIdx.x] + by;
 }
 
+// GroupClose.  A run of 16 solves ended in 16 counter launches and 16 copies,
+// each a trip of its own through the queue; a thread moves four pairs.
+static __global__ __launch_bounds__(256) void k_group_close(GroupClose g)
+{
+  int d = 0;
+  while (d + 1 < g.n && blockIdx.x >= g.start[d + 1]) ++d;
+  const unsigned b = blockIdx.x - g.start[d];
+  if (b == 0 && threadIdx.x == 0 && g.step[d]) *g.step[d] += g.by;
+  for (int q = 0; q < 4; ++q) {
+    const long long i = b * 1024ll + q * 256 + threadIdx.x;
+    if (i >= g.pairs[d]) return;
+    const long long r = g.at[d] + i;
+    g.dst[d][i] = g.src[d][r < g.ring[d] ? r : r - g.ring[d]];
+  }
+}
+
+// One observer's spectrum, re then im, into the pinned buffer it is read from.
+static __global__ __launch_bounds__(256) void k_read_spectrum(const double *re, const double *im, double *out, int n)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < 2 * n) out[i] = i < n ? re[i] : im[i - n];
+}
+
 }  // namespace vgpu

@@ -1192,8 +1192,7 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
     if (rowH[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, false>), blocks(rowH[0]), b, 0, s, rowH[0]);
     if (rowH[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, false>), blocks(rowH[1]), b, 0, s, rowH[1]);
   }
-  for (int i = 0; i < n; ++i)
-    hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(64), 0, s, A[i].stepp, (unsigned long long)nsteps);
+  // (the step counters advance with the group's close)
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return set_error(cs[0], VGPU_EDEVICE, "kernel launch failed: %s", hipGetErrorString(err));
   return VGPU_OK;
