@@ -1518,14 +1518,6 @@ template <typename T, bool ZERO> __global__ __launch_bounds__(256) void k_sibc_e
   sibc_e_block<T, ZERO>(a, blockIdx.x);
 }
 
-// The SIBC faces' blocks, then the E rows.
-template <typename T, bool IDX>
-__global__ __launch_bounds__(256) void k_sibc_rows(SibcEArgs<T> a, const XArgs<T> *x, unsigned nSibc)
-{
-  if (blockIdx.x < nSibc) sibc_e_block<T, false>(a, blockIdx.x);
-  else x_rows<T, IDX, true>(cp(x), blockIdx.x - nSibc);
-}
-
 // SIBC: gathered H corrections (sibc.c:616-776).
 template <typename T> __global__ void k_sibc_h(SibcHArgs<T> a)
 {
@@ -1756,6 +1748,31 @@ __global__ __launch_bounds__(256) void k_e_sweep(FastE<T> f, const ShellDev *pcs
   if (b < nSide) side_block<T, IDX, true, (X >= 3)>(sd, cp(x), (int)b, soff, last, pi);
   else if (b < n1) e_shell_column<T, IDX, X, false, false>(pcs, work, ap, cp(x), b - nSide);
   else e_fast_tile<T, IDX, X, false>(f, cp(x), b - n1);
+}
+
+// The E sweep of a grid with SIBC faces, whose E pass reads the old H and its
+// own states and writes no field: its blocks (a multiple of eight) come
+// second, so their chains of dependent loads run under the sweep's streams.
+// 96x81x64 box FP64: 38.4 us a step in a launch of their own, with the E rows,
+// and the sweep's, 28.5 in one; 256x256x160 box FP32, where both move bytes
+// (270 MB of states) all the time, 200 and 197.  FP32 keeps five wavefronts a
+// SIMD (97 registers without the bound).
+template <typename T, bool IDX, int X>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 5 : 3) void k_e_sweep_sibc(FastE<T> f, const ShellDev *pcs, const ShellWork *work,
+                                                      const EArgs<T> *ap, const XArgs<T> *x, unsigned nSide,
+                                                      unsigned nSibc, unsigned nShell, SideArgs<T> sd, SibcEArgs<T> se,
+                                                      unsigned sibcBlocks, int soff, int last, double pi)
+{
+  const unsigned b = blockIdx.x, n0 = nSide + nSibc, n1 = n0 + nShell;
+  if (b < nSide) {
+    side_block<T, IDX, true, (X >= 3)>(sd, cp(x), (int)b, soff, last, pi);
+  } else if (b < n0) {
+    if (b - nSide < sibcBlocks) sibc_e_block<T, false>(se, b - nSide);
+  } else if (b < n1) {
+    e_shell_column<T, IDX, X, false, false>(pcs, work, ap, cp(x), b - n0);
+  } else {
+    e_fast_tile<T, IDX, X, false>(f, cp(x), b - n1);
+  }
 }
 
 template <typename T, bool IDX, bool X>

@@ -869,13 +869,23 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   const bool apart = sweeps_apart(c);
   auto sweep_e = [&](int soff, int last) {
     const unsigned ns = A.nside[0], nw = (unsigned)c->nEwork;
-    const dim3 b(256), g(ns + nw + (apart ? 0u : eg1.x));
+    const unsigned nb = c->sibcFaces ? (unsigned)c->sibcBlocks : 0u, nb8 = (nb + 7) / 8 * 8;
+    const dim3 b(256), g(ns + nb8 + nw + (apart ? 0u : eg1.x));
     if (!g.x) return;
     const int x = c->xlevel();
     const FastE<T> &f = fe[0];
     const SideArgs<T> &sd = A.side[0];
     auto go = [&](auto k) { hipLaunchKernelGGL(k, g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi); };
-    if (!c->indexed) go(k_e_sweep<T, false, 3>);
+    auto sibc = [&](auto k) {
+      hipLaunchKernelGGL(k, g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nb8, nw, sd, A.se[0], nb, soff, last, pi);
+    };
+    if (nb && !c->indexed) sibc(k_e_sweep_sibc<T, false, 3>);
+    else if (nb && x == 0) sibc(k_e_sweep_sibc<T, true, 0>);
+    else if (nb && x == 1) sibc(k_e_sweep_sibc<T, true, 1>);
+    else if (nb && x == 2) sibc(k_e_sweep_sibc<T, true, 2>);
+    else if (nb && x == 3) sibc(k_e_sweep_sibc<T, true, 3>);
+    else if (nb) sibc(k_e_sweep_sibc<T, true, 4>);
+    else if (!c->indexed) go(k_e_sweep<T, false, 3>);
     else if (x == 0) go(k_e_sweep<T, true, 0>);
     else if (x == 1) go(k_e_sweep<T, true, 1>);
     else if (x == 2) go(k_e_sweep<T, true, 2>);
@@ -959,12 +969,6 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   auto &da = A.da;
   const auto &se = A.se;
   const auto &sh = A.sh;
-  auto sibc_rows = [&]() {
-    const unsigned nb = (unsigned)c->sibcBlocks;
-    const dim3 b(256), g(nb + (unsigned)((c->nXrow[0] + c->nXgroup[0] + 255) / 256));
-    if (c->indexed) hipLaunchKernelGGL((k_sibc_rows<T, true>), g, b, 0, s, se[0], xe, nb);
-    else hipLaunchKernelGGL((k_sibc_rows<T, false>), g, b, 0, s, se[0], xe, nb);
-  };
   auto &ce = A.ce;
   auto &xa = A.xa;
   const bool anyAux = A.anyAux;
@@ -994,8 +998,7 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     if (apart) fast_e(0);
     else sweep_e(soff, last);
     mark(c->evE, 2 * ne++ + 1);
-    if (c->sibcFaces) sibc_rows();
-    else rows(0);
+    rows(0);
     mark(c->evH, 2 * nh);
     if (apart) fast_h(0);
     else sweep_h(soff, last);
