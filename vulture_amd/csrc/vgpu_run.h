@@ -518,7 +518,7 @@ template <typename T> struct StepArgs {
 // for more: 537 against 529 us at 272^3 in FP32 (85 MB a field).
 static bool sweeps_apart(const Ctx *c) { return c->ncell * c->esz > ((size_t)64 << 20); }
 
-template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun *chk)
+template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun *chk, bool packed = false)
 {
   const double dt = c->grid.dt;
   // argument sets by the field set a step reads (index 0/1)
@@ -528,6 +528,12 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   // Fast kernels: 64x4 tiles (64 x ty) over the fast boxes, marching z in
   // chunks of 4 planes, or 2 where they have launches of their own (272^3 FP32:
   // 505 us a step with 4, 501 with 2, 514 with 8; merged grids within 1 %).
+  // Where chunks of 4 make fewer than seven blocks a CU there is little else to
+  // run under a block's chain of planes, and one plane a block is faster: a
+  // step of the 53x41x62 request 24.8 us against 27.5, 101x115x108 67.6 and
+  // 70.9, the FP64 96x81x64 box 49.9 and 52.6; with more blocks the planes' shared loads count (FP64 128^3
+  // Debye volume 162 and 167).  Packed launches have their members' blocks
+  // together and keep 4 (364 and 383 for 16 requests).
   // rows per block (tuning override VGPU_FAST_TY: 1..8)
   int ty = 4;
   if (const char *ev = getenv("VGPU_FAST_TY")) ty = std::max(1, std::min(atoi(ev), 8));
@@ -535,7 +541,7 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   auto fast_grid = [&](const int *fb, int &kchunk) {
     if (fb[0] > fb[1] || fb[2] > fb[3] || fb[4] > fb[5]) return dim3(0, 0, 0);
     const int gx = (fb[1] - fb[0] + 64) / 64, gy = (fb[3] - fb[2] + ty) / ty, nz = fb[5] - fb[4] + 1;
-    kchunk = std::min(sweeps_apart(c) ? 2 : 4, nz);
+    kchunk = std::min(sweeps_apart(c) ? 2 : !packed && gx * gy * ((nz + 3) / 4) < 1792 ? 1 : 4, nz);
     if (const char *ev = getenv("VGPU_FAST_KCHUNK"))  // tuning override: planes per block
       kchunk = std::max(1, std::min(atoi(ev), nz));
     return dim3(gx, gy, (nz + kchunk - 1) / kchunk);
@@ -1075,7 +1081,7 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
 template <typename T> int upload_pack(Ctx *c)
 {
   StepArgs<T> A{};
-  fill_step_args<T>(c, A, nullptr);
+  fill_step_args<T>(c, A, nullptr, true);
   // shells at SHELL_KC planes per block: a packed launch fills the device
   // with many grids' blocks, where a small grid's own plan used one plane
   std::vector<ShellDev> ep, hp;
@@ -1135,7 +1141,7 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
     }
   }
   std::vector<StepArgs<T>> A(n);
-  for (int i = 0; i < n; ++i) fill_step_args<T>(cs[i], A[i], nullptr);
+  for (int i = 0; i < n; ++i) fill_step_args<T>(cs[i], A[i], nullptr, true);
   // One packed launch: the solves with a positive block count, in order.
   auto plan = [&](auto blocks) {
     PackMap m{};
