@@ -59,9 +59,9 @@ def _traffic(kernel, prec):
 
 
 def debye_site_words(st):
-    """Compulsory words per Debye site: lastE read and written, J read and
-    written per pole (two words per pole when complex)."""
-    return 2 + 2 * max(st["debye_poles"], 1) * (2 if st["debye_complex"] else 1)
+    """Compulsory words per Debye site: J read and written per pole (two words
+    per pole when complex); the last E is the E the sweep reads anyway."""
+    return 2 * max(st["debye_poles"], 1) * (2 if st["debye_complex"] else 1)
 
 
 def kernel_bytes(st, esz):
@@ -74,9 +74,11 @@ def kernel_bytes(st, esz):
     and its H class (2 B; 3 words of gamma) and writes new H (3) of each H
     cell updated again after the E corrections.
 
-    Separate sweeps (k_e_fast, k_h_fast): fast E reads E and H (6 words) and
+    Separate sweeps (k_e_fast, k_h_fast; on fields up to 64 MB the times are
+    those of the whole sweeps, k_e_sweep and k_h_sweep, priced by their fast
+    cells alone): fast E reads E and H (6 words) and
     the class (2 B; 6 words of alpha/beta without classes), writes E (3),
-    plus the fused Debye sites; fast H reads H and E (6), the class (2 B; 3
+    plus the Debye sites in line; fast H reads H and E (6), the class (2 B; 3
     words of gamma), writes H (3)."""
     ce, ch = st["fast_cells"]
     if st.get("leap"):

@@ -217,9 +217,9 @@ typedef struct {
   uint64_t correction_rows[2]; /* source / TF/SF correction rows, E and H */
   uint64_t bytes;              /* device footprint */
   uint64_t fast_cells[2];      /* cells of the E and H fast sweep kernels */
-  uint64_t debye_fused_sites;  /* Debye sites applied inside the fast E kernel */
+  uint64_t debye_fused_sites;  /* Debye sites of the fast E tiles that they apply in line */
   int indexed_media;           /* 1: coefficients read as 16-bit classes */
-  int debye_fused;             /* 1: first Debye layer fused into the E sweep */
+  int debye_fused;             /* 1: the E sweep applies one-pole Debye sites in line */
   int sibc_state;              /* SIBC filter state: 0 complex per filter, 1 real per filter, 2 real per input */
   int leap;                    /* 1: fused leapfrog sweep (E then H in one pass over the fast box) */
   uint64_t fix_cells;          /* H cells of the fused box updated again after the E corrections */
@@ -229,7 +229,9 @@ typedef struct {
 int vgpu_get_stats(const vgpu_ctx *c, vgpu_stats *out);
 
 /* Time of the kernels of the last vgpu_run, from events on its stream (ms),
- * and the average duration of the E and H volume kernels in it (ms). */
+ * and the average duration of the E and H volume kernels in it (ms): the fast
+ * tiles where they have launches of their own (fields over 64 MB), else each
+ * half-step's whole sweep. */
 int vgpu_last_run_timing(const vgpu_ctx *c, double *total_ms, double *volume_e_ms, double *volume_h_ms);
 
 /* Update-once check of the field sweeps.  Replaces the reference's

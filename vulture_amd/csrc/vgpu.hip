@@ -1743,7 +1743,7 @@ int vgpu_get_stats(const vgpu_ctx *c, vgpu_stats *out)
                              ? (uint64_t)(fb[1] - fb[0] + 1) * (uint64_t)(fb[3] - fb[2] + 1) * (uint64_t)(fb[5] - fb[4] + 1)
                              : 0;
   }
-  out->debye_fused_sites = (uint64_t)c->debyeSimple;
+  out->debye_fused_sites = (uint64_t)c->debyeFast;
   out->indexed_media = c->indexed ? 1 : 0;
   out->debye_fused = c->debyeSimple > 0 ? 1 : 0;
   out->sibc_state = c->sibcFactored ? 2 : c->sibcReal ? 1 : 0;

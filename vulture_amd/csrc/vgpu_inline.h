@@ -362,6 +362,12 @@ template <typename T> int build_inline(Ctx *c)
   }
   c->indexed = indexed;
   c->debyeSimple = (long long)simple.size();
+  c->debyeFast = 0;
+  for (const Ctx::XSite &s : simple) {
+    int n[3];
+    geo.unlin(s.key / 3, n);
+    c->debyeFast += in_box(c->fastE, n[0], n[1], n[2]);
+  }
   c->debyeSites = listed;
   if (listed > INT32_MAX) return set_error(c, VGPU_EINVAL, "too many Debye sites");
   if (listed) {

@@ -653,6 +653,7 @@ struct Ctx {
   // sites as well; 3 and 4 the same with update rows
   int xlevel() const { return xflag0 == ~0u ? 0 : (debyeSimple ? 2 : 1) + (xskip ? 2 : 0); }
   long long debyeSimple = 0;                 // one-pole Debye sites applied from the class table
+  long long debyeFast = 0;                   // those of them in the fast E box
   // an operation on one field value, before rows are made of them
   // (key: ((cell * 3 + component) * 4 + order); kept in the reference's order within one key)
   struct XEnt {
