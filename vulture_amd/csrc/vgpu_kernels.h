@@ -489,6 +489,27 @@ VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, XPre<T> &p, T o
 // instead of storing them, and leaves every field and auxiliary untouched.
 VG_DEV void visit(unsigned *v, long long id) { atomicAdd(v + id, 1u); }
 
+// The Mur E values that a flagged cell's thread writes (x_inline_e), counted.
+template <typename T>
+VG_DEV void count_mur(const VG_CONST XArgs<T> *x, long long id, unsigned fl, unsigned *const *vis)
+{
+  for (int f = 0; f < 6; ++f)
+    for (int s = 0; s < 2; ++s) {
+      const int C = ((f >> 1) + 1 + s) % 3;
+      if ((fl >> (XF_MUR_SHIFT + 2 * f + s)) & 1u) visit(vis[C], XPre<T>::mur_at(x, id, f));
+    }
+}
+
+// The values of update-row block b, counted.
+template <typename T> VG_DEV void count_updates(const VG_CONST XArgs<T> *x, unsigned b, unsigned *const *vis)
+{
+  const long long q = b * 256ll + threadIdx.x;
+  if (q >= x->nupd) return;
+  const VG_GLOBAL XRow *row = gp(x->row) + q;
+  const int c = (int)(row->opc & 3u);
+  visit(c == 0 ? vis[0] : c == 1 ? vis[1] : vis[2], row->cell);
+}
+
 // Fast E tile: inner grid (grid.c:709-797).  X: in-line corrections, 0 none,
 // 1 Mur faces and zeroed E, 2 Debye sites as well, 3 and 4 the same with
 // values left to update rows.
@@ -548,9 +569,9 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
     T e2 = a2 * o2 + b2 * (idhx * (hy - hyx) + idhy * (hxy - hx));
     if (vx) {
       if (CHK) {
-        visit(f.vis[0], id);
-        visit(f.vis[1], id);
-        visit(f.vis[2], id);
+        if (flagged) count_mur(x, id, pre.fl, f.vis);
+        for (int C = 0; C < 3; ++C)
+          if (X < 3 || !(pre.fl & (XF_SKIP << C))) visit(f.vis[C], id);
       } else {
         if (flagged) x_inline_e<T, (X == 2 || X == 4)>(x, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
         if (X < 3 || !(pre.fl & XF_SKIP)) f.E[0][id] = e0;
@@ -615,9 +636,8 @@ template <typename T, bool IDX, bool X, bool CHK> VG_DEV void h_fast_tile(const 
     T h2 = I2[id] + g2 * (idey * (exy - ex) + idex * (ey - eyx));
     if (vx) {
       if (CHK) {
-        visit(f.vis[0], id);
-        visit(f.vis[1], id);
-        visit(f.vis[2], id);
+        for (int C = 0; C < 3; ++C)
+          if (!(fl & (XF_SKIP << C))) visit(f.vis[C], id);
       } else {
         if (fl & XF_ZERO) h0 = T(0);
         if (fl & (XF_ZERO << 1)) h1 = T(0);
@@ -1080,8 +1100,9 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
     c1.load(g, rg[1], n3, id, cls);
     c2.load(g, rg[2], n3, id, cls);
     if (CHK) {
+      if (flagged) count_mur(x, id, pre.fl, a.vis);
       for (int C = 0; C < 3; ++C)
-        if (rg[C].reg >= 0) visit(a.vis[C], id);
+        if (rg[C].reg >= 0 && (X < 3 || !(pre.fl & (XF_SKIP << C)))) visit(a.vis[C], id);
     } else {
       T e0 = c0.value(g, rg[0], idh1 * (hz - hzy) + idh2 * (hym - hy));
       T e1 = c1.value(g, rg[1], idh2 * (hx - hxm) + idh0 * (hzx - hz));
@@ -1225,7 +1246,7 @@ VG_DEV void h_shell_column(const ShellDev *pcs, const ShellWork *work, const HAr
     c2.load(q, rg[2], n3, id, cls);
     if (CHK) {
       for (int C = 0; C < 3; ++C)
-        if (rg[C].reg >= 0) visit(a.vis[C], id);
+        if (rg[C].reg >= 0 && !(fl & (XF_SKIP << C))) visit(a.vis[C], id);
     } else {
       c0.store(q, rg[0], id, fl, ide2 * (eyp1 - eyc) + ide1 * (ez - ezy));
       c1.store(q, rg[1], id, fl, ide0 * (ezx - ez) + ide2 * (exc - exp1));
@@ -1784,6 +1805,41 @@ __global__ __launch_bounds__(256) void k_h_sweep(FastH<T> f, const ShellDev *pcs
   if (b < nSide) side_block<T, IDX, false, X>(sd, cp(x), (int)b, soff, last, pi);
   else if (b < n1) h_shell_column<T, IDX, X, false, false>(pcs, work, ap, b - nSide);
   else h_fast_tile<T, IDX, X, false>(f, b - n1);
+}
+
+// The update-once check's form of the two sweeps: the grid of k_e_sweep
+// (k_e_sweep_sibc with nSibc > 0) or k_h_sweep, each block counting the updates
+// that its block there stores.  Update rows are the side blocks from updFirst
+// on.  E takes the flags of every level (X = 3; a level without update rows
+// flags none of their cells).
+template <typename T, bool IDX>
+__global__ __launch_bounds__(256) void k_e_sweep_chk(FastE<T> f, const ShellDev *pcs, const ShellWork *work,
+                                                     const EArgs<T> *ap, const XArgs<T> *x, unsigned nSide,
+                                                     unsigned nSibc, unsigned nShell, unsigned updFirst)
+{
+  const unsigned b = blockIdx.x, n0 = nSide + nSibc, n1 = n0 + nShell;
+  if (b < nSide) {
+    if (b >= updFirst) count_updates(cp(x), b - updFirst, f.vis);
+  } else if (b >= n0 && b < n1) {
+    e_shell_column<T, IDX, 3, true, false>(pcs, work, ap, cp(x), b - n0);
+  } else if (b >= n1) {
+    e_fast_tile<T, IDX, 3, true>(f, cp(x), b - n1);
+  }
+}
+
+template <typename T, bool IDX, bool X>
+__global__ __launch_bounds__(256) void k_h_sweep_chk(FastH<T> f, const ShellDev *pcs, const ShellWork *work,
+                                                     const HArgs<T> *ap, const XArgs<T> *x, unsigned nSide,
+                                                     unsigned nShell, unsigned updFirst)
+{
+  const unsigned b = blockIdx.x, n1 = nSide + nShell;
+  if (b < nSide) {
+    if (X && b >= updFirst) count_updates(cp(x), b - updFirst, f.vis);
+  } else if (b < n1) {
+    h_shell_column<T, IDX, X, true, false>(pcs, work, ap, b - nSide);
+  } else {
+    h_fast_tile<T, IDX, X, true>(f, b - n1);
+  }
 }
 
 // Ghost plane copy for one face (surface.c:569-812).

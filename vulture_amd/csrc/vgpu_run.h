@@ -835,7 +835,10 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     const FastE<T> &f = fe[q];
     if (!egrid.x) return;
     const int x = c->xlevel();
-    if (chk && c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 0, true>), eg1, vblk, 0, s, f, xe);
+    // (the check counts Mur's E with level 1's flags)
+    if (chk && c->inl && c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 1, true>), eg1, vblk, 0, s, f, xe);
+    else if (chk && c->inl) hipLaunchKernelGGL((k_e_fast<T, false, 1, true>), eg1, vblk, 0, s, f, xe);
+    else if (chk && c->indexed) hipLaunchKernelGGL((k_e_fast<T, true, 0, true>), eg1, vblk, 0, s, f, xe);
     else if (chk) hipLaunchKernelGGL((k_e_fast<T, false, 0, true>), eg1, vblk, 0, s, f, xe);
     // (grids whose fast tiles launch apart have no update rows)
     else if (c->indexed && x == 2) hipLaunchKernelGGL((k_e_fast<T, true, 2>), eg1, vblk, 0, s, f, xe);
@@ -881,6 +884,14 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     const int x = c->xlevel();
     const FastE<T> &f = fe[0];
     const SideArgs<T> &sd = A.side[0];
+    if (chk) {
+      auto count = [&](auto k) {
+        hipLaunchKernelGGL(k, g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nb8, nw, (unsigned)sd.b[3]);
+      };
+      if (c->indexed) count(k_e_sweep_chk<T, true>);
+      else count(k_e_sweep_chk<T, false>);
+      return;
+    }
     auto go = [&](auto k) { hipLaunchKernelGGL(k, g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nw, sd, soff, last, pi); };
     auto sibc = [&](auto k) {
       hipLaunchKernelGGL(k, g, b, 0, s, f, epc, ewk, eap[0], xe, ns, nb8, nw, sd, A.se[0], nb, soff, last, pi);
@@ -903,6 +914,16 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     const dim3 b(256), g(ns + nw + (apart ? 0u : hg1.x));
     if (!g.x) return;
     const SideArgs<T> &sd = A.side[1];
+    if (chk) {
+      auto count = [&](auto k) {
+        hipLaunchKernelGGL(k, g, b, 0, s, fh[0], hpc, hwk, hap[0], xh, ns, nw, (unsigned)sd.b[3]);
+      };
+      if (c->indexed && c->xflagH) count(k_h_sweep_chk<T, true, true>);
+      else if (c->indexed) count(k_h_sweep_chk<T, true, false>);
+      else if (c->xflagH) count(k_h_sweep_chk<T, false, true>);
+      else count(k_h_sweep_chk<T, false, false>);
+      return;
+    }
     auto go = [&](auto k) { hipLaunchKernelGGL(k, g, b, 0, s, fh[0], hpc, hwk, hap[0], xh, ns, nw, sd, soff, last, pi); };
     if (c->indexed && c->xflagH) go(k_h_sweep<T, true, true>);
     else if (c->indexed) go(k_h_sweep<T, true, false>);
@@ -956,8 +977,15 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   const dim3 murGrid = A.murGrid;
   if (chk) {
     const int q = c->par;
-    if (c->murmask) hipLaunchKernelGGL((k_mur_e<T, true>), murGrid, dim3(16, 16), 0, s, ma[q]);
-    if (c->leap) {
+    if (c->murmask && !c->murPush) hipLaunchKernelGGL((k_mur_e<T, true>), murGrid, dim3(16, 16), 0, s, ma[q]);
+    if (c->inl) {
+      sweep_e(0, 0);
+      if (apart) {
+        fast_e(0);
+        fast_h(0);
+      }
+      sweep_h(0, 0);
+    } else if (c->leap) {
       leap(q);
       shell_e(q);
       shell_h(q);
@@ -1209,10 +1237,11 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
 
 // Update-once check (the reference's CHECK_LIMITS build: grid.h:181-191, and
 // checkGrid, grid.c:951-1025).  One step of the field sweeps -- Mur E, the E
-// sweep, the H sweep, as the loop launches them -- runs in its counting form,
-// which adds one to a per-cell count for each update instead of storing it;
-// each component's counts are then tallied against its outer field limits
-// folim.  Fields, UPML auxiliaries and Debye state are left as they were.
+// sweep, the H sweep, in the grids that the loop launches them in -- runs in
+// its counting form, which adds one to a per-cell count for each update instead
+// of storing it: a value left to an update row counts there, a Mur value where
+// its inner neighbour's thread or Mur's own launch writes it.  Each component's
+// counts are then tallied against its outer field limits folim.  Fields, UPML auxiliaries and Debye state are left as they were.
 // Bytes of device memory one update-once check uses: visit counts per
 // component (device layout), the two sweep argument blocks, the tally and,
 // with counts, their staging in the counts layout; each part 256-byte aligned.
