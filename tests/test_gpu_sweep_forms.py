@@ -1,5 +1,8 @@
 """The launch forms of the step that the default sizes of the other tests do
 not take (needs an MI355X)."""
+import filecmp
+import os
+
 import numpy as np
 import pytest
 
@@ -18,6 +21,7 @@ def _fields(mesh, precision, steps=80):
 
 
 def _write(tmp_path, text):
+    tmp_path.mkdir(parents=True, exist_ok=True)
     p = tmp_path / "m.mesh"
     p.write_text(text)
     return str(p)
@@ -38,3 +42,33 @@ def test_check_counts_the_loops_launches(precision, ty, tmp_path, monkeypatch):
     clean = rep["missed"] == rep["repeated"] == rep["outside"] == [0] * 6
     same = all(np.array_equal(a, b) for a, b in zip(ref, got))
     assert clean == same, (rep, same)
+
+
+@pytest.mark.parametrize("ty", ["1", "3", "5", "8"])
+@pytest.mark.parametrize("precision,n", [("fp64", 40), ("fp32", 40), ("fp64", 208)])
+def test_rows_per_tile(precision, n, ty, tmp_path, monkeypatch):
+    """VGPU_FAST_TY changes no field, where the fast tiles share the sweep's
+    launch (40^3) and where they have their own (208^3 in FP64, 85 MB a field)."""
+    mesh = _write(tmp_path, meshgen.freespace(n=n, steps=80))
+    print(f"case fields of {ty} rows per tile {n} {precision}", flush=True)
+    ref, _ = _fields(mesh, precision)
+    monkeypatch.setenv("VGPU_FAST_TY", ty)
+    got, rep = _fields(mesh, precision)
+    assert rep["missed"] == rep["repeated"] == rep["outside"] == [0] * 6, rep
+    for a, b in zip(ref, got):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("ty", ["2", "8"])
+def test_rows_per_tile_packed(ty, tmp_path, monkeypatch):
+    """The same for a packed group."""
+    meshes = [_write(tmp_path / str(q), meshgen.freespace(n=n, steps=60)) for q, n in enumerate((17, 24, 40))]
+    print(f"case packed, {ty} rows per tile", flush=True)
+    vulture_amd.run_meshes_group(meshes, [str(tmp_path / f"a{q}") for q in range(3)], precision="fp64")
+    monkeypatch.setenv("VGPU_FAST_TY", ty)
+    vulture_amd.run_meshes_group(meshes, [str(tmp_path / f"b{q}") for q in range(3)], precision="fp64")
+    for q in range(3):
+        a, b = str(tmp_path / f"a{q}"), str(tmp_path / f"b{q}")
+        files = sorted(os.listdir(a))
+        assert files and files == sorted(os.listdir(b))
+        assert filecmp.cmpfiles(a, b, files, shallow=False)[0] == files

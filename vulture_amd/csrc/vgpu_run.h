@@ -534,9 +534,12 @@ template <typename T> void fill_step_args(Ctx *c, StepArgs<T> &A, const VisitRun
   // 70.9, the FP64 96x81x64 box 49.9 and 52.6; with more blocks the planes' shared loads count (FP64 128^3
   // Debye volume 162 and 167).  Packed launches have their members' blocks
   // together and keep 4 (364 and 383 for 16 requests).
-  // rows per block (tuning override VGPU_FAST_TY: 1..8)
+  // Rows per block: four, a wavefront each, in the 256 threads of a launch that
+  // the tiles share with the shell and the side blocks.  Launches of their own
+  // take another number (tuning override VGPU_FAST_TY: 1..8).
   int ty = 4;
-  if (const char *ev = getenv("VGPU_FAST_TY")) ty = std::max(1, std::min(atoi(ev), 8));
+  if (!c->inl || (sweeps_apart(c) && !packed))
+    if (const char *ev = getenv("VGPU_FAST_TY")) ty = std::max(1, std::min(atoi(ev), 8));
   A.vblk = dim3(64 * ty);
   auto fast_grid = [&](const int *fb, int &kchunk) {
     if (fb[0] > fb[1] || fb[2] > fb[3] || fb[4] > fb[5]) return dim3(0, 0, 0);
