@@ -72,3 +72,35 @@ def test_rows_per_tile_packed(ty, tmp_path, monkeypatch):
         files = sorted(os.listdir(a))
         assert files and files == sorted(os.listdir(b))
         assert filecmp.cmpfiles(a, b, files, shallow=False)[0] == files
+
+
+def _box(n, body, bt="PML 5", steps=40):
+    c = n // 2
+    lines = ["VM 1.0.0", "CE sweep forms", f"DM {n} {n} {n}", "GS"]
+    lines += [f"BT {f} {bt}" for f in ("XLO", "XHI", "YLO", "YHI", "ZLO", "ZHI")]
+    lines += ["WF wf1 GAUSSIAN_PULSE 1.0 3.0e-11 1.0e-11",
+              f"EX {c} {c + 1} {c} {c + 1} {c} {c + 1} a JZ wf1 1.0 0.0", *body, f"OP {c} {c} {c} {c} {c} {c} t TDOM_ASCII"]
+    return "\n".join(lines + ["GE", f"NT {steps}", "CN 0.95", "MS 1e-3", "EN"]) + "\n"
+
+
+@pytest.mark.parametrize("classes", [True, False])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_listed_debye_site_memory(precision, classes, tmp_path, monkeypatch):
+    """Debye sites outside the sweeps' lines (two poles, or one without
+    classes) take no more than their list, coefficient and state did in
+    launches of their own: 8 bytes and 2 + poles reals a site."""
+    if not classes:
+        monkeypatch.setenv("VGPU_NO_INDEXED_MEDIA", "1")
+    print(f"case Debye site memory {precision} {classes}", flush=True)
+    medium = "2.0 0.01 1.0 1e9 -1e9" + (" 4e9 -3e9" if classes else "")
+    used = []
+    for mt in (f"MT m DEBYE {medium}", "MT m SIMPLE 2.0 0.01 1.0"):
+        mesh = _write(tmp_path, _box(112, [mt, "MB 20 90 25 95 30 100 m"]))
+        with vulture_amd.DeviceSolve(mesh, precision=precision) as ds:
+            st = ds.stats()
+            used.append(st["bytes"])
+            if len(used) == 1:
+                sites, poles = st["debye_sites"], st["debye_poles"]
+                assert poles == (2 if classes else 1) and sites > 3 * 70 ** 3 and not st["debye_fused"]
+    real = 8 if precision == "fp64" else 4
+    assert used[0] - used[1] <= sites * (8 + (2 + poles) * real) + 4096, (used, sites)

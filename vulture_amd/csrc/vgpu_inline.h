@@ -192,7 +192,8 @@ template <typename T> int build_inline(Ctx *c)
         } else {
           for (size_t k = a; k < b; ++k) {
             if (st[k].med >= 1 << 21) return set_error(c, VGPU_EINVAL, "Debye site index out of range");
-            add.push_back({st[k].key * 4, XO_DEBYE | st[k].med << 8, (int)listed++, 0, 0});
+            add.push_back({st[k].key * 4, XO_DEBYE | st[k].med << 8, 0, 0, 0});
+            ++listed;
           }
         }
       }
@@ -350,7 +351,8 @@ template <typename T> int build_inline(Ctx *c)
   plan(0);
   plan(1);
   if (!(indexed && fits())) {
-    for (const Ctx::XSite &s : simple) c->xent[0].push_back({s.key * 4, XO_DEBYE | s.med << 8, (int)listed++, 0, 0});
+    for (const Ctx::XSite &s : simple) c->xent[0].push_back({s.key * 4, XO_DEBYE | s.med << 8, 0, 0, 0});
+    listed += (long long)simple.size();
     simple.clear();
     sort_by_key(c->xent[0]);
     plan(0);
@@ -400,19 +402,33 @@ template <typename T> int build_inline(Ctx *c)
         a = b;
       }
     }
+    // Debye sites alone on their value, component by component; the sites of
+    // rows hold the state slots behind theirs
+    auto alone = [&](size_t q) { return !grouped[q] && R[q].b == R[q].a + 1 && kind(v[R[q].a]) == XO_DEBYE; };
+    std::vector<XSiteDev> site;
+    for (int C = 0; C < 3 && e == 0; ++C)
+      for (size_t q = 0; q < R.size(); ++q)
+        if (alone(q) && v[R[q].a].comp() == C)
+          site.push_back({(int)v[R[q].a].cell(), (unsigned)(v[R[q].a].code >> 8) << 2 | (unsigned)C});
+    if (e == 0) {
+      c->nXsite = (long long)site.size();
+      if (!up(c->d_xsite, site.data(), site.size() * sizeof(XSiteDev))) return fail("Debye sites");
+    }
+    int slot = (int)site.size();
     std::vector<XRow> row;
     std::vector<XOp<T>> op;
     std::vector<int> gstart;
-    row.reserve(upd[e].size() + R.size() + 1);
-    op.reserve(v.size());
+    row.reserve(upd[e].size() + R.size() - site.size() + 1);
+    op.reserve(v.size() - site.size());
     auto take = [&](const Value &r) {
       row.push_back({(int)v[r.a].cell(), (unsigned)op.size() << 2 | (unsigned)v[r.a].comp()});
-      for (size_t k = r.a; k < r.b; ++k) op.push_back({v[k].code, v[k].arg, T(v[k].a), T(v[k].b)});
+      for (size_t k = r.a; k < r.b; ++k)
+        op.push_back({v[k].code, kind(v[k]) == XO_DEBYE ? slot++ : v[k].arg, T(v[k].a), T(v[k].b)});
     };
     for (const Value &r : upd[e]) take(r);
     c->nXupd[e] = (long long)row.size();
     for (size_t q = 0; q < R.size(); ++q)
-      if (!grouped[q]) take(R[q]);
+      if (!grouped[q] && !alone(q)) take(R[q]);
     c->nXrow[e] = (long long)row.size() - c->nXupd[e];
     for (const Src &s : by)
       if (grouped[s.q]) {

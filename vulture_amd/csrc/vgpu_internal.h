@@ -95,7 +95,8 @@ template <typename T> struct HArgs {
 //    lane of a wavefront at a time at the x faces.)
 //  - Rows, for what is left (ghost planes, values that are not ordinary
 //    updates): a launch after the sweep, a thread per value, ghosts behind the
-//    row of their source.
+//    row of their source.  Debye sites alone on their value (of several poles,
+//    or without classes) have a list of their own in it.
 enum XKind { XO_SRC, XO_AUX, XO_WAVE, XO_ZERO, XO_DEBYE, XO_GHOST, XO_SIBC };
 // flags of a flagged class (E: dtab slot 6, H: the class table's slot 3):
 // one-pole Debye sites of components 0-2 (bits 0-2), zeroed components (3-5),
@@ -121,6 +122,13 @@ struct XRow {
   unsigned opc;          // first operation << 2 | component
 };
 
+// A Debye site that is its value's only operation: what a row would have to
+// look up -- its one operation, where that ends -- is known.
+struct XSiteDev {
+  int cell;
+  unsigned mc;           // medium << 2 | component
+};
+
 // A value of the incident field or of a source at one time: scale *
 // wf_value(t) in double, rounded once (a source), or its two factors rounded
 // first, the time less `geo` (an analytic plane wave's, at one edge).
@@ -138,6 +146,8 @@ template <typename T> struct XArgs {
   long long plane;
   T mzeta[6];            // Mur factors
   long long nupd, nrow, ngroup;  // update rows, rows, then groups of rows (a row and its ghosts)
+  long long nsite;       // sites alone on their value (E); they hold the first state slots
+  const XSiteDev *site;
   const int *gstart;     // first row of each group
   const XRow *row;
   const XOp<T> *op;
@@ -675,9 +685,14 @@ struct Ctx {
   bool xskip = false;                        // values may be left to update rows
   bool xflagH = false;                       // some H cells are flagged (with xskip)
   void *d_xargs[2] = {}, *d_xval[2] = {}, *d_xvals[2] = {}, *d_xcls[2] = {};
-  void *d_xgstart[2] = {}, *d_xrow[2] = {}, *d_xop[2] = {};
+  void *d_xgstart[2] = {}, *d_xrow[2] = {}, *d_xop[2] = {}, *d_xsite = nullptr;
   void *d_xdtab = nullptr, *d_xJ = nullptr;
-  long long nXval[2] = {}, nXupd[2] = {}, nXrow[2] = {}, nXgroup[2] = {};
+  long long nXval[2] = {}, nXupd[2] = {}, nXrow[2] = {}, nXgroup[2] = {}, nXsite = 0;
+  // blocks of half-step e's launch of rows: rows and groups, then sites
+  long long row_blocks(int e) const
+  {
+    return (nXrow[e] + nXgroup[e] + 255) / 256 + (e == 0 ? (nXsite + 255) / 256 : 0);
+  }
   std::vector<double> hflags;                // [H class] flags
   // fused leapfrog sweep: the fast boxes are its fused box, H cells to
   // update again after the E corrections

@@ -361,6 +361,7 @@ template <typename T> static void fill_correction_args(Ctx *c, XArgs<T> &x, int 
   x.cls = P<uint16_t>(c->indexed ? (e == 0 ? c->d_ecls : c->d_hcls) : c->d_xcls[e]);
   x.PX = c->PX; x.plane = c->plane;
   x.nupd = c->nXupd[e]; x.nrow = c->nXrow[e]; x.ngroup = c->nXgroup[e];
+  x.nsite = e == 0 ? c->nXsite : 0; x.site = P<XSiteDev>(e == 0 ? c->d_xsite : nullptr);
   x.gstart = P<int>(c->d_xgstart[e]); x.row = P<XRow>(c->d_xrow[e]); x.op = P<XOp<T>>(c->d_xop[e]);
   for (int d = 0; d < 3; ++d) {
     x.F[d] = P<T>(c->fld(0, 3 * e + d));
@@ -934,7 +935,7 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     else go(k_h_sweep<T, false, false>);
   };
   auto rows = [&](int e) {
-    const dim3 b(256), g((unsigned)((c->nXrow[e] + c->nXgroup[e] + 255) / 256));
+    const dim3 b(256), g((unsigned)c->row_blocks(e));
     if (!g.x) return;
     if (c->indexed && e == 0) hipLaunchKernelGGL((k_rows<T, true, true>), g, b, 0, s, xe);
     else if (c->indexed) hipLaunchKernelGGL((k_rows<T, true, false>), g, b, 0, s, xh);
@@ -1199,8 +1200,7 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
       sweepH[2 * x + f] = plan([&](int i) {
         return cs[i]->indexed == idx && cs[i]->xflagH == (f == 0)
                    ? (long long)A[i].nside[1] + cs[i]->nHworkPk + A[i].hg1.x : 0LL; });
-    auto nrows = [&](int i, int e) {
-      return cs[i]->indexed == idx ? (cs[i]->nXrow[e] + cs[i]->nXgroup[e] + 255) / 256 : 0LL; };
+    auto nrows = [&](int i, int e) { return cs[i]->indexed == idx ? cs[i]->row_blocks(e) : 0LL; };
     rowE[x] = plan([&](int i) { return nrows(i, 0); });
     rowH[x] = plan([&](int i) { return nrows(i, 1); });
   }
