@@ -104,3 +104,44 @@ def test_listed_debye_site_memory(precision, classes, tmp_path, monkeypatch):
                 assert poles == (2 if classes else 1) and sites > 3 * 70 ** 3 and not st["debye_fused"]
     real = 8 if precision == "fp64" else 4
     assert used[0] - used[1] <= sites * (8 + (2 + poles) * real) + 4096, (used, sites)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_one_pole_site_memory(precision, tmp_path):
+    """One-pole sites in the sweeps' lines: a small block in a large grid
+    holds currents for its own cells, not for the grid's."""
+    print(f"case one-pole site memory {precision}", flush=True)
+    used = []
+    for mt in ("MT m DEBYE 2.0 0.01 1.0 1e9 -1e9", "MT m SIMPLE 2.0 0.01 1.0"):
+        mesh = _write(tmp_path, _box(112, [mt, "MB 40 60 45 65 50 70 m"]))
+        with vulture_amd.DeviceSolve(mesh, precision=precision) as ds:
+            st = ds.stats()
+            used.append(st["bytes"])
+            if len(used) == 1:
+                sites = st["debye_sites"]
+                assert sites >= 3 * 20 ** 3 and st["debye_fused"]
+    real = 8 if precision == "fp64" else 4
+    assert used[0] - used[1] <= sites * (8 + 3 * real) + 4096, (used, sites)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("body", [
+    ["MT m DEBYE 2.0 0.01 1.0 1e9 -1e9", "MB 1 2 1 2 1 2 m"],
+    ["MT m DEBYE 2.0 0.01 1.0 1e9 -1e9", "MB 9 10 9 10 9 10 m"],
+    ["MT m DEBYE 2.0 0.01 1.0 1e9 -1e9", "MB 0 1 3 9 5 6 m", "EX 2 8 0 10 0 10 b =EZ wf1 0.2 0.0"],
+    ["MT m DEBYE 2.0 0.01 1.0 1e9 -1e9", "MT t DEBYE 3.0 0.0 1.0 1e9 -1e9 4e9 -3e9", "MB 0 10 0 10 0 10 m",
+     "MB 2 5 2 5 2 5 t", "MB 4 8 4 8 4 8 m"],
+], ids=["low", "high", "edge", "mixed"])
+@pytest.mark.parametrize("bt", ["PML 5", "MUR", "PEC"])
+def test_one_pole_boxes(bt, body, precision, tmp_path, monkeypatch):
+    """Currents over the sites' box: blocks at the ends of the grid, flagged
+    cells (Mur, sources) outside the box, blocks of other media among them.
+    Without classes the same sites are listed; the fields agree bit by bit."""
+    mesh = _write(tmp_path, _box(10, body, bt))
+    print(f"case one-pole box {bt} {body[1]} {precision}", flush=True)
+    a, _ = _fields(mesh, precision, 40)
+    monkeypatch.setenv("VGPU_NO_INDEXED_MEDIA", "1")
+    b, _ = _fields(mesh, precision, 40)
+    assert any(np.count_nonzero(f) for f in a)
+    for f, g in zip(a, b):
+        assert np.array_equal(f, g)

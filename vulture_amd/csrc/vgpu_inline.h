@@ -365,11 +365,17 @@ template <typename T> int build_inline(Ctx *c)
   c->indexed = indexed;
   c->debyeSimple = (long long)simple.size();
   c->debyeFast = 0;
+  int jhi[3] = {-1, -1, -1};
   for (const Ctx::XSite &s : simple) {
     int n[3];
     geo.unlin(s.key / 3, n);
     c->debyeFast += in_box(c->fastE, n[0], n[1], n[2]);
+    for (int a = 0; a < 3; ++a) {
+      c->jlo[a] = jhi[a] < 0 ? n[a] : std::min(c->jlo[a], n[a]);
+      jhi[a] = std::max(jhi[a], n[a]);
+    }
   }
+  for (int a = 0; a < 3; ++a) c->jn[a] = jhi[a] < 0 ? 0 : jhi[a] - c->jlo[a] + 1;
   c->debyeSites = listed;
   if (listed > INT32_MAX) return set_error(c, VGPU_EINVAL, "too many Debye sites");
   if (listed) {
@@ -483,7 +489,8 @@ template <typename T> int build_inline(Ctx *c)
       dt[k * DTAB_STRIDE + 6] = T(made[e][k][4]);
     }
     if (!up(c->d_xdtab, dt.data(), dt.size() * sizeof(T))) return fail("class table");
-    if (!simple.empty() && !(c->d_xJ = dev_alloc(c, 3 * c->ncell * sizeof(T)))) return fail("Debye state");
+    if (!simple.empty() && !(c->d_xJ = dev_alloc(c, (size_t)c->jn[0] * c->jn[1] * c->jn[2] * 3 * sizeof(T))))
+      return fail("Debye state");
   }
   return VGPU_OK;
 }

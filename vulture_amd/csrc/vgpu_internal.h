@@ -80,8 +80,8 @@ template <typename T> struct HArgs {
 //  - In line: the thread that sweeps a cell applies them right after its
 //    update, with no second pass over the field.  This takes what needs no
 //    look-up chain: a single one-pole Debye site per value (its alpha and beta
-//    in the class table, its J in a dense array, its previous E the old E the
-//    sweep has in a register), an E to zero (SIBC), and Mur's E, which the
+//    in the class table, its J in a dense array over the sites' box, its
+//    previous E the old E the sweep has in a register), an E to zero (SIBC), and Mur's E, which the
 //    thread of the face's inner neighbour writes, having both of that
 //    neighbour's values Mur's equation takes.  Such cells have coefficient
 //    classes of their own (from `flag0` on), so the others pay one comparison.
@@ -141,13 +141,11 @@ template <typename T> struct XArgs {
   unsigned flag0;        // first flagged class (E)
   const uint16_t *cls;   // per cell: class, or without classes E 0 / 1 + dtab row, H its flags
   const T *dtab;         // [class - flag0][8]: alpha, beta of J per component, flags
-  T *J;                  // [cell][component] (null without one-pole sites)
+  T *J;                  // [cell of the one-pole sites' box][component]
   int PX;
   long long plane;
   T mzeta[6];            // Mur factors
   long long nupd, nrow, ngroup;  // update rows, rows, then groups of rows (a row and its ghosts)
-  long long nsite;       // sites alone on their value (E); they hold the first state slots
-  const XSiteDev *site;
   const int *gstart;     // first row of each group
   const XRow *row;
   const XOp<T> *op;
@@ -166,6 +164,10 @@ template <typename T> struct XArgs {
   const int *dnp;
   int dmaxP, dcplx;
   const T *Etan;
+  long long nsite;       // sites alone on their value (E); they hold the first state slots
+  const XSiteDev *site;
+  int jlo[3], jn[2], jplane;  // first cell of the one-pole sites' box, its extents in x and y, their product
+  unsigned jlast;        // the box's last cell
 };
 
 // Values of a half-step's sources and analytic plane waves, evaluated ahead
@@ -682,6 +684,7 @@ struct Ctx {
   std::vector<double> dhost[2];              // its alpha and beta (real part)
   std::vector<XVal> xval[2];
   unsigned xflag0 = ~0u;
+  int jlo[3] = {}, jn[3] = {};               // box of the one-pole sites
   bool xskip = false;                        // values may be left to update rows
   bool xflagH = false;                       // some H cells are flagged (with xskip)
   void *d_xargs[2] = {}, *d_xval[2] = {}, *d_xvals[2] = {}, *d_xcls[2] = {};

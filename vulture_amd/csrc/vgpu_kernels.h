@@ -430,9 +430,9 @@ template <typename T> VG_DEV void x_debye(T &j, T da, T db, T be, T eo, T &e)
 }
 
 // What a flagged cell's corrections read, loaded together with the update's
-// own operands: its class's row of dtab, J -- dense and interleaved, so its
-// address needs nothing but the cell and it is one stream -- and the E of the
-// first Mur face beside it.
+// own operands: its class's row of dtab, J -- dense over the sites' box and
+// interleaved, so its address needs nothing but the cell and it is one stream
+// -- and the E of the first Mur face beside it.
 template <typename T> struct XPre {
   T j[3], d[6], m0, m1, mz;
   unsigned fl;
@@ -446,12 +446,18 @@ template <typename T> struct XPre {
     const int C = ((f >> 1) + 1 + s) % 3;
     return gp(C == 0 ? x->F[0] : C == 1 ? x->F[1] : x->F[2]);
   }
-  template <bool DEBYE> VG_DEV void load(const VG_CONST XArgs<T> *x, long long id, unsigned cls)
+  // place of a cell in J
+  VG_DEV static int j_at(const VG_CONST XArgs<T> *x, int i, int j, int k)
+  {
+    return (k - x->jlo[2]) * x->jplane + (j - x->jlo[1]) * x->jn[0] + (i - x->jlo[0]);
+  }
+  template <bool DEBYE> VG_DEV void load(const VG_CONST XArgs<T> *x, long long id, int jid, unsigned cls)
   {
     const VG_GLOBAL T *q = gp(x->dtab) + (cls - x->flag0) * DTAB_STRIDE;
     fl = (unsigned)q[6];
     if (DEBYE) {
-      const VG_GLOBAL T *J = gp(x->J) + 3 * id;
+      // (flagged cells without a site may lie outside the box)
+      const VG_GLOBAL T *J = gp(x->J) + 3ull * min((unsigned)jid, x->jlast);
       for (int c = 0; c < 3; ++c) j[c] = J[c];
       for (int c = 0; c < 6; ++c) d[c] = q[c];
     }
@@ -469,7 +475,7 @@ template <typename T> struct XPre {
 // beta): the Mur faces that take its update (mur.c:135-395), its one-pole
 // Debye sites, its zeroed components.
 template <typename T, bool DEBYE>
-VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, XPre<T> &p, T o0, T o1, T o2, T b0, T b1, T b2, T &e0,
+VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, int jid, XPre<T> &p, T o0, T o1, T o2, T b0, T b1, T b2, T &e0,
                        T &e1, T &e2)
 {
   const unsigned fl = p.fl;
@@ -496,7 +502,7 @@ VG_DEV void x_inline_e(const VG_CONST XArgs<T> *x, long long id, XPre<T> &p, T o
     if (fl & XF_DEBYE) x_debye(p.j[0], p.d[0], p.d[1], b0, o0, e0);
     if (fl & (XF_DEBYE << 1)) x_debye(p.j[1], p.d[2], p.d[3], b1, o1, e1);
     if (fl & (XF_DEBYE << 2)) x_debye(p.j[2], p.d[4], p.d[5], b2, o2, e2);
-    VG_GLOBAL T *J = gp(x->J) + 3 * id;  // this thread's alone: the others go back as they came
+    VG_GLOBAL T *J = gp(x->J) + 3ll * jid;  // this thread's alone: the others go back as they came
     for (int c = 0; c < 3; ++c) J[c] = p.j[c];
   }
   if (fl & XF_ZERO) e0 = T(0);
@@ -554,6 +560,8 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
   const T idhx = f.idh[0][ic], idhy = f.idh[1][j];
   const unsigned flag0 = X ? x->flag0 : ~0u;
   long long id = ((long long)kb * f.NY + j) * SJ + ic;
+  constexpr bool DEBYE = X == 2 || X == 4;
+  int jid = DEBYE ? XPre<T>::j_at(x, ic, j, kb) : 0;
   // The fast box starts at index 1 or more on every axis, so the i-1, j-1
   // and k-1 neighbours are inside the allocation.
   T hxm = Hx[id - P], hym = Hy[id - P];
@@ -565,7 +573,7 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
     const unsigned cls = cnext;
     XPre<T> pre{};
     const bool flagged = X && cls >= flag0;
-    if (flagged) pre.template load<(X == 2 || X == 4)>(x, id, cls);
+    if (flagged) pre.template load<DEBYE>(x, id, jid, cls);
     const T hx = Hx[id], hy = Hy[id], hz = Hz[id];
     const T hzy = Hz[id - SJ], hzx = Hz[id - 1], hyx = Hy[id - 1], hxy = Hx[id - SJ];
     if (pc) cnext = (unsigned)pc[id + P];
@@ -593,7 +601,7 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
         for (int C = 0; C < 3; ++C)
           if (X < 3 || !(pre.fl & (XF_SKIP << C))) visit(f.vis[C], id);
       } else {
-        if (flagged) x_inline_e<T, (X == 2 || X == 4)>(x, id, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
+        if (flagged) x_inline_e<T, DEBYE>(x, id, jid, pre, o0, o1, o2, b0, b1, b2, e0, e1, e2);
         if (X < 3 || !(pre.fl & XF_SKIP)) f.E[0][id] = e0;
         if (X < 3 || !(pre.fl & (XF_SKIP << 1))) f.E[1][id] = e1;
         if (X < 3 || !(pre.fl & (XF_SKIP << 2))) f.E[2][id] = e2;
@@ -601,6 +609,7 @@ VG_DEV void e_fast_tile(const FastE<T> &f, const VG_CONST XArgs<T> *x, unsigned 
     }
     hxm = hx;
     hym = hy;
+    if (DEBYE) jid += x->jplane;
   }
 }
 
@@ -1091,7 +1100,9 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
   const bool xm = i > 0, ym = j > 0;
   const T idh0 = g.idh[0][i], idh1 = g.idh[1][j];
   const unsigned flag0 = X ? x->flag0 : ~0u;
+  constexpr bool DEBYE = X == 2 || X == 4;
   int k = pc->z0 + dk0;
+  int jid = DEBYE ? XPre<T>::j_at(x, i, j, k) : 0;
   long long id = ((long long)k * NY + j) * SJ + i;
   T hxm = k > 0 ? Hx[id - P] : T(0), hym = k > 0 ? Hy[id - P] : T(0);  // plane k-1, carried
   EShellCell<T, IDX, 0> c0;
@@ -1115,7 +1126,7 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
     const int n3[3] = {i, j, k};
     XPre<T> pre{};
     const bool flagged = X && cls >= flag0;
-    if (flagged) pre.template load<(X == 2 || X == 4)>(x, id, cls);
+    if (flagged) pre.template load<DEBYE>(x, id, jid, cls);
     c0.load(g, rg[0], n3, id, cls);
     c1.load(g, rg[1], n3, id, cls);
     c2.load(g, rg[2], n3, id, cls);
@@ -1127,13 +1138,14 @@ VG_DEV void e_shell_column(const ShellDev *pcs, const ShellWork *work, const EAr
       T e0 = c0.value(g, rg[0], idh1 * (hz - hzy) + idh2 * (hym - hy));
       T e1 = c1.value(g, rg[1], idh2 * (hx - hxm) + idh0 * (hzx - hz));
       T e2 = c2.value(g, rg[2], idh0 * (hy - hyx) + idh1 * (hxy - hx));
-      if (flagged) x_inline_e<T, (X == 2 || X == 4)>(x, id, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
+      if (flagged) x_inline_e<T, DEBYE>(x, id, jid, pre, c0.e, c1.e, c2.e, c0.be, c1.be, c2.be, e0, e1, e2);
       if (rg[0].reg >= 0 && (X < 3 || !(pre.fl & XF_SKIP))) g.E[0][id] = e0;
       if (rg[1].reg >= 0 && (X < 3 || !(pre.fl & (XF_SKIP << 1)))) g.E[1][id] = e1;
       if (rg[2].reg >= 0 && (X < 3 || !(pre.fl & (XF_SKIP << 2)))) g.E[2][id] = e2;
     }
     hxm = hx;
     hym = hy;
+    if (DEBYE) jid += x->jplane;
     rg[0].q += rg[0].psz;
     rg[1].q += rg[1].psz;
     rg[2].q += rg[2].psz;

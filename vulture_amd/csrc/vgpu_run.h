@@ -377,6 +377,10 @@ template <typename T> static void fill_correction_args(Ctx *c, XArgs<T> &x, int 
   x.flag0 = ~0u;
   if (e) return;
   x.flag0 = c->xflag0;
+  for (int a = 0; a < 3; ++a) x.jlo[a] = c->jlo[a];
+  for (int a = 0; a < 2; ++a) x.jn[a] = c->jn[a];
+  x.jplane = c->jn[0] * c->jn[1];
+  x.jlast = (unsigned)((long long)x.jplane * c->jn[2] - 1);
   x.dtab = P<T>(c->d_xdtab); x.J = P<T>(c->d_xJ);
   for (int f = 0; f < 6; ++f) x.mzeta[f] = T(c->zeta[f]);
   x.dlast = P<T>(c->d_dlast); x.dJ = P<T>(c->d_dJ); x.dstride = c->debyeSites;

@@ -94,15 +94,24 @@ static size_t estimate_bytes(const vh_solve *s, int prec)
   const size_t gi = (size_t)(s->gibox[XHI] - s->gibox[XLO]) * (s->gibox[YHI] - s->gibox[YLO]) *
                     (s->gibox[ZHI] - s->gibox[ZLO]);
   b += (go - gi) * 9 * esz;
-  if (s->numDebye > 0) b += ncell * 3 * esz;  /* dense polarisation currents */
+  /* one-pole sites: currents over the sites' box, or listed like the others */
+  size_t listed = 0, onePole = 0, box = 0;
+  int lo[3] = {0, 0, 0}, hi[3] = {-1, -1, -1};
   for (int d = 0; d < s->numDebye; d++) {
+    const bool one = s->media[s->debye[d].medium].numPoles == 1;
     size_t n = 0;
     for (int f = 0; f < 3; f++) {
       const int *l = s->debye[d].flim[f];
       n += (size_t)(l[XHI] - l[XLO] + 1) * (l[YHI] - l[YLO] + 1) * (l[ZHI] - l[ZLO] + 1);
+      for (int a = 0; a < 3 && one; a++) {
+        if (hi[a] < 0 || l[2 * a] < lo[a]) lo[a] = l[2 * a];
+        if (l[2 * a + 1] > hi[a]) hi[a] = l[2 * a + 1];
+      }
     }
-    b += n * (esz * 3 + 16);
+    *(one ? &onePole : &listed) += n * (esz * 3 + 16);
   }
+  if (onePole) box = (size_t)(hi[0] - lo[0] + 1) * (hi[1] - lo[1] + 1) * (hi[2] - lo[2] + 1) * 3 * esz;
+  b += listed + (box > onePole ? box : onePole);
   b += (size_t)s->numObs * (s->numTimeSteps * 6 * 8 + 12 * s->numFreq * 8);
   return b + b / 8 + ((size_t)64 << 20);
 }
