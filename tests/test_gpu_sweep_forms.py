@@ -1,6 +1,8 @@
 """The launch forms of the step that the default sizes of the other tests do
 not take (needs an MI355X)."""
+import ctypes
 import filecmp
+import math
 import os
 
 import numpy as np
@@ -145,3 +147,136 @@ def test_one_pole_boxes(bt, body, precision, tmp_path, monkeypatch):
     assert any(np.count_nonzero(f) for f in a)
     for f, g in zip(a, b):
         assert np.array_equal(f, g)
+
+
+class _Grid(ctypes.Structure):
+    """vgpu_grid_desc (include/vgpu.h)."""
+    _I6, _D = ctypes.c_int * 6, ctypes.POINTER(ctypes.c_double)
+    _fields_ = [("nx", ctypes.c_int), ("ny", ctypes.c_int), ("nz", ctypes.c_int), ("gibox", _I6), ("gobox", _I6),
+                ("gfilim", _I6 * 6), ("dt", ctypes.c_double), ("c0", ctypes.c_double), ("eps0", ctypes.c_double),
+                ("mu0", ctypes.c_double), ("eta0", ctypes.c_double), ("grid_type", ctypes.c_int),
+                ("xlines", _D), ("ylines", _D), ("zlines", _D), ("nlines", ctypes.c_int * 3),
+                ("dex", _D), ("dey", _D), ("dez", _D), ("idex", _D), ("idey", _D), ("idez", _D),
+                ("idhx", _D), ("idhy", _D), ("idhz", _D)]
+
+
+N, ALPHA, BETA, GAMMA, SIZE = 8, 0.9, 0.4, 0.3, 2.0
+
+
+def _context(v, lim, ghosts):
+    """A uniform N^3 grid of unit edges in FP64, a hard Ez source at (3, 4, 4)
+    that holds SIZE from the second step on (a compact step of tiny width)."""
+    ones = np.ones(N + 1)
+    dp = ones.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    g = _Grid(nx=N, ny=N, nz=N, dt=1.0, c0=1.0, eps0=1.0, mu0=1.0, eta0=1.0, grid_type=0)
+    for q in range(6):
+        g.gibox[q] = g.gobox[q] = 1 if q % 2 == 0 else N - 1
+        for c in range(6):
+            g.gfilim[c][q] = lim[c][q]
+    g.nlines = (ctypes.c_int * 3)(N, N, N)
+    for f in ("xlines", "ylines", "zlines", "dex", "dey", "dez", "idex", "idey", "idez", "idhx", "idhy", "idhz"):
+        setattr(g, f, dp)
+    ctx = ctypes.c_void_p()
+    assert v.vgpu_create(ctypes.byref(g), 0, 0, ctypes.byref(ctx)) == 0
+    arrays = [np.full(N ** 3, x) for x in (ALPHA, BETA, GAMMA)]
+    p3 = ctypes.c_void_p * 3
+    assert v.vgpu_set_media(ctx, *[p3(*[a.ctypes.data] * 3) for a in arrays]) == 0
+    assert v.vgpu_set_ghosts(ctx, (ctypes.c_int * 6)(*ghosts)) == 0
+    d = ctypes.c_double
+    assert v.vgpu_add_waveform(ctx, 8, d(1.0), d(0.0), d(1e-9), d(0.25), None, ctypes.c_ulong(0)) == 0
+    assert v.vgpu_add_source(ctx, 2, 0, 0, d(SIZE), 0, d(0.0), (ctypes.c_int * 6)(3, 3, 4, 4, 4, 4)) == 0
+    assert v.vgpu_finalize(ctx, ctypes.c_uint64(64), ctypes.c_uint64(64)) == 0, v.vgpu_last_error(ctx)
+    return ctx
+
+
+def _expected(lim, ghosts, steps):
+    """The same steps in numpy: sweeps over the limits, source, ghost copies."""
+    E, H = np.zeros((3, N, N, N)), np.zeros((3, N, N, N))
+
+    def sweep(F, G, e):
+        new = F.copy()
+        for c in range(3):
+            l = lim[3 * (not e) + c]
+            at = tuple(slice(l[2 * a], l[2 * a + 1] + 1) for a in range(3))
+            a1, a2 = (c + 1) % 3, (c + 2) % 3
+            s = 1 if e else -1  # E reads the value below, H the one above
+
+            def diff(g, a):
+                return (g - np.roll(g, s, a))[at] * (1 if e else -1)
+            curl = diff(G[a2], a1) - diff(G[a1], a2)
+            new[c][at] = (ALPHA * F[c][at] + BETA * curl) if e else F[c][at] - GAMMA * curl
+        F[:] = new
+
+    def copy(F, e):
+        for f, t in enumerate(ghosts):
+            a, hi = f >> 1, f & 1
+            if not t:
+                continue
+            dst, src = (N - 1, N - 2) if hi else (0, 1)
+            if t == 3:
+                src = 1 if hi else N - 2
+            for c in range(3):
+                if (c == a) == e:
+                    i, j = [slice(None)] * 3, [slice(None)] * 3
+                    i[a], j[a] = dst, src
+                    F[c][tuple(i)] = (-1.0 if t == 2 else 1.0) * F[c][tuple(j)]
+
+    for n in range(steps):
+        sweep(E, H, True)
+        # a compact step of no width times sin(2 pi n / 4)
+        E[2][3, 4, 4] = SIZE * math.sin(2.0 * 4.0 * math.atan(1.0) * 0.25 * n) if n else 0.0
+        copy(E, True)
+        sweep(H, E, False)
+        copy(H, False)
+    return list(E) + list(H)
+
+
+def _download(v, ctx):
+    out = []
+    for c in range(6):
+        a = np.empty((N, N, N))
+        assert v.vgpu_download_field(ctx, c, a.ctypes.data_as(ctypes.c_void_p)) == 0
+        out.append(a)
+    return out
+
+
+@pytest.mark.parametrize("ghosts", [(1, 2, 3, 3, 2, 1), (3, 3, 1, 1, 2, 2)])
+@pytest.mark.parametrize("inside", [False, True])
+def test_ghost_planes_and_limits(inside, ghosts):
+    """Ghost planes beside the sweeps' limits, and inside them, where the
+    sweep's value is overwritten by the copy: alone and in a group run."""
+    vulture_amd.load_host()
+    v = vulture_amd.load_vgpu()
+    v.vgpu_create.restype = v.vgpu_finalize.restype = v.vgpu_set_media.restype = ctypes.c_int
+    v.vgpu_destroy.argtypes = [ctypes.c_void_p]
+    steps = 12
+    usual = [[1, N - 2] * 3 for _ in range(6)]
+    lim = [l[:] for l in usual]
+    if inside:  # each ghost component over its ghost planes too
+        for c in range(6):
+            for a in range(3):
+                if (c < 3) == (c % 3 == a):
+                    lim[c][2 * a + 1] = N - 1
+                    if c < 3:
+                        lim[c][2 * a] = 1
+    print(f"case ghost planes inside {inside} {ghosts}", flush=True)
+    ctxs = [_context(v, l, ghosts) for l in (lim, lim, usual, usual)]
+    try:
+        for ctx in (ctxs[0], ctxs[2]):
+            assert v.vgpu_run(ctx, 0, steps, None) == 0
+        first = (ctypes.c_uint64 * 2)(0, 0)
+        group = (ctypes.c_void_p * 2)(ctxs[1], ctxs[3])
+        for n in range(0, steps, 4):
+            first[0] = first[1] = n
+            assert v.vgpu_run_group(group, 2, first, ctypes.c_uint64(4)) == 0
+        for ctx in ctxs:
+            assert v.vgpu_synchronize(ctx) == 0
+        alone, grouped = _download(v, ctxs[0]), _download(v, ctxs[1])
+        exp = _expected(lim, ghosts, steps)
+        for a, b, x in zip(alone, grouped, exp):
+            assert np.array_equal(a, b)
+            assert np.max(np.abs(a - x)) <= 1e-13 * max(1.0, np.max(np.abs(x)))
+        assert any(np.count_nonzero(a) > 100 for a in alone)
+    finally:
+        for ctx in ctxs:
+            v.vgpu_destroy(ctx)

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <array>
 #include <map>
+#include <new>
 #include <atomic>
 #include <mutex>
 #include <shared_mutex>
@@ -1293,6 +1294,34 @@ static int build_leap(Ctx *c)
   return VGPU_OK;
 }
 
+// The corrections' lists and the class tables, in the form c->inl names.
+static int build_lists(Ctx *c)
+{
+  try {
+    int r;
+    if ((r = build_debye(c)) || (r = build_sibc(c)) || (r = build_corrections(c)) ||
+        (r = c->prec == VGPU_FP64 ? build_inline<double>(c) : build_inline<float>(c)))
+      return r;
+    return build_class_tables(c);
+  } catch (const std::bad_alloc &) {
+    return set_error(c, VGPU_ENOMEM, "corrections: host memory");
+  }
+}
+
+// Takes back what build_lists made, device memory from allocation `mark` on
+// included, and leaves the context to the separate launches.  (Classes that
+// build_inline added beside the host's stay: their coefficients are those of
+// the classes they came from.)
+static void drop_inline(Ctx *c, size_t mark, size_t bytes)
+{
+  for (size_t q = mark; q < c->allocs.size(); ++q) hipFree(c->allocs[q]);
+  c->allocs.resize(mark);
+  c->bytes = bytes;
+  (void)hipGetLastError();
+  static_cast<InlineState &>(*c) = InlineState();
+  c->debyeSites = 0;
+}
+
 int vgpu_finalize(vgpu_ctx *c, uint64_t total_steps, uint64_t max_steps_per_run)
 {
   if (!c || c->finalized) return VGPU_ESTATE;
@@ -1303,10 +1332,18 @@ int vgpu_finalize(vgpu_ctx *c, uint64_t total_steps, uint64_t max_steps_per_run)
   c->d_step = dev_alloc(c, 64);
   if (!c->d_step) return set_error(c, VGPU_ENOMEM, "step counter");
   int r;
-  if ((r = build_debye(c)) || (r = build_sibc(c)) || (r = build_corrections(c)) || (r = build_observers(c)) ||
-      (r = c->prec == VGPU_FP64 ? build_inline<double>(c) : build_inline<float>(c)) || (r = build_class_tables(c)) ||
-      (r = build_leap(c)))
-    return r;
+  if ((r = build_observers(c))) return r;
+  const size_t mark = c->allocs.size(), bytes = c->bytes;
+  r = build_lists(c);
+  if (r && c->inl) {
+    // what the in-line form does not hold -- a ghost plane that a sweep updates,
+    // more operations than a row's number counts, more memory than there is --
+    // the launches of their own may
+    drop_inline(c, mark, bytes);
+    r = build_lists(c);
+    if (!r) c->err.clear();
+  }
+  if (r || (r = build_leap(c))) return r;
   if ((r = c->prec == VGPU_FP64 ? prepare_sweeps<double>(c) : prepare_sweeps<float>(c))) return r;
   if (c->inl && (r = c->prec == VGPU_FP64 ? upload_pack<double>(c) : upload_pack<float>(c)))
     return r;

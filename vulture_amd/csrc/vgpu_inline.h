@@ -22,6 +22,7 @@ template <typename T> struct InlineGeom {
   int ein[3][1][6];
   struct Ghost { int axis, dst, src; double sign; };
   std::vector<Ghost> ghosts[6];  // per component, in face order
+  int glo[3], ghi[3];            // the copied planes' extents
 
   explicit InlineGeom(Ctx *ctx) : c(ctx)
   {
@@ -29,6 +30,11 @@ template <typename T> struct InlineGeom {
     for (int C = 0; C < 3; ++C)
       for (int q = 0; q < 6; ++q) ein[C][0][q] = ea.in[C][q];
     // ghost planes as launch_ghosts copies them (surface.c:569-812)
+    const int N[3] = {c->NX, c->NY, c->NZ};
+    for (int a = 0; a < 3; ++a) {
+      glo[a] = std::max(0, c->grid.gobox[2 * a] - 1);
+      ghi[a] = std::min(N[a] - 1, c->grid.gobox[2 * a + 1]);
+    }
     for (int f = 0; f < 6; ++f) {
       const int t = c->ghost[f], a = f >> 1;
       if (!t) continue;
@@ -53,6 +59,8 @@ template <typename T> struct InlineGeom {
   }
   bool ghost_dst(int C, const int n[3]) const
   {
+    for (int a = 0; a < 3; ++a)
+      if (n[a] < glo[a] || n[a] > ghi[a]) return false;
     for (const Ghost &g : ghosts[C])
       if (n[g.axis] == g.dst) return true;
     return false;
@@ -211,7 +219,11 @@ template <typename T> int build_inline(Ctx *c)
     for (int C = 0; C < 3; ++C) {
       const auto &gs = geo.ghosts[3 * e + C];
       for (size_t g = 0; g < gs.size(); ++g) {
-        int lo[3] = {0, 0, 0}, hi[3] = {N[0] - 1, N[1] - 1, N[2] - 1}, n[3];
+        int lo[3], hi[3], n[3];
+        for (int a = 0; a < 3; ++a) {
+          lo[a] = geo.glo[a];
+          hi[a] = geo.ghi[a];
+        }
         lo[gs[g].axis] = hi[gs[g].axis] = gs[g].dst;
         for (n[2] = lo[2]; n[2] <= hi[2]; ++n[2])
           for (n[1] = lo[1]; n[1] <= hi[1]; ++n[1])

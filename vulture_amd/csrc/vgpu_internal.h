@@ -619,46 +619,10 @@ inline void leap_box(const int gfilim[6][6], const int N[3], int fb[6])
   if (w >= 63 && w % 63 <= 16) fb[1] = fb[0] + w / 63 * 63 - 1;
 }
 
-struct Ctx {
-  std::string err;
-  vgpu_prec prec;
-  int device;
-  size_t esz;            // bytes per stored real
-  int NX, NY, NZ, PX;
-  long long plane;
-  size_t ncell;          // PX*NY*NZ
-  vgpu_grid_desc grid;
-  std::vector<double> xl, yl, zl, dex, dey, dez, idex, idey, idez, idhx, idhy, idhz;
-  hipStream_t stream = nullptr;
-  std::vector<hipEvent_t> evE, evH;
-  double last_total_ms = 0, last_e_ms = 0, last_h_ms = 0;
-  bool finalized = false;
-  size_t bytes = 0;
-
-  // device allocations
-  std::vector<void *> allocs;
-  // the field sets (Ex..Hz each): set `par` holds the current fields; with
-  // the fused sweep there are two and every step flips it, otherwise F1 is F
-  void *F[6] = {}, *F1[6] = {};
-  int par = 0;
-  void *fld(int set, int d) const { return set ? F1[d] : F[d]; }
-  int next(int set) const { return leap ? set ^ 1 : set; }  // the set a step writes
-  void *alpha[3] = {}, *beta[3] = {}, *gamma[3] = {};
-  void *ide[3] = {}, *idh[3] = {};
-  bool media_set = false;
-
-  // Coefficient classes (the reference's indexed-media representation,
-  // grid.h:108-135): every cell's (alpha, beta) triple of E components and
-  // gamma triple of H components is one entry of a small table.  Built on
-  // the host in vgpu_set_media, refined with the layer-0 Debye block of each
-  // E component in vgpu_finalize, uploaded as uint16 per cell when both
-  // tables fit.
-  std::vector<uint32_t> ecls, hcls;          // host, per device cell
-  std::vector<double> etab, htab;            // host: [class][6] alpha/beta, [class][3] gamma (device: padded to 8, 4)
-  bool indexed = false;
-  void *d_ecls = nullptr, *d_hcls = nullptr, *d_etab = nullptr, *d_htab = nullptr;
-  int nEcls = 0, nHcls = 0;
-  // corrections as XArgs has them: every context but those with the fused sweep
+// The in-line form of a context's corrections (XArgs).
+struct InlineState {
+  // every context but those with the fused sweep, those too large for it, and
+  // those whose set-up it does not hold
   bool inl = false;
   bool murPush = false;                      // Mur E written by its inner neighbour's thread
   // in-line corrections of the E sweep: 0 none, 1 Mur and zeros, 2 Debye
@@ -697,6 +661,47 @@ struct Ctx {
     return (nXrow[e] + nXgroup[e] + 255) / 256 + (e == 0 ? (nXsite + 255) / 256 : 0);
   }
   std::vector<double> hflags;                // [H class] flags
+};
+
+struct Ctx : InlineState {
+  std::string err;
+  vgpu_prec prec;
+  int device;
+  size_t esz;            // bytes per stored real
+  int NX, NY, NZ, PX;
+  long long plane;
+  size_t ncell;          // PX*NY*NZ
+  vgpu_grid_desc grid;
+  std::vector<double> xl, yl, zl, dex, dey, dez, idex, idey, idez, idhx, idhy, idhz;
+  hipStream_t stream = nullptr;
+  std::vector<hipEvent_t> evE, evH;
+  double last_total_ms = 0, last_e_ms = 0, last_h_ms = 0;
+  bool finalized = false;
+  size_t bytes = 0;
+
+  // device allocations
+  std::vector<void *> allocs;
+  // the field sets (Ex..Hz each): set `par` holds the current fields; with
+  // the fused sweep there are two and every step flips it, otherwise F1 is F
+  void *F[6] = {}, *F1[6] = {};
+  int par = 0;
+  void *fld(int set, int d) const { return set ? F1[d] : F[d]; }
+  int next(int set) const { return leap ? set ^ 1 : set; }  // the set a step writes
+  void *alpha[3] = {}, *beta[3] = {}, *gamma[3] = {};
+  void *ide[3] = {}, *idh[3] = {};
+  bool media_set = false;
+
+  // Coefficient classes (the reference's indexed-media representation,
+  // grid.h:108-135): every cell's (alpha, beta) triple of E components and
+  // gamma triple of H components is one entry of a small table.  Built on
+  // the host in vgpu_set_media, refined with the layer-0 Debye block of each
+  // E component in vgpu_finalize, uploaded as uint16 per cell when both
+  // tables fit.
+  std::vector<uint32_t> ecls, hcls;          // host, per device cell
+  std::vector<double> etab, htab;            // host: [class][6] alpha/beta, [class][3] gamma (device: padded to 8, 4)
+  bool indexed = false;
+  void *d_ecls = nullptr, *d_hcls = nullptr, *d_etab = nullptr, *d_htab = nullptr;
+  int nEcls = 0, nHcls = 0;
   // fused leapfrog sweep: the fast boxes are its fused box, H cells to
   // update again after the E corrections
   bool leap = false;
