@@ -47,15 +47,18 @@ METRIC = "Mcells/s FP64 vs FP32 at 256^3 + %HBM peak; p50/p99 sweep-solve latenc
 HBM_PEAK_GBS = 8000.0
 
 
-def _traffic(kernel, prec):
-    """HBM bytes per launch from a committed rocprofv3 --pmc summary, or None."""
+def _traffic(kernel, prec, algorithmic):
+    """HBM bytes per launch from a committed rocprofv3 --pmc summary; None
+    without one of a launch of the same compulsory bytes (a summary of another
+    grid, or of the kernel before it did other work, says nothing here)."""
     path = os.path.join(HERE, "profiles", f"traffic_{kernel}_debye256_{prec}.txt")
     if not os.path.exists(path):
         return None
-    for line in open(path):
-        if line.startswith("traffic_bytes_per_launch"):
-            return float(line.split()[1])
-    return None
+    with open(path) as f:
+        vals = dict(line.split() for line in f if len(line.split()) == 2 and line[0] != "#")
+    if float(vals.get("algorithmic_bytes", 0)) != algorithmic:
+        return None
+    return float(vals["traffic_bytes_per_launch"])
 
 
 def debye_site_words(st):
@@ -123,7 +126,7 @@ def measure(mesh, prec, steps, warmup):
     achieved = kb / (kms * 1e-3) / 1e9
     sb = step_bytes(st, esz)
     step_gbs = sb / (ms_step * 1e-3) / 1e9
-    traffic = _traffic(name, prec)
+    traffic = _traffic(name, prec, kb)
     return {
         "prec": prec, "setup_s": round(setup_s, 2), "stats": st,
         "value": st["cells"] * steps / (total_ms * 1e-3) / 1e6,

@@ -15,11 +15,13 @@
       launch of kernel NAME, each request counter scaled by the bytes the copy
       moves per request.
   python -m vulture_amd.profiling traffic --kernel NAME --fetch DIR --write DIR
-          --copy-fetch DIR --copy-write DIR [--mib N]
+          --copy-fetch DIR --copy-write DIR [--mib N] [--algorithmic BYTES]
       From four `rocprofv3 --pmc FETCH_SIZE|WRITE_SIZE -d DIR` runs (the
       workload and the copy kernel), print the HBM bytes per launch of
       kernel NAME: each counter (KiB per dispatch) scaled by what it reads
-      for the copy of known size.
+      for the copy of known size.  --algorithmic notes the compulsory bytes
+      that bench.py gave the launch in that run, by which it knows the summary
+      again.
 """
 import argparse
 import csv
@@ -103,6 +105,8 @@ def cmd_traffic(args):
     fetch = kf * 1024.0 * ff
     write = kw * 1024.0 * fw
     print(f"kernel {args.kernel}")
+    if args.algorithmic:
+        print(f"algorithmic_bytes {args.algorithmic}")
     print(f"dispatches_fetch {nf}")
     print(f"dispatches_write {nw}")
     print(f"copy_FETCH_SIZE_KiB {cf:.1f}")
@@ -153,6 +157,7 @@ def main(argv=None):
     p.add_argument("--write", required=True)
     p.add_argument("--copy-fetch", required=True)
     p.add_argument("--copy-write", required=True)
+    p.add_argument("--algorithmic", type=int)
     p.add_argument("--copy-kernel", default="elementwise")
     p.add_argument("--mib", type=int, default=1024)
     p = sub.add_parser("requests")
