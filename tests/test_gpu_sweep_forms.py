@@ -280,3 +280,131 @@ def test_ghost_planes_and_limits(inside, ghosts):
     finally:
         for ctx in ctxs:
             v.vgpu_destroy(ctx)
+
+
+# ---------------------------------------------------------------------------
+# The sweeps' forms by size.  The fused leapfrog sweep (VGPU_LEAP=1) keeps the
+# corrections in launches of their own, with operands and order of its own
+# arrays; its fields are the separate sweeps' to the bit.
+# ---------------------------------------------------------------------------
+def _mesh(dm, bt, body, steps):
+    nx, ny, nz = dm
+    lines = ["VM 1.0.0", "CE sweep forms", "DM %d %d %d" % dm, "GS"]
+    lines += [f"BT {f} {t}" for f, t in zip(("XLO", "XHI", "YLO", "YHI", "ZLO", "ZHI"), bt)]
+    lines += ["WF wf1 GAUSSIAN_PULSE 1.0 3.0e-11 1.0e-11", *body,
+              f"PW 5 {nx - 5} 4 {ny - 6} 6 {nz - 4} pw1 wf1 35.0 20.0 40.0 111111 1.0 0.0",
+              f"EX 1 3 1 {ny - 1} 1 {nz - 1} b JZ wf1 1.0 0.0", f"EX {nx - 2} {nx - 1} 2 6 1 3 c =EZ wf1 0.5 1.0e-12",
+              f"EX 7 8 3 5 {nz - 1} {nz - 1} e =JMY wf1 250.0 2.0e-12",
+              f"OP {nx // 2} {nx // 2} {ny // 2} {ny // 2} {nz // 2} {nz // 2} t TDOM_ASCII"]
+    return "\n".join(lines + ["GE", f"NT {steps}", "CN 0.95", "MS 1e-3", "EN"]) + "\n"
+
+
+def _cells(dm, bt, precision):
+    """Cells of the allocation: layers and a ghost each side, whole lines in x."""
+    layers = [sum(int(t.split()[1]) for t in bt[2 * a:2 * a + 2] if t.startswith("PML")) for a in range(3)]
+    n = [dm[a] + layers[a] + 2 for a in range(3)]
+    line = 16 if precision == "fp64" else 32
+    return (n[0] + line - 1) // line * line * n[1] * n[2]
+
+
+MEDIA = ["MT one DEBYE 2.0 0.01 1.0 1e9 -1e9", "MT two DEBYE 3.0 0.0 1.0 1e9 -1e9 4e9 -3e9"]
+BLOCKS = ["MB 3 40 10 50 12 60 one", "MB 30 60 20 62 5 40 two", "MB 38 46 15 25 20 30 one", "MB 50 55 4 9 60 70 one"]
+PML = ["PML 5"] * 6
+MIXED = ["PML 4", "MUR", "PMC", "PEC", "MUR", "PML 6"]
+MUR = ["MUR"] * 6
+ROWS_MAX = 1000000  # cells of the largest grids with update rows
+APART = 64 << 20    # bytes of a field beyond which the fast tiles launch apart
+
+
+def _agree_with_fused_sweep(dm, bt, body, precision, steps, tmp_path, monkeypatch, files=()):
+    mesh = _write(tmp_path, _mesh(dm, bt, body, steps))
+    for name, text in files:
+        (tmp_path / name).write_text(text)
+    with vulture_amd.DeviceSolve(mesh, precision=precision, steps=steps) as ds:
+        st = ds.stats()
+        ds.run(0, steps)
+        ds.synchronize()
+        a = [ds.download(c) for c in range(6)]
+    assert not st["leap"]
+    monkeypatch.setenv("VGPU_LEAP", "1")
+    with vulture_amd.DeviceSolve(mesh, precision=precision, steps=steps) as ds:
+        assert ds.stats()["leap"]
+        ds.run(0, steps)
+        ds.synchronize()
+        for c in range(6):
+            b = ds.download(c)
+            assert np.count_nonzero(b) > b.size // 20
+            assert np.array_equal(a[c], b), c
+    return st
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("bt", [PML, MIXED, MUR], ids=["pml", "mixed", "mur"])
+@pytest.mark.parametrize("debye", [False, True])
+@pytest.mark.parametrize("side", ["below", "above"])
+def test_forms_either_side_of_the_update_rows(side, debye, bt, precision, tmp_path, monkeypatch):
+    """The largest grid with update rows and the smallest without: the same
+    x and y extents, one plane more."""
+    dm = [84, 84, 90]
+    while _cells(dm, bt, precision) <= ROWS_MAX:
+        dm[2] += 1
+    dm[2] -= side == "below"
+    dm = tuple(dm)
+    assert (_cells(dm, bt, precision) <= ROWS_MAX) == (side == "below")
+    print(f"case forms at {dm} {bt[1]} Debye {debye} {precision}", flush=True)
+    st = _agree_with_fused_sweep(dm, bt, (MEDIA + BLOCKS if debye else []), precision, 30, tmp_path, monkeypatch)
+    assert bool(st["debye_fused"]) == debye
+
+
+@pytest.mark.parametrize("precision,n", [("fp64", 208), ("fp32", 260)])
+@pytest.mark.parametrize("bt", [PML, MIXED], ids=["pml", "mixed"])
+@pytest.mark.parametrize("debye", [False, True])
+def test_forms_with_tiles_apart(debye, bt, precision, n, tmp_path, monkeypatch):
+    """Fields past 64 MB: shell and side blocks, then the fast tiles."""
+    dm = (n, n, n)
+    assert _cells(dm, bt, precision) * (8 if precision == "fp64" else 4) > APART
+    print(f"case tiles apart {dm} {bt[1]} Debye {debye} {precision}", flush=True)
+    st = _agree_with_fused_sweep(dm, bt, (MEDIA + BLOCKS if debye else []), precision, 100, tmp_path, monkeypatch)
+    assert bool(st["debye_fused"]) == debye
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [40, 104])
+def test_forms_with_sibc(n, precision, tmp_path, monkeypatch):
+    """SIBC faces with their H terms in update rows (40^3) and in rows (104^3)."""
+    from vulture_amd import pfe
+    dm = (n, n, n)
+    assert (_cells(dm, MIXED, precision) <= ROWS_MAX) == (n == 40)
+    body = ['BT s0 SIBC "slab.pfe"', "BT s1 SIBC -0.5 0.25 0.25 -0.5", f"TB 12 12 8 {n - 9} 7 {n - 8} s0",
+            f"TB 14 {n - 8} 9 {n - 12} 15 15 s0", f"TB 15 {n - 7} 13 13 18 {n - 6} s1"]
+    slab = pfe.pfe_text(pfe.fit_slab(1e6, 5e-4, fmax=3e10, per_decade=2))
+    print(f"case SIBC {dm} {precision}", flush=True)
+    st = _agree_with_fused_sweep(dm, MIXED, body, precision, 60, tmp_path, monkeypatch, [("slab.pfe", slab)])
+    assert st["sibc_faces"] > 1000
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("chunk", [0, 14])
+def test_corrections_packed(chunk, precision, tmp_path):
+    """The meshes of the corrections' oracle tests in one packed group: each
+    one's files are its own run's, byte for byte."""
+    import shutil
+
+    from conftest import GOLDEN
+    from test_gpu_inline import MESHES
+    names = sorted(MESHES)
+    meshes = []
+    for name in names:
+        d = tmp_path / name
+        meshes.append(_write(d, MESHES[name]))
+        shutil.copy(os.path.join(GOLDEN, "ref_inputs", "closedbox_go04", "go04.pfe"), str(d))
+    print(f"case packed corrections {precision} {chunk}", flush=True)
+    for name, m in zip(names, meshes):
+        vulture_amd.run_mesh(m, str(tmp_path / name / "alone"), precision=precision, chunk=chunk)
+    vulture_amd.run_meshes_group(meshes, [str(tmp_path / name / "group") for name in names], precision=precision,
+                                 chunk=chunk)
+    for name in names:
+        a, b = str(tmp_path / name / "alone"), str(tmp_path / name / "group")
+        files = sorted(os.listdir(a))
+        assert files and files == sorted(os.listdir(b))
+        assert filecmp.cmpfiles(a, b, files, shallow=False)[0] == files, name
