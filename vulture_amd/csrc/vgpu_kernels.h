@@ -1916,8 +1916,9 @@ template <typename S> VG_DEV S ld_args(const VG_CONST S *p)
 {
   static_assert(sizeof(S) % 4 == 0, "argument blocks are whole words");
   S out;
-  const VG_CONST unsigned *w = reinterpret_cast<const VG_CONST unsigned *>(p);
-  unsigned *o = reinterpret_cast<unsigned *>(&out);
+  typedef unsigned word __attribute__((may_alias));  // of whatever types the block has
+  const VG_CONST word *w = reinterpret_cast<const VG_CONST word *>(p);
+  word *o = reinterpret_cast<word *>(&out);
 #pragma unroll
   for (int i = 0; i < (int)(sizeof(S) / 4); ++i) o[i] = w[i];
   return out;
