@@ -738,6 +738,24 @@ static int build_sibc(Ctx *c)
   std::vector<long long> zeroKeys;
   long long f = 0, seq = 0;
   const std::vector<double> *ide[3] = {&c->idex, &c->idey, &c->idez};
+  // in line: a term is an operation on its value, a zeroed normal H another;
+  // build_inline sorts them and drops the terms of zeroed values
+  auto term = [&](long long key, const SibcHEnt &e) {
+    if (c->inl) {
+      const std::vector<double> &id = *ide[(e.bits >> 9) & 3];
+      c->xent[1].push_back({(key / 6 * 3 + key % 6 - 3) * 4 + 1, XO_SIBC | e.bits << 3, e.face, id[e.ia], id[e.ib]});
+    } else {
+      hents.push_back({key, seq++, e});
+    }
+  };
+  auto zero = [&](long long key) {
+    if (c->inl) c->xent[1].push_back({(key / 6 * 3 + key % 6 - 3) * 4, XO_ZERO, 0, 0, 0});
+    else zeroKeys.push_back(key);
+  };
+  if (c->inl) {
+    c->xent[0].reserve(3 * (size_t)NF);
+    c->xent[1].reserve(10 * (size_t)NF);
+  }
   std::vector<SibcBlock> blocks;
   for (int s = 0; s < ns; ++s) {
     const vgpu_sibc_desc &d = c->sibc[s].d;
@@ -788,10 +806,17 @@ static int build_sibc(Ctx *c)
             // cell along the other tangential axis
             const long long o1 = d.normal == 0 ? P : d.normal == 1 ? 1 : SJ;
             const long long o2 = d.normal == 0 ? SJ : d.normal == 1 ? P : 1;
-            for (const auto &[at, comp] : {std::pair<long long, int>(id, t1), {id + o1, t1}, {id, t2}, {id + o2, t2}}) {
+            // (the next cell's at the surface's end only: elsewhere it is the next face's own)
+            const int n3[3] = {i, j, k};
+            const bool e1 = n3[t2] + 1 == d.gbbox[2 * t2 + 1], e2 = n3[t1] + 1 == d.gbbox[2 * t1 + 1];
+            auto touch = [&](long long at, int comp) {
               if (c->leap) c->eTouched.push_back(at * 3 + comp);
               if (c->inl) c->xent[0].push_back({(at * 3 + comp) * 4 + 1, XO_ZERO, 0, 0, 0});
-            }
+            };
+            touch(id, t1);
+            touch(id, t2);
+            if (e1) touch(id + o1, t1);
+            if (e2) touch(id + o2, t2);
           }
           const unsigned char *a = &c->sibc[s].adjA[4 * lf], *b = &c->sibc[s].adjB[4 * lf];
           for (int r = 0; r < 4; ++r) { adjA[4 * f + r] = a[r]; adjB[4 * f + r] = b[r]; }
@@ -802,22 +827,26 @@ static int build_sibc(Ctx *c)
             e.face = (int)f;
             e.bits = 0 | slot << 1 | slot << 3 | (sign < 0) << 5 | wbit(w) << 6 | idaxis << 9;
             e.ia = e.ib = idi;
-            hents.push_back({c->lin(ci, cj, ck) * 6 + comp, seq++, e});
+            term(c->lin(ci, cj, ck) * 6 + comp, e);
           };
           auto adj = [&](int comp, int ci, int cj, int ck, double sign, double w, int sa, int sb, int idaxis,
                          int ia, int ib, int r) {
+            // (the value is another face's normal H: zeroed)
+            if (c->inl && ci >= d.gbbox[0] && ci < d.gbbox[1] && cj >= d.gbbox[2] && cj < d.gbbox[3] &&
+                ck >= d.gbbox[4] && ck < d.gbbox[5])
+              return;
             SibcHEnt e{};
             e.face = (int)f;
             e.bits = 1 | sa << 1 | sb << 3 | (sign < 0) << 5 | wbit(w) << 6 | (a[r] ? 0 : 1) << 7 |
                      (b[r] ? 0 : 1) << 8 | idaxis << 9;
             e.ia = ia;
             e.ib = ib;
-            hents.push_back({c->lin(ci, cj, ck) * 6 + comp, seq++, e});
+            term(c->lin(ci, cj, ck) * 6 + comp, e);
           };
           if (d.normal == 0) {
             const double wyl = 0.5 * (1 + pmc(2, k)), wyh = 0.5 * (1 + pmc(2, k + 1));
             const double wzl = 0.5 * (1 + pmc(1, j)), wzh = 0.5 * (1 + pmc(1, j + 1));
-            zeroKeys.push_back(c->lin(i, j, k) * 6 + 3);
+            zero(c->lin(i, j, k) * 6 + 3);
             edge(4, i - 1, j, k, +1, wzl, 2, 0, i - 1);
             edge(4, i - 1, j + 1, k, +1, wzh, 2, 0, i - 1);
             edge(4, i, j, k, -1, wzl, 3, 0, i);
@@ -833,7 +862,7 @@ static int build_sibc(Ctx *c)
           } else if (d.normal == 1) {
             const double wzl = 0.5 * (1 + pmc(0, i)), wzh = 0.5 * (1 + pmc(0, i + 1));
             const double wxl = 0.5 * (1 + pmc(2, k)), wxh = 0.5 * (1 + pmc(2, k + 1));
-            zeroKeys.push_back(c->lin(i, j, k) * 6 + 4);
+            zero(c->lin(i, j, k) * 6 + 4);
             edge(5, i, j - 1, k, +1, wxl, 2, 1, j - 1);
             edge(5, i, j - 1, k + 1, +1, wxh, 2, 1, j - 1);
             edge(5, i, j, k, -1, wxl, 3, 1, j);
@@ -850,7 +879,7 @@ static int build_sibc(Ctx *c)
           } else {
             const double wxl = 0.5 * (1 + pmc(1, j)), wxh = 0.5 * (1 + pmc(1, j + 1));
             const double wyl = 0.5 * (1 + pmc(0, i)), wyh = 0.5 * (1 + pmc(0, i + 1));
-            zeroKeys.push_back(c->lin(i, j, k) * 6 + 5);
+            zero(c->lin(i, j, k) * 6 + 5);
             edge(3, i, j, k - 1, +1, wyl, 2, 2, k - 1);
             edge(3, i + 1, j, k - 1, +1, wyh, 2, 2, k - 1);
             edge(3, i, j, k, -1, wyl, 3, 2, k);
@@ -866,21 +895,6 @@ static int build_sibc(Ctx *c)
           }
         }
     f = f0 + lf;
-  }
-  if (c->inl) {
-    // a normal H set to zero takes no other term
-    std::sort(zeroKeys.begin(), zeroKeys.end());
-    zeroKeys.erase(std::unique(zeroKeys.begin(), zeroKeys.end()), zeroKeys.end());
-    for (long long key : zeroKeys) c->xent[1].push_back({(key / 6 * 3 + key % 6 - 3) * 4, XO_ZERO, 0, 0, 0});
-    c->xent[1].reserve(zeroKeys.size() + hents.size());
-    for (const HE &h : hents) {
-      if (std::binary_search(zeroKeys.begin(), zeroKeys.end(), h.key)) continue;
-      const std::vector<double> &id = *ide[(h.e.bits >> 9) & 3];
-      c->xent[1].push_back({(h.key / 6 * 3 + h.key % 6 - 3) * 4 + 1, XO_SIBC | h.e.bits << 3, h.e.face, id[h.e.ia],
-                            id[h.e.ib]});
-    }
-    hents.clear();
-    zeroKeys.clear();
   }
   std::stable_sort(hents.begin(), hents.end(), [](const HE &a, const HE &b) { return a.key < b.key; });
   std::sort(zeroKeys.begin(), zeroKeys.end());
@@ -994,6 +1008,39 @@ static int build_corrections(Ctx *c)
   std::vector<RowEntry> rows[2];
   long long seq = 0;
   const bool cubic = c->grid.grid_type == 0;
+  // In line an entry is an operation on its value; sources' and analytic waves'
+  // values are evaluated ahead, a source's once for all its cells.
+  std::vector<int> srcVal(c->src.size(), -1);
+  for (size_t s = 0; s < c->src.size() && c->inl; ++s) {
+    std::vector<XVal> &val = c->xval[c->src[s].field < 3 ? 0 : 1];
+    srcVal[s] = (int)val.size();
+    val.push_back({0.0, c->src[s].delay, c->src[s].size, c->src[s].waveform, 0});
+  }
+  bool many = false;  // more sources or plane waves than an entry's number counts
+  auto entry = [&](int e, long long key, const CorrEntry &ce) {
+    if (!c->inl) {
+      rows[e].push_back({key, seq++, ce});
+      return;
+    }
+    many = many || ce.idx >= (1 << 23);
+    std::vector<XVal> &val = c->xval[e];
+    Ctx::XEnt x{key * 4 + 2, 0, 0, 0, 0};
+    if (ce.kind <= 1) {
+      x.code = XO_SRC | ce.kind << 3 | c->src[ce.idx].soft << 4;
+      x.arg = srcVal[ce.idx];
+    } else if (ce.kind == 2) {
+      x.code = XO_AUX | ce.inc << 3 | (ce.sign < 0 ? 1 : 0) << 6 | ce.idx << 8;
+      x.arg = ce.auxid;
+      x.a = ce.geo;
+      x.b = ce.il;
+    } else {
+      x.code = XO_WAVE | (ce.sign < 0 ? 1 : 0) << 6;
+      x.arg = (int)val.size();
+      x.b = ce.il;
+      val.push_back({ce.geo, c->pw[ce.idx].d.delay, c->pw[ce.idx].d.Finc[ce.inc], c->pw[ce.idx].d.waveform, 1});
+    }
+    c->xent[e].push_back(x);
+  };
   // sources first (source.c:602-753)
   for (size_t s = 0; s < c->src.size(); ++s) {
     const Ctx::Src &src = c->src[s];
@@ -1008,8 +1055,23 @@ static int build_corrections(Ctx *c)
           CorrEntry ce{};
           ce.kind = src.kind;
           ce.idx = (int)s;
-          rows[e].push_back({c->lin(i, j, k) * 3 + comp, seq++, ce});
+          entry(e, c->lin(i, j, k) * 3 + comp, ce);
         }
+  }
+  // (room for the plane waves' entries at once)
+  for (int e = 0; e < 2 && c->inl; ++e) {
+    size_t n = 0, waves = 0;
+    for (const Ctx::Pw &p : c->pw)
+      for (int q = 0; q < 12; ++q) {
+        const int *t = e == 0 ? TFSF_E[q] : TFSF_H[q];
+        if (!p.d.active[t[0]]) continue;
+        const int *l = p.d.flim[t[0]][t[1]], a = t[0] >> 1, a1 = (a + 1) % 3, a2 = (a + 2) % 3;
+        const size_t cells = (size_t)std::max(0, l[2 * a1 + 1] - l[2 * a1] + 1) * std::max(0, l[2 * a2 + 1] - l[2 * a2] + 1);
+        n += cells;
+        if (!(cubic && p.d.use_aux)) waves += cells;
+      }
+    c->xent[e].reserve(c->xent[e].size() + n);
+    c->xval[e].reserve(c->xval[e].size() + waves);
   }
   // then plane waves, face by face
   const std::vector<double> *idh[3] = {&c->idhx, &c->idhy, &c->idhz};
@@ -1068,47 +1130,13 @@ static int build_corrections(Ctx *c)
                 ce.kind = 3;
                 ce.geo = dd / d.phase_velocity;
               }
-              rows[e].push_back({c->lin(i, j, k) * 3 + comp % 3, seq++, ce});
+              entry(e, c->lin(i, j, k) * 3 + comp % 3, ce);
             }
       }
     }
+  if (many) return set_error(c, VGPU_EINVAL, "too many sources or plane waves");
   if (c->leap)
     for (const RowEntry &r : rows[0]) c->eTouched.push_back(r.key);
-  for (int e = 0; e < 2 && c->inl; ++e) {
-    // operations on the rows' values; sources' and analytic waves' values are
-    // evaluated ahead, a source's once for all its cells
-    std::vector<XVal> &val = c->xval[e];
-    std::vector<int> srcVal(c->src.size(), -1);
-    for (size_t s = 0; s < c->src.size(); ++s)
-      if ((c->src[s].field < 3 ? 0 : 1) == e) {
-        srcVal[s] = (int)val.size();
-        val.push_back({0.0, c->src[s].delay, c->src[s].size, c->src[s].waveform, 0});
-      }
-    for (const RowEntry &r : rows[e]) {
-      const CorrEntry &ce = r.e;
-      if (ce.idx < 0 || ce.idx >= (1 << 23)) return set_error(c, VGPU_EINVAL, "too many sources or plane waves");
-      Ctx::XEnt x{r.key * 4 + 2, 0, 0, 0, 0};
-      if (ce.kind <= 1) {
-        x.code = XO_SRC | ce.kind << 3 | c->src[ce.idx].soft << 4;
-        x.arg = srcVal[ce.idx];
-      } else if (ce.kind == 2) {
-        x.code = XO_AUX | ce.inc << 3 | (ce.sign < 0 ? 1 : 0) << 6 | ce.idx << 8;
-        x.arg = ce.auxid;
-        x.a = ce.geo;
-        x.b = ce.il;
-      } else {
-        x.code = XO_WAVE | (ce.sign < 0 ? 1 : 0) << 6;
-        x.arg = (int)val.size();
-        x.b = ce.il;
-        val.push_back({ce.geo, c->pw[ce.idx].d.delay, c->pw[ce.idx].d.Finc[ce.inc], c->pw[ce.idx].d.waveform, 1});
-      }
-      c->xent[e].push_back(x);
-    }
-    std::vector<long long> keys;
-    for (const RowEntry &r : rows[e]) keys.push_back(r.key);
-    std::sort(keys.begin(), keys.end());
-    c->corrRows[e] = std::unique(keys.begin(), keys.end()) - keys.begin();
-  }
   for (int e = 0; e < 2 && !c->inl; ++e) {
     std::stable_sort(rows[e].begin(), rows[e].end(), [](const RowEntry &a, const RowEntry &b) { return a.key < b.key; });
     std::vector<int> rstart;

@@ -157,14 +157,25 @@ template <typename T> int build_inline(Ctx *c)
     return false;
   };
 
-  // operations but Debye, by value; a ghost value takes its source's, so what
-  // else would change it is lost
+  // operations but Debye, by value; an H set to zero by SIBC takes none of its
+  // terms; a ghost value takes its source's, so what else would change it is lost
   for (int e = 0; e < 2; ++e) {
     std::vector<Ent> &v = c->xent[e];
     sort_by_key(v);
     size_t k = 0;
+    long long corrected = -1, zeroed = -1;
+    c->corrRows[e] = 0;
     for (const Ent &x : v) {
-      if (k && kind(x) == XO_ZERO && kind(v[k - 1]) == XO_ZERO && v[k - 1].key == x.key) continue;
+      const int what = kind(x);
+      if (what == XO_ZERO) {
+        if (k && kind(v[k - 1]) == XO_ZERO && v[k - 1].key == x.key) continue;
+        zeroed = x.value();
+      } else if (what == XO_SIBC) {
+        if (zeroed == x.value()) continue;
+      } else if (corrected != x.value()) {  // sources and TF/SF
+        corrected = x.value();
+        ++c->corrRows[e];
+      }
       if (!geo.ghosts[3 * e + x.comp()].empty()) {
         int n[3];
         geo.unlin(x.cell(), n);
@@ -278,13 +289,18 @@ template <typename T> int build_inline(Ctx *c)
     for (size_t a = 0; a < v.size();) {
       size_t b = a;
       while (b < v.size() && v[b].value() == v[a].value()) ++b;
+      size_t from = a;
+      if (!small && (e == 1 || kind(v[a]) != XO_ZERO)) {  // a row wherever it lies
+        rest[e].push_back({a, b, kind(v[a]) == XO_GHOST});
+        a = b;
+        continue;
+      }
       const long long cell = v[a].cell();
       const int C = v[a].comp();
       int n[3];
       geo.unlin(cell, n);
       const int reg = geo.region(3 * e + C, n);
       const bool inside = n[0] > 0 && n[1] > 0 && n[2] > 0 && n[0] < N[0] - 1 && n[1] < N[1] - 1 && n[2] < N[2] - 1;
-      size_t from = a;
       if (reg >= 0 && kind(v[a]) == XO_ZERO && (small || e == 0) && (b == a + 1 || !small || reg != 6 || !inside)) {
         fl.push_back({cell, (unsigned)XF_ZERO << C});
         ++from;
