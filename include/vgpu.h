@@ -158,14 +158,16 @@ int vgpu_synchronize(vgpu_ctx *c);
 
 /* Advance up to VGPU_GROUP_MAX solves by nsteps each in lockstep, context i
  * over steps [first[i], first[i]+nsteps): one packed launch per step kernel
- * over all of them (fast and shell sweeps, Debye layers, corrections,
- * observers) instead of one launch per solve, for grids too small to fill
- * the device alone.  Each context ends as after vgpu_run(ctxs[i], first[i],
+ * over all of them (the sweeps, with corrections, observers and incident
+ * fields beside them, and the rows behind them) instead of one launch per
+ * solve, for grids too small to fill the device alone.  Each context ends as after vgpu_run(ctxs[i], first[i],
  * nsteps, NULL), bit for bit, with its own run record (vgpu_run_result).
  * Runs on the first context's stream after the work queued on every
  * member's stream; each member's stream waits for the group's end.  Every
- * member must use the separate sweeps (not VGPU_LEAP, not a fused Debye
- * layer) and share device and precision.  No counterpart in the reference,
+ * member must use the separate sweeps (not VGPU_LEAP) and share device and
+ * precision; a member whose corrections have launches of their own (2^31
+ * cells and more, set-ups that the in-line form does not hold) runs its own
+ * launches on the group's stream.  No counterpart in the reference,
  * which runs one solve per process (src/simulation.c:136-230); it serves
  * many small solves on one GPU. */
 #define VGPU_GROUP_MAX 16

@@ -271,11 +271,15 @@ template <typename T> int build_inline(Ctx *c)
   // alone on a swept value, which are a flag.  Update rows take values of the
   // ordinary update with both neighbours inside on every axis, unless a Mur
   // face takes them too: its thread, the sweep's, reads the old value.
-  // They pay where a launch is what a step waits for, in grids up to a million
-  // cells: 53x41x62 request 35.6 -> 28.9 us a step, 40^3 free space FP64 28.6
-  // -> 26.5.  Beyond, reading the other field's neighbours again costs more
-  // than the rows' launch: 256^3 Debye volume 497 -> 531, 173x211x158 request
-  // 204 -> 215, FP64 128^3 Debye volume 159 -> 168.
+  // They pay where a launch is what a step waits for: 53x41x62 request 35.6 ->
+  // 28.9 us a step, 40^3 free space FP64 28.6 -> 26.5.  In large grids reading
+  // the other field's neighbours again costs more than the rows' launch: 256^3
+  // Debye volume 497 -> 531, 173x211x158 request 204 -> 215.  The line is drawn
+  // at a million cells; between there and about three million it depends on
+  // what is corrected.  Sources and TF/SF would still gain (2.0 M-cell request
+  // 71.4 -> 66.2, 2.7 M-cell Debye volume FP64 156.5 -> 153.7, 140^3 with a
+  // one-pole block FP32 63.4 -> 59.3), sites of several poles lose (the same
+  // block, two poles: 75.3 -> 92.4 FP32, 133 -> 186 FP64; 108^3 44.6 -> 51.0).
   const bool small = c->xskip = c->ncell <= 1000000;
   struct Value { size_t a, b; bool ghost; };
   struct Entry { int cell; int med[3]; unsigned fl; };

@@ -31,7 +31,7 @@ struct WaveformDev;
 struct PwDev;
 
 // Full argument block of the E sweep, kept in device memory and read through
-// a pointer by the shell kernel and the fused Debye step.
+// a pointer by the shell blocks.
 template <typename T> struct EArgs {
   int NX, NY, NZ, PX;
   long long plane;
@@ -694,9 +694,8 @@ struct Ctx : InlineState {
   // Coefficient classes (the reference's indexed-media representation,
   // grid.h:108-135): every cell's (alpha, beta) triple of E components and
   // gamma triple of H components is one entry of a small table.  Built on
-  // the host in vgpu_set_media, refined with the layer-0 Debye block of each
-  // E component in vgpu_finalize, uploaded as uint16 per cell when both
-  // tables fit.
+  // the host in vgpu_set_media, refined in vgpu_finalize with what the sweeps
+  // do in line (build_inline), uploaded as uint16 per cell when both tables fit.
   std::vector<uint32_t> ecls, hcls;          // host, per device cell
   std::vector<double> etab, htab;            // host: [class][6] alpha/beta, [class][3] gamma (device: padded to 8, 4)
   bool indexed = false;

@@ -183,8 +183,9 @@ VG_DEV double wf_value(const WaveformDev &w, double t, double delay, double pi)
 
 // ---------------------------------------------------------------------------
 // 1-D auxiliary grids of the TF/SF plane waves (planewave.c:1315-1372).
-// One block per plane wave; the blocks ride in other launches (k_head for E,
-// the H corrections' k_corr for H), whose own work they do not touch.
+// One block per plane wave; the blocks ride in other launches, whose own work
+// they do not touch: among the side blocks of the E sweep for E and of the H
+// sweep for H (with corrections in launches of their own in k_head and k_corr_aux).
 // ---------------------------------------------------------------------------
 template <typename T> VG_DEV void aux_e_block(const AuxArgs<T> &a, int p, double t, double pi)
 {
@@ -230,24 +231,20 @@ template <typename T> VG_DEV void aux_h_block(const AuxArgs<T> &a, int p)
 }
 
 // ===========================================================================
-// Volume sweeps.  Each half-step is two kernels over disjoint cells:
-//  - the fast kernel over the fast box, where every component takes the
-//    ordinary update (inner grid).  A 64x4 thread tile covers 64 x-cells by
-//    4 y-rows and marches along z over a chunk of planes, carrying the plane
-//    below (E) or above (H) in registers; its arguments are a few pointers
-//    and integers passed by value, so they stay in scalar registers.
-//  - the shell kernel over everything else (UPML slabs, Mur normal H, cells
-//    of one component's inner grid only, ghost layers), planned on the host
-//    as pieces of x runs (ShellPiece), reading its pointers from the argument
-//    block in device memory.
+// Volume sweeps.  A half-step covers the grid with two kinds of blocks over
+// disjoint cells, in one launch (k_e_sweep, k_h_sweep) or, in large grids, the
+// fast tiles in one of their own (k_e_fast, k_h_fast; sweeps_apart):
+//  - fast tiles over the fast box, where every component takes the ordinary
+//    update (inner grid).  A 64x4 thread tile covers 64 x-cells by 4 y-rows and
+//    marches along z over a chunk of planes, carrying the plane below (E) or
+//    above (H) in registers; its arguments are a few pointers and integers
+//    passed by value, so they stay in scalar registers.
+//  - shell blocks over everything else (UPML slabs, Mur normal H, cells of one
+//    component's inner grid only, ghost layers), planned on the host as pieces
+//    of x runs (ShellPiece), reading their pointers from the argument block in
+//    device memory.
 // ===========================================================================
 
-// XCD-aware block order.  Workgroups are dealt to the eight XCDs round-robin
-// by launch index, and each XCD has its own L2, so consecutive launch indices
-// would scatter neighbouring rows and planes over different L2s.  The grid is
-// padded to a multiple of eight and launch index b runs logical block
-// (b % 8) * (n / 8) + b / 8: every XCD sweeps one contiguous range of blocks
-// (a z range of the domain), where neighbouring rows and planes share its L2.
 // Tile of fast block b: z chunk bz, y tile by, x chunk bx.  Workgroups are
 // dealt to the eight XCDs round-robin by launch index, and each XCD has its
 // own L2.  All XCDs sweep one z chunk at a time, each an eighth of its tiles
@@ -271,8 +268,10 @@ VG_DEV bool fast_block(unsigned b, int nchx, int gy, int gz, int per, bool down,
   return true;
 }
 
-// The fused sweep's order: its grid is padded to a multiple of eight and every
-// XCD runs one contiguous range of logical blocks.
+// The fused sweep's order: its grid is padded to a multiple of eight and launch
+// index b runs logical block (b % 8) * (n / 8) + b / 8, so every XCD sweeps one
+// contiguous range of blocks (a z range of the domain), whose neighbouring rows
+// and planes share its L2.
 VG_DEV unsigned xcd_block()
 {
   const unsigned per = gridDim.x / 8;
@@ -949,8 +948,8 @@ VG_DEV bool shell_column(const ShellDev *pcs, const ShellWork *work, unsigned b,
   return true;
 }
 
-// Region of component C at x = i of a piece: reg 6 ordinary, 0..5 UPML slab
-// (p its slab index at plane dk of the piece, psz the step of p per plane,
+// Region of component C at x = i of a piece, as the host's checks of the plan
+// take it: reg 6 ordinary, 0..5 UPML slab (p its slab index at plane dk of the piece, psz the step of p per plane,
 // a/b the slab's auxiliaries); reg -1 not updated.
 struct ColRegion {
   int reg;
@@ -1000,8 +999,7 @@ template <typename T> struct EShellPtrs {
   VG_GLOBAL const T *Ein[3], *H[3], *alpha[3], *beta[3], *ad[3], *bd[3], *ah[3], *ibh[3], *idh[3], *etab;
   VG_GLOBAL const uint16_t *ecls;
   // sep false: the step reads and writes one field set (no fused sweep), so
-  // the old E is read through E itself; one pointer fewer per component
-  // keeps FP32 k_e_shell at 78 VGPRs, six waves per SIMD, instead of 86
+  // the old E is read through E itself, one pointer fewer per component
   VG_DEV explicit EShellPtrs(const EArgs<T> &a, bool sep)
   {
     PP = gp(a.PPpool);
@@ -1808,8 +1806,10 @@ __global__ __launch_bounds__(256) void k_e_sweep(FastE<T> f, const ShellDev *pcs
 // second, so their chains of dependent loads run under the sweep's streams.
 // 96x81x64 box FP64: 38.4 us a step in a launch of their own, with the E rows,
 // and the sweep's, 28.5 in one; 256x256x160 box FP32, where both move bytes
-// (270 MB of states) all the time, 200 and 197.  FP32 keeps five wavefronts a
-// SIMD (97 registers without the bound).
+// (270 MB of states) all the time, 200 and 197.  FP32 is held to 96 registers,
+// five wavefronts a SIMD (97 without the bound); it spills up to 19 scalar
+// registers and no vector ones.  FP64 has four with X = 1 and 3 (127), three
+// with the others (130 to 147).
 template <typename T, bool IDX, int X>
 __global__ __launch_bounds__(256, sizeof(T) == 4 ? 5 : 3) void k_e_sweep_sibc(FastE<T> f, const ShellDev *pcs, const ShellWork *work,
                                                       const EArgs<T> *ap, const XArgs<T> *x, unsigned nSide,

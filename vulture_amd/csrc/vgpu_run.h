@@ -1,13 +1,14 @@
-// Per-precision time-step driver: launches one step's kernels in the
-// reference's order (simulation.c:157-222):
-//   observers -> Mur E -> E sweep (fast box with the first Debye layer, then
-//   the shell: inner-grid edges and UPML) -> remaining Debye layers -> SIBC E
-//   -> sources/TF-SF E -> ghost E -> H sweep (fast box, shell: Mur normal H
-//   and UPML) -> SIBC H -> sources/TF-SF H -> ghost H
-// The aux grids of the plane waves touch nothing but their own arrays: their
-// E update rides in the observers' launch and their H update in the H
-// corrections' launch, which keeps the order in which each aux array is
-// written and read.
+// Per-precision time-step driver.  The reference's step (simulation.c:157-222) is
+//   observers -> Mur E -> E update (inner grid, UPML) -> Debye blocks -> SIBC E
+//   -> sources/TF-SF E -> ghost E -> H update (inner grid, Mur normal H, UPML)
+//   -> SIBC H -> sources/TF-SF H -> ghost H
+// A step here is the E sweep, the E rows, the H sweep and the H rows.  Each value
+// takes its operations in the reference's order: in the sweep's thread, in an
+// update row beside it or in a row behind it (XArgs).  What reads and writes
+// nothing of a sweep rides in blocks beside it (SideArgs): the observers' samples,
+// the values of sources and analytic waves, the aux grids of the plane waves.
+// Contexts with the fused sweep, of 2^31 cells and more, or with a set-up that
+// the rows do not hold launch the step's parts one after another.
 #pragma once
 #include "vgpu_kernels.h"
 #include <algorithm>
@@ -514,8 +515,9 @@ template <typename T> struct StepArgs {
 };
 
 // Whether a context's fast tiles have launches of their own.  In one launch
-// the tiles share the shell's register count (FP32 E 104 and H 62 VGPRs
-// against 62 and 53 alone), but its blocks fill the device together with
+// the tiles share the shell's register count (FP32 with Debye sites E 96 and H
+// 62 VGPRs against 49 and 53 alone, five and eight wavefronts a SIMD against
+// eight), but its blocks fill the device together with
 // theirs and one launch fewer is on the step's critical path: 48.6 -> 39.8 us
 // a step on a 53x41x62 request, 82 -> 71 on 101x115x108, 298 -> 283 on the
 // FP64 200x160x120 enclosure, 377 -> 368 on the 256x256x160 box.  Where the
@@ -838,7 +840,6 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   const ShellDev *epc = A.epc, *hpc = A.hpc;
   const ShellWork *ewk = A.ewk, *hwk = A.hwk;
   const XArgs<T> *xe = P<XArgs<T>>(c->d_xargs[0]), *xh = P<XArgs<T>>(c->d_xargs[1]);
-  const unsigned nHshell = (unsigned)c->nHwork;
   auto fast_e = [&](int q) {
     const FastE<T> &f = fe[q];
     if (!egrid.x) return;
@@ -1048,7 +1049,8 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
     if (apart) sweep_h(soff, last);
     rows(1);
   }
-  // Steps with the fused leapfrog sweep.
+  // Steps with corrections in launches of their own: the fused leapfrog sweep,
+  // grids of 2^31 cells and more, set-ups that the in-line form does not hold.
   for (uint64_t n = 0; !c->inl && n < nsteps; ++n) {
     const int soff = (int)n;
     const int q = c->leap ? c->par ^ (int)(n & 1) : c->par;  // field set this step reads
@@ -1160,10 +1162,11 @@ template <typename T> int upload_pack(Ctx *c)
 
 // Steps of several solves in lockstep on one stream (vgpu_run_group): the
 // same kernels in the same order per solve as run_steps, with the sweeps and
-// what rides along, and the rows, of all solves in one packed launch each; SIBC E, and Mur E where it keeps its launch, stay one per
-// solve.  Solves share no memory, so only each solve's own order matters, and
-// every block does what it does in the solve's own launch.  Members without
-// PackArgs (grids too large to index in line) run their own launches.
+// what rides along, and the rows, of all solves in one packed launch each; SIBC
+// E, and Mur E where it keeps its launch, stay one per solve.  Solves share no
+// memory, so only each solve's own order matters, and every block does what it
+// does in the solve's own launch.  Members without PackArgs (corrections in
+// launches of their own) run alone.
 template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t nsteps, hipStream_t s)
 {
   const double pi = 4.0 * atan(1.0);
