@@ -1360,7 +1360,6 @@ int vgpu_finalize(vgpu_ctx *c, uint64_t total_steps, uint64_t max_steps_per_run)
   c->d_step = dev_alloc(c, 64);
   if (!c->d_step) return set_error(c, VGPU_ENOMEM, "step counter");
   int r;
-  if ((r = build_observers(c))) return r;
   const size_t mark = c->allocs.size(), bytes = c->bytes;
   r = build_lists(c);
   if (r && c->inl) {
@@ -1371,7 +1370,7 @@ int vgpu_finalize(vgpu_ctx *c, uint64_t total_steps, uint64_t max_steps_per_run)
     r = build_lists(c);
     if (!r) c->err.clear();
   }
-  if (r || (r = build_leap(c))) return r;
+  if (r || (r = build_observers(c)) || (r = build_leap(c))) return r;
   if ((r = c->prec == VGPU_FP64 ? prepare_sweeps<double>(c) : prepare_sweeps<float>(c))) return r;
   if (c->inl && (r = c->prec == VGPU_FP64 ? upload_pack<double>(c) : upload_pack<float>(c)))
     return r;

@@ -450,7 +450,7 @@ template <typename T> int build_inline(Ctx *c)
           site.push_back({(int)v[R[q].a].cell(), (unsigned)(v[R[q].a].code >> 8) << 2 | (unsigned)C});
     if (e == 0) {
       c->nXsite = (long long)site.size();
-      if (!up(c->d_xsite, site.data(), site.size() * sizeof(XSiteDev))) return fail("Debye sites");
+      if (!site.empty() && !up(c->d_xsite, site.data(), site.size() * sizeof(XSiteDev))) return fail("Debye sites");
     }
     int slot = (int)site.size();
     std::vector<XRow> row;

@@ -378,10 +378,11 @@ VG_DEV void x_row(const VG_CONST XArgs<T> *x, const VG_GLOBAL XRow *row)
 // operation a site (32 in FP64), one look-up after another and the three
 // components of a cell side by side; a site is 8 bytes, component by component.
 // A 256^3 grid, 4.9 M cells of it of a two-pole medium: 572 us a step against
-// 653 in FP32, 966 against 1024 in FP64.
-template <typename T, bool IDX, bool ELEC> VG_DEV void x_rows(const VG_CONST XArgs<T> *x, unsigned b)
+// 653 in FP32, 966 against 1024 in FP64.  Rows without such sites (SITES false)
+// are spared the question: 11.8 against 11.2 us on the FP64 enclosure's E rows.
+template <typename T, bool IDX, bool ELEC, bool SITES> VG_DEV void x_rows(const VG_CONST XArgs<T> *x, unsigned b)
 {
-  if (ELEC) {
+  if (SITES) {
     const unsigned n = (unsigned)((x->nrow + x->ngroup + 255) >> 8);
     if (b >= n) {
       const long long g = (b - n) * 256ll + threadIdx.x;
@@ -413,9 +414,10 @@ template <typename T, bool IDX, bool ELEC> VG_DEV void x_update(const VG_CONST X
   if (q < x->nupd) x_row<T, IDX, ELEC, true>(x, gp(x->row) + q);
 }
 
-template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) void k_rows(const XArgs<T> *x)
+template <typename T, bool IDX, bool ELEC, bool SITES = false>
+__global__ __launch_bounds__(256) void k_rows(const XArgs<T> *x)
 {
-  x_rows<T, IDX, ELEC>(cp(x), blockIdx.x);
+  x_rows<T, IDX, ELEC, SITES>(cp(x), blockIdx.x);
 }
 
 // A one-pole Debye site (debye.c:243-307, as debye_site with one real pole):
@@ -1961,11 +1963,12 @@ template <typename T> __global__ __launch_bounds__(256) void k_first_samples_pk(
   sample_value_block<T, 0>(a, (int)(blockIdx.x - m.start[d]), *a.o.step, pi);
 }
 
-template <typename T, bool IDX, bool ELEC> __global__ __launch_bounds__(256) void k_rows_pk(PackMap m)
+template <typename T, bool IDX, bool ELEC, bool SITES = false>
+__global__ __launch_bounds__(256) void k_rows_pk(PackMap m)
 {
   const int d = pack_member(m, blockIdx.x);
   const VG_CONST PackArgs<T> *a = pack_args<T>(m, d);
-  x_rows<T, IDX, ELEC>(cp(ELEC ? a->xe : a->xh), blockIdx.x - m.start[d]);
+  x_rows<T, IDX, ELEC, SITES>(cp(ELEC ? a->xe : a->xh), blockIdx.x - m.start[d]);
 }
 
 // Device step counter: set before a run that does not continue the previous

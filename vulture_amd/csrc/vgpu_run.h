@@ -942,7 +942,9 @@ template <typename T> int run_steps(Ctx *c, uint64_t nsteps, hipStream_t s, bool
   auto rows = [&](int e) {
     const dim3 b(256), g((unsigned)c->row_blocks(e));
     if (!g.x) return;
-    if (c->indexed && e == 0) hipLaunchKernelGGL((k_rows<T, true, true>), g, b, 0, s, xe);
+    if (c->indexed && e == 0 && c->nXsite) hipLaunchKernelGGL((k_rows<T, true, true, true>), g, b, 0, s, xe);
+    else if (e == 0 && c->nXsite) hipLaunchKernelGGL((k_rows<T, false, true, true>), g, b, 0, s, xe);
+    else if (c->indexed && e == 0) hipLaunchKernelGGL((k_rows<T, true, true>), g, b, 0, s, xe);
     else if (c->indexed) hipLaunchKernelGGL((k_rows<T, true, false>), g, b, 0, s, xh);
     else if (e == 0) hipLaunchKernelGGL((k_rows<T, false, true>), g, b, 0, s, xe);
     else hipLaunchKernelGGL((k_rows<T, false, false>), g, b, 0, s, xh);
@@ -1197,7 +1199,7 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
   };
   // packs by kernel form: with classes, the E sweep's by the level of its
   // in-line corrections
-  PackMap sweepE[6], sweepH[4], rowE[2], rowH[2];
+  PackMap sweepE[6], sweepH[4], rowE[4], rowH[2];
   for (int x = 0; x < 6; ++x)
     sweepE[x] = plan([&](int i) {
       return (cs[i]->indexed ? cs[i]->xlevel() : 5) == x ? (long long)A[i].nside[0] + cs[i]->nEworkPk + A[i].eg1.x : 0LL; });
@@ -1208,7 +1210,8 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
         return cs[i]->indexed == idx && cs[i]->xflagH == (f == 0)
                    ? (long long)A[i].nside[1] + cs[i]->nHworkPk + A[i].hg1.x : 0LL; });
     auto nrows = [&](int i, int e) { return cs[i]->indexed == idx ? cs[i]->row_blocks(e) : 0LL; };
-    rowE[x] = plan([&](int i) { return nrows(i, 0); });
+    for (int f = 0; f < 2; ++f)  // with Debye sites of the list or without
+      rowE[2 * x + f] = plan([&](int i) { return (cs[i]->nXsite > 0) == (f == 0) ? nrows(i, 0) : 0LL; });
     rowH[x] = plan([&](int i) { return nrows(i, 1); });
   }
   const PackMap first = plan([&](int i) { return (long long)A[i].side[1].b[2]; });
@@ -1227,8 +1230,10 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
     if (sweepE[3].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 3>), blocks(sweepE[3]), b, 0, s, sweepE[3], pi);
     if (sweepE[4].n) hipLaunchKernelGGL((k_e_sweep_pk<T, true, 4>), blocks(sweepE[4]), b, 0, s, sweepE[4], pi);
     if (sweepE[5].n) hipLaunchKernelGGL((k_e_sweep_pk<T, false, 3>), blocks(sweepE[5]), b, 0, s, sweepE[5], pi);
-    if (rowE[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, true>), blocks(rowE[0]), b, 0, s, rowE[0]);
-    if (rowE[1].n) hipLaunchKernelGGL((k_rows_pk<T, false, true>), blocks(rowE[1]), b, 0, s, rowE[1]);
+    if (rowE[0].n) hipLaunchKernelGGL((k_rows_pk<T, true, true, true>), blocks(rowE[0]), b, 0, s, rowE[0]);
+    if (rowE[1].n) hipLaunchKernelGGL((k_rows_pk<T, true, true>), blocks(rowE[1]), b, 0, s, rowE[1]);
+    if (rowE[2].n) hipLaunchKernelGGL((k_rows_pk<T, false, true, true>), blocks(rowE[2]), b, 0, s, rowE[2]);
+    if (rowE[3].n) hipLaunchKernelGGL((k_rows_pk<T, false, true>), blocks(rowE[3]), b, 0, s, rowE[3]);
     for (int i = 0; i < n; ++i)
       if (cs[i]->sibcFaces)
         hipLaunchKernelGGL((k_sibc_e<T, false>), dim3((unsigned)cs[i]->sibcBlocks), dim3(256), 0, s, A[i].se[0]);
