@@ -141,7 +141,7 @@ template <typename T> struct XArgs {
   unsigned flag0;        // first flagged class (E)
   const uint16_t *cls;   // per cell: class, or without classes E 0 / 1 + dtab row, H its flags
   const T *dtab;         // [class - flag0][8]: alpha, beta of J per component, flags
-  T *J;                  // [cell of the one-pole sites' box][component]
+  T *J;                  // [cell of the one-pole sites' box][component], from the box's would-be cell (0, 0, 0)
   int PX;
   long long plane;
   T mzeta[6];            // Mur factors
@@ -166,8 +166,8 @@ template <typename T> struct XArgs {
   const T *Etan;
   long long nsite;       // sites alone on their value (E); they hold the first state slots
   const XSiteDev *site;
-  int jlo[3], jn[2], jplane;  // first cell of the one-pole sites' box, its extents in x and y, their product
-  unsigned jlast;        // the box's last cell
+  int jrow, jplane;      // the one-pole sites' box: cells a row and a plane
+  int jfirst, jlast;     // the places of its first and last cell
 };
 
 // Values of a half-step's sources and analytic plane waves, evaluated ahead

@@ -448,17 +448,14 @@ template <typename T> struct XPre {
     return gp(C == 0 ? x->F[0] : C == 1 ? x->F[1] : x->F[2]);
   }
   // place of a cell in J
-  VG_DEV static int j_at(const VG_CONST XArgs<T> *x, int i, int j, int k)
-  {
-    return (k - x->jlo[2]) * x->jplane + (j - x->jlo[1]) * x->jn[0] + (i - x->jlo[0]);
-  }
+  VG_DEV static int j_at(const VG_CONST XArgs<T> *x, int i, int j, int k) { return k * x->jplane + j * x->jrow + i; }
   template <bool DEBYE> VG_DEV void load(const VG_CONST XArgs<T> *x, long long id, int jid, unsigned cls)
   {
     const VG_GLOBAL T *q = gp(x->dtab) + (cls - x->flag0) * DTAB_STRIDE;
     fl = (unsigned)q[6];
     if (DEBYE) {
       // (flagged cells without a site may lie outside the box)
-      const VG_GLOBAL T *J = gp(x->J) + 3ull * min((unsigned)jid, x->jlast);
+      const VG_GLOBAL T *J = gp(x->J) + 3ll * max(x->jfirst, min(jid, x->jlast));
       for (int c = 0; c < 3; ++c) j[c] = J[c];
       for (int c = 0; c < 6; ++c) d[c] = q[c];
     }

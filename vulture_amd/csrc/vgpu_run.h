@@ -378,11 +378,13 @@ template <typename T> static void fill_correction_args(Ctx *c, XArgs<T> &x, int 
   x.flag0 = ~0u;
   if (e) return;
   x.flag0 = c->xflag0;
-  for (int a = 0; a < 3; ++a) x.jlo[a] = c->jlo[a];
-  for (int a = 0; a < 2; ++a) x.jn[a] = c->jn[a];
-  x.jplane = c->jn[0] * c->jn[1];
-  x.jlast = (unsigned)((long long)x.jplane * c->jn[2] - 1);
-  x.dtab = P<T>(c->d_xdtab); x.J = P<T>(c->d_xJ);
+  if (c->d_xJ) {
+    x.jrow = c->jn[0]; x.jplane = c->jn[0] * c->jn[1];
+    x.jfirst = c->jlo[2] * x.jplane + c->jlo[1] * x.jrow + c->jlo[0];
+    x.jlast = x.jfirst + c->jn[2] * x.jplane - 1;
+    x.J = P<T>(c->d_xJ) - 3ll * x.jfirst;
+  }
+  x.dtab = P<T>(c->d_xdtab);
   for (int f = 0; f < 6; ++f) x.mzeta[f] = T(c->zeta[f]);
   x.dlast = P<T>(c->d_dlast); x.dJ = P<T>(c->d_dJ); x.dstride = c->debyeSites;
   x.dalpha = P<double>(c->d_dalpha); x.dbeta = P<double>(c->d_dbeta); x.dnp = P<int>(c->d_dnp);
