@@ -80,7 +80,12 @@ static inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, int k,
 template <typename V> static inline hipError_t hipGetSymbolAddress(void **p, V *s) { *p = (void *)s; return hipSuccess; }
 static inline hipError_t hipSetDevice(int) { return hipSuccess; }
 static inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
-static inline hipError_t hipGetLastError() { return hipSuccess; }
+// (an error at every look with CPU_HIP_ERROR=1)
+static inline hipError_t hipGetLastError()
+{
+  const char *e = getenv("CPU_HIP_ERROR");
+  return e && e[0] == '1' ? hipErrorCpu : hipSuccess;
+}
 static inline const char *hipGetErrorString(hipError_t) { return "cpu"; }
 static inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)malloc(1); return hipSuccess; }
 static inline hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }

@@ -186,3 +186,29 @@ def test_packed_against_alone(cpu, tmp_path):
             files = sorted(os.listdir(a))
             assert files and files == sorted(os.listdir(b))
             assert filecmp.cmpfiles(a, b, files, shallow=False)[0] == files
+
+
+@pytest.mark.parametrize("inside", [False, True])
+def test_group_reports_failed_launches(cpu, inside):
+    """A group run whose launches fail says so, also where no member has its
+    corrections in line (ghost planes inside the sweeps' limits)."""
+    import ctypes
+
+    from test_gpu_sweep_forms import N, _context
+    vulture_amd.load_host()
+    v = vulture_amd.load_vgpu()
+    v.vgpu_create.restype = v.vgpu_finalize.restype = v.vgpu_set_media.restype = ctypes.c_int
+    v.vgpu_destroy.argtypes = [ctypes.c_void_p]
+    lim = [[1, N - 2] * 3 for _ in range(6)]
+    if inside:
+        lim[0][1] = N - 1
+    ctxs = [_context(v, lim, (1, 1, 3, 3, 2, 2)) for _ in range(2)]
+    group, first = (ctypes.c_void_p * 2)(*ctxs), (ctypes.c_uint64 * 2)(0, 0)
+    assert v.vgpu_run_group(group, 2, first, ctypes.c_uint64(4)) == 0
+    first[0] = first[1] = 4
+    cpu.setenv("CPU_HIP_ERROR", "1")
+    assert v.vgpu_run_group(group, 2, first, ctypes.c_uint64(4)) == -3
+    assert b"kernel launch failed" in v.vgpu_last_error(ctxs[0])
+    cpu.setenv("CPU_HIP_ERROR", "0")
+    for c in ctxs:
+        v.vgpu_destroy(c)

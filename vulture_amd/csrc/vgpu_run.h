@@ -1248,7 +1248,7 @@ template <typename T> int run_group_steps(Ctx *const *all, int nall, uint64_t ns
   }
   // (the step counters advance with the group's close)
   const hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return set_error(cs[0], VGPU_EDEVICE, "kernel launch failed: %s", hipGetErrorString(err));
+  if (err != hipSuccess) return set_error(all[0], VGPU_EDEVICE, "kernel launch failed: %s", hipGetErrorString(err));
   return VGPU_OK;
 }
 
